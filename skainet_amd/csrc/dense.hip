@@ -1,5 +1,8 @@
 // Dense fp32 matmul entries of the kernel SPI. No decoder configuration routes through them (every linear layer
-// there is packed). Two kernels:
+// there is packed). Three kernels:
+//   sgemm_mfma_skinny_kernel  fp32 operands on v_mfma_f32_16x16x4_f32, K split over the waves of a workgroup and nothing
+//                      staged through LDS: products whose 64 x 128 tiles would leave CUs idle (few rows, or few columns
+//                      with a long K), any stride, alignment and remainder;
 //   sgemm_mfma_kernel  fp32 operands on the fp32 matrix instruction (v_mfma_f32_32x32x2_f32: exact fp32 products, fp32
 //                      accumulation), 128 x 128 x 16 tiles, for products of at least 64 rows whose operands are 16-byte
 //                      aligned with strides and K (and N, when B is read along its rows) multiples of four;
@@ -163,6 +166,144 @@ __global__ __launch_bounds__(256) void sgemm_mfma_kernel(const float* __restrict
             }
 }
 
+// Few rows (or few output columns with a long K): what bounds these products is the one read of the weight, and with
+// 64-wide tiles it was latency -- 32 x 4096 x 4096 is 64 tiles, each a chain of 256 K slices behind barriers (720 us).
+// Here a workgroup owns 16 NT output columns x 16 MTILES rows and its NW waves split K, 32 elements at a time in turn,
+// so that the workgroup reads NW x 128 consecutive bytes of each of its weight rows per round; 4096 columns are 256
+// workgroups. Operands go from global memory straight into the matrix instruction's registers: lane (r, q) = (l % 16,
+// l / 16) loads floats 4 q .. 4 q + 3 and 16 + 4 q .. of a step of row r of either operand (64 consecutive bytes of 16
+// rows per load; dword alignment is enough), and instruction j multiplies everybody's j-th float -- the contraction
+// index is a free permutation as long as both operands use the same one. One step is requested ahead of the one that
+// multiplies. Partial tiles meet in LDS once. A: [m, k] rows; BT: B(p, j) = b[j * b_stride + p], else b[p * b_stride + j].
+// Measured: 32 rows x 4096 x 4096: 720 -> 24 us (2.8 TB/s of operands); one row 17 us (3.9 TB/s);
+// 256 rows 101 us (85 TFLOP/s).
+struct __attribute__((packed, aligned(4))) f32x4_a4 { float v[4]; };
+
+template <bool BT, int MTILES, int NT, int NW>
+__global__ __launch_bounds__(64 * NW) void sgemm_mfma_skinny_kernel(const float* __restrict__ a, int64_t a_stride, const float* __restrict__ b,
+                                                                    int64_t b_stride, float* __restrict__ c, int64_t c_stride, int m, int n, int k) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    __shared__ float part[NW][MTILES * NT][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int j0 = blockIdx.x * (16 * NT), i0 = blockIdx.y * (16 * MTILES);
+    // rows and columns past the end are copies of the last one that nobody stores
+    const float* pa[MTILES];
+    const float* pb[NT];
+#pragma unroll
+    for (int t = 0; t < MTILES; ++t) {
+        const int row = i0 + 16 * t + r;
+        pa[t] = a + (int64_t)(row < m ? row : m - 1) * a_stride + 4 * q;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int col = j0 + 16 * t + r < n ? j0 + 16 * t + r : n - 1;
+        pb[t] = BT ? b + (int64_t)col * b_stride + 4 * q : b + (int64_t)(4 * q) * b_stride + col;
+    }
+    struct Step { float a[MTILES][8], b[NT][8]; };
+    auto load = [&](Step& s, int64_t p) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if constexpr (BT) {
+                const f32x4_a4 x = *reinterpret_cast<const f32x4_a4*>(pb[t] + p), y = *reinterpret_cast<const f32x4_a4*>(pb[t] + p + 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { s.b[t][e] = x.v[e]; s.b[t][4 + e] = y.v[e]; }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { s.b[t][e] = pb[t][(p + e) * b_stride]; s.b[t][4 + e] = pb[t][(p + 16 + e) * b_stride]; }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < MTILES; ++t) {
+            const f32x4_a4 x = *reinterpret_cast<const f32x4_a4*>(pa[t] + p), y = *reinterpret_cast<const f32x4_a4*>(pa[t] + p + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { s.a[t][e] = x.v[e]; s.a[t][4 + e] = y.v[e]; }
+        }
+    };
+    f32x4 acc[MTILES][NT];
+#pragma unroll
+    for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Step& s) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.a[t][e], s.b[u][e], acc[t][u], 0, 0, 0);
+    };
+    const int full = k >> 5;                       // whole steps; wave w takes w, w + NW, ...
+    if (wave < full) {
+        Step s0, s1;
+        load(s0, (int64_t)wave * 32);
+        int st = wave;
+        for (; st + NW < full; st += 2 * NW) {
+            load(s1, (int64_t)(st + NW) * 32);
+            multiply(s0);
+            // the request past the last step repeats it: in bounds and never multiplied
+            load(s0, (int64_t)(st + 2 * NW < full ? st + 2 * NW : st + NW) * 32);
+            multiply(s1);
+        }
+        if (st < full) multiply(s0);
+    }
+    if ((k & 31) && wave == full % NW) {           // the last, partial step: elements past K are zeros on both sides
+        Step s;
+        const int64_t p = (int64_t)full * 32;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t at = p + (e < 4 ? e : 12 + e);
+            const bool in = at + 4 * q < k;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) s.b[t][e] = in ? (BT ? pb[t][at] : pb[t][at * b_stride]) : 0.f;
+#pragma unroll
+            for (int t = 0; t < MTILES; ++t) s.a[t][e] = in ? pa[t][at] : 0.f;
+        }
+        multiply(s);
+    }
+    // accumulator element e of lane (r, q): row 4 q + e, column r of the tile
+#pragma unroll
+    for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[wave][t * NT + u][(4 * q + e) * 16 + r] = acc[t][u][e];
+    __syncthreads();
+    for (int at = threadIdx.x; at < MTILES * NT * 256; at += 64 * NW) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += (&part[w][0][0])[at];
+        const int tile = at >> 8;
+        const int row = i0 + 16 * (tile / NT) + ((at >> 4) & 15), cc = j0 + 16 * (tile % NT) + (at & 15);
+        if (row < m && cc < n) c[(int64_t)row * c_stride + cc] = sum;
+    }
+}
+
+template <bool BT, int MTILES, int NT>
+static void launch_skinny(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
+                          int m, int n, int k) {
+    const dim3 grid((n + 16 * NT - 1) / (16 * NT), (m + 16 * MTILES - 1) / (16 * MTILES));
+    // waves per workgroup: enough for eight waves per CU over the whole grid, as long as every wave has a step of K
+    const int64_t groups = (int64_t)grid.x * grid.y;
+    int nw = 4;
+    while (nw < 16 / NT && groups * nw < 8 * (int64_t)num_cus() && 32 * nw < k) nw *= 2;
+    if (NT == 1 && nw == 16) sgemm_mfma_skinny_kernel<BT, MTILES, 1, 16><<<grid, dim3(1024), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    else if (nw == 8) sgemm_mfma_skinny_kernel<BT, MTILES, NT, 8><<<grid, dim3(512), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    else sgemm_mfma_skinny_kernel<BT, MTILES, NT, 4><<<grid, dim3(256), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+}
+// The largest tile whose grid still gives every CU a workgroup (a larger tile reads its operands less often, an idle CU
+// costs more than that), and no more rows than the product has.
+template <bool BT>
+static void launch_skinny_rows(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
+                               int m, int n, int k) {
+    auto groups = [&](int mt, int nt) { return (int64_t)((n + 16 * nt - 1) / (16 * nt)) * ((m + 16 * mt - 1) / (16 * mt)); };
+    const int cus = num_cus();
+    if (m > 32 && groups(4, 2) >= cus) launch_skinny<BT, 4, 2>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    else if (m > 32 && groups(4, 1) >= cus) launch_skinny<BT, 4, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    else if (m > 16 && groups(2, 1) >= cus) launch_skinny<BT, 2, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    else launch_skinny<BT, 1, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+}
+
 static std::atomic<int> g_dense_mfma{1};
 void set_dense_mfma(int v) { g_dense_mfma = v != 0; }
 
@@ -172,6 +313,17 @@ int launch_fp32_matmul(const float* a, int64_t a_stride, const float* b, int64_t
     if (k < 0) k = 0;
     const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && (a_stride & 3) == 0 &&
                          (b_stride & 3) == 0 && (k & 3) == 0 && (b_transposed || (n & 3) == 0);
+    // 64 x 128 tiles that do not fill the CUs leave the product to the kernel that splits K over waves; where they fill
+    // them the tile kernel reads each operand less often
+    const int64_t tiles64 = (int64_t)((n + MT - 1) / MT) * ((m + 63) / 64);
+    // (B read along its rows at an odd alignment and 64 rows or more: the LDS tile kernel, whose loads do not mind)
+    if (g_dense_mfma && k >= 1 && tiles64 < num_cus() && (b_transposed || aligned || m < 64)) {
+        note_kernel("sgemm_mfma_kernel");
+        if (b_transposed) launch_skinny_rows<true>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+        else launch_skinny_rows<false>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+        SKH_CHECK(hipGetLastError());
+        return 0;
+    }
     if (g_dense_mfma && aligned && m >= 64 && n >= 32 && k >= 4) {
         // 128-row tiles where they give every CU at least one; else 64-row tiles
         const int tiles128 = ((n + MT - 1) / MT) * ((m + 127) / 128);

@@ -441,6 +441,31 @@ def test_dense_fp32_matmul_on_the_matrix_cores(hip_backend, torch_cuda, m, n, k,
         close(out.cpu().numpy(), want, rel=1e-5, abs_=2e-6 * np.sqrt(k) * 16)
 
 
+@pytest.mark.parametrize("wt", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 17, 31), (3, 16, 32), (16, 33, 33), (17, 100, 2047), (33, 4100, 65), (64, 8200, 96),
+                                   (65, 5, 8192), (130, 4097, 161)])
+def test_dense_fp32_products_with_k_split_over_waves(hip_backend, torch_cuda, m, n, k, wt):
+    """Few rows or few columns: K is split over the waves of a workgroup, at every tile size (1, 2, 4 row tiles, 1 or 2
+    column tiles), with partial last steps of K, ragged edges and rows that are not 16-byte aligned. An fp32 sum of k
+    products in any order is within k * 2^-24 of the sum of magnitudes (about 0.8^2 k for N(0, 1) operands); the written
+    bound takes a quarter of that worst case."""
+    torch = torch_cuda
+    rng = np.random.default_rng(7 * m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k) if wt else (k, n)).astype(np.float32)
+    want = a.astype(np.float64) @ (b.astype(np.float64).T if wt else b.astype(np.float64))
+    out = torch.full((m + 1, n), float("nan"), dtype=torch.float32, device="cuda")
+    if wt:
+        hip_backend.fp32_matmul_wt_dev(dev(torch, a), 0, dev(torch, b), 0, out, 0, m, n, k)
+    else:
+        hip_backend.fp32_matmul_dev(dev(torch, a), 0, k, dev(torch, b), 0, n, out, 0, n, m, n, k)
+    if wt or m < 64:                                    # unaligned rows of B at 64 rows and more stay on the tile kernel
+        assert hip_backend.last_kernel() == "sgemm_mfma_kernel"
+    got = out.cpu().numpy()
+    assert np.isnan(got[m]).all()                       # nothing past the last row
+    assert np.abs(got[:m] - want).max() <= max(1, k / 4) * 2.0 ** -24 * 0.64 * k + 1e-6
+
+
 @pytest.mark.parametrize("kind,codec", [("bf16", "BFloat16"), ("fp16", "Float16")])
 def test_narrow_float_matmuls(hip_backend, torch_cuda, kind, codec):
     """Bf16MatmulKernel / Fp16MatmulKernel through the host entry: the oracle on the recorded inputs (with the formats'
