@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <thread>
 
@@ -51,6 +52,7 @@ int launch_sdpa_prefill(const float* q, const float* k, const float* v, float* o
                         const int32_t* lengths, const float* mask, int mask_b, int mask_h, int mask_q, int mask_k, int out_rows);
 int launch_i32_increment(int32_t* v, int32_t delta);
 int launch_stream_read(const void* p, int64_t bytes, int grid, uint32_t* sink);
+int launch_host_copy(void* dst, const void* src, size_t bytes, uint32_t* counter, uint32_t* flag, uint32_t ticket);   // hostio.hip
 int launch_relayout_to_row_major(const uint8_t* src, uint8_t* dst, int rows, int bpr, int block_bytes);
 int launch_fp32_matmul(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
                        int m, int n, int k, bool b_transposed);
@@ -277,6 +279,62 @@ static int staged_h2d(void* dst, const uint8_t* src, size_t bytes) {
         if (check_hip(result[t], "hipMemcpy(weight, staged)") != 0) return -1;
     return 0;
 }
+// Small host <-> device copies: a kernel moves them between device memory and page-locked staging on the caller's stream,
+// and the host polls a page-locked flag that the kernel's last workgroup sets. A launch costs 2.8 us here, a launch with
+// hipStreamSynchronize behind it 11.3, a launch that sets a flag the host polls 6.5 (a kernel with nothing to do). Both
+// directions still return only when the bytes are where they belong. Measured against the runtime's copy and wait, up /
+// down: 4 KB 15.3 / 21.8 -> 9.8 / 9.2 us, 16 KB 14.2 / 21.2 -> 10.5 / 10.3, 64 KB 10.9 / 11.9 -> 12.0 / 12.0, 256 KB
+// 15.6 / 19.9 -> 21.0 / 22.7 (the runtime overlaps its staging with the bus), so callers' memory goes this way up to
+// COPY_KERNEL_MAX; data that lies in page-locked staging anyway up to PINNED_KERNEL_MAX.
+constexpr size_t COPY_KERNEL_MAX = 32u << 10, PINNED_KERNEL_MAX = 256u << 10;
+static thread_local Scratch t_link[2];            // page-locked: bytes on their way down / up
+static thread_local Scratch t_flag;               // page-locked: the ticket of the last finished flagged copy
+static thread_local uint32_t t_ticket = 0;
+static bool copy_kernel_fits(size_t bytes, size_t most = COPY_KERNEL_MAX) { return bytes <= most && !t_capture_stream; }
+// Queues the copy with a completion ticket; wait_copy waits for it.
+static int queue_flagged_copy(void* dst, const void* src, size_t bytes) {
+    const bool fresh = t_flag.ptr == nullptr;
+    uint32_t* flag = static_cast<uint32_t*>(pinned_get(t_flag, 64));
+    uint8_t* sync = static_cast<uint8_t*>(sync_scratch(SYNC_SCRATCH_BYTES));
+    if (!flag || !sync) return -1;
+    if (fresh) { *flag = 0; t_ticket = 0; }
+    return launch_host_copy(dst, src, bytes, reinterpret_cast<uint32_t*>(sync + SYNC_SCRATCH_BYTES - 64), flag, ++t_ticket);
+}
+static int wait_copy() {
+    const uint32_t* flag = static_cast<const uint32_t*>(t_flag.ptr);
+    auto arrived = [&] { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == t_ticket; };
+    // polled for as long as a short queue of kernels takes; behind more work than that the thread sleeps in the runtime
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    do {
+        for (int i = 0; i < 256; ++i) {
+            if (arrived()) return 0;
+            __builtin_ia32_pause();
+        }
+    } while (std::chrono::steady_clock::now() < until);
+    if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
+    return arrived() ? 0 : set_error("host copy: the stream drained without the copy's completion");
+}
+static int copy_h2d(void* dst, const void* src, size_t bytes) {
+    if (!copy_kernel_fits(bytes)) {
+        if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
+        return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
+    }
+    void* pin = pinned_get(t_link[0], bytes);
+    if (!pin) return -1;
+    memcpy(pin, src, bytes);
+    if (queue_flagged_copy(dst, pin, bytes) != 0) return -1;
+    return wait_copy();
+}
+static int copy_d2h(void* dst, const void* src, size_t bytes) {
+    if (!copy_kernel_fits(bytes)) {
+        if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
+        return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
+    }
+    void* pin = pinned_get(t_link[1], bytes);
+    if (!pin || queue_flagged_copy(pin, src, bytes) != 0 || wait_copy() != 0) return -1;
+    memcpy(dst, pin, bytes);
+    return 0;
+}
 float* sdpa_workspace(size_t bytes) { return static_cast<float*>(scratch_get(t_workspace, bytes)); }
 void* kernel_workspace(size_t bytes) { return scratch_get(t_workspace, bytes); }
 
@@ -353,6 +411,8 @@ int32_t skainet_hip_thread_release(void) {
         sc.ptr = nullptr; sc.cap = 0;
     };
     for (Scratch& sc : t_pinned) drop_pinned(sc);
+    for (Scratch& sc : t_link) drop_pinned(sc);
+    drop_pinned(t_flag);
     if (t_sync && check_hip(hipFree(t_sync), "hipFree(sync scratch)") != 0) rc = -1;
     t_sync = nullptr;
     if (t_ev0 && check_hip(hipEventDestroy(t_ev0), "hipEventDestroy") != 0) rc = -1;
@@ -387,14 +447,12 @@ int32_t skainet_hip_host_free(void* p) {
 int32_t skainet_hip_memcpy_h2d(void* dst, const void* src, size_t bytes) {
     if (ensure_device() != 0) return -1;
     if (bytes == 0) return 0;
-    if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
-    return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
+    return copy_h2d(dst, src, bytes);
 }
 int32_t skainet_hip_memcpy_d2h(void* dst, const void* src, size_t bytes) {
     if (ensure_device() != 0) return -1;
     if (bytes == 0) return 0;
-    if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
-    return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
+    return copy_d2h(dst, src, bytes);
 }
 int32_t skainet_hip_memcpy_d2d(void* dst, const void* src, size_t bytes) {
     if (ensure_device() != 0) return -1;
@@ -496,9 +554,9 @@ int32_t skainet_hip_matmul_dev(const skainet_hip_weight* w, const float* x, int3
     return skainet_hip_matmul_kind_dev(w, x, m, out, m <= 8 ? 0 : 1);
 }
 // The view-kernel route of the SPI on a resident weight: activations and result live in host memory, the weight stays
-// on the device. One call = copy the rows into page-locked staging, one asynchronous upload, the product, one
-// asynchronous download, one wait; every buffer belongs to the calling thread and is reused, so a call allocates
-// nothing once the thread has seen its largest shape.
+// on the device. One call = copy the rows into page-locked staging, one upload and one download on the stream (copy kernels
+// for small payloads, see above: 4096 x 4096 at one row 23.4 -> 20.4 us), one wait; every buffer belongs to the calling
+// thread and is reused, so a call allocates nothing once the thread has seen its largest shape.
 int32_t skainet_hip_matmul_host(const skainet_hip_weight* w, const float* x_host, int32_t m, float* out_host) {
     if (ensure_device() != 0) return -1;
     if (!w) return set_error("matmul_host: null weight handle");
@@ -511,10 +569,18 @@ int32_t skainet_hip_matmul_host(const skainet_hip_weight* w, const float* x_host
     float* yd = static_cast<float*>(scratch_get(t_stage[2], out_bytes));
     if (!pin_in || !pin_out || !xd || !yd) return -1;
     memcpy(pin_in, x_host, in_bytes);
-    if (check_hip(hipMemcpyAsync(xd, pin_in, in_bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
+    if (copy_kernel_fits(in_bytes, PINNED_KERNEL_MAX)) {
+        if (launch_host_copy(xd, pin_in, in_bytes, nullptr, nullptr, 0) != 0) return -1;
+    } else if (check_hip(hipMemcpyAsync(xd, pin_in, in_bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) {
+        return -1;
+    }
     if (skainet_hip_matmul_dev(w, xd, m, yd) != 0) return -1;
-    if (check_hip(hipMemcpyAsync(pin_out, yd, out_bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
-    if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
+    if (copy_kernel_fits(out_bytes, PINNED_KERNEL_MAX)) {
+        if (queue_flagged_copy(pin_out, yd, out_bytes) != 0 || wait_copy() != 0) return -1;
+    } else {
+        if (check_hip(hipMemcpyAsync(pin_out, yd, out_bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
+        if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
+    }
     memcpy(out_host, pin_out, out_bytes);
     return 0;
 }
@@ -962,8 +1028,7 @@ static void* stage_in(int slot, const void* host, size_t bytes) {
     return d;
 }
 static int stage_out(void* host, const void* dev, size_t bytes) {
-    if (check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
-    return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
+    return copy_d2h(host, dev, bytes);
 }
 
 static void packed_matmul_host(int enc, int order, const float* input, int32_t input_offset, const uint8_t* weight,

@@ -79,14 +79,25 @@ class ForwardScope:
         self._slab.close()
 
 
+def _count(shape) -> int:
+    n = 1
+    for s in shape:
+        n *= s
+    return n
+
+
+_F32 = np.dtype(np.float32)
+
+
 class HipTensor:
     """A dense tensor whose bytes are resident on the device (fp32 unless `dtype` says int32). `owner` keeps the
     allocation alive: an `_Allocation`, a `ForwardScope`, or another tensor (views)."""
 
-    __slots__ = ("shape", "_ptr", "owner", "dtype", "_scope", "_generation")
+    __slots__ = ("shape", "_ptr", "owner", "dtype", "_scope", "_generation", "volume")
 
     def __init__(self, shape: Sequence[int], ptr: int, owner, dtype=np.float32):
         self.shape = tuple(int(s) for s in shape)
+        self.volume = _count(self.shape)
         self._ptr = int(ptr)
         self.owner = owner
         self.dtype = np.dtype(dtype)
@@ -101,13 +112,6 @@ class HipTensor:
         if self._scope is not None and self._scope.generation != self._generation:
             raise HipError(f"tensor {self.shape} belongs to a forward scope that has been reset since")
         return self._ptr
-
-    @property
-    def volume(self) -> int:
-        n = 1
-        for s in self.shape:
-            n *= s
-        return n
 
     @property
     def nbytes(self) -> int:
@@ -130,10 +134,9 @@ class HipTensor:
         return HipTensor((count,) + self.shape[1:], self.ptr + start * inner * self.dtype.itemsize, self, self.dtype)
 
     def numpy(self) -> np.ndarray:
-        """The heap mirror: one synchronous download."""
+        """The heap mirror: one synchronous download, behind everything this thread's stream holds."""
         out = np.empty(self.shape, dtype=self.dtype)
         if out.size:
-            check(_lib.hip().skainet_hip_sync(), "sync")
             check(_lib.hip().skainet_hip_memcpy_d2h(out.ctypes.data, self.ptr, out.nbytes), "d2h")
         return out
 
@@ -163,11 +166,24 @@ class HipOps:
                 t.ptr
 
     def _out(self, shape: Sequence[int], dtype=np.float32) -> HipTensor:
-        n = int(np.prod(shape, dtype=np.int64)) * np.dtype(dtype).itemsize
+        n = _count(shape) * np.dtype(dtype).itemsize
         if self.scope is not None:
             return HipTensor(shape, self.scope.allocate(n), self.scope, dtype)
         a = _Allocation(n)
         return HipTensor(shape, a.ptr, a, dtype)
+
+    def _out_f32(self, shape: Tuple[int, ...], volume: int) -> HipTensor:
+        """_out for an fp32 output whose shape is a tuple of ints already (an operand's, or made of operands'): a chain of
+        small ops is bound by the interpreter, so its outputs skip the constructor's conversions."""
+        scope = self.scope
+        t = HipTensor.__new__(HipTensor)
+        t.shape, t.volume, t.dtype = shape, volume, _F32
+        if scope is not None:
+            t._ptr, t.owner, t._scope, t._generation = scope.allocate(4 * volume), scope, scope, scope.generation
+        else:
+            a = _Allocation(4 * volume)
+            t._ptr, t.owner, t._scope, t._generation = a.ptr, a, None, 0
+        return t
 
     def to_resident(self, array: np.ndarray) -> HipTensor:
         """Upload once (WasmCpuOps.kt:154 toResident): an input that many ops will read."""
@@ -189,16 +205,17 @@ class HipOps:
             raise ValueError(f"Matrix multiplication shape mismatch: {a.shape} vs {b.shape}")
         m, k = a.shape
         n = b.shape[1]
-        self._live(a, b)
-        out = self._out((m, n))
+        ap, bp = a.ptr, b.ptr
+        out = self._out_f32((m, n), m * n)
         if m and n:
-            check(self._lib.skainet_hip_fp32_matmul_dev(a.ptr, 0, k, b.ptr, 0, n, out.ptr, 0, n, m, n, k), "matmul")
+            check(self._lib.skainet_hip_fp32_matmul_dev(ap, 0, k, bp, 0, n, out._ptr, 0, n, m, n, k), "matmul")
         return out
 
     def matmul_weight_transposed(self, x: HipTensor, weight: Weight) -> HipTensor:
         """x(..., k) . W(n, k)^T. A dense weight is a HipTensor; a packed one (Q4_K, Q6_K, Q8_0, ...) a DeviceWeight, which
         takes the product its view kernel runs: GEMV kernels up to 8 rows, the MFMA dequant-GEMM above."""
-        if isinstance(weight, HipTensor):
+        dense = isinstance(weight, HipTensor)
+        if dense:
             if len(weight.shape) != 2:
                 raise ValueError(f"weight must be [n, k]; got {weight.shape}")
             n, k = weight.shape
@@ -207,13 +224,14 @@ class HipOps:
         if not x.shape or x.shape[-1] != k:
             raise ValueError(f"matmulWeightTransposed shape mismatch: {x.shape} vs weight [{n}, {k}]")
         m = x.volume // k if k else 0
-        self._live(x, weight)
-        out = self._out(x.shape[:-1] + (n,))
+        xp, wp = x.ptr, weight.ptr if dense else weight._h
+        shape = x.shape[:-1] + (n,)
+        out = self._out_f32(shape, m * n if k else _count(shape))
         if m and n:
-            if isinstance(weight, HipTensor):
-                check(self._lib.skainet_hip_fp32_matmul_wt_dev(x.ptr, 0, weight.ptr, 0, out.ptr, 0, m, n, k), "matmul_wt")
+            if dense:
+                check(self._lib.skainet_hip_fp32_matmul_wt_dev(xp, 0, wp, 0, out._ptr, 0, m, n, k), "matmul_wt")
             else:
-                check(self._lib.skainet_hip_matmul_dev(weight._h, x.ptr, m, out.ptr), "matmul")
+                check(self._lib.skainet_hip_matmul_dev(wp, xp, m, out._ptr), "matmul")
         return out
 
     # ---- elementwise (WasmCpuOps.kt:240-277) -------------------------------------------------------------------------
@@ -222,20 +240,27 @@ class HipOps:
         """The operand's index mode against the broadcast output shape (WasmCpuOps.kt:232-238)."""
         if s == out:
             return kernels.MODE_FULL
-        if int(np.prod(s, dtype=np.int64)) == 1:
+        if _count(s) == 1:
             return kernels.MODE_SCALAR
         if s and out and s[-1] == out[-1] and all(d == 1 for d in s[:-1]):
             return kernels.MODE_BIAS
         raise ValueError(f"broadcast of {s} to {out} is not one of full / scalar / last-dimension bias")
 
     def _binary(self, op: str, a: HipTensor, b: HipTensor) -> HipTensor:
-        shape = _broadcast_shape(a.shape, b.shape)
-        am, bm = self._mode(a.shape, shape), self._mode(b.shape, shape)
-        self._live(a, b)
-        out = self._out(shape)
-        n = out.volume
+        sa, sb = a.shape, b.shape
+        if sa == sb:
+            shape, am, bm = sa, kernels.MODE_FULL, kernels.MODE_FULL
+        elif len(sb) == 1 and sa and sb[0] == sa[-1] and sb[0] > 1:      # a layer's bias
+            shape, am, bm = sa, kernels.MODE_FULL, kernels.MODE_BIAS
+        else:
+            shape = _broadcast_shape(sa, sb)
+            am, bm = self._mode(sa, shape), self._mode(sb, shape)
+        ap, bp = a.ptr, b.ptr
+        n = a.volume if shape is sa else _count(shape)
+        out = self._out_f32(shape, n)
         if n:
-            kernels.binary_dev(op, a, b, out, n, am, bm, shape[-1] if shape else 1)
+            check(self._lib.skainet_hip_f32_binary_dev(kernels.BINARY_OPS[op], ap, am, bp, bm, out._ptr, n, shape[-1] if shape else 1),
+                  "binary")
         return out
 
     def add(self, a, b): return self._binary("add", a, b)
@@ -245,10 +270,10 @@ class HipOps:
 
     # ---- activations (WasmCpuOps.kt:281-312) -------------------------------------------------------------------------
     def _unary(self, op: str, t: HipTensor) -> HipTensor:
-        self._live(t)
-        out = self._out(t.shape)
-        if t.volume:
-            kernels.unary_dev(op, t, out, t.volume)
+        tp, n = t.ptr, t.volume
+        out = self._out_f32(t.shape, n)
+        if n:
+            check(self._lib.skainet_hip_f32_unary_dev(kernels.UNARY_OPS[op], tp, out._ptr, n), "unary")
         return out
 
     def relu(self, t): return self._unary("relu", t)
@@ -286,10 +311,10 @@ class HipOps:
         if rank == 0 or dim % rank != rank - 1:
             raise ValueError("softmax runs over the last dimension")
         cols = t.shape[-1]
-        self._live(t)
-        out = self._out(t.shape)
-        if t.volume:
-            kernels.softmax_rows_dev(t, out, t.volume // cols, cols, log)
+        tp, n = t.ptr, t.volume
+        out = self._out_f32(t.shape, n)
+        if n:
+            check(self._lib.skainet_hip_f32_softmax_rows_dev(tp, out._ptr, n // cols, cols, int(log)), "softmax_rows")
         return out
 
     def softmax(self, t, dim: int = -1): return self._softmax(t, dim, False)
@@ -301,10 +326,10 @@ class HipOps:
         cols = x.shape[-1]
         if gamma is not None and gamma.volume != cols:
             raise ValueError(f"gamma of {gamma.shape} against rows of {cols}")
-        self._live(x, gamma)
-        out = self._out(x.shape)
-        if x.volume:
-            kernels.rms_norm_dev(x, gamma, out, x.volume // cols, cols, eps)
+        xp, gp, n = x.ptr, gamma.ptr if gamma is not None else 0, x.volume
+        out = self._out_f32(x.shape, n)
+        if n:
+            check(self._lib.skainet_hip_f32_rms_norm_dev(xp, gp, out._ptr, n // cols, cols, eps), "rms_norm")
         return out
 
     def layer_norm(self, x: HipTensor, gamma: Optional[HipTensor], beta: Optional[HipTensor], eps: float) -> HipTensor:
@@ -314,10 +339,11 @@ class HipOps:
         for name, p in (("gamma", gamma), ("beta", beta)):
             if p is not None and p.volume != cols:
                 raise ValueError(f"{name} of {p.shape} against rows of {cols}")
-        self._live(x, gamma, beta)
-        out = self._out(x.shape)
-        if x.volume:
-            kernels.layer_norm_dev(x, gamma, beta, out, x.volume // cols, cols, eps)
+        xp, n = x.ptr, x.volume
+        gp, bp = gamma.ptr if gamma is not None else 0, beta.ptr if beta is not None else 0
+        out = self._out_f32(x.shape, n)
+        if n:
+            check(self._lib.skainet_hip_f32_layer_norm_dev(xp, gp, bp, out._ptr, n // cols, cols, eps), "layer_norm")
         return out
 
     # ---- attention (WasmCpuOps.kt:428) -------------------------------------------------------------------------------

@@ -178,3 +178,27 @@ def test_llama_stack_through_the_generic_ops_matches_the_checker_and_the_fused_d
         assert outs[0][0][0] == first_fused
         assert outs[0][0][1:] == [int(t) for t in fused.decode(6, use_graph=False)]
     assert OpsLlamaDecoder.launches_per_token(type("D", (), {"cfg": cfg})()) == 17 * cfg.layers + 5
+
+
+@pytest.mark.parametrize("offset", [0, 4, 1])
+@pytest.mark.parametrize("nbytes", [1, 15, 16, 17, 1023, 16384, 32768, 32769, 65536, 300001])
+def test_host_copies_of_every_size_and_alignment_are_byte_exact(hip_backend, nbytes, offset):
+    """Small copies are made by a kernel between device memory and page-locked staging (16-byte pieces with a byte tail, or
+    bytes where the device side is not aligned), larger ones by the runtime: neighbours untouched, bytes equal."""
+    from skainet_amd import _lib
+    lib = _lib.hip()
+    rng = np.random.default_rng(nbytes + offset)
+    src, around = rng.integers(0, 256, nbytes, dtype=np.uint8), np.full(nbytes + 64, 0xA5, np.uint8)
+    p = lib.skainet_hip_malloc(around.size)
+    try:
+        for a in (around, src):
+            at = p if a is around else p + 16 + offset
+            assert lib.skainet_hip_memcpy_h2d(at, a.ctypes.data, a.size) == 0
+        got, part = np.empty_like(around), np.empty_like(src)
+        assert lib.skainet_hip_memcpy_d2h(got.ctypes.data, p, got.size) == 0
+        assert lib.skainet_hip_memcpy_d2h(part.ctypes.data, p + 16 + offset, nbytes) == 0
+        want = around.copy()
+        want[16 + offset:16 + offset + nbytes] = src
+        assert np.array_equal(got, want) and np.array_equal(part, src)
+    finally:
+        lib.skainet_hip_free(p)
