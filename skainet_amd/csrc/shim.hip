@@ -282,27 +282,34 @@ static int staged_h2d(void* dst, const uint8_t* src, size_t bytes) {
 // Small host <-> device copies: a kernel moves them between device memory and page-locked staging on the caller's stream,
 // and the host polls a page-locked flag that the kernel's last workgroup sets. A launch costs 2.8 us here, a launch with
 // hipStreamSynchronize behind it 11.3, a launch that sets a flag the host polls 6.5 (a kernel with nothing to do). Both
-// directions still return only when the bytes are where they belong. Measured against the runtime's copy and wait, up /
-// down: 4 KB 15.3 / 21.8 -> 9.8 / 9.2 us, 16 KB 14.2 / 21.2 -> 10.5 / 10.3, 64 KB 10.9 / 11.9 -> 12.0 / 12.0, 256 KB
-// 15.6 / 19.9 -> 21.0 / 22.7 (the runtime overlaps its staging with the bus), so callers' memory goes this way up to
-// COPY_KERNEL_MAX; data that lies in page-locked staging anyway up to PINNED_KERNEL_MAX.
-constexpr size_t COPY_KERNEL_MAX = 32u << 10, PINNED_KERNEL_MAX = 256u << 10;
+// directions still return only when the bytes are where they belong. More than COPY_CHUNK bytes go in pieces, the host
+// filling (or emptying) one piece of staging while the kernel of another is on the bus. Measured against the runtime's copy
+// and wait, up / down: 4 KB 15.3 / 21.8 -> 8.6 / 7.9 us, 16 KB 14.2 / 21.2 -> 9.0 / 8.8, 128 KB 87 (an array
+// the runtime pins for the call) -> 14.5 up, 1 MB 40.8 / 59.8 -> 42 / 43. Above COPY_KERNEL_MAX the
+// copy engine's rate counts for more than its hand-over.
+constexpr size_t COPY_KERNEL_MAX = 1u << 20, COPY_CHUNK = 128u << 10;
 static thread_local Scratch t_link[2];            // page-locked: bytes on their way down / up
 static thread_local Scratch t_flag;               // page-locked: the ticket of the last finished flagged copy
-static thread_local uint32_t t_ticket = 0;
-static bool copy_kernel_fits(size_t bytes, size_t most = COPY_KERNEL_MAX) { return bytes <= most && !t_capture_stream; }
-// Queues the copy with a completion ticket; wait_copy waits for it.
-static int queue_flagged_copy(void* dst, const void* src, size_t bytes) {
+static thread_local uint32_t t_ticket = 0;        // the last one handed out
+static bool copy_kernel_fits(size_t bytes) { return bytes <= COPY_KERNEL_MAX && !t_capture_stream; }
+static size_t copy_chunk(size_t bytes) {          // at most four pieces: a piece costs a launch
+    const size_t quarter = (bytes / 4 + 4095) & ~(size_t)4095;
+    return quarter > COPY_CHUNK ? quarter : COPY_CHUNK;
+}
+// Queues the copy with a completion ticket (0: failed); wait_copy waits for it.
+static uint32_t queue_flagged_copy(void* dst, const void* src, size_t bytes) {
     const bool fresh = t_flag.ptr == nullptr;
     uint32_t* flag = static_cast<uint32_t*>(pinned_get(t_flag, 64));
     uint8_t* sync = static_cast<uint8_t*>(sync_scratch(SYNC_SCRATCH_BYTES));
-    if (!flag || !sync) return -1;
+    if (!flag || !sync) return 0;
     if (fresh) { *flag = 0; t_ticket = 0; }
-    return launch_host_copy(dst, src, bytes, reinterpret_cast<uint32_t*>(sync + SYNC_SCRATCH_BYTES - 64), flag, ++t_ticket);
+    if (++t_ticket == 0) ++t_ticket;
+    return launch_host_copy(dst, src, bytes, reinterpret_cast<uint32_t*>(sync + SYNC_SCRATCH_BYTES - 64), flag, t_ticket) == 0 ? t_ticket : 0;
 }
-static int wait_copy() {
+static int wait_copy(uint32_t ticket) {
+    if (!ticket) return -1;
     const uint32_t* flag = static_cast<const uint32_t*>(t_flag.ptr);
-    auto arrived = [&] { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == t_ticket; };
+    auto arrived = [&] { return (int32_t)(__atomic_load_n(flag, __ATOMIC_ACQUIRE) - ticket) >= 0; };
     // polled for as long as a short queue of kernels takes; behind more work than that the thread sleeps in the runtime
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     do {
@@ -314,16 +321,43 @@ static int wait_copy() {
     if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
     return arrived() ? 0 : set_error("host copy: the stream drained without the copy's completion");
 }
+// The two halves: `pin` is page-locked staging of at least `bytes`. The way up is only queued (the last piece with a ticket
+// when the caller wants to wait for it), the way down is complete on return.
+static int copy_up(void* dst, const void* src, void* pin, size_t bytes, bool wait) {
+    const size_t chunk = copy_chunk(bytes);
+    for (size_t off = 0; off < bytes; off += chunk) {
+        const size_t len = bytes - off < chunk ? bytes - off : chunk;
+        uint8_t* stage = static_cast<uint8_t*>(pin) + off;
+        memcpy(stage, static_cast<const uint8_t*>(src) + off, len);
+        if (wait && off + len == bytes) return wait_copy(queue_flagged_copy(static_cast<uint8_t*>(dst) + off, stage, len));
+        if (launch_host_copy(static_cast<uint8_t*>(dst) + off, stage, len, nullptr, nullptr, 0) != 0) return -1;
+    }
+    return 0;
+}
+static int copy_down(void* dst, const void* src, void* pin, size_t bytes) {
+    const size_t chunk = copy_chunk(bytes);
+    uint32_t tickets[4];
+    int n = 0;
+    for (size_t off = 0; off < bytes; off += chunk, ++n) {
+        const size_t len = bytes - off < chunk ? bytes - off : chunk;
+        tickets[n] = queue_flagged_copy(static_cast<uint8_t*>(pin) + off, static_cast<const uint8_t*>(src) + off, len);
+        if (!tickets[n]) return -1;
+    }
+    n = 0;
+    for (size_t off = 0; off < bytes; off += chunk, ++n) {
+        const size_t len = bytes - off < chunk ? bytes - off : chunk;
+        if (wait_copy(tickets[n]) != 0) return -1;
+        memcpy(static_cast<uint8_t*>(dst) + off, static_cast<uint8_t*>(pin) + off, len);
+    }
+    return 0;
+}
 static int copy_h2d(void* dst, const void* src, size_t bytes) {
     if (!copy_kernel_fits(bytes)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }
     void* pin = pinned_get(t_link[0], bytes);
-    if (!pin) return -1;
-    memcpy(pin, src, bytes);
-    if (queue_flagged_copy(dst, pin, bytes) != 0) return -1;
-    return wait_copy();
+    return pin ? copy_up(dst, src, pin, bytes, true) : -1;
 }
 static int copy_d2h(void* dst, const void* src, size_t bytes) {
     if (!copy_kernel_fits(bytes)) {
@@ -331,9 +365,7 @@ static int copy_d2h(void* dst, const void* src, size_t bytes) {
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }
     void* pin = pinned_get(t_link[1], bytes);
-    if (!pin || queue_flagged_copy(pin, src, bytes) != 0 || wait_copy() != 0) return -1;
-    memcpy(dst, pin, bytes);
-    return 0;
+    return pin ? copy_down(dst, src, pin, bytes) : -1;
 }
 float* sdpa_workspace(size_t bytes) { return static_cast<float*>(scratch_get(t_workspace, bytes)); }
 void* kernel_workspace(size_t bytes) { return scratch_get(t_workspace, bytes); }
@@ -568,19 +600,16 @@ int32_t skainet_hip_matmul_host(const skainet_hip_weight* w, const float* x_host
     float* xd = static_cast<float*>(scratch_get(t_stage[1], in_bytes));
     float* yd = static_cast<float*>(scratch_get(t_stage[2], out_bytes));
     if (!pin_in || !pin_out || !xd || !yd) return -1;
-    memcpy(pin_in, x_host, in_bytes);
-    if (copy_kernel_fits(in_bytes, PINNED_KERNEL_MAX)) {
-        if (launch_host_copy(xd, pin_in, in_bytes, nullptr, nullptr, 0) != 0) return -1;
-    } else if (check_hip(hipMemcpyAsync(xd, pin_in, in_bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) {
-        return -1;
+    if (copy_kernel_fits(in_bytes)) {
+        if (copy_up(xd, x_host, pin_in, in_bytes, false) != 0) return -1;
+    } else {
+        memcpy(pin_in, x_host, in_bytes);
+        if (check_hip(hipMemcpyAsync(xd, pin_in, in_bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
     }
     if (skainet_hip_matmul_dev(w, xd, m, yd) != 0) return -1;
-    if (copy_kernel_fits(out_bytes, PINNED_KERNEL_MAX)) {
-        if (queue_flagged_copy(pin_out, yd, out_bytes) != 0 || wait_copy() != 0) return -1;
-    } else {
-        if (check_hip(hipMemcpyAsync(pin_out, yd, out_bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
-        if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
-    }
+    if (copy_kernel_fits(out_bytes)) return copy_down(out_host, yd, pin_out, out_bytes);
+    if (check_hip(hipMemcpyAsync(pin_out, yd, out_bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
+    if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
     memcpy(out_host, pin_out, out_bytes);
     return 0;
 }
