@@ -1,4 +1,4 @@
-// Decode-shape attention (one query position per sequence) over a KV cache: bandwidth-bound split-K.
+// Decode-shape attention (one query position per sequence, or the few of a draft) over a KV cache: bandwidth-bound split-K.
 //
 // Same contract as the general kernel in sdpa.hip (reference: skainet_f32_sdpa,
 //   /root/reference/skainet-backends/skainet-backend-native-cpu/native/src/f32_fused.c:290-396, rules of
@@ -22,6 +22,8 @@
 //     the second launch costs at 10 splits and far more at 64 (4096 keys: 21.8 us against 12.3).
 #include "gemv_q4k.h"
 
+#include <cmath>
+
 namespace skh {
 
 constexpr float SDPA_DECODE_MASKED = -1.0e30f;
@@ -35,8 +37,9 @@ struct SdpaDecodeParams {
     int window, right_context;
     const int32_t* lengths;
     int splits;
-    float* part;          // [batch * heads][splits][D] unnormalised outputs; null: one split, the normalised result goes to out
-    float* ml;            // [batch * heads][splits][2] running maximum (in units of ln 2) and sum of each split
+    float* part;          // [query rows][splits][D] unnormalised outputs; null: one split, the normalised result goes to out
+    float* ml;            // [query rows][splits][2] running maximum (in units of ln 2) and sum of each split
+    int seq_q, causal;    // queries per sequence (the last ones of its positions) and whether a later key is hidden from them
 };
 
 // Scores are kept in units of ln 2 (the query is scaled by scale * log2(e) once), so every exponential of the softmax is
@@ -50,7 +53,10 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
     return m_old == -INFINITY ? 0.f : e;
 }
 
-template <int GS, int DPL>
+// MQ: several queries per sequence (a draft of a few tokens). The rows that share a KV head are then its query heads times
+// the queries, GS of them to a workgroup: each has a key range of its own (causal and window move with the query), the
+// workgroup walks the union and a key outside a row's range scores -inf for that row.
+template <int GS, int DPL, bool MQ>
 __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     constexpr int D = 16 * DPL;
     constexpr int U = 2;                       // groups of 4 keys a wave has in flight
@@ -63,20 +69,36 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     const int sub = lane & 15, kg = lane >> 4;
     const int split = blockIdx.x, b = blockIdx.z;
     const int per_kv = p.heads / p.kv_heads;
-    const int subs = per_kv / GS;
+    const int rows_kv = MQ ? per_kv * p.seq_q : per_kv;        // query rows that share a KV head
+    const int subs = MQ ? (rows_kv + GS - 1) / GS : per_kv / GS;
     const int kvh = blockIdx.y / subs;
-    const int h0 = kvh * per_kv + (blockIdx.y % subs) * GS;
-
-    // attended key range of this sequence's single query (absolute position seq_kv - 1, so causal cuts nothing)
-    int first = 0, end = p.seq_kv;
-    if (p.window > 0) {
-        first = max(first, p.seq_kv - p.window);
-        end = min(end, p.seq_kv + p.right_context);
+    const int r0 = (blockIdx.y % subs) * GS;
+    // row g of the workgroup: its place among the [batch, heads, seq_q] query rows (rows past the last are copies of it)
+    int64_t row_of[GS];
+    int first_of[GS], end_of[GS];
+    bool uniform_of[GS];
+    int first = 0x7FFFFFFF, end = 0;
+#pragma unroll
+    for (int g = 0; g < GS; ++g) {
+        const int r = MQ ? min(r0 + g, rows_kv - 1) : r0 + g;
+        const int qi = MQ ? r % p.seq_q : 0, h = MQ ? r / p.seq_q : r;
+        row_of[g] = MQ ? ((int64_t)b * p.heads + kvh * per_kv + h) * p.seq_q + qi : (int64_t)b * p.heads + kvh * per_kv + h;
+        // attended key range of this row's query (one query: absolute position seq_kv - 1, so causal cuts nothing)
+        const int pos = MQ ? p.seq_kv - p.seq_q + qi : p.seq_kv - 1;
+        int f = 0, e = p.seq_kv;
+        if (p.window > 0) {
+            f = max(f, pos - p.window + 1);
+            e = min(e, pos + p.right_context + 1);
+        }
+        if (MQ && p.causal) e = min(e, pos + 1);
+        if (p.lengths) e = min(e, p.lengths[b]);
+        e = max(e, 0);
+        uniform_of[g] = f >= e;                // nothing attended: every key scores the same finite value
+        if (uniform_of[g]) { f = 0; e = p.seq_kv; }
+        first_of[g] = f; end_of[g] = e;
+        first = min(first, f); end = max(end, e);
     }
-    if (p.lengths) end = min(end, p.lengths[b]);
-    end = max(end, 0);
-    const bool uniform = first >= end;         // nothing attended: every key scores the same finite value
-    if (uniform) { first = 0; end = p.seq_kv; }
+    const bool uniform = uniform_of[0];        // one query: the same for all rows of the workgroup
     const int chunk = ((end - first + p.splits - 1) / p.splits + 15) & ~15;
     const int lo = first + split * chunk;
     const int hi = min(end, lo + chunk);
@@ -85,7 +107,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     float qr[GS][DPL];
 #pragma unroll
     for (int g = 0; g < GS; ++g) {
-        const float* qp = p.q + ((int64_t)b * p.heads + h0 + g) * D + sub * 4;
+        const float* qp = p.q + row_of[g] * D + sub * 4;
 #pragma unroll
         for (int d = 0; d < DPL; d += 4) {
             const float4 t = *reinterpret_cast<const float4*>(qp + 16 * d);   // float4 number d / 4 of the lane: elements 64 (d / 4) + 4 sub ..
@@ -122,9 +144,14 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         }
     };
     auto consume = [&](const float (&kr)[U][DPL], const float (&vr)[U][DPL], int k0) {
-        bool valid[U];
+        bool valid[U][MQ ? GS : 1];
 #pragma unroll
-        for (int u = 0; u < U; ++u) valid[u] = k0 + 16 * u + kg < hi;
+        for (int u = 0; u < U; ++u) {
+            const int key = k0 + 16 * u + kg;
+#pragma unroll
+            for (int g = 0; g < (MQ ? GS : 1); ++g)
+                valid[u][g] = MQ ? key < min(hi, end_of[g]) && key >= first_of[g] : key < hi;
+        }
         // Branch-free from here to the end of the body: the U x GS score chains (dot product, row reduction, exponentials)
         // are independent and the compiler interleaves them; behind a per-key branch each ran on its own, one
         // dependent instruction at a time -- with one wave per SIMD that chain, not the memory, set the pace.
@@ -137,8 +164,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
 #pragma unroll
                 for (int d = 0; d < DPL; ++d) s = fmaf(qr[g][d], kr[u][d], s);
                 s = row16_sum(s);
-                if (uniform) s = SDPA_DECODE_MASKED;
-                sc[u][g] = valid[u] ? s : -INFINITY;
+                if (MQ ? uniform_of[g] : uniform) s = SDPA_DECODE_MASKED;
+                sc[u][g] = valid[u][MQ ? g : 0] ? s : -INFINITY;
             }
         }
 #pragma unroll
@@ -152,7 +179,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const float e = exp2_raw(sc[u][g] - m_new);        // NaN for (-inf) - (-inf): discarded by the select
-                pr[u] = valid[u] ? e : 0.f;
+                pr[u] = valid[u][MQ ? g : 0] ? e : 0.f;
                 psum += pr[u];
             }
             l[g] = fmaf(l[g], alpha, psum);
@@ -223,8 +250,11 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         for (int st = 0; st < 16; ++st)
 #pragma unroll
             for (int e = 0; e < EPT; ++e) o[e] = fmaf(wacc[st][g][i0 + e], c[st], o[e]);
+        if (MQ && r0 + g >= rows_kv) return;
         const float mm = wmm[g], ls = wls[g];
-        const int64_t row = (int64_t)b * p.heads + h0 + g;
+        int64_t row = row_of[0];
+#pragma unroll
+        for (int e = 1; e < GS; ++e) row = g == e ? row_of[e] : row;
 #pragma unroll
         for (int e = 0; e < EPT; ++e) {
             const int d = i0 + e;                                   // a state's layout in LDS is the row's own element order
@@ -285,21 +315,29 @@ float* sdpa_workspace(size_t bytes);   // shim.hip: per-thread scratch, grown on
 static std::atomic<int> g_sdpa_decode_split_keys{64};   // least keys per split (a multiple of 16)
 void set_sdpa_decode_split_keys(int v) { if (v >= 16) g_sdpa_decode_split_keys = (v + 15) & ~15; }
 
-template <int GS, int DPL>
+template <int GS, int DPL, bool MQ>
 static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge) {
     constexpr int D = 16 * DPL;
     note_kernel("sdpa_decode_kernel");
-    sdpa_decode_kernel<GS, DPL><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
+    sdpa_decode_kernel<GS, DPL, MQ><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
     SKH_CHECK(hipGetLastError());
     if (merge) {
-        sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits);
+        sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits);
         SKH_CHECK(hipGetLastError());
     }
     return 1;
 }
+template <int DPL, bool MQ>
+static int launch_decode_d(const SdpaDecodeParams& p, int gs, int subs, bool merge) {
+    if constexpr (DPL <= 8) { if (gs == 4) return launch_decode_variant<4, DPL, MQ>(p, subs, merge); }
+    if (gs == 2) return launch_decode_variant<2, DPL, MQ>(p, subs, merge);
+    return launch_decode_variant<1, DPL, MQ>(p, subs, merge);
+}
 
 static std::atomic<int> g_sdpa_decode_gs{0};            // query heads per workgroup: 0 = chosen from the shape, else 1 / 2 / 4
 void set_sdpa_decode_gs(int v) { if (v == 0 || v == 1 || v == 2 || v == 4) g_sdpa_decode_gs = v; }
+static std::atomic<int> g_sdpa_decode_one_launch{1};
+void set_sdpa_decode_one_launch(int v) { g_sdpa_decode_one_launch = v != 0; }
 static std::atomic<int> g_attn_merge_max_keys{176};    // most keys per split the unmerged form accepts (a multiple of 16)
 void set_attn_merge_max_keys(int v) { if (v >= 16) g_attn_merge_max_keys = (v + 15) & ~15; }
 // most splits the unmerged form uses. Measured in a Llama-3-8B decode step at 520 to 650 keys (ms per token): 2 splits 1.637,
@@ -313,63 +351,86 @@ void set_attn_merge_splits(int v) { if (v >= 1 && v <= ATTN_MERGE_MAX_SPLITS) g_
 // its own activation load (at most ATTN_MERGE_MAX_SPLITS splits, one sequence): `out` is not written, *leave describes
 // where the partials are; 0 when the key count would need more splits than that.
 int launch_sdpa_decode(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
-                       int seq_kv, int kv_capacity, int head_dim, float scale, int window, int right_context,
+                       int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window, int right_context,
                        const int32_t* lengths, AttnMergePrologue* leave) {
+    if (seq_q > seq_kv) return 0;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return 0;
     if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) return 0;
     const int per_kv = heads / kv_heads;
     const int gs_max = head_dim == 256 ? 2 : 4;
     int gs = g_sdpa_decode_gs.load() > 0 ? min(g_sdpa_decode_gs.load(), gs_max) : gs_max;
-    while (per_kv % gs != 0) gs >>= 1;
+    const bool draft = seq_q > 1;
+    // one query: GS divides the heads of a KV head; several: the last workgroup of a KV head may be padded, so a group is
+    // only not wider than the rows there are
+    while (draft ? gs > 2 && per_kv * seq_q <= gs / 2 : per_kv % gs != 0) gs >>= 1;
+    // keys that a query can attend: a window bounds them whatever the cache holds
+    const int keys = window > 0 ? (int)min((int64_t)seq_kv, (int64_t)window + right_context + seq_q - 1) : seq_kv;
+    // One split, no merge behind it: the merge is a second launch (2.8 us of a host's time, and about that between two
+    // dependent kernels on the device), which buys the parallelism of the splits. Estimates in us, fitted to 1 / 2 / 8 / 16
+    // sequences x 6 to 64 heads x 64 to 4096 keys at D 64 and 128. One split with GS rows per workgroup: 2.7 and its passes
+    // of 32 keys (a chain of loads and arithmetic, longer with more rows) or its traffic (every workgroup of a KV head reads
+    // it, mostly through another die's L2), 4.4 at least (the host's launch). With splits: 4.9 and the traffic, 6.8 at
+    // least. Measured, 32 heads over 8, D 128, one sequence: 128 keys 7.1 -> 4.6 us, 512 keys 6.8 -> 6.0, 640 keys 6.7 (6.9
+    // with one split); 16 sequences at 1024 keys: 25.1 -> 20.6.
+    bool single = false;
+    const int cols = draft ? per_kv * seq_q : per_kv;           // rows that share a KV head
+    if (g_sdpa_decode_one_launch && !leave && g_sdpa_decode_gs.load() == 0 && keys > g_sdpa_decode_split_keys && keys <= 2048) {
+        const double once = 8e-6 * batch * kv_heads * keys * head_dim;      // MB of K and V
+        double best = 0.95 * fmax(6.8, 4.9 + once * ((cols + gs - 1) / gs) / 6.9);
+        const int most = gs;
+        for (int g = 1; g <= most; g *= 2) {
+            if (draft ? g > 1 && cols <= g / 2 : per_kv % g != 0) break;
+            const double groups_kv = (cols + g - 1) / g, wgs = groups_kv * batch * kv_heads;
+            const double slope = head_dim == 64 ? (g == 1 ? 0.137 : g == 2 ? 0.21 : 0.32) : (g == 1 ? 0.21 : g == 2 ? 0.30 : 0.54) * head_dim / 128;
+            const double rate = wgs >= 128 ? 7.5 : 6.3 * fmin(1.0, sqrt(wgs / 64));
+            const double t = fmax(4.4, 2.7 + fmax((keys + 31) / 32 * slope, once * groups_kv / rate));
+            if (t < best) { best = t; gs = g; single = true; }
+        }
+    }
     // Few workgroups (one sequence at a short context, or splits capped for the projection that merges them): two query
     // heads per workgroup instead of four. The K / V rows are then fetched by two workgroups (the second from L2), each
     // with half the arithmetic per pass, and twice as many CUs take part: 1.502 against 1.526 ms per token in a
     // Llama-3-8B decode step at 520 to 650 keys (one head per workgroup: 1.529).
-    if (g_sdpa_decode_gs.load() == 0 && gs == 4) {
+    if (g_sdpa_decode_gs.load() == 0 && gs == 4 && !draft && !single) {
         const int64_t groups4 = (int64_t)batch * kv_heads * (per_kv / 4);
         const int most = leave ? g_attn_merge_splits.load() : SDPA_DECODE_MAX_SPLITS;
-        const int splits4 = min(most, (seq_kv + g_sdpa_decode_split_keys - 1) / g_sdpa_decode_split_keys);
+        const int splits4 = min(most, (keys + g_sdpa_decode_split_keys - 1) / g_sdpa_decode_split_keys);
         if (groups4 * splits4 < num_cus()) gs = 2;
     }
-    const int subs = per_kv / gs;
-    if (batch > 65535) return 0;
+    const int subs = (cols + gs - 1) / gs;
+    if (batch > 65535 || (int64_t)kv_heads * subs > 65535) return 0;
     SdpaDecodeParams p{q, k, v, out, batch, heads, kv_heads, seq_kv, kv_capacity, scale, window, right_context, lengths, 1,
-                       nullptr, nullptr};
+                       nullptr, nullptr, seq_q, causal};
     // enough workgroups to put every CU on the cache, at least 64 keys per split (measured in the decoder at 500 to 650
     // keys: 32 or 48 keys per split 2.5 % slower per token, 96 and 128 keys the same as 64)
     const int64_t groups = (int64_t)batch * kv_heads * subs;
     int splits = (int)((2 * (int64_t)num_cus() + groups - 1) / groups);
-    splits = min(splits, min(SDPA_DECODE_MAX_SPLITS, (seq_kv + g_sdpa_decode_split_keys - 1) / g_sdpa_decode_split_keys));
+    splits = min(splits, min(SDPA_DECODE_MAX_SPLITS, (keys + g_sdpa_decode_split_keys - 1) / g_sdpa_decode_split_keys));
     if (splits < 1) splits = 1;
+    // what the partials of this many splits take is held by the one-split form as well: a cache that grows into splits then
+    // does not move the scratch under a graph recorded before
+    if (splits > 1 && !sdpa_workspace(sizeof(float) * (size_t)batch * heads * seq_q * splits * (head_dim + 2))) return -1;
+    if (single) splits = 1;
     if (leave) {
         if (batch != 1) return 0;
         const int most = g_attn_merge_splits;
         if (splits > most) {
-            if ((seq_kv + most - 1) / most > g_attn_merge_max_keys) return 0;
+            if ((keys + most - 1) / most > g_attn_merge_max_keys) return 0;
             splits = most;
         }
     }
     p.splits = splits;
     if (splits > 1 || leave) {
-        const size_t rows = (size_t)batch * heads;
+        const size_t rows = (size_t)batch * heads * seq_q;
         p.part = sdpa_workspace(sizeof(float) * rows * splits * (head_dim + 2));
         if (!p.part) return -1;
         p.ml = p.part + rows * splits * head_dim;
     }
     if (leave) *leave = AttnMergePrologue{p.part, p.ml, splits, head_dim};
     const bool merge = splits > 1 && !leave;
-    if (head_dim == 64) {
-        if (gs == 4) return launch_decode_variant<4, 4>(p, subs, merge);
-        if (gs == 2) return launch_decode_variant<2, 4>(p, subs, merge);
-        return launch_decode_variant<1, 4>(p, subs, merge);
-    }
-    if (head_dim == 128) {
-        if (gs == 4) return launch_decode_variant<4, 8>(p, subs, merge);
-        if (gs == 2) return launch_decode_variant<2, 8>(p, subs, merge);
-        return launch_decode_variant<1, 8>(p, subs, merge);
-    }
-    if (gs == 2) return launch_decode_variant<2, 16>(p, subs, merge);
-    return launch_decode_variant<1, 16>(p, subs, merge);
+    if (head_dim == 64) return draft ? launch_decode_d<4, true>(p, gs, subs, merge) : launch_decode_d<4, false>(p, gs, subs, merge);
+    if (head_dim == 128) return draft ? launch_decode_d<8, true>(p, gs, subs, merge) : launch_decode_d<8, false>(p, gs, subs, merge);
+    return draft ? launch_decode_d<16, true>(p, gs, subs, merge) : launch_decode_d<16, false>(p, gs, subs, merge);
 }
 
 int launch_q4k_gemv_mfma(const uint8_t* w, const float* x, float* y, int k, int n, const float* gain, float eps,
@@ -393,7 +454,7 @@ int launch_attn_out_proj_q4k(const uint8_t* wo, int n, int k, const float* q, co
     if ((reinterpret_cast<uintptr_t>(wo) & 15) || !q4k_gemv_mfma_accepts_merge(k, n, head_dim)) return 0;
     if (residual && (reinterpret_cast<uintptr_t>(residual) & 3)) return 0;
     AttnMergePrologue am{};
-    const int r = launch_sdpa_decode(q, k_cache, v_cache, nullptr, 1, heads, kv_heads, seq_kv, kv_capacity, head_dim, scale, window, 0,
+    const int r = launch_sdpa_decode(q, k_cache, v_cache, nullptr, 1, heads, kv_heads, 1, seq_kv, kv_capacity, head_dim, scale, 1, window, 0,
                                      lengths, &am);
     if (r <= 0) return r;
     const int g = launch_q4k_gemv_mfma(wo, nullptr, out, k, n, nullptr, 0.f, residual, residual ? EPI_RESIDUAL : EPI_NONE, nullptr, &am);

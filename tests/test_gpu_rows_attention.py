@@ -126,6 +126,30 @@ def test_attention_decode_kernel_shapes_and_rules(hip_backend, torch_cuda, heads
         close(got, L.sdpa(q, k, v, scale, causal, win, rc, lens), rel=2e-5, abs_=2e-6)
 
 
+@pytest.mark.parametrize("one_launch", [1, 0])
+@pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv", [(1, 8, 2, 128, 2, 65), (2, 6, 2, 64, 3, 300), (1, 4, 4, 128, 8, 8), (1, 3, 1, 64, 15, 700),
+                                                           (3, 2, 1, 256, 5, 129), (1, 32, 8, 128, 4, 1500), (2, 1, 1, 64, 2, 40)])
+def test_attention_of_a_few_queries_over_a_cache(hip_backend, torch_cuda, batch, heads, kv_heads, d, sq, skv, one_launch):
+    """2 to 15 queries per sequence on the cache-streaming kernel: rows of several queries and heads share a workgroup, each
+    with a key range of its own (causal and window move with the query, lengths cut some of them to nothing, one sequence
+    to no key at all), padded last workgroups, one split and several."""
+    rng = np.random.default_rng(heads * d + skv + sq)
+    q = rng.standard_normal((batch, heads, sq, d)).astype(np.float32)
+    k = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
+    v = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
+    scale = float(1 / np.sqrt(d))
+    lengths = np.array([skv - sq // 2, 0, skv // 3][:batch], np.int32)
+    hip_backend.set_tuning("sdpa_decode_one_launch", one_launch)
+    try:
+        for causal, win, rc, lens in ((True, 0, 0, None), (False, 0, 0, None), (True, 0, 0, lengths), (True, max(1, skv // 5), 0, None),
+                                      (False, 3, 2, lengths), (True, 2, 0, lengths)):
+            got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, scale, causal, win, rc, lens)
+            assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+            close(got, L.sdpa(q, k, v, scale, causal, win, rc, lens), rel=2e-5, abs_=2e-6)
+    finally:
+        hip_backend.set_tuning("sdpa_decode_one_launch", 1)
+
+
 def test_attention_prefill_config_against_torch_fp32(hip_backend, torch_cuda):
     """Prefill: seq 2048 causal, 32 / 8 heads, head_dim 128. The oracle checks a 256-long prefix problem exactly;
     the full size is compared with torch's fp32 attention on the same device (textbook softmax(QK^T)V)."""
