@@ -19,6 +19,8 @@
 // (fp32 atomic adds into C cost more than the K loop at these sizes, and their order is not reproducible).
 #include "common.h"
 
+#include <cmath>
+
 namespace skh {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -683,6 +685,11 @@ int launch_q4k_gemm_frag(const uint8_t* a, const uint8_t* w, float* c, int m, in
 bool gemm_frag_enabled();
 bool gemm_frag_fits(int m, int n, int k);
 bool gemm_frag_forced();
+int launch_gemm_skinny(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* c, const float* gain, float eps,
+                       const float* residual, int epilogue, bool x_pairs);                                       // gemm_skinny.hip
+bool gemm_skinny_fits(int enc, int m, int n, int k);
+double gemm_skinny_estimate(int enc, int m, int n, int k);
+int gemm_skinny_mode();
 
 static std::atomic<int> g_gemm_ksplit{0};   // 0 = choose from the tile count
 void set_gemm_ksplit(int v) { g_gemm_ksplit = v; }
@@ -713,6 +720,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
         (gain && ((reinterpret_cast<uintptr_t>(gain) & 15) || k > 256 * 4 * 16)) || (epilogue == GEMM_EPI_SWIGLU && (n & 1)) ||
         (epilogue != GEMM_EPI_NONE && !tmp))
         return fused ? 1 : launch_gemv(enc, w, x, m, k, n, y);
+    if (gemm_skinny_mode() >= 2 && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     hipStream_t s = current_stream();
     auto round_activations = [&](__bf16* a) -> int {            // fp32 -> bf16, with the RMSNorm of a fused call folded in
         const int64_t n4 = (int64_t)m * k / 4;                  // k is a multiple of 64
@@ -777,6 +785,20 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
             if (ks == 1 || t < best) { best = t; ksplit = ks; }
         }
         tile_estimate = best;
+    }
+    // Few rows: the kernel without a row tile to fill, where its estimate is below that of what the rules underneath would
+    // take (tile kernel: its own launch, the pass in front and the sum of the splits; fragment-order kernel: likewise)
+    const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 && gemm_ksw_enabled() && gemm_frag_enabled();
+    if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k)) {
+        // (the epilogue plays no part: a product takes one kernel, and sums in one order, whatever is done to it on the way out)
+        double other = tile_estimate + (ksplit > 1 ? 5.5 : 2.75);
+        if (frag_ok) {
+            // (its four-wave form, two workgroups per CU, loses about half of an unfilled round)
+            const double tiles = (double)((m + 127) / 128) * ((n + 63) / 64) / num_cus();
+            const double rounds = tiles <= 1.0 ? 1.0 : 0.5 * (tiles + ceil(tiles));
+            other = fmin(other, rounds * (8.0 + (k <= 4096 ? 0.20 : 0.27) * (k / GK)) + 2.75);
+        }
+        if (gemm_skinny_estimate(enc, m, n, k) < 0.95 * other) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     }
     if (ksw_ok && gemm_ksw_enabled() && g_gemm_ksplit.load() <= 0) {
         // The kernel that splits K over the waves of a workgroup fills the chip with 128 x 64 tiles and parks no partial

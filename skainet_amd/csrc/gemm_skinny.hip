@@ -1,0 +1,511 @@
+// Packed-weight GEMM for prompts and batches of few rows (9 to about 128), every format:
+//   C[m, n] = sum_k A[m, k] * dequant(W[n, k]),  A fp32 [M, K] rounded to bf16 once, W packed in canonical row-major GGUF
+//   order, products bf16 x bf16 on v_mfma_f32_16x16x32_bf16, fp32 accumulation, C fp32 [M, N].
+// The decode is the block arithmetic of the reference (code * (d * sc) - dmin * m and its siblings) in fp32, rounded to
+// bf16 (nearest even). Semantics: m rows = m scalar GEMVs,
+//   skainet-backends/skainet-backend-cpu/src/commonMain/kotlin/sk/ainet/exec/kernel/PackedViewMatmulKernel.kt:69-108.
+//
+// What bounds it: every weight is decoded once per row block (2.3 to 3.7 vector instructions each), the weight is read
+// once, and a workgroup reads its rows' activations for every 16 NT columns. The 256- and 128-row tiles of the other
+// kernels spend their matrix work, their activation traffic and their LDS round trips on rows that do not exist here.
+//   * A workgroup owns 16 MT rows x 16 NT columns; its NW waves split K by 256-element super-blocks (w, w + NW, ...).
+//   * Lane (c, q) = (l % 16, l / 16) of a wave holds, of each of its NT weight rows c, the 64 weights of the super-block
+//     that its own B operands need: it loads their bytes straight from memory (48 to 80 bytes in 16-byte loads; the four
+//     lanes of a row read one consecutive run), decodes eight of them per matrix instruction, and no weight passes
+//     through LDS. The next super-block's bytes are requested before the current one is decoded.
+//   * The contraction index is a free permutation as long as both operands agree: step u (0..7) of a super-block takes,
+//     from lane q, elements 64 q + 8 u .. + 7 (a lane owns 64 consecutive elements), or for Q6_K, whose bytes interleave
+//     quarters, 128 (q / 2) + 32 (u / 2) + 16 (q % 2) + 8 (u % 2) .. + 7. The pass in front writes the activations in that
+//     order, 1 KB of consecutive memory per (16 rows, step), so an A operand is one 16-byte load per lane.
+//   * The waves' partial tiles meet in LDS once; residual or SwiGLU are applied where the sums are stored.
+// Measured (product and pass in front): Q4_K 24 x 14336 x 4096 22.4 -> 17 us (the weight in 8 us behind two
+// launches of 2.75), 64 x 4096 x 4096 19.5 -> 10.8, 9 x 4096 x 14336 27.8 -> 13.6; Q8_0 64 x 4096 x 4096 21.4 -> 14.1.
+#include "common.h"
+
+#include <cmath>
+#include <type_traits>
+
+namespace skh {
+
+typedef __bf16 skn_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 skn_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float skn_f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 skn_h2 __attribute__((ext_vector_type(2)));
+
+void* kernel_workspace(size_t bytes);   // shim.hip
+
+enum { SKN_EPI_NONE = 0, SKN_EPI_RESIDUAL = 1, SKN_EPI_SWIGLU = 2 };
+
+__device__ __forceinline__ uint32_t skn_pack(float a, float b) { return __builtin_bit_cast(uint32_t, skn_bf16x2{(__bf16)a, (__bf16)b}); }
+__device__ __forceinline__ float skn_silu(float g) { return g * (1.0f / (1.0f + expf(-g))); }
+
+// ---------------------------------------------------------------------------------------------- activations
+// Element offset inside a super-block of the eight elements of step u, lane group q.
+template <bool Q6>
+__device__ __forceinline__ int skn_elem(int q, int u) {
+    return Q6 ? 128 * (q >> 1) + 32 * (u >> 1) + 16 * (q & 1) + 8 * (u & 1) : 64 * q + 8 * u;
+}
+// Inverse: 8-element piece j (0..31) of a super-block -> byte offset of its 16 bytes (row r of the tile) in the 8 KB of
+// (row tile, super-block).
+template <bool Q6>
+__device__ __forceinline__ int skn_piece(int j, int r) {
+    const int q = Q6 ? 2 * (j >> 4) + ((j >> 1) & 1) : j >> 3, u = Q6 ? 2 * ((j >> 2) & 3) + (j & 1) : j & 7;
+    return u * 1024 + (r + 16 * q) * 16;
+}
+// One workgroup per (super-block, row tile of 16): 512 pieces, two per thread. PAIRS: rows of interleaved (gate, up)
+// pairs, the activation is their SwiGLU.
+template <bool Q6, bool PAIRS>
+__global__ __launch_bounds__(256) void skinny_prepass_kernel(const float* __restrict__ x, uint8_t* __restrict__ out, int m, int k) {
+    const int sb = blockIdx.x, mt = blockIdx.y, nsb = k >> 8;
+    uint8_t* dst = out + ((int64_t)mt * nsb + sb) * 8192;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int r = (threadIdx.x >> 5) + 8 * p, j = threadIdx.x & 31, row = 16 * mt + r;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (row < m) {
+            const int64_t at = (int64_t)row * k + 256 * sb + 8 * j;
+            if constexpr (PAIRS) {
+                const float4* s = reinterpret_cast<const float4*>(x + 2 * at);
+                const float4 a = s[0], b = s[1], c = s[2], d = s[3];
+                v = make_uint4(skn_pack(skn_silu(a.x) * a.y, skn_silu(a.z) * a.w), skn_pack(skn_silu(b.x) * b.y, skn_silu(b.z) * b.w),
+                               skn_pack(skn_silu(c.x) * c.y, skn_silu(c.z) * c.w), skn_pack(skn_silu(d.x) * d.y, skn_silu(d.z) * d.w));
+            } else {
+                const float4* s = reinterpret_cast<const float4*>(x + at);
+                const float4 a = s[0], b = s[1];
+                v = make_uint4(skn_pack(a.x, a.y), skn_pack(a.z, a.w), skn_pack(b.x, b.y), skn_pack(b.z, b.w));
+            }
+        }
+        *reinterpret_cast<uint4*>(dst + skn_piece<Q6>(j, r)) = v;
+    }
+}
+// The same with an RMSNorm folded in: one workgroup per row (rows past m: zeros), V pieces per thread held in registers.
+template <bool Q6, int V>
+__global__ __launch_bounds__(256) void skinny_prepass_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ gain,
+                                                                     uint8_t* __restrict__ out, int m, int k, float eps) {
+    __shared__ float red[4];
+    const int row = blockIdx.x, mt = row >> 4, r = row & 15, pieces = k >> 3;
+    float4 a[V], b[V];
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int p = threadIdx.x + 256 * i;
+        const bool in = p < pieces && row < m;
+        const float4* src = reinterpret_cast<const float4*>(x + (int64_t)row * k) + 2 * p;
+        a[i] = in ? src[0] : make_float4(0.f, 0.f, 0.f, 0.f);
+        b[i] = in ? src[1] : make_float4(0.f, 0.f, 0.f, 0.f);
+        s = fmaf(a[i].x, a[i].x, s); s = fmaf(a[i].y, a[i].y, s); s = fmaf(a[i].z, a[i].z, s); s = fmaf(a[i].w, a[i].w, s);
+        s = fmaf(b[i].x, b[i].x, s); s = fmaf(b[i].y, b[i].y, s); s = fmaf(b[i].z, b[i].z, s); s = fmaf(b[i].w, b[i].w, s);
+    }
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    const float scale = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) * (1.0f / (float)k) + eps);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int p = threadIdx.x + 256 * i;
+        if (p >= pieces) continue;
+        const float4* g4 = reinterpret_cast<const float4*>(gain) + 2 * p;
+        const float4 g = g4[0], h = g4[1];
+        const uint4 v = make_uint4(skn_pack(a[i].x * scale * g.x, a[i].y * scale * g.y), skn_pack(a[i].z * scale * g.z, a[i].w * scale * g.w),
+                                   skn_pack(b[i].x * scale * h.x, b[i].y * scale * h.y), skn_pack(b[i].z * scale * h.z, b[i].w * scale * h.w));
+        *reinterpret_cast<uint4*>(out + ((int64_t)mt * (k >> 8) + (p >> 5)) * 8192 + skn_piece<Q6>(p & 31, r)) = v;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------- weight formats
+// Per format: Raw (the bytes a lane needs of one super-block of one row), load, Scales (worked out once per super-block),
+// and decode<U>: the eight weights of step U as four dwords of bf16 pairs.
+template <int I> __device__ __forceinline__ float skn_byte(uint32_t v) { return ubyte_to_float<I>(v); }
+// four codes, one per byte, times scale plus add
+__device__ __forceinline__ void skn_bytes4(uint32_t v, float scale, float add, uint32_t& lo, uint32_t& hi) {
+    lo = skn_pack(fmaf(skn_byte<0>(v), scale, add), fmaf(skn_byte<1>(v), scale, add));
+    hi = skn_pack(fmaf(skn_byte<2>(v), scale, add), fmaf(skn_byte<3>(v), scale, add));
+}
+// The four codes of one nibble plane of a dword (PLANE 0: low nibbles, 1: high): masked into 16-bit fields they are the fp16
+// subnormals code * 2^-24 (2^-20), which the mixed-precision multiply-add widens exactly; `scale` carries the power of two.
+template <int PLANE>
+__device__ __forceinline__ void skn_nibbles4(uint32_t c, float scale, float add, uint32_t& lo, uint32_t& hi) {
+    constexpr uint32_t mask = PLANE ? 0x00F000F0u : 0x000F000Fu;
+    const skn_h2 b02 = __builtin_bit_cast(skn_h2, c & mask), b13 = __builtin_bit_cast(skn_h2, (c >> 8) & mask);
+    lo = skn_pack(fmaf((float)b02.x, scale, add), fmaf((float)b13.x, scale, add));
+    hi = skn_pack(fmaf((float)b02.y, scale, add), fmaf((float)b13.y, scale, add));
+}
+constexpr float SKN_2P24 = 16777216.0f, SKN_2P20 = 1048576.0f;
+
+// d * sc and dmin * m of sub-blocks 2 q and 2 q + 1 from a K-quant header (ggml get_scale_min_k4)
+struct SknK4 { float s0, s1, m0, m1; };
+__device__ __forceinline__ SknK4 skn_k4(const uint4& hdr, int q) {
+    const float d = half_bits_to_float_fast(hdr.x & 0xFFFFu), dmin = half_bits_to_float_fast(hdr.x >> 16);
+    const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, mn_lo = hdr.z & 0x3F3F3F3Fu;
+    const uint32_t sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u), mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+    const int sh = 16 * (q & 1);
+    const uint32_t sc = (q < 2 ? sc_lo : sc_hi) >> sh, mn = (q < 2 ? mn_lo : mn_hi) >> sh;
+    return SknK4{d * (float)(sc & 0xFFu), d * (float)((sc >> 8) & 0xFFu), dmin * (float)(mn & 0xFFu), dmin * (float)((mn >> 8) & 0xFFu)};
+}
+
+struct SknQ4K {
+    static constexpr int BYTES = Q4K_BYTES;
+    static constexpr bool Q6 = false;
+    struct Raw { uint4 hdr; uint32_t c[8]; };
+    struct Scales { float s0, a0, s1, a1; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* blk, int q) {
+        r.hdr = *reinterpret_cast<const uint4*>(blk);
+        const uint4 a = *reinterpret_cast<const uint4*>(blk + 16 + 32 * q), b = *reinterpret_cast<const uint4*>(blk + 32 + 32 * q);
+        r.c[0] = a.x; r.c[1] = a.y; r.c[2] = a.z; r.c[3] = a.w; r.c[4] = b.x; r.c[5] = b.y; r.c[6] = b.z; r.c[7] = b.w;
+    }
+    static __device__ __forceinline__ Scales scales(const Raw& r, int q) {
+        const SknK4 k = skn_k4(r.hdr, q);
+        return Scales{k.s0 * SKN_2P24, -k.m0, k.s1 * SKN_2P20, -k.m1};
+    }
+    template <int U> static __device__ __forceinline__ void decode(const Raw& r, const Scales& s, uint32_t (&o)[4]) {
+        const uint32_t c0 = r.c[2 * (U & 3)], c1 = r.c[2 * (U & 3) + 1];
+        if constexpr (U < 4) { skn_nibbles4<0>(c0, s.s0, s.a0, o[0], o[1]); skn_nibbles4<0>(c1, s.s0, s.a0, o[2], o[3]); }
+        else { skn_nibbles4<1>(c0, s.s1, s.a1, o[0], o[1]); skn_nibbles4<1>(c1, s.s1, s.a1, o[2], o[3]); }
+    }
+};
+struct SknQ5K {
+    static constexpr int BYTES = Q5K_BYTES;
+    static constexpr bool Q6 = false;
+    struct Raw { uint4 hdr; uint32_t c[8], h[8]; };
+    struct Scales { float s0, a0, s1, a1; int bit; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* blk, int q) {
+        r.hdr = *reinterpret_cast<const uint4*>(blk);
+        const uint4 h0 = *reinterpret_cast<const uint4*>(blk + 16), h1 = *reinterpret_cast<const uint4*>(blk + 32);
+        const uint4 a = *reinterpret_cast<const uint4*>(blk + 48 + 32 * q), b = *reinterpret_cast<const uint4*>(blk + 64 + 32 * q);
+        r.c[0] = a.x; r.c[1] = a.y; r.c[2] = a.z; r.c[3] = a.w; r.c[4] = b.x; r.c[5] = b.y; r.c[6] = b.z; r.c[7] = b.w;
+        r.h[0] = h0.x; r.h[1] = h0.y; r.h[2] = h0.z; r.h[3] = h0.w; r.h[4] = h1.x; r.h[5] = h1.y; r.h[6] = h1.z; r.h[7] = h1.w;
+    }
+    static __device__ __forceinline__ Scales scales(const Raw& r, int q) {
+        const SknK4 k = skn_k4(r.hdr, q);
+        return Scales{k.s0, -k.m0, k.s1, -k.m1, 2 * q};
+    }
+    template <int U> static __device__ __forceinline__ void decode(const Raw& r, const Scales& s, uint32_t (&o)[4]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int at = 2 * (U & 3) + i;
+            const uint32_t v = ((r.c[at] >> (U < 4 ? 0 : 4)) & 0x0F0F0F0Fu) | (((r.h[at] >> (s.bit + (U < 4 ? 0 : 1))) & 0x01010101u) << 4);
+            skn_bytes4(v, U < 4 ? s.s0 : s.s1, U < 4 ? s.a0 : s.a1, o[2 * i], o[2 * i + 1]);
+        }
+    }
+};
+// 16 bytes from an address that is 0 or 2 bytes past a dword boundary (`odd`): dword-aligned loads and a byte shift. A
+// 16-byte load at an odd half-word address takes the memory pipe about twice as long (Q8_0, 32 x 4096 x 4096: 14.5 us with
+// such loads, 11.3 with these). With an even address the fifth dword is the fourth again: nothing past the run is read.
+struct SknQ6K {
+    static constexpr int BYTES = Q6K_BYTES;
+    static constexpr bool Q6 = true;
+    struct Raw { u32x4_vec a, b, h; u32x2_vec sc; uint32_t a4, b4, h4, sc2, d; int odd; };
+    struct Scales { float s[4]; uint32_t a[4], b[4], h[4]; };
+    static __device__ __forceinline__ void run(u32x4_vec& v, uint32_t& last, const uint8_t* base, int odd) {
+        v = load_u32x4_a4(base);
+        last = *reinterpret_cast<const uint32_t*>(base + 12 + 4 * odd);
+    }
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* blk, int q) {
+        const int half = q >> 1, off = 16 * (q & 1);
+        r.odd = (int)(reinterpret_cast<uintptr_t>(blk) >> 1) & 1;
+        const uint8_t* base = blk - 2 * r.odd;
+        run(r.a, r.a4, base + 64 * half + off, r.odd);
+        run(r.b, r.b4, base + 64 * half + 32 + off, r.odd);
+        run(r.h, r.h4, base + 128 + 32 * half + off, r.odd);
+        const uint32_t* sc = reinterpret_cast<const uint32_t*>(base + 192 + 8 * half);
+        r.sc = u32x2_vec{sc[0], sc[1]};
+        r.sc2 = sc[1 + r.odd];
+        r.d = load_u16(blk + 208);
+    }
+    static __device__ __forceinline__ void align(uint32_t (&o)[4], const u32x4_vec& v, uint32_t last, uint32_t sh) {
+        o[0] = __builtin_amdgcn_alignbyte(v.y, v.x, sh);
+        o[1] = __builtin_amdgcn_alignbyte(v.z, v.y, sh);
+        o[2] = __builtin_amdgcn_alignbyte(v.w, v.z, sh);
+        o[3] = __builtin_amdgcn_alignbyte(last, v.w, sh);
+    }
+    static __device__ __forceinline__ Scales scales(const Raw& r, int q) {
+        const float d = half_bits_to_float_fast(r.d);
+        const uint32_t sh = 2 * r.odd, s0 = __builtin_amdgcn_alignbyte(r.sc.y, r.sc.x, sh), s1 = __builtin_amdgcn_alignbyte(r.sc2, r.sc.y, sh);
+        const int b = 8 * (q & 1);
+        Scales s{{d * (float)(int8_t)(s0 >> b), d * (float)(int8_t)(s0 >> (16 + b)), d * (float)(int8_t)(s1 >> b), d * (float)(int8_t)(s1 >> (16 + b))}, {}, {}, {}};
+        align(s.a, r.a, r.a4, sh); align(s.b, r.b, r.b4, sh); align(s.h, r.h, r.h4, sh);
+        return s;
+    }
+    template <int U> static __device__ __forceinline__ void decode(const Raw&, const Scales& s, uint32_t (&o)[4]) {
+        constexpr int Q = U >> 1, E = 2 * (U & 1);
+        const float sc = s.s[Q], add = -32.f * sc;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t l = (Q & 1) ? s.b[E + i] : s.a[E + i];
+            const uint32_t v = ((l >> (Q < 2 ? 0 : 4)) & 0x0F0F0F0Fu) | (((s.h[E + i] >> (2 * Q)) & 0x03030303u) << 4);
+            skn_bytes4(v, sc, add, o[2 * i], o[2 * i + 1]);
+        }
+    }
+};
+// The formats of 32-element blocks: a lane's two blocks are 68, 36, 44 or 48 consecutive bytes from a dword boundary, and
+// the second block's codes lie on dwords themselves; the first block's are shifted into place (Q5_1: no shift).
+struct SknQ80 {
+    static constexpr int BYTES = 8 * Q80_BYTES;
+    static constexpr bool Q6 = false;
+    struct Raw { uint32_t v[17]; };
+    struct Scales { float d[2]; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* blk, int q) {
+        const uint8_t* b = blk + 68 * q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32x4_vec x = load_u32x4_a4(b + 16 * i);
+            r.v[4 * i] = x.x; r.v[4 * i + 1] = x.y; r.v[4 * i + 2] = x.z; r.v[4 * i + 3] = x.w;
+        }
+        r.v[16] = *reinterpret_cast<const uint32_t*>(b + 64);
+    }
+    static __device__ __forceinline__ Scales scales(const Raw& r, int) { return Scales{{half_bits_to_float_fast(r.v[0] & 0xFFFFu), half_bits_to_float_fast(r.v[8] >> 16)}}; }
+    template <int U> static __device__ __forceinline__ void decode(const Raw& r, const Scales& s, uint32_t (&o)[4]) {
+        const float d = s.d[U >> 2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t v = U < 4 ? __builtin_amdgcn_alignbyte(r.v[2 * U + i + 1], r.v[2 * U + i], 2) : r.v[2 * U + i + 1];
+            o[2 * i] = skn_pack((float)(int8_t)v * d, (float)(int8_t)(v >> 8) * d);
+            o[2 * i + 1] = skn_pack((float)(int8_t)(v >> 16) * d, (float)(int8_t)(v >> 24) * d);
+        }
+    }
+};
+// Q4_0 / Q5_0 / Q5_1 (FMT 0 / 1 / 2): low nibbles of the 16 code bytes are elements 0..15 of a block, high nibbles 16..31
+template <int FMT> struct SknQ45 {
+    static constexpr int BB = FMT == 0 ? Q40_BYTES : FMT == 1 ? Q50_BYTES : Q51_BYTES;
+    static constexpr int BYTES = 8 * BB, DWORDS = BB / 2;
+    static constexpr bool Q6 = false;
+    struct Raw { uint32_t v[DWORDS]; };
+    struct Scales { float d[2], add[2]; uint32_t h[2]; };
+    static __device__ __forceinline__ void load(Raw& r, const uint8_t* blk, int q) {
+        const uint8_t* b = blk + 2 * BB * q;
+#pragma unroll
+        for (int i = 0; i < DWORDS / 4; ++i) {
+            const u32x4_vec x = load_u32x4_a4(b + 16 * i);
+            r.v[4 * i] = x.x; r.v[4 * i + 1] = x.y; r.v[4 * i + 2] = x.z; r.v[4 * i + 3] = x.w;
+        }
+#pragma unroll
+        for (int i = DWORDS / 4 * 4; i < DWORDS; ++i) r.v[i] = reinterpret_cast<const uint32_t*>(b)[i];
+    }
+    static __device__ __forceinline__ Scales scales(const Raw& r, int) {
+        Scales s;
+        const uint32_t d0 = r.v[0] & 0xFFFFu, d1 = FMT == 0 ? r.v[4] >> 16 : FMT == 1 ? r.v[5] >> 16 : r.v[6] & 0xFFFFu;
+        s.d[0] = half_bits_to_float_fast(d0);
+        s.d[1] = half_bits_to_float_fast(d1);
+        s.add[0] = FMT == 0 ? -8.f * s.d[0] : FMT == 1 ? -16.f * s.d[0] : half_bits_to_float_fast(r.v[0] >> 16);
+        s.add[1] = FMT == 0 ? -8.f * s.d[1] : FMT == 1 ? -16.f * s.d[1] : half_bits_to_float_fast(r.v[FMT == 2 ? 6 : 0] >> 16);
+        s.h[0] = FMT == 1 ? __builtin_amdgcn_alignbyte(r.v[1], r.v[0], 2) : r.v[1];
+        s.h[1] = FMT == 1 ? r.v[6] : r.v[FMT == 2 ? 7 : 1];
+        return s;
+    }
+    template <int B> static __device__ __forceinline__ uint32_t code_dword(const Raw& r, int e) {      // dword e of block B's 16 code bytes
+        if constexpr (FMT == 2) return r.v[6 * B + 2 + e];
+        else if constexpr (B == 1) return r.v[(FMT == 0 ? 5 : 7) + e];
+        else return __builtin_amdgcn_alignbyte(r.v[(FMT == 0 ? 1 : 2) + e], r.v[(FMT == 0 ? 0 : 1) + e], 2);
+    }
+    template <int U> static __device__ __forceinline__ void decode(const Raw& r, const Scales& s, uint32_t (&o)[4]) {
+        constexpr int B = U >> 2, P = (U >> 1) & 1, E = 2 * (U & 1);       // block, nibble plane, first code dword
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t c = code_dword<B>(r, E + i);
+            if constexpr (FMT == 0) skn_nibbles4<P>(c, s.d[B] * (P ? SKN_2P20 : SKN_2P24), s.add[B], o[2 * i], o[2 * i + 1]);
+            else {
+                const uint32_t v = ((c >> (4 * P)) & 0x0F0F0F0Fu) | (((((s.h[B] >> (8 * (U & 3) + 4 * i)) & 0xFu) * 0x00204081u) & 0x01010101u) << 4);
+                skn_bytes4(v, s.d[B], s.add[B], o[2 * i], o[2 * i + 1]);
+            }
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------------------------- the product
+constexpr int SKN_WAVES = 8;      // one wave of a workgroup per super-block in turn (four waves measured the same or up to 10 % slower)
+template <class F, int MT, int NT>
+__global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, float* c,
+                                                                     const float* residual, int m, int n, int k, int epilogue) {
+    constexpr int NW = SKN_WAVES;
+    extern __shared__ __attribute__((aligned(16))) float skn_part[];       // [NW][MT * NT][256]
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * (16 * NT), mt0 = blockIdx.y * MT;
+    const int nsb = k >> 8;
+    const int mtiles = (m + 15) >> 4;
+    const uint32_t row_bytes = (uint32_t)nsb * F::BYTES;
+    uint32_t row[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) row[t] = (uint32_t)min(n0 + 16 * t + col, n - 1) * row_bytes;    // rows past N: a valid copy, never stored
+    // A operands of (row tile, super-block): 8 KB; row tiles past the last are copies of it, never stored
+    const uint8_t* at[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) at[i] = a + (int64_t)min(mt0 + i, mtiles - 1) * nsb * 8192 + 16 * lane;
+    skn_f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = skn_f32x4{0.f, 0.f, 0.f, 0.f};
+
+    constexpr int AR = MT >= 4 ? 2 : 4;                                   // steps of A operands in flight or in use
+    if (wave < nsb) {
+        typename F::Raw raw[2][NT];
+        auto load_w = [&](int set, int sb) __attribute__((always_inline)) {
+            const uint8_t* base = w + (int64_t)sb * F::BYTES;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) F::load(raw[set][t], base + row[t], q);
+        };
+        skn_bf16x8 af[AR][MT];
+        auto load_a = [&](int slot, int sb, int u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) af[slot][i] = *reinterpret_cast<const skn_bf16x8*>(at[i] + (int64_t)sb * 8192 + 1024 * u);
+        };
+        // one super-block: `set` holds its bytes, `next` (clamped to this wave's last) is requested meanwhile
+        auto body = [&](auto set_c, int sb, int next) __attribute__((always_inline)) {
+            constexpr int SET = decltype(set_c)::value;
+            load_w(SET ^ 1, next);
+            typename F::Scales sc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sc[t] = F::scales(raw[SET][t], q);
+            auto step = [&](auto uc) __attribute__((always_inline)) {
+                constexpr int U = decltype(uc)::value;
+                constexpr int AHEAD = U + AR - 1;
+                if constexpr (AHEAD < 8) load_a(AHEAD % AR, sb, AHEAD);
+                else load_a(AHEAD % AR, next, AHEAD - 8);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    uint32_t o[4];
+                    F::template decode<U>(raw[SET][t], sc[t], o);
+                    const skn_bf16x8 b = __builtin_bit_cast(skn_bf16x8, uint4{o[0], o[1], o[2], o[3]});
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[U % AR][i], b, acc[i][t], 0, 0, 0);
+                }
+            };
+            step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{}); step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 4>{}); step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 6>{}); step(std::integral_constant<int, 7>{});
+        };
+        load_w(0, wave);
+#pragma unroll
+        for (int u = 0; u < AR - 1; ++u) load_a(u, wave, u);
+        for (int sb = wave; sb < nsb; sb += 2 * NW) {
+            const int second = sb + NW, third = sb + 2 * NW;
+            body(std::integral_constant<int, 0>{}, sb, second < nsb ? second : sb);
+            if (second >= nsb) break;
+            body(std::integral_constant<int, 1>{}, second, third < nsb ? third : second);
+        }
+    }
+    // accumulator element e of lane (col, q): row 4 q + e, column col of its 16 x 16 tile
+    float* mine = skn_part + (size_t)wave * (MT * NT * 256);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine[(i * NT + t) * 256 + (4 * q + e) * 16 + col] = acc[i][t][e];
+    __syncthreads();
+    for (int p = threadIdx.x; p < MT * NT * 128; p += 64 * NW) {          // two adjacent columns each
+        float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            const float2 t = *reinterpret_cast<const float2*>(skn_part + (size_t)v * (MT * NT * 256) + 2 * p);
+            s.x += t.x; s.y += t.y;
+        }
+        const int tile = p >> 7, gr = 16 * (mt0 + tile / NT) + ((p >> 3) & 15), gc = n0 + 16 * (tile % NT) + 2 * (p & 7);
+        if (gr >= m || gc >= n) continue;
+        if (epilogue == SKN_EPI_SWIGLU) {                                 // n is even: (gate, up) pairs
+            c[(int64_t)gr * (n >> 1) + (gc >> 1)] = skn_silu(s.x) * s.y;
+            continue;
+        }
+        const int64_t o = (int64_t)gr * n + gc;
+        if (epilogue == SKN_EPI_RESIDUAL) { s.x += residual[o]; if (gc + 1 < n) s.y += residual[o + 1]; }
+        c[o] = s.x;
+        if (gc + 1 < n) c[o + 1] = s.y;
+    }
+}
+
+size_t gemm_skinny_activation_bytes(int m, int k) { return (size_t)((m + 15) / 16) * 16 * (size_t)k * 2; }
+// k in whole super-blocks, byte offsets of a weight row in 32 bits
+bool gemm_skinny_fits(int enc, int m, int n, int k) {
+    return k % 256 == 0 && (uint64_t)n * (uint64_t)(k / block_elems(enc)) * block_bytes(enc) < ((uint64_t)1 << 32) && (m + 15) / 16 <= 65535;
+}
+
+template <bool Q6>
+static int skinny_prepass(const float* x, const float* gain, float eps, uint8_t* a, int m, int k, bool pairs, hipStream_t s) {
+    const int mtiles = (m + 15) / 16;
+    if (pairs) skinny_prepass_kernel<Q6, true><<<dim3(k / 256, mtiles), dim3(256), 0, s>>>(x, a, m, k);
+    else if (!gain) skinny_prepass_kernel<Q6, false><<<dim3(k / 256, mtiles), dim3(256), 0, s>>>(x, a, m, k);
+    else if (k <= 256 * 8 * 2) skinny_prepass_rmsnorm_kernel<Q6, 2><<<dim3(16 * mtiles), dim3(256), 0, s>>>(x, gain, a, m, k, eps);
+    else skinny_prepass_rmsnorm_kernel<Q6, 8><<<dim3(16 * mtiles), dim3(256), 0, s>>>(x, gain, a, m, k, eps);
+    SKH_CHECK(hipGetLastError());
+    return 0;
+}
+
+template <class F, int MT, int NT>
+static int launch_skinny_tile(const uint8_t* a, const uint8_t* w, float* c, const float* residual, int m, int n, int k, int epilogue, hipStream_t s) {
+    constexpr size_t smem = (size_t)SKN_WAVES * MT * NT * 256 * sizeof(float);
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&packed_gemm_skinny_kernel<F, MT, NT>), smem);
+    packed_gemm_skinny_kernel<F, MT, NT><<<dim3((n + 16 * NT - 1) / (16 * NT), ((m + 15) / 16 + MT - 1) / MT), dim3(64 * SKN_WAVES), smem, s>>>(
+        a, w, c, residual, m, n, k, epilogue);
+    SKH_CHECK(hipGetLastError());
+    return 0;
+}
+
+// The tile of a shape and what it is estimated to take, in us. A wave's time for one super-block of its tile, measured per
+// format on 4096 x 4096, 4096 x 14336 and 14336 x 4096 (time of the call without its two launches' 5.5 us, per super-block
+// of a wave and round of one workgroup per CU): columns are tiles of 16 MT rows x 16 NT columns.
+struct SknTile { int mt, nt; double us; };
+SknTile gemm_skinny_tile(int enc, int m, int n, int k) {
+    static const int shapes[6][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 2}, {2, 2}, {4, 2}};
+    static const double q4k[6] = {1.3, 2.2, 3.8, 2.2, 2.95, 4.4}, q5k[6] = {1.7, 2.3, 4.0, 3.4, 4.0, 5.7}, q6k[6] = {2.1, 2.8, 4.2, 4.3, 5.0, 6.7};
+    static const double q80[6] = {2.1, 3.0, 5.3, 3.8, 4.7, 6.4}, q40[6] = {1.3, 2.0, 3.6, 2.2, 3.0, 4.7}, q50[6] = {1.5, 2.1, 4.0, 2.7, 3.4, 5.0};
+    static const double q51[6] = {1.6, 2.2, 4.1, 2.8, 3.7, 5.3};
+    const double* cost = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
+                       : enc == ENC_Q5_1 ? q51 : q80;
+    const int mtiles = (m + 15) / 16, iters = ((k >> 8) + SKN_WAVES - 1) / SKN_WAVES;
+    // weights that do not stay in the 256 MB memory-side cache between calls were measured a fifth slower
+    const double slow = (double)n * (k / block_elems(enc)) * block_bytes(enc) > 64e6 ? 1.2 : 1.0;
+    SknTile best{1, 1, 0.0};
+    for (int i = 0; i < 6; ++i) {
+        const int mt = shapes[i][0], nt = shapes[i][1];
+        if (mt > 1 && mt >= 2 * mtiles) continue;                         // more rows than there are
+        const double groups = (double)((mtiles + mt - 1) / mt) * ((n + 16 * nt - 1) / (16 * nt)) / num_cus();
+        const double rounds = groups <= 1.0 ? 1.0 : mt * nt >= 4 ? ceil(groups) : groups;     // the large tiles run one workgroup per CU
+        const double us = 5.5 + iters * rounds * cost[i] * slow;
+        if (best.us == 0.0 || us < best.us) best = SknTile{mt, nt, us};
+    }
+    return best;
+}
+double gemm_skinny_estimate(int enc, int m, int n, int k) { return gemm_skinny_tile(enc, m, n, k).us; }
+
+static std::atomic<int> g_gemm_skinny{1};   // 0 never, 1 where the estimate favours it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits
+void set_gemm_skinny(int v) { g_gemm_skinny = v; }
+int gemm_skinny_mode() { return g_gemm_skinny.load(); }
+
+template <class F>
+static int launch_skinny_format(int enc, const float* x, const float* gain, float eps, bool pairs, uint8_t* a, const uint8_t* w, float* c,
+                                const float* residual, int m, int n, int k, int epilogue, hipStream_t s) {
+    if (skinny_prepass<F::Q6>(x, gain, eps, a, m, k, pairs, s) != 0) return -1;
+    SknTile t = gemm_skinny_tile(enc, m, n, k);
+    if (const int forced = g_gemm_skinny.load(); forced >= 11) { t.mt = forced / 10; t.nt = forced % 10; }
+    note_kernel("packed_gemm_skinny_kernel");
+    if (t.nt == 2) {
+        if (t.mt == 4) return launch_skinny_tile<F, 4, 2>(a, w, c, residual, m, n, k, epilogue, s);
+        if (t.mt == 2) return launch_skinny_tile<F, 2, 2>(a, w, c, residual, m, n, k, epilogue, s);
+        return launch_skinny_tile<F, 1, 2>(a, w, c, residual, m, n, k, epilogue, s);
+    }
+    if (t.mt == 4) return launch_skinny_tile<F, 4, 1>(a, w, c, residual, m, n, k, epilogue, s);
+    if (t.mt == 2) return launch_skinny_tile<F, 2, 1>(a, w, c, residual, m, n, k, epilogue, s);
+    return launch_skinny_tile<F, 1, 1>(a, w, c, residual, m, n, k, epilogue, s);
+}
+
+// c = epilogue(prologue(x) . W^T), all of it: the pass in front and the product. `c` is [m, n] ([m, n / 2] with SwiGLU).
+int launch_gemm_skinny(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* c, const float* gain, float eps,
+                       const float* residual, int epilogue, bool x_pairs) {
+    uint8_t* a = static_cast<uint8_t*>(kernel_workspace(gemm_skinny_activation_bytes(m, k)));
+    if (!a) return -1;
+    hipStream_t s = current_stream();
+    switch (enc) {
+        case ENC_Q4_K: return launch_skinny_format<SknQ4K>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_K: return launch_skinny_format<SknQ5K>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q6_K: return launch_skinny_format<SknQ6K>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q4_0: return launch_skinny_format<SknQ45<0>>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_0: return launch_skinny_format<SknQ45<1>>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_1: return launch_skinny_format<SknQ45<2>>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+        default: return launch_skinny_format<SknQ80>(enc, x, gain, eps, x_pairs, a, w, c, residual, m, n, k, epilogue, s);
+    }
+}
+
+}  // namespace skh

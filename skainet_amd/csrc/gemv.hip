@@ -165,6 +165,7 @@ void set_gemm_wide(int v);
 void set_gemm_ksplit(int v);
 void set_gemm_rows(int v);
 void set_gemm_ksw(int v);
+void set_gemm_skinny(int v);
 void set_gemm_ksw_teams(int v);
 void set_gemm_ksw_stages(int v);
 void set_gemm_frag(int v);
@@ -210,6 +211,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "q4k_rows_enable")) { g_q4k_rows_enable = value; return 0; }
     if (!strcmp(key, "gemm_ksplit")) { set_gemm_ksplit(value); return 0; }
     if (!strcmp(key, "gemm_rows")) { set_gemm_rows(value); return 0; }
+    if (!strcmp(key, "gemm_skinny")) { set_gemm_skinny(value); return 0; }
     if (!strcmp(key, "gemm_ksw")) { set_gemm_ksw(value); return 0; }
     if (!strcmp(key, "gemm_ksw_teams")) { set_gemm_ksw_teams(value); return 0; }
     if (!strcmp(key, "gemm_ksw_stages")) { set_gemm_ksw_stages(value); return 0; }

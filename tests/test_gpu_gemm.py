@@ -197,3 +197,39 @@ def test_q4k_gemm_with_activations_in_fragment_order(hip_backend, torch_cuda, m,
     if (m, n, k) == (512, 4096, 4096):
         gpu_gemm(hip_backend, torch_cuda, "Q4_K", packed, n, k, x)
         assert hip_backend.last_kernel() == "q4k_gemm_frag_kernel"     # the launcher's own choice for this shape
+
+
+@pytest.mark.parametrize("enc", ALL_ENCS)
+@pytest.mark.parametrize("m,n,k", [(9, 5, 256), (16, 16, 2048), (17, 33, 2304), (33, 130, 768), (64, 31, 4352), (100, 70, 512), (150, 40, 256)])
+def test_gemm_of_few_rows(hip_backend, torch_cuda, enc, m, n, k):
+    """The kernel whose lanes decode their own operands, forced at each of its tiles (1, 2 or 4 row tiles x 1 or 2 column
+    tiles of 16) on ragged rows and columns, fewer super-blocks than waves and uneven counts per wave (1, 2, 8, 9, 17 over
+    8 waves), Q6_K rows that start on odd half words; against the oracle (2e-2) and the product of bf16-rounded operands
+    (2e-4); with RMSNorm, residual and SwiGLU against the same product finished in float64."""
+    torch, kx = torch_cuda, hip_backend
+    packed = gaussian_weight(kx, enc, n, k, 700 + n)
+    rng = np.random.default_rng(m + n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    want = L.gemv(enc, x, packed, n)
+    gain, res = (1 + 0.2 * rng.standard_normal(k)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    try:
+        for tile in (2, 11, 12, 21, 22, 41, 42):
+            kx.set_tuning("gemm_skinny", tile)
+            got = gpu_gemm(kx, torch, enc, packed, n, k, x)
+            assert kx.last_kernel() == "packed_gemm_skinny_kernel"
+            check(got, want)
+            check_exact(torch, enc, got, x, packed, n)
+        w = kx.DeviceWeight.upload(enc, packed, n, k)
+        xn = (x.astype(np.float64) / np.sqrt((x.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-5) * gain).astype(np.float32)
+        p = bf16_round(torch, xn) @ bf16_round(torch, L.dequant(enc, packed).reshape(n, -1)).T
+        out = torch.full((m, n), float("nan"), device="cuda")
+        w.matmul_fused(dev(torch, x), m, out, gain=dev(torch, gain), eps=1e-5, residual=dev(torch, res), epilogue=kx.EPI_RESIDUAL)
+        # a normalised activation that two fp32 evaluations round to neighbouring bf16 values moves one product by 2^-8 of it,
+        # at most 2^-8 * 4.5 * 0.08 = 1.4e-3 for these operands, against a largest output above 1
+        assert normalized_err(out.cpu().numpy(), p + res, eps=1.0) <= 2e-3
+        if n % 2 == 0:
+            half = torch.full((m, n // 2), float("nan"), device="cuda")
+            w.matmul_fused(dev(torch, x), m, half, gain=dev(torch, gain), eps=1e-5, epilogue=kx.EPI_SWIGLU)
+            assert normalized_err(half.cpu().numpy(), p[:, 0::2] / (1 + np.exp(-p[:, 0::2])) * p[:, 1::2], eps=1.0) <= 4e-3
+    finally:
+        kx.set_tuning("gemm_skinny", 1)
