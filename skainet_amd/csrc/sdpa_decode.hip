@@ -371,10 +371,13 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     // of 32 keys (a chain of loads and arithmetic, longer with more rows) or its traffic (every workgroup of a KV head reads
     // it, mostly through another die's L2), 4.4 at least (the host's launch). With splits: 4.9 and the traffic, 6.8 at
     // least. Measured, 32 heads over 8, D 128, one sequence: 128 keys 7.1 -> 4.6 us, 512 keys 6.8 -> 6.0, 640 keys 6.7 (6.9
-    // with one split); 16 sequences at 1024 keys: 25.1 -> 20.6.
+    // with one split); 16 sequences at 1024 keys: 25.1 -> 20.6. A key count on the device (a decode step over a growing cache)
+    // stays with splits above 256: `keys` is then only a bound, and between a layer's products the cache comes from memory,
+    // where a chain of passes waits longer (19 layers at 430 keys: 608 us per step with splits, 664 with one).
     bool single = false;
     const int cols = draft ? per_kv * seq_q : per_kv;           // rows that share a KV head
-    if (g_sdpa_decode_one_launch && !leave && g_sdpa_decode_gs.load() == 0 && keys > g_sdpa_decode_split_keys && keys <= 2048) {
+    if (g_sdpa_decode_one_launch && !leave && g_sdpa_decode_gs.load() == 0 && keys > g_sdpa_decode_split_keys &&
+        keys <= (lengths ? 256 : 2048)) {
         const double once = 8e-6 * batch * kv_heads * keys * head_dim;      // MB of K and V
         double best = 0.95 * fmax(6.8, 4.9 + once * ((cols + gs - 1) / gs) / 6.9);
         const int most = gs;

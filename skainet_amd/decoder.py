@@ -409,11 +409,14 @@ class LlamaDecoder:
         return int(self.token.download(np.int32, 1)[0])
 
     KEY_BUCKET = 512
+    SHORT_KEYS = 256      # a first, shorter bucket: up to here one launch attends a layer's keys, above it splits and a merge
 
     def _key_bound(self, keys: int) -> int:
         """The key count a step is laid out for: the next multiple of KEY_BUCKET (the device-side length picks the keys
         that exist, the bound decides how attention splits them)."""
         b = self.KEY_BUCKET
+        if keys <= self.SHORT_KEYS < b:
+            b = self.SHORT_KEYS
         return min(self.cfg.ctx_max, (keys + b - 1) // b * b)
 
     def _decode_step(self, bound: Optional[int] = None) -> None:

@@ -77,6 +77,7 @@ class OpsLlamaDecoder:
     """Prefill + greedy decode for batch 1 through `HipOps` alone; KV cache, position and current token on the device."""
 
     KEY_BUCKET = 512
+    SHORT_KEYS = 256      # a first, shorter bucket: up to here one launch attends a layer's keys, above it splits and a merge
 
     def __init__(self, weights: OpsLlamaWeights, max_prefill: int = 512):
         c = self.cfg = weights.cfg
@@ -156,6 +157,8 @@ class OpsLlamaDecoder:
 
     def _key_bound(self, keys: int) -> int:
         b = self.KEY_BUCKET
+        if keys <= self.SHORT_KEYS < b:
+            b = self.SHORT_KEYS
         return min(self.cfg.ctx_max, (keys + b - 1) // b * b)
 
     def _decode_step(self, bound: Optional[int] = None) -> None:
