@@ -286,16 +286,18 @@ static int staged_h2d(void* dst, const uint8_t* src, size_t bytes) {
 // filling (or emptying) one piece of staging while the kernel of another is on the bus. Measured against the runtime's copy
 // and wait, up / down: 4 KB 15.3 / 21.8 -> 8.6 / 7.9 us, 16 KB 14.2 / 21.2 -> 9.0 / 8.8, 128 KB 87 (an array
 // the runtime pins for the call) -> 14.5 up, 1 MB 40.8 / 59.8 -> 42 / 43. Above COPY_KERNEL_MAX the
-// copy engine's rate counts for more than its hand-over.
-constexpr size_t COPY_KERNEL_MAX = 1u << 20, COPY_CHUNK = 128u << 10;
+// copy engine's rate counts for more than its hand-over; where the bytes pass through page-locked staging anyway (a product
+// on host arrays) the pieces hide the bus behind the host's memcpy up to STAGED_KERNEL_MAX.
+constexpr size_t COPY_KERNEL_MAX = 1u << 20, STAGED_KERNEL_MAX = 8u << 20, COPY_CHUNK = 128u << 10;
 static thread_local Scratch t_link[2];            // page-locked: bytes on their way down / up
 static thread_local Scratch t_flag;               // page-locked: the ticket of the last finished flagged copy
 static thread_local uint32_t t_ticket = 0;        // the last one handed out
-static bool copy_kernel_fits(size_t bytes) { return bytes <= COPY_KERNEL_MAX && !t_capture_stream; }
-static size_t copy_chunk(size_t bytes) {          // at most four pieces: a piece costs a launch
+static bool copy_kernel_fits(size_t bytes, size_t most = COPY_KERNEL_MAX) { return bytes <= most && !t_capture_stream; }
+static size_t copy_chunk(size_t bytes) {          // four pieces of 128 to 256 KB, then more of 256: a piece costs a launch
     const size_t quarter = (bytes / 4 + 4095) & ~(size_t)4095;
-    return quarter > COPY_CHUNK ? quarter : COPY_CHUNK;
+    return quarter > 2 * COPY_CHUNK ? 2 * COPY_CHUNK : quarter > COPY_CHUNK ? quarter : COPY_CHUNK;
 }
+constexpr int COPY_MAX_PIECES = (int)(STAGED_KERNEL_MAX / (2 * COPY_CHUNK)) + 1;
 // Queues the copy with a completion ticket (0: failed); wait_copy waits for it.
 static uint32_t queue_flagged_copy(void* dst, const void* src, size_t bytes) {
     const bool fresh = t_flag.ptr == nullptr;
@@ -336,7 +338,7 @@ static int copy_up(void* dst, const void* src, void* pin, size_t bytes, bool wai
 }
 static int copy_down(void* dst, const void* src, void* pin, size_t bytes) {
     const size_t chunk = copy_chunk(bytes);
-    uint32_t tickets[4];
+    uint32_t tickets[COPY_MAX_PIECES];
     int n = 0;
     for (size_t off = 0; off < bytes; off += chunk, ++n) {
         const size_t len = bytes - off < chunk ? bytes - off : chunk;
@@ -600,14 +602,14 @@ int32_t skainet_hip_matmul_host(const skainet_hip_weight* w, const float* x_host
     float* xd = static_cast<float*>(scratch_get(t_stage[1], in_bytes));
     float* yd = static_cast<float*>(scratch_get(t_stage[2], out_bytes));
     if (!pin_in || !pin_out || !xd || !yd) return -1;
-    if (copy_kernel_fits(in_bytes)) {
+    if (copy_kernel_fits(in_bytes, STAGED_KERNEL_MAX)) {
         if (copy_up(xd, x_host, pin_in, in_bytes, false) != 0) return -1;
     } else {
         memcpy(pin_in, x_host, in_bytes);
         if (check_hip(hipMemcpyAsync(xd, pin_in, in_bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
     }
     if (skainet_hip_matmul_dev(w, xd, m, yd) != 0) return -1;
-    if (copy_kernel_fits(out_bytes)) return copy_down(out_host, yd, pin_out, out_bytes);
+    if (copy_kernel_fits(out_bytes, STAGED_KERNEL_MAX)) return copy_down(out_host, yd, pin_out, out_bytes);
     if (check_hip(hipMemcpyAsync(pin_out, yd, out_bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
     if (check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize") != 0) return -1;
     memcpy(out_host, pin_out, out_bytes);
