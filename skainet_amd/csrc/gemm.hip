@@ -698,6 +698,46 @@ void set_gemm_wide(int v) { g_gemm_wide = v; }
 static std::atomic<int> g_gemm_rows{0};     // 0 = choose from the shape, 2 / 4 = 128 / 256 activation rows per tile
 void set_gemm_rows(int v) { if (v == 0 || v == 2 || v == 4) g_gemm_rows = v; }
 
+// What a product takes on the tile kernel, in us, the pass in front and both launches (5.5) included. A round is one
+// workgroup per CU; a step of 64 elements of K costs more the fuller the round (clocks and memory are shared): the two
+// numbers per format and tile are for 64 and for 256 tiles, measured at K 2048 and 4096, and a round spends 3 us outside its
+// loop. Two of the 128 x 128 workgroups fit a CU: two rounds of them take 1.42 (half of the second full) to 1.67 of one.
+static double gemm_round_us(const double (&step)[2], double tiles, double steps) {
+    const double fill = tiles <= 64 ? 0.0 : tiles >= 256 ? 1.0 : (tiles - 64) / 192;
+    return 3.0 + (step[0] + (step[1] - step[0]) * fill) * steps;
+}
+static double gemm_tile_us(int enc, int wtm, int wtn, double tiles, double steps) {
+    // [128 x 128, 128 x 256, 256 x 128, 256 x 256][64 tiles, 256 tiles]
+    static const double q4k[4][2] = {{0.586, 0.739}, {0.99, 1.29}, {0.825, 1.10}, {1.44, 1.99}}, q5k[4][2] = {{0.623, 0.783}, {1.14, 1.42}, {0.872, 1.19}, {1.58, 2.17}};
+    static const double q6k[4][2] = {{0.68, 0.805}, {1.25, 1.51}, {0.908, 1.23}, {1.69, 2.35}}, q80[4][2] = {{0.803, 0.894}, {1.39, 1.96}, {1.03, 1.29}, {1.83, 2.68}};
+    static const double q40[4][2] = {{0.539, 0.705}, {0.994, 1.24}, {0.806, 1.08}, {1.38, 1.95}}, q50[4][2] = {{0.628, 0.764}, {1.22, 1.43}, {0.853, 1.15}, {1.63, 2.17}};
+    static const double q51[4][2] = {{0.602, 0.764}, {1.14, 1.46}, {0.84, 1.17}, {1.57, 2.26}};
+    const double (*table)[2] = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
+                             : enc == ENC_Q5_1 ? q51 : q80;
+    const int shape = (wtm == 4 ? 2 : 0) + (wtn == 4 ? 1 : 0);
+    const double cus = num_cus(), one = gemm_round_us(table[shape], 256, steps);
+    tiles *= 256 / cus;                                          // the measurements are for 256 CUs
+    double t = 5.5;
+    if (shape == 0) {
+        const double pairs = floor(tiles / 512);
+        t += pairs * 1.67 * one;
+        tiles -= 512 * pairs;
+        if (tiles > 256) return t + one * (tiles <= 384 ? 1.42 : 1.42 + 0.5 * (tiles - 384) / 256);
+    } else {
+        const double rounds = floor(tiles / 256);
+        t += rounds * one;
+        tiles -= 256 * rounds;
+    }
+    return tiles > 0 ? t + gemm_round_us(table[shape], tiles, steps) : t;
+}
+// The same for the fragment-order kernel (Q4_K, 128 x 64 tiles), measured at 64 to 1024 tiles, K 1024 to 14336.
+static double gemm_frag_us(int m, int n, int k) {
+    const double tiles = (double)((m + 127) / 128) * ((n + 63) / 64) * 256 / num_cus(), steps = k / GK;
+    if (tiles <= 128) return 8.8 + 0.19 * steps;
+    if (tiles <= 256) return 8.8 + 0.7 * (tiles - 128) / 128 + (0.19 + 0.085 * (tiles - 128) / 128) * steps;
+    return 8.5 + tiles / 256 + (0.2575 * tiles / 256 + (tiles < 512 ? 0.06 : 0.0)) * steps;
+}
+
 // y = epilogue(prologue(x) . W^T): gain != null normalises every activation row first (RMSNorm, folded into the pass that
 // rounds the activations to bf16); epilogue is one of GEMM_EPI_* (residual [m, n] may be y; SwiGLU: y is [m, n / 2]).
 // `tmp` ([m, n] floats, needed when an epilogue is asked for) takes the plain product when K is not split.
@@ -755,62 +795,41 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     const bool frag_ok = ksw_ok && gemm_frag_fits(m, n, k);
     if (frag_ok && gemm_frag_forced()) return run_frag();
     if (ksw_ok && gemm_ksw_forced()) return run_ksw();
-    // 128 activation rows per tile where there are no more than that (the weight is then decoded once, and half the
-    // matrix work of the taller tile is not spent on rows that do not exist); the wide tile where it alone fills most of
-    // the chip in one round
-    const int wtm = g_gemm_rows.load() != 0 ? g_gemm_rows.load() : (m <= 128 ? 2 : 4);
-    const int tiles_m = (m + gemm_gm(wtm) - 1) / gemm_gm(wtm);
-    const int wide_tiles = tiles_m * ((n + gemm_gn(4) - 1) / gemm_gn(4));
-    const bool wide = g_gemm_wide.load() >= 0 ? g_gemm_wide.load() != 0 : 4 * wide_tiles >= 3 * num_cus();
-    const int wtn = wide ? 4 : 2;
-    const int tiles_n = (n + gemm_gn(wtn) - 1) / gemm_gn(wtn);
-    const int tiles = tiles_m * tiles_n;
-    // K chunks are whole 256-element groups so every encoding's blocks stay intact
+    // The tile shape and the number of K splits with the least estimate. K chunks are whole 256-element groups so every
+    // encoding's blocks stay intact; the launch that sums the splits takes 5 us and (splits + 1) m n floats at 8 bytes per ns.
     const int kgroups = (k + 255) / 256;
-    int ksplit = g_gemm_ksplit;
+    int wtm = 2, wtn = 2, ksplit = 1;
     double tile_estimate = 0.0;
-    if (ksplit <= 0) {
-        // One workgroup is resident per CU, so the tile grid runs in rounds of num_cus() workgroups. Measured on this
-        // kernel: about 8 us per round outside the K loop, 1.04 us per 64-element K step, and for the launch that sums
-        // the splits 2.3 us plus its (splits + 1) * m * n floats at 8 bytes per ns. Take the split with the least estimate.
-        const int cus = num_cus();
-        double best = 0.0;
-        ksplit = 1;
-        for (int ks = 1; ks <= 8 && ks <= kgroups; ++ks) {
-            const int rounds = (tiles * ks + cus - 1) / cus;
-            const int steps = ((kgroups + ks - 1) / ks) * (256 / GK);
-            const double step_us = wtm == 4 ? (wide ? 2.0 : 1.04) : (wide ? 1.13 : 0.65);   // measured per tile shape
-            double t = rounds * (8.0 + step_us * steps);
-            if (ks > 1) t += 2.3 + (double)(ks + 1) * m * n * 4.0 / 8.0e6;
-            if (ks == 1 || t < best) { best = t; ksplit = ks; }
+    for (int tm = 2; tm <= 4; tm += 2) {
+        if (g_gemm_rows.load() != 0 && tm != g_gemm_rows.load()) continue;
+        for (int tn = 2; tn <= 4; tn += 2) {
+            if (g_gemm_wide.load() >= 0 && (tn == 4) != (g_gemm_wide.load() != 0)) continue;
+            const double tiles = (double)((m + gemm_gm(tm) - 1) / gemm_gm(tm)) * ((n + gemm_gn(tn) - 1) / gemm_gn(tn));
+            for (int ks = 1; ks <= 8 && ks <= kgroups; ++ks) {
+                if (g_gemm_ksplit.load() > 0 && ks != (g_gemm_ksplit.load() < kgroups ? g_gemm_ksplit.load() : kgroups)) continue;
+                double t = gemm_tile_us(enc, tm, tn, tiles * ks, ((kgroups + ks - 1) / ks) * (256 / GK));
+                if (ks > 1) t += 5.0 + (double)(ks + 1) * m * n * 4.0 / 8.0e6;
+                if (tile_estimate == 0.0 || t < tile_estimate) { tile_estimate = t; wtm = tm; wtn = tn; ksplit = ks; }
+            }
         }
-        tile_estimate = best;
     }
-    // Few rows: the kernel without a row tile to fill, where its estimate is below that of what the rules underneath would
-    // take (tile kernel: its own launch, the pass in front and the sum of the splits; fragment-order kernel: likewise)
+    if (g_gemm_ksplit.load() > 8) ksplit = g_gemm_ksplit.load();
+    const bool frag_by_rule = frag_ok && gemm_frag_enabled() && gemm_ksw_enabled() && g_gemm_ksplit.load() <= 0;
+    const double frag_estimate = frag_by_rule ? gemm_frag_us(m, n, k) : tile_estimate;
+    // Few rows: the kernel without a row tile to fill. (The epilogue plays no part in the choice: a product takes one
+    // kernel, and sums in one order, whatever is done to it on the way out.)
     const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 && gemm_ksw_enabled() && gemm_frag_enabled();
-    if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k)) {
-        // (the epilogue plays no part: a product takes one kernel, and sums in one order, whatever is done to it on the way out)
-        double other = tile_estimate + (ksplit > 1 ? 5.5 : 2.75);
-        if (frag_ok) {
-            // (its four-wave form, two workgroups per CU, loses about half of an unfilled round)
-            const double tiles = (double)((m + 127) / 128) * ((n + 63) / 64) / num_cus();
-            const double rounds = tiles <= 1.0 ? 1.0 : 0.5 * (tiles + ceil(tiles));
-            other = fmin(other, rounds * (8.0 + (k <= 4096 ? 0.20 : 0.27) * (k / GK)) + 2.75);
-        }
-        if (gemm_skinny_estimate(enc, m, n, k) < 0.95 * other) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
-    }
-    if (ksw_ok && gemm_ksw_enabled() && g_gemm_ksplit.load() <= 0) {
-        // The kernel that splits K over the waves of a workgroup fills the chip with 128 x 64 tiles and parks no partial
-        // products; its step is slower per tile row (0.31 us per 64 elements of K measured, 6.5 us per round outside the loop).
-        // It wins where the tile kernel would have to split K across workgroups: 512 x 4096 x 4096 is such a shape.
+    if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k) &&
+        gemm_skinny_estimate(enc, m, n, k) < 0.95 * fmin(tile_estimate, frag_estimate))
+        return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
+    if (frag_by_rule && frag_estimate < tile_estimate) return run_frag();
+    if (ksw_ok && gemm_ksw_enabled() && !gemm_frag_enabled() && g_gemm_ksplit.load() <= 0) {
+        // with the fragment-order kernel switched off, its predecessor where it would beat the tile kernel (0.31 us per 64
+        // elements of K, 6.5 us per round outside the loop)
         const int rounds = (((m + 127) / 128) * ((n + 63) / 64) + num_cus() - 1) / num_cus();
-        // the same tiles with the activations in fragment order: measured 8 us per round outside the loop and 0.20 us per
-        // 64 elements of K (0.27 on rows longer than two super-blocks per wave, whose weight ring is refilled under way)
-        if (frag_ok && gemm_frag_enabled()) {
-            if (rounds * (8.0 + (k <= 4096 ? 0.20 : 0.27) * (k / GK)) < tile_estimate) return run_frag();
-        } else if (rounds * (6.5 + 0.31 * (k / GK)) < tile_estimate) return run_ksw();
+        if (rounds * (6.5 + 0.31 * (k / GK)) + 5.5 < tile_estimate) return run_ksw();
     }
+    const int tiles_m = (m + gemm_gm(wtm) - 1) / gemm_gm(wtm), tiles_n = (n + gemm_gn(wtn) - 1) / gemm_gn(wtn);
     if (ksplit > kgroups) ksplit = kgroups;
     const int k_chunk = ((kgroups + ksplit - 1) / ksplit) * 256;
     ksplit = (k + k_chunk - 1) / k_chunk;

@@ -32,6 +32,8 @@ typedef __bf16 frg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 frg_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float frg_f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t frg_u32x4 __attribute__((ext_vector_type(4)));
+typedef float frg_f32x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(4))) frg_f32x4_a4 { frg_f32x4 v; };
 
 constexpr int FRG_M = 128, FRG_N = 64;
 constexpr int FRG_SLOT = FRG_N * 144;                         // one raw super-block of the tile's 64 weight rows: 9 wave loads
@@ -411,9 +413,10 @@ __global__ __launch_bounds__(64 * FRG_WAVES, 2) void q4k_gemm_frag_kernel(const 
             // residual (may be c itself: every element is read and then written by this one thread): c = residual + product
             float* dst = c + (int64_t)gr * n + gc;
             const float* res = residual ? residual + (int64_t)gr * n + gc : nullptr;
-            if (gc + 3 < n && ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(res)) & 15) == 0) {
-                if (res) { const float4 t = *reinterpret_cast<const float4*>(res); sum.x = t.x + sum.x; sum.y = t.y + sum.y; sum.z = t.z + sum.z; sum.w = t.w + sum.w; }
-                *reinterpret_cast<float4*>(dst) = sum;
+            if (gc + 3 < n) {
+                // four floats at dword alignment are one access as well (rows of an n that is no multiple of four)
+                if (res) { const frg_f32x4_a4 t = *reinterpret_cast<const frg_f32x4_a4*>(res); sum.x = t.v.x + sum.x; sum.y = t.v.y + sum.y; sum.z = t.v.z + sum.z; sum.w = t.v.w + sum.w; }
+                *reinterpret_cast<frg_f32x4_a4*>(dst) = frg_f32x4_a4{frg_f32x4{sum.x, sum.y, sum.z, sum.w}};
             } else {
                 if (gc < n) dst[0] = (res ? res[0] : 0.f) + sum.x;
                 if (gc + 1 < n) dst[1] = (res ? res[1] : 0.f) + sum.y;
