@@ -184,7 +184,9 @@ void* sync_scratch(size_t bytes) {
         }
         void* p = nullptr;
         if (check_hip(hipMalloc(&p, SYNC_SCRATCH_BYTES), "hipMalloc(sync scratch)") != 0) return nullptr;
-        if (check_hip(hipMemset(p, 0, SYNC_SCRATCH_BYTES), "hipMemset(sync scratch)") != 0) { (void)hipFree(p); return nullptr; }
+        // (waited for: the caller's stream may be one that does not order itself behind the default stream)
+        if (check_hip(hipMemset(p, 0, SYNC_SCRATCH_BYTES), "hipMemset(sync scratch)") != 0 ||
+            check_hip(hipStreamSynchronize(nullptr), "hipStreamSynchronize") != 0) { (void)hipFree(p); return nullptr; }
         t_sync = p;
     }
     return t_sync;
@@ -353,8 +355,28 @@ static int copy_down(void* dst, const void* src, void* pin, size_t bytes) {
     }
     return 0;
 }
+// A kernel that is handed a bad range faults where the runtime's copy returns an error, so the copy kernel gets only what
+// the runtime knows as one allocation of this device, `bytes` long from there, against memory that is the host's. Everything
+// else (another device's or managed memory, mapped ranges, stale addresses, runs past an allocation) is the runtime's, which
+// copies or refuses it.
+static bool device_range(const void* p, size_t bytes) {
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t off = (size_t)(static_cast<const uint8_t*>(p) - static_cast<const uint8_t*>(base));
+    return at.type == hipMemoryTypeDevice && at.device == g_device && off <= size && bytes <= size - off;
+}
+static bool host_memory(const void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) { (void)hipGetLastError(); return true; }      // unknown to the runtime: pageable
+    return at.type == hipMemoryTypeUnregistered || at.type == hipMemoryTypeHost;
+}
 static int copy_h2d(void* dst, const void* src, size_t bytes) {
-    if (!copy_kernel_fits(bytes)) {
+    if (!copy_kernel_fits(bytes) || !device_range(dst, bytes) || !host_memory(src)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }
@@ -362,7 +384,7 @@ static int copy_h2d(void* dst, const void* src, size_t bytes) {
     return pin ? copy_up(dst, src, pin, bytes, true) : -1;
 }
 static int copy_d2h(void* dst, const void* src, size_t bytes) {
-    if (!copy_kernel_fits(bytes)) {
+    if (!copy_kernel_fits(bytes) || !device_range(src, bytes) || !host_memory(dst)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }

@@ -202,3 +202,23 @@ def test_host_copies_of_every_size_and_alignment_are_byte_exact(hip_backend, nby
         assert np.array_equal(got, want) and np.array_equal(part, src)
     finally:
         lib.skainet_hip_free(p)
+
+
+@pytest.mark.parametrize("nbytes", [300, 5000, 70000])
+def test_host_copies_past_an_allocation_are_refused(hip_backend, nbytes):
+    """A run that leaves its allocation, and an address that is none of the device's, return an error as the runtime's copy
+    does: they never reach the copy kernel. Device memory in the host's place is the runtime's to copy."""
+    from skainet_amd import _lib
+    lib = _lib.hip()
+    host = np.arange(nbytes, dtype=np.uint8)
+    p, other = lib.skainet_hip_malloc(256), lib.skainet_hip_malloc(nbytes)
+    try:
+        assert lib.skainet_hip_memcpy_h2d(p, host.ctypes.data, nbytes) != 0
+        assert lib.skainet_hip_memcpy_d2h(host.ctypes.data, p, nbytes) != 0
+        assert lib.skainet_hip_memcpy_h2d(p, host.ctypes.data, 256) == 0           # and the thread goes on
+        back = np.zeros(256, np.uint8)
+        assert lib.skainet_hip_memcpy_d2h(back.ctypes.data, p, 256) == 0
+        assert np.array_equal(back, host[:256])
+    finally:
+        lib.skainet_hip_free(p)
+        lib.skainet_hip_free(other)
