@@ -126,18 +126,19 @@ SKAINET_HIP_API int64_t skainet_hip_weight_nbytes(const skainet_hip_weight* w);
 /* out[m, rows] = x[m, cols] . W^T, fp32 in and out, device pointers. What a ViewKernel registered for
  * matmul(F32 dense x packed BLOCKED_ROW_MAJOR) runs (API/MatmulKernels.kt:11-40; CPU twin
  * REF/skainet-backend-native-cpu/src/jvmMain/kotlin/sk/ainet/exec/kernel/FfmRowMajorKernels.kt:52-106).
- * m <= 8 streams the weight once per 4 (Q4_K: 8) rows, within 1e-3 of the exact fp32 product; the arithmetic class
- * depends on format and m:
+ * m <= 8 is within 1e-3 of the exact fp32 product and streams the weight once (m = 5 .. 8 of Q6_K and Q5_K twice on a few
+ * shapes); the arithmetic class depends on format and m:
  *   - Q4_K, m = 1, K a multiple of 1024 up to 16384, and Q8_0, m = 1, K a multiple of 1024 up to 4096: codes stay
  *     integers, the activations are rounded to 22-bit fixed point against the largest magnitude of their 64-element
  *     group and contracted on the int8 matrix instruction; scales and minima are applied in fp32 (measured 4e-5 / 2e-5
  *     in the GEMV parity metric). A NaN or an infinity among the activations makes every output NaN.
- *   - Q4_K, m = 3 .. 8: codes exact, an activation enters as bf16 hi + bf16 lo (16 to 17 significant bits) on the bf16
- *     matrix instructions, fp32 sums (2e-4 in the metric).
- *   - everything else (Q4_K m = 2 or other K, Q6_K, Q5_K, Q4_0, Q5_0, Q5_1, Q8_0 at other K): fp32 multiply-adds on
- *     decoded codes, the reference's exact-fp32 products in another summation order.
+ *   - Q4_K, m = 3 .. 8 at K = 4096 and most other K above 2048: codes exact, an activation enters as bf16 hi + bf16 lo (16 to
+ *     17 significant bits) on the bf16 matrix instructions, fp32 sums (2e-4 in the metric).
+ *   - everything else (Q4_K m = 2 or other K, Q6_K, Q5_K, Q4_0, Q5_0, Q5_1, Q8_0 at other K or m): fp32 multiply-adds on
+ *     decoded codes or decoded weights on the fp32 matrix instruction ("gemv_few"), the reference's exact-fp32 products in
+ *     another summation order.
  *   skainet_hip_set_tuning("q4k_mfma_enable", 0) / ("q8_0_mfma_enable", 0) force the fp32 kernels at m = 1,
- *   ("q4k_wide_enable", 0) + ("q4k_quads_stream_enable", 0) + ("q4k_rows_enable", 0) the fp32 slot kernel at every m.
+ *   ("gemv_few", 0) + ("q4k_wide_enable", 0) + ("q4k_quads_stream_enable", 0) + ("q4k_rows_enable", 0) the fp32 slot kernel at every m.
  * Larger m uses the MFMA dequant-GEMM, which rounds activations and decoded weights to bf16 and accumulates in fp32
  * (within 2e-2 of the largest output): the switch at m = 9 is a switch of precision class as well as of kernel, and
  * skainet_hip_matmul_kind_dev pins either one. */
@@ -429,9 +430,10 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * and more instead of eight),
  * "q4k_mfma_window" (row quads the one-row integer matrix-core kernel keeps in flight per wave: 2 or 3,
  * 0 = chosen from K), "gemm_ksplit" (K splits of the MFMA GEMM,
- * 0 = automatic), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
+ * 0 = automatic), "gemv_few" (products of 2 to 8 rows on the fp32 matrix instruction: 0 never, 1 where they are the faster ones,
+ * 2 wherever they fit), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
  * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2), "gemm_wide" (1 / 0: force the 256-column / 128-column tile, -1 = chosen from the shape), "gemm_rows" (2 / 4: 128 / 256
- * activation rows per tile, 0 = 128 up to 128 rows and 256 above), "gemm_ksw" (the Q4_K kernel that splits K over the
+ * activation rows per tile, 0 = chosen from the shape), "gemm_ksw" (the Q4_K kernel that splits K over the
  * waves of a workgroup: 0 never, 1 where the launcher's estimate favours it, 2 wherever it fits), "gemm_ksw_teams" (teams
  * of four waves per workgroup of that kernel, each with its own share of K: 1 or 2, default 2; rows with an odd number
  * of 256-element super-blocks always run one team), "gemm_ksw_stages" (activation tiles the one-team form keeps in LDS: 3 to 7,

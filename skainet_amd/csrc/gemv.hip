@@ -197,6 +197,8 @@ int launch_q8_0_gemv_mfma(const uint8_t* w, const float* x, float* y, int k, int
 void set_q8_0_mfma_enable(int v);
 void set_q8_0_mfma_per_cu(int v);
 void set_dense_mfma(int v);
+int launch_gemv_few(int enc, const uint8_t* w, const float* x, float* y, int m, int n, int k);         // gemv_few.hip
+void set_gemv_few(int v);
 
 // Experiment knobs (defaults are the measured best): returns 0 when the key is known.
 int set_tuning(const char* key, int value) {
@@ -211,6 +213,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "q4k_rows_enable")) { g_q4k_rows_enable = value; return 0; }
     if (!strcmp(key, "gemm_ksplit")) { set_gemm_ksplit(value); return 0; }
     if (!strcmp(key, "gemm_rows")) { set_gemm_rows(value); return 0; }
+    if (!strcmp(key, "gemv_few")) { set_gemv_few(value); return 0; }
     if (!strcmp(key, "gemm_skinny")) { set_gemm_skinny(value); return 0; }
     if (!strcmp(key, "gemm_ksw")) { set_gemm_ksw(value); return 0; }
     if (!strcmp(key, "gemm_ksw_teams")) { set_gemm_ksw_teams(value); return 0; }
@@ -251,6 +254,13 @@ int launch_gemv(int enc, const uint8_t* w, const float* x, int m, int k, int n, 
         const float* xb = x + (int64_t)b0 * k;
         float* yb = y + (int64_t)b0 * n;
         int rc;
+        if (left >= 2) {
+            // 2 to 8 rows, K in whole super-blocks: decoded to fp32 in front of the fp32 matrix instruction
+            const int nf = left < 8 ? left : 8;
+            rc = launch_gemv_few(enc, w, xb, yb, nf, n, k);
+            if (rc < 0) return rc;
+            if (rc == 1) { b0 += nf; continue; }
+        }
         if (enc == ENC_Q4_K && g_q4k_rows_enable) {
             // 3 to 8 rows: the fp32 matrix-instruction kernel; 1 or 2: the row-streaming kernel
             const int nq = left < 8 ? left : 8;

@@ -598,3 +598,34 @@ def test_q4k_one_row_fixed_point_kernel_keeps_non_finite_activations_loud(hip_ba
     x[0, 128:192] = np.float32(1e-41) * rng.standard_normal(64).astype(np.float32)      # one group of subnormals
     got = gpu_matmul(hip_backend, torch_cuda, "Q4_K", packed, n, k, x)
     assert np.isfinite(got).all() and normalized_err(got, L.gemv("Q4_K", x, packed, n)) <= GEMV_TOL
+
+
+@pytest.mark.parametrize("enc", ENCS + MORE_ENCS)
+@pytest.mark.parametrize("n,k,m", [(1, 256, 2), (5, 512, 3), (67, 1280, 8), (130, 5120, 5), (33, 6400, 4), (70, 7168, 6), (1030, 4096, 4),
+                                   (300, 11008, 7), (9, 14336, 3), (40, 16640, 8)])
+def test_products_of_two_to_eight_rows_on_the_fp32_matrix_instruction(hip_backend, torch_cuda, enc, n, k, m):
+    """The few-rows kernel, forced: ragged quads, fewer super-blocks than a pass, passes shared by teams of waves (5, 7, 11 and
+    17 passes over four or eight waves), Q6_K rows on odd half words. Against float64 sums of the oracle's decoded weights: a
+    product passes fewer than 96 fp32 roundings (two of the decode, at most 32 sums per pass and three rounds of passes in a
+    lane, then the fold), each at most 2^-24 of the sum of magnitudes. An infinite scale at the end of row 0 stays in row 0."""
+    kx, bs = hip_backend, G.PACKED[enc][0]
+    packed = random_valid_blocks(enc, n * k // bs, 900 + n)
+    x = np.random.default_rng(n + k).standard_normal((m, k)).astype(np.float32)
+    w = L.dequant(enc, packed).reshape(n, k).astype(np.float64)
+    want, magnitude = x.astype(np.float64) @ w.T, np.abs(x).astype(np.float64) @ np.abs(w).T
+    try:
+        kx.set_tuning("gemv_few", 2)
+        got = gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0)
+        assert kx.last_kernel() == "packed_gemv_few_kernel"
+        assert (np.abs(got - want) <= 96 * 2.0 ** -24 * magnitude).all()
+        rows = packed.reshape(n, -1).copy()
+        d_off = G.PACKED[enc][2]
+        at = rows.shape[1] - G.PACKED[enc][1] + d_off
+        rows[0, at:at + 2] = np.array([np.inf], np.float16).view(np.uint8)
+        loud = gpu_matmul(kx, torch_cuda, enc, rows.reshape(-1), n, k, x, kind=0)
+        assert not np.isfinite(loud[:, 0]).any()
+        assert np.array_equal(loud[:, 1:], got[:, 1:])
+        kx.set_tuning("gemv_few", 0)                        # the kernels behind it, at the same sizes
+        assert normalized_err(gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0), want) <= GEMV_TOL
+    finally:
+        kx.set_tuning("gemv_few", 1)
