@@ -135,7 +135,7 @@ SKAINET_HIP_API int64_t skainet_hip_weight_nbytes(const skainet_hip_weight* w);
  *   - Q4_K, m = 3 .. 8 at K = 4096 and most other K above 2048: codes exact, an activation enters as bf16 hi + bf16 lo (16 to
  *     17 significant bits) on the bf16 matrix instructions, fp32 sums (2e-4 in the metric).
  *   - everything else (Q4_K m = 2 or other K, Q6_K, Q5_K, Q4_0, Q5_0, Q5_1, Q8_0 at other K or m): fp32 multiply-adds on
- *     decoded codes or decoded weights on the fp32 matrix instruction ("gemv_few"), the reference's exact-fp32 products in
+ *     decoded codes, or decoded weights on the fp32 matrix instruction or multiply-adds ("gemv_few"), the reference's exact-fp32 products in
  *     another summation order.
  *   skainet_hip_set_tuning("q4k_mfma_enable", 0) / ("q8_0_mfma_enable", 0) force the fp32 kernels at m = 1,
  *   ("gemv_few", 0) + ("q4k_wide_enable", 0) + ("q4k_quads_stream_enable", 0) + ("q4k_rows_enable", 0) the fp32 slot kernel at every m.
@@ -430,7 +430,7 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * and more instead of eight),
  * "q4k_mfma_window" (row quads the one-row integer matrix-core kernel keeps in flight per wave: 2 or 3,
  * 0 = chosen from K), "gemm_ksplit" (K splits of the MFMA GEMM,
- * 0 = automatic), "gemv_few" (products of 2 to 8 rows on the fp32 matrix instruction: 0 never, 1 where they are the faster ones,
+ * 0 = automatic), "gemv_few" (products of 1 to 8 rows by lanes that decode 64 weights at a time: 0 never, 1 where they are the faster ones,
  * 2 wherever they fit), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
  * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2), "gemm_wide" (1 / 0: force the 256-column / 128-column tile, -1 = chosen from the shape), "gemm_rows" (2 / 4: 128 / 256
  * activation rows per tile, 0 = chosen from the shape), "gemm_ksw" (the Q4_K kernel that splits K over the

@@ -254,8 +254,8 @@ int launch_gemv(int enc, const uint8_t* w, const float* x, int m, int k, int n, 
         const float* xb = x + (int64_t)b0 * k;
         float* yb = y + (int64_t)b0 * n;
         int rc;
-        if (left >= 2) {
-            // 2 to 8 rows, K in whole super-blocks: decoded to fp32 in front of the fp32 matrix instruction
+        {
+            // 1 to 8 rows, K in whole super-blocks, where its rule says so: lanes that decode 64 weights at a time
             const int nf = left < 8 ? left : 8;
             rc = launch_gemv_few(enc, w, xb, yb, nf, n, k);
             if (rc < 0) return rc;

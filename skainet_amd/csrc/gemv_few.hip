@@ -1,4 +1,4 @@
-// Packed-weight products of 2 to 8 activation rows (a few sequences decoded together, a draft), fp32 throughout:
+// Packed-weight products of 1 to 8 activation rows (a few sequences decoded together, a draft), fp32 throughout:
 //   y[b, o] = sum_j x[b, j] * dequant(W[o, j])      fp32 activations, weights decoded to fp32, fp32 products and sums.
 // Semantics: m rows = m scalar GEMVs of the reference's exact-fp32 kernels,
 //   skainet-backends/skainet-backend-cpu/src/commonMain/kotlin/sk/ainet/exec/kernel/PackedViewMatmulKernel.kt:69-108.
@@ -13,6 +13,8 @@
 //   * A slot is the 64 weights that one lane decodes (packed_lane64.h). Its activations (64 floats per four batch rows) stay
 //     in registers while the wave walks the workgroup's rows; 16 slots are a pass of 1024 elements of K and the waves of a
 //     workgroup share the passes. R quads of weight rows are requested ahead.
+//   * One and two rows would leave the instruction half empty: the vector unit multiplies, same lanes and loads (Q8_0
+//     2 x 10000 x 4096 13.9 us on the row kernel, 12 on the matrix instruction, 10.7 here).
 //   * The 16 blocks' sums fold inside a DPP row; the four DPP rows and the waves meet in LDS once, summed in a fixed order.
 #include "packed_lane64.h"
 
@@ -27,11 +29,14 @@ constexpr int FEW_MAX_WAVES = 8;      // two per SIMD: 256 registers each
 
 constexpr int FEW_STAGE_FLOATS = 2 * 16 * 68;      // two batch rows x 16 slots of 64 floats, each padded by four against bank conflicts
 
-// MB: batch rows in fours (1 or 2), R: quads in flight.
-template <class F, int MB, int R>
+// ROWS: batch rows computed (4 or 8 on the matrix instruction; 1 or 2 on the vector unit, every lane with the rows' activations of
+// its slot), R: quads in flight.
+template <class F, int ROWS, int R>
 __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                                              float* __restrict__ y, int m, int n, int k, int rows_per_wg) {
-    extern __shared__ __attribute__((aligned(16))) float few_smem[];      // [wave][FEW_STAGE_FLOATS], then [wave][row][DPP row][4 MB]
+    constexpr bool VECTOR = ROWS <= 2;
+    constexpr int MB = VECTOR ? 1 : ROWS / 4, NX = VECTOR ? ROWS : MB;    // batch rows in fours; sets of 64 activations in a lane
+    extern __shared__ __attribute__((aligned(16))) float few_smem[];      // [wave][FEW_STAGE_FLOATS], then [wave][row][DPP row][ROWS]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
     const int blk = lane >> 2, j = lane & 3, q = blk & 3;                 // a pass starts on a super-block: slot % 4 is the lane's own
     const int nsb = k >> 8, passes = (nsb + 3) >> 2;
@@ -40,7 +45,7 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
     const int nrows = min(n - r0, rows_per_wg), quads = (nrows + 3) >> 2;
     float4* const stage = reinterpret_cast<float4*>(few_smem + (size_t)wave * FEW_STAGE_FLOATS);
     float* const few_part = few_smem + (size_t)nwaves * FEW_STAGE_FLOATS;
-    float* const mine = few_part + (size_t)wave * rows_per_wg * 16 * MB;
+    float* const mine = few_part + (size_t)wave * rows_per_wg * 4 * ROWS;
 
     // Rounds of one pass per wave; where the last round has fewer passes than waves, several waves share one and its rows
     // (five waves would leave three of four SIMDs idle half the time: 4 x 30000 x 5120, Q4_0: 38 -> 27 us).
@@ -53,16 +58,17 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
         // The wave's activations: whole kilobytes of a batch row per load (a lane's own 64 floats would take a line per lane
         // and load, 128 KB of a CU's waves through a 32 KB L1: Q4_0 4 x 14336 x 4096 16.9 -> 14.2 us), the first four rows in
         // front of the weights, whose loads must not hold them up; then through LDS into the lanes' order, two rows at a time.
-        float4 xr[4][4];
+        constexpr int PAIR = ROWS < 2 ? ROWS : 2;
+        float4 xr[VECTOR ? PAIR : 4][4];
         auto load_x = [&](int four, int b0) __attribute__((always_inline)) {     // two rows
 #pragma unroll
-            for (int b = b0; b < b0 + 2; ++b)
+            for (int b = b0; b < b0 + PAIR; ++b)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)                               // past K and past m: copies of the last
                     xr[b][i] = *reinterpret_cast<const float4*>(x + (int64_t)min(4 * four + b, m - 1) * k + min(1024 * pass + 4 * (64 * i + lane), k - 4));
         };
         load_x(0, 0);
-        load_x(0, 2);
+        if constexpr (!VECTOR) load_x(0, 2);
         __builtin_amdgcn_sched_barrier(0);
         // super-blocks past the last are copies of it whose bytes and activations become zeros
         const int sb = 4 * pass + (blk >> 2);
@@ -74,14 +80,14 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
         };
         load(0, q0);
         __builtin_amdgcn_sched_barrier(0);
-        float xa[MB][64];
+        float xa[NX][64];
 #pragma unroll
         for (int four = 0; four < MB; ++four) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < (VECTOR ? 1 : 2); ++h) {
                 if (four) load_x(four, 2 * h);                            // two rows at a time: all eight at once would spill
 #pragma unroll
-                for (int b = 0; b < 2; ++b)
+                for (int b = 0; b < PAIR; ++b)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int f = 64 * i + lane;                      // float4 of the pass; slot f / 16
@@ -91,15 +97,21 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
                     }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");    // wave-private: LDS serves a wave's accesses in order
                 __builtin_amdgcn_wave_barrier();
-                if ((j >> 1) == h) {
+                auto take = [&](float (&d)[64], int row) __attribute__((always_inline)) {      // the lane's slot of a staged row
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
                         const int f = 64 * (blk >> 2) + (skn_elem<F::Q6>(q, u) >> 2);
-                        const float4* src = stage + (j & 1) * 272 + (f >> 4) * 17 + (f & 15);
+                        const float4* src = stage + row * 272 + (f >> 4) * 17 + (f & 15);
                         const float4 lo = src[0], hi = src[1];
-                        float* d = &xa[four][8 * u];
-                        d[0] = lo.x; d[1] = lo.y; d[2] = lo.z; d[3] = lo.w; d[4] = hi.x; d[5] = hi.y; d[6] = hi.z; d[7] = hi.w;
+                        d[8 * u] = lo.x; d[8 * u + 1] = lo.y; d[8 * u + 2] = lo.z; d[8 * u + 3] = lo.w;
+                        d[8 * u + 4] = hi.x; d[8 * u + 5] = hi.y; d[8 * u + 6] = hi.z; d[8 * u + 7] = hi.w;
                     }
+                };
+                if constexpr (VECTOR) {
+#pragma unroll
+                    for (int b = 0; b < ROWS; ++b) take(xa[b], b);
+                } else {
+                    if ((j >> 1) == h) take(xa[four], j & 1);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -111,49 +123,77 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
         for (int i = 1; i < R; ++i) load(i, min(q0 + i, q1 - 1));
         __builtin_amdgcn_sched_barrier(0);
         auto compute = [&](int slot, int quad) __attribute__((always_inline)) {
-            constexpr int NA = 4 / MB;                                    // independent sums per four batch rows
-            few_f32x4 acc[MB][NA];
-#pragma unroll
-            for (int b = 0; b < MB; ++b)
-#pragma unroll
-                for (int a = 0; a < NA; ++a) acc[b][a] = few_f32x4{0.f, 0.f, 0.f, 0.f};
             if (ragged && !in) __builtin_memset(&raw[slot], 0, sizeof(raw[slot]));      // zero times an infinite scale would be a NaN
             const typename F::Scales sc = F::scales(raw[slot], q);
-            // Matrix and vector instructions do not overlap here and changing from one to the other costs 1 to 2 ns
-            // (4x4x1 alone 4.2 ns; one and two multiply-adds in turn 7.8, of which the latter 1.9): the decode of 16 or 32
-            // weights and their products stay apart (Q4_0, 4 x 14336 x 4096: 14.2 -> 12.2 us).
-            constexpr int G = MB == 1 ? 4 : 2;                            // steps of eight weights at a time
-            auto step = [&](auto uc) __attribute__((always_inline)) {
-                constexpr int U = decltype(uc)::value;
-                SknF32 o[G];
-                F::template decode<U>(raw[slot], sc, o[0]);
-                F::template decode<U + 1>(raw[slot], sc, o[1]);
-                if constexpr (G == 4) { F::template decode<U + 2>(raw[slot], sc, o[2]); F::template decode<U + 3>(raw[slot], sc, o[3]); }
-                __builtin_amdgcn_sched_barrier(0);
+            float* const dst = mine + ((4 * quad + j) * 4 + (lane >> 4)) * ROWS;          // the four blocks of a DPP row fold in registers
+            if constexpr (VECTOR) {
+                float acc[ROWS][4];
 #pragma unroll
-                for (int e = 0; e < 8 * G; ++e)
+                for (int b = 0; b < ROWS; ++b) acc[b][0] = acc[b][1] = acc[b][2] = acc[b][3] = 0.f;
+                auto step = [&](auto uc) __attribute__((always_inline)) {
+                    constexpr int U = decltype(uc)::value;
+                    SknF32 o;
+                    F::template decode<U>(raw[slot], sc, o);
 #pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        acc[b][e % NA] = __builtin_amdgcn_mfma_f32_4x4x1f32(xa[b][8 * U + e], o[e >> 3].w[e & 7], acc[b][e % NA], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            step(std::integral_constant<int, 0>{});
-            if constexpr (G == 2) step(std::integral_constant<int, 2>{});
-            step(std::integral_constant<int, 4>{});
-            if constexpr (G == 2) step(std::integral_constant<int, 6>{});
-            // element e of lane (blk, j): batch row e, weight row j, K slot blk; the four blocks of a DPP row fold here
+                    for (int e = 0; e < 8; ++e)
 #pragma unroll
-            for (int b = 0; b < MB; ++b) {
-                few_f32x4 s = acc[b][0] + acc[b][1];
-                if constexpr (NA == 4) s += acc[b][2] + acc[b][3];
+                        for (int b = 0; b < ROWS; ++b) acc[b][e & 3] = fmaf(xa[b][8 * U + e], o.w[e], acc[b][e & 3]);
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
+                step(std::integral_constant<int, 2>{}); step(std::integral_constant<int, 3>{});
+                step(std::integral_constant<int, 4>{}); step(std::integral_constant<int, 5>{});
+                step(std::integral_constant<int, 6>{}); step(std::integral_constant<int, 7>{});
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s[e] += dpp_row_move<0x128>(s[e]);                    // row_ror:8
-                    s[e] += dpp_row_move<0x124>(s[e]);                    // row_ror:4
+                for (int b = 0; b < ROWS; ++b) {
+                    float s = (acc[b][0] + acc[b][1]) + (acc[b][2] + acc[b][3]);
+                    s += dpp_row_move<0x128>(s);                          // row_ror:8
+                    s += dpp_row_move<0x124>(s);                          // row_ror:4
+                    if ((lane & 12) == 0) dst[b] = round == 0 ? s : dst[b] + s;
                 }
-                if ((lane & 12) == 0) {
-                    few_f32x4* dst = reinterpret_cast<few_f32x4*>(mine + ((4 * quad + j) * 4 + (lane >> 4)) * 4 * MB + 4 * b);
-                    *dst = round == 0 ? s : *dst + s;
+            } else {
+                constexpr int NA = 4 / MB;                                // independent sums per four batch rows
+                few_f32x4 acc[MB][NA];
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int a = 0; a < NA; ++a) acc[b][a] = few_f32x4{0.f, 0.f, 0.f, 0.f};
+                // Matrix and vector instructions do not overlap here and changing from one to the other costs 1 to 2 ns
+                // (4x4x1 alone 4.2 ns; one and two multiply-adds in turn 7.8, of which the latter 1.9): the decode of 16 or 32
+                // weights and their products stay apart (Q4_0, 4 x 14336 x 4096: 14.2 -> 12.2 us).
+                constexpr int G = MB == 1 ? 4 : 2;                        // steps of eight weights at a time
+                auto step = [&](auto uc) __attribute__((always_inline)) {
+                    constexpr int U = decltype(uc)::value;
+                    SknF32 o[G];
+                    F::template decode<U>(raw[slot], sc, o[0]);
+                    F::template decode<U + 1>(raw[slot], sc, o[1]);
+                    if constexpr (G == 4) { F::template decode<U + 2>(raw[slot], sc, o[2]); F::template decode<U + 3>(raw[slot], sc, o[3]); }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 8 * G; ++e)
+#pragma unroll
+                        for (int b = 0; b < MB; ++b)
+                            acc[b][e % NA] = __builtin_amdgcn_mfma_f32_4x4x1f32(xa[b][8 * U + e], o[e >> 3].w[e & 7], acc[b][e % NA], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                step(std::integral_constant<int, 0>{});
+                if constexpr (G == 2) step(std::integral_constant<int, 2>{});
+                step(std::integral_constant<int, 4>{});
+                if constexpr (G == 2) step(std::integral_constant<int, 6>{});
+                // element e of lane (blk, j): batch row e, weight row j, K slot blk
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    few_f32x4 s = acc[b][0] + acc[b][1];
+                    if constexpr (NA == 4) s += acc[b][2] + acc[b][3];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        s[e] += dpp_row_move<0x128>(s[e]);                // row_ror:8
+                        s[e] += dpp_row_move<0x124>(s[e]);                // row_ror:4
+                    }
+                    if ((lane & 12) == 0) {
+                        few_f32x4* const d4 = reinterpret_cast<few_f32x4*>(dst) + b;
+                        *d4 = round == 0 ? s : *d4 + s;
+                    }
                 }
             }
         };
@@ -170,19 +210,19 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
             if (t + i < q1) compute(i, t + i);
     }
     __syncthreads();
-    for (int at = threadIdx.x; at < rows_per_wg * 4 * MB; at += blockDim.x) {
+    for (int at = threadIdx.x; at < rows_per_wg * ROWS; at += blockDim.x) {
         const int row = at % rows_per_wg, b = at / rows_per_wg;           // consecutive threads: consecutive outputs of a batch row
         if (row >= nrows || b >= m) continue;
         float s = 0.f;
         for (int v = 0; v < nwaves; ++v) {
-            const float* src = few_part + (((size_t)v * rows_per_wg + row) * 4) * 4 * MB + b;
-            s += (src[0] + src[4 * MB]) + (src[8 * MB] + src[12 * MB]);
+            const float* src = few_part + (((size_t)v * rows_per_wg + row) * 4) * ROWS + b;
+            s += (src[0] + src[ROWS]) + (src[2 * ROWS] + src[3 * ROWS]);
         }
         y[(int64_t)b * n + r0 + row] = s;
     }
 }
 
-template <class F, int MB, int R>
+template <class F, int ROWS, int R>
 static int launch_few_rows(const uint8_t* w, const float* x, float* y, int m, int n, int k) {
     const int passes = (k / 256 + 3) / 4;
     // a wave per pass up to four and for eight; else rounds of four or eight and a shared rest, so that the SIMDs get the same
@@ -191,52 +231,70 @@ static int launch_few_rows(const uint8_t* w, const float* x, float* y, int m, in
     const int resident = num_cus() * (FEW_MAX_WAVES / nwaves);
     const int turns = (int)(((int64_t)n + (int64_t)resident * FEW_MAX_ROWS - 1) / ((int64_t)resident * FEW_MAX_ROWS));
     const int rows = (int)(((int64_t)n + (int64_t)resident * turns - 1) / ((int64_t)resident * turns) + 3) & ~3;      // at most FEW_MAX_ROWS
-    const size_t smem = (size_t)nwaves * (FEW_STAGE_FLOATS + rows * 16 * MB) * sizeof(float);
-    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&packed_gemv_few_kernel<F, MB, R>), (size_t)FEW_MAX_WAVES * (FEW_STAGE_FLOATS + FEW_MAX_ROWS * 16 * MB) * sizeof(float));
+    const size_t smem = (size_t)nwaves * (FEW_STAGE_FLOATS + rows * 4 * ROWS) * sizeof(float);
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&packed_gemv_few_kernel<F, ROWS, R>), (size_t)FEW_MAX_WAVES * (FEW_STAGE_FLOATS + FEW_MAX_ROWS * 4 * ROWS) * sizeof(float));
     note_kernel("packed_gemv_few_kernel");
-    packed_gemv_few_kernel<F, MB, R><<<dim3((n + rows - 1) / rows), dim3(64 * nwaves), smem, current_stream()>>>(w, x, y, m, n, k, rows);
+    packed_gemv_few_kernel<F, ROWS, R><<<dim3((n + rows - 1) / rows), dim3(64 * nwaves), smem, current_stream()>>>(w, x, y, m, n, k, rows);
     SKH_CHECK(hipGetLastError());
     return 1;
 }
-// Three quads ahead, or two beside the activations of eight rows. (Four to six for four rows: the same to 6 % slower.)
+// Quads ahead: what the registers hold beside the activations. (Four to six for four rows: the same to 6 % slower.)
 template <class F>
 static int launch_few(const uint8_t* w, const float* x, float* y, int m, int n, int k) {
-    return m > 4 ? launch_few_rows<F, 2, 2>(w, x, y, m, n, k) : launch_few_rows<F, 1, 3>(w, x, y, m, n, k);
+    if (m == 1) return launch_few_rows<F, 1, 4>(w, x, y, m, n, k);
+    if (m == 2) return launch_few_rows<F, 2, 2>(w, x, y, m, n, k);
+    return m > 4 ? launch_few_rows<F, 8, 2>(w, x, y, m, n, k) : launch_few_rows<F, 4, 3>(w, x, y, m, n, k);
 }
 
 static std::atomic<int> g_gemv_few{1};      // 0 never, 1 by rule, 2 wherever it fits
 void set_gemv_few(int v) { g_gemv_few = v; }
 
-// Where this kernel is faster than the row kernel, measured over n 1500 to 32000, K 512 to 14336 (row kernel -> this one, us).
-// Three rows and more of a format of 32-element blocks: everywhere (Q8_0 4 x 4096 x 11008 26.1 -> 14.9, 8 x 32000 x 4096
-// 111 -> 41; Q4_0 3 x 4000 x 512 5.8 -> 4.3). The row kernel holds its own where it multiplies little and loads well:
-//   * two rows, half of this kernel's products for nothing: only with enough rows of weights per wave to cover the start, and
-//     K beyond the row kernel's eight full waves (Q5_K 2 x 10000 x 12800 44.5 -> 33.4, but x 8192 16.0 -> 19.3), or for the
-//     32-element blocks its two (Q8_0 2 x 14336 x 4096 17.3 -> 15.0, x 2048 7.7 -> 9.5);
-//   * the K-quants, whose lanes decode more per byte: few weight rows with a K that takes this kernel a shared round (Q6_K
-//     5 x 1500 x 7168 13.2 -> 15.0, x 8192 13.6 -> 11.4), and Q6_K up to four rows outside 4096 < K <= 6144 and K > 8192
-//     (4 x 14336 x 4096 15.9 -> 16.8, 3 x 10000 x 11008 49.5 -> 30.4);
-//   * Q4_K has batched kernels of its own (K 4096; any K): this one on rows shorter than a wave's share there (8 x 30000 x 512
-//     35.5 -> 12.6, 3 x 4000 x 2048 6.3 -> 5.5; 4 x 10000 x 2560 8.4 -> 9.4) and on few long ones (4 x 2048 x 14336 15.3 -> 10.9;
-//     4 x 10000 x 14336 27.3 -> 28.3).
+// Where this kernel is faster than the ones behind it (row kernel, for one row of 32-element blocks the streaming kernel), measured
+// over n 1500 to 30000, K 512 to 14336 in us, theirs -> this one's. It is where they multiply much or load badly: many activation
+// rows, rows of few kilobytes, K that leaves their waves unequal shares (more than 8192, 4096 to 5120). They hold their own with
+// few products on full waves, and where K takes this kernel a second round that few waves share (6144 to 8192).
+//   32-element blocks, 3 to 8 rows: everywhere (Q8_0 4 x 4096 x 11008 26.1 -> 14.6, 8 x 32000 x 4096 111 -> 41)
+//     2 rows: Q4_0 everywhere (4000 x 4096 7.2 -> 5.3), the others outside 6144 < K <= 8192 (Q8_0 10000 x 4096 13.9 -> 10.7, x
+//     7168 16.2 -> 17.2)
+//     1 row: many weight rows (Q5_0 30000 x 4096 27.7 -> 20.7; Q8_0 has the integer kernel at multiples of 1024), and for formats of
+//     4 and 5 bits a K beyond the streaming kernel's (Q4_0 4000 x 11008 11.7 -> 9.9, Q5_0 10000 x 8192 15.2 -> 15.8)
+//   Q6_K, Q5_K: their decode costs more, so 5 to 8 rows (Q6_K 8 x 4096 x 11008 53 -> 24; 5 x 1500 x 7168 13.2 -> 15.0), 3 and 4 of Q5_K,
+//     and below that rows that leave the row kernel's lanes idle (Q6_K 1 x 30000 x 768 18.0 -> 10.0, 2 x 10000 x 11008 36.6 -> 25.6;
+//     4 x 14336 x 4096 15.9 -> 16.8)
+//   Q4_K has batched kernels of its own: rows shorter than a wave's share there (8 x 30000 x 512 35.5 -> 12.6) and few long ones (4 x 2048
+//     x 14336 15.3 -> 10.9; 4 x 10000 x 14336 27.3 -> 28.3).
+// Besides: rows go in fours per workgroup, so a little more than 16 per CU costs a quarter (Q6_K 4 x 4147 x 6144 13.6 -> 16.2, x 4000
+// 12.1 -> 12.2), and products of 4 us are as long as their launch on either side (within 0.3 us).
 static bool few_by_rule(int enc, int m, int n, int k) {
-    const bool block32 = block_elems(enc) == 32, many = n >= 12 * num_cus();
+    const int cus = num_cus();
+    const bool many = n >= 12 * cus, lots = n >= 48 * cus, uneven = n > 16 * cus && n < 24 * cus;
     if (enc == ENC_Q4_K) {
-        if (m == 2) return many && k <= 1280;
-        return k <= 2048 || (n < 20 * num_cus() && k > 4096 && (k <= 5120 || k > 7168));
+        if (m == 1) return false;
+        if (m == 2 && k <= 4096) return many && k <= 2048;
+        return k <= 2048 || (k > 4096 && (k <= 5120 || (n < 16 * cus && (k > 7168 || (m == 2 && k <= 6144)))));
     }
-    if (m == 2) return many && (k > 8192 || (block32 && k > 2048 && k <= 5120));
-    if (block32) return true;
-    if (m >= 5) return many || k <= 4096 || (k > 7168 && k <= 12288);
-    if (enc == ENC_Q5_K) return many || k <= 4096;
-    return k <= 768 || (many && (k > 8192 || (k > 4096 && k <= 6144)));
+    if (block_elems(enc) == 32) {
+        if (m >= 3) return true;
+        if (m == 2) {
+            if (k <= 1024) return many;
+            if (enc == ENC_Q8_0 && k <= 2048) return !lots;
+            return k <= 4096 || (n >= 4 * cus && (k <= 6144 || (k > 8192 && (k <= 12288 || !lots))));
+        }
+        if (k <= 4096) return lots && (enc != ENC_Q8_0 || (k % 1024 != 0 && (k < 1024 || k > 2048)));
+        return many && !lots && enc != ENC_Q8_0 && (k <= 6144 || k > 8192);
+    }
+    if (m >= 5) return many || k <= 4096 || (k > 7168 && k <= 11264);
+    if (m >= 3 && enc == ENC_Q5_K) return k <= 4096 || (many && !(uneven && k <= 8192));
+    if (!many) return m >= 2 && k <= 768 && n >= 4 * cus;
+    if (m == 1) return enc == ENC_Q6_K ? k <= 768 || (k <= 1792 && n >= 32 * cus) : k > 8192 && k <= 12288 && !lots;
+    return k <= 768 || (k > 8192 && (k <= 12288 || !lots)) || (k > 4096 && k <= (m == 2 ? 5120 : 6144) && !uneven);
 }
 
 // Returns 1 when this kernel took the product, 0 when the row kernel is the faster one or the shape is outside its range, -1 on
 // a launch error.
 int launch_gemv_few(int enc, const uint8_t* w, const float* x, float* y, int m, int n, int k) {
     const int mode = g_gemv_few.load();
-    if (!mode || m < 2 || m > 8 || n < 1 || k < 256 || k % 256 != 0) return 0;
+    if (!mode || m < 1 || m > 8 || n < 1 || k < 256 || k % 256 != 0) return 0;
     if ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) return 0;
     if ((uint64_t)n * (uint64_t)(k / block_elems(enc)) * block_bytes(enc) >= ((uint64_t)1 << 32)) return 0;      // 32-bit byte offsets
     if (mode == 1 && !few_by_rule(enc, m, n, k)) return 0;

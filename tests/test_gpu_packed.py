@@ -602,8 +602,9 @@ def test_q4k_one_row_fixed_point_kernel_keeps_non_finite_activations_loud(hip_ba
 
 @pytest.mark.parametrize("enc", ENCS + MORE_ENCS)
 @pytest.mark.parametrize("n,k,m", [(1, 256, 2), (5, 512, 3), (67, 1280, 8), (130, 5120, 5), (33, 6400, 4), (70, 7168, 6), (1030, 4096, 4),
-                                   (300, 11008, 7), (9, 14336, 3), (40, 16640, 8)])
-def test_products_of_two_to_eight_rows_on_the_fp32_matrix_instruction(hip_backend, torch_cuda, enc, n, k, m):
+                                   (300, 11008, 7), (9, 14336, 3), (40, 16640, 8), (1, 256, 1), (70, 3328, 1), (1030, 5120, 1),
+                                   (21, 11008, 2), (6, 16640, 1)])
+def test_products_of_one_to_eight_rows_by_lanes_that_decode_64_weights(hip_backend, torch_cuda, enc, n, k, m):
     """The few-rows kernel, forced: ragged quads, fewer super-blocks than a pass, passes shared by teams of waves (5, 7, 11 and
     17 passes over four or eight waves), Q6_K rows on odd half words. Against float64 sums of the oracle's decoded weights: a
     product passes fewer than 96 fp32 roundings (two of the decode, at most 32 sums per pass and three rounds of passes in a
