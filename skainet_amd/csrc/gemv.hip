@@ -175,6 +175,7 @@ void set_gemm_frag_waves(int v);
 void set_gemm_frag_gm(int v);
 void set_sdpa_prefill_mfma(int v);
 void set_sdpa_prefill_teams(int v);
+void set_sdpa_prefill_splits(int v);
 void set_sdpa_decode_split_keys(int v);
 void set_q4k_ksplit_enable(int v);
 void set_q4k_mfma_enable(int v);
@@ -224,6 +225,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "gemm_frag_waves")) { set_gemm_frag_waves(value); return 0; }
     if (!strcmp(key, "gemm_frag_gm")) { set_gemm_frag_gm(value); return 0; }
     if (!strcmp(key, "sdpa_prefill_mfma")) { set_sdpa_prefill_mfma(value); return 0; }
+    if (!strcmp(key, "sdpa_prefill_splits")) { set_sdpa_prefill_splits(value); return 0; }
     if (!strcmp(key, "sdpa_prefill_teams")) { set_sdpa_prefill_teams(value); return 0; }
     if (!strcmp(key, "q4k_ksplit_enable")) { set_q4k_ksplit_enable(value); return 0; }
     if (!strcmp(key, "q4k_mfma_enable")) { set_q4k_mfma_enable(value); return 0; }

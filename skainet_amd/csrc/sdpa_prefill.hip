@@ -13,7 +13,7 @@
 // the reference's arithmetic is kept as it stands: every key of the sequence takes part, an excluded one at -1e30
 // plus its mask value (the mask is added to every score), so no key block is skipped.
 //
-// Two launches:
+// Two launches (three where keys are split over workgroups, see the kernel):
 //   1. kv_to_bf16_kernel: K -> bf16 [kv head][key][D], V -> bf16 transposed [kv head][D][key], keys padded with
 //      zeros to a multiple of 64. (The PV product contracts over keys, and an MFMA operand wants 8 consecutive
 //      contraction values per lane: V has to be read along keys, hence the transpose, done once per call.)
@@ -99,6 +99,9 @@ struct PrefillParams {
     int heads_per_wg;      // 1, 2 or 4 query heads of one KV head per workgroup
     const float* mask;         // additive mask or null; dims 1 or the full extent (heads: 1, kv_heads or heads)
     int mask_b, mask_h, mask_q, mask_k;
+    int splits;                // workgroups that share a query group's keys (one team only)
+    float* part;               // [row][splits][D] unnormalised outputs, row = (b, head, query); splits > 1 only
+    float* ml;                 // [row][splits][2] running maximum (in units of ln 2) and sum
     int out_rows;              // 0: out is [batch, heads, seq_q, D]; 1: [batch, seq_q, heads, D], token rows of a projection's input
 };
 
@@ -136,7 +139,9 @@ __device__ __forceinline__ void pf_store_block(const pf_u32x4 (&kreg)[PF_KB * (D
 }
 
 // TEAMS 2: the paired form described above. TEAMS 1: one query group per workgroup of four waves (two workgroups per
-// CU), for calls whose paired grid would leave CUs without a workgroup.
+// CU), for calls whose paired grid would leave CUs without a workgroup; where that leaves CUs idle too, several workgroups
+// share a group's keys (splits) and sdpa_prefill_merge_kernel puts their outputs together: what bounds such a call is the
+// chain of blocks a workgroup walks.
 template <int D, int TEAMS>
 __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_kernel(PrefillParams p) {
     constexpr int PF_THREADS = 256 * TEAMS;
@@ -160,7 +165,7 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
     const int head_groups = per_kv / hpw;
     const int kvh = blockIdx.y / head_groups;
     const int head = kvh * per_kv + (blockIdx.y % head_groups) * hpw + wave % hpw;
-    const int b = blockIdx.z;
+    const int b = TEAMS == 1 ? blockIdx.z / p.splits : blockIdx.z;
     // query groups (a team's share of the query positions). Causal over the whole prefix: team 0 takes group G - 1 - i,
     // team 1 group i (equal work in every workgroup). Under a sliding window, or without the causal rule, every group
     // has about the same work and neighbours share most of their key blocks: groups 2 i + 1 and 2 i. With an odd number
@@ -205,8 +210,14 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
     const bool all_keys = wg_uniform || masked;
     const int e_beg = first_of(group_first(g_early)) / PF_KB, e_end = (end_of(group_last(g_early)) + PF_KB - 1) / PF_KB;
     const int l_beg = first_of(group_first(g_late)) / PF_KB, l_end = (end_of(group_last(g_late)) + PF_KB - 1) / PF_KB;
-    const int blk_begin = all_keys ? 0 : min(e_beg, l_beg);
-    const int nblocks = all_keys ? (p.seq_kv + PF_KB - 1) / PF_KB : max(max(e_end, l_end), blk_begin);
+    int blk_begin = all_keys ? 0 : min(e_beg, l_beg);
+    int nblocks = all_keys ? (p.seq_kv + PF_KB - 1) / PF_KB : max(max(e_end, l_end), blk_begin);
+    const int split = TEAMS == 1 ? blockIdx.z % p.splits : 0;
+    if (TEAMS == 1 && p.splits > 1) {                                       // this workgroup's share of the group's blocks (may be none)
+        const int share = (nblocks - blk_begin + p.splits - 1) / p.splits;
+        blk_begin += split * share;
+        nblocks = min(nblocks, blk_begin + share);
+    }
     auto needed = [&](int blk) { return all_keys || (blk >= e_beg && blk < e_end) || (blk >= l_beg && blk < l_end); };
     auto next_needed = [&](int blk) { int nb = blk + 1; while (nb < nblocks && !needed(nb)) ++nb; return nb; };
     // this wave's 32 positions: the keys any of them attends, and the keys all of them attend
@@ -364,6 +375,20 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
 
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    if (TEAMS == 1 && p.splits > 1) {
+        if (my_q < p.seq_q) {
+            const int64_t at = (((int64_t)b * p.heads + head) * p.seq_q + my_q) * p.splits + split;
+            float* op = p.part + at * D;
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    *reinterpret_cast<float4*>(op + 32 * i + 8 * e4 + 4 * h) =
+                        make_float4(oacc[i][4 * e4], oacc[i][4 * e4 + 1], oacc[i][4 * e4 + 2], oacc[i][4 * e4 + 3]);
+            if (h == 0) *reinterpret_cast<float2*>(p.ml + 2 * at) = make_float2(m_run, l_tot);
+        }
+        return;
+    }
     if (my_q < p.seq_q && team_active) {
         float* op = p.out + (p.out_rows ? (((int64_t)b * p.seq_q + my_q) * p.heads + head) : (((int64_t)b * p.heads + head) * p.seq_q + my_q)) * D;
 #pragma unroll
@@ -377,12 +402,63 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
     }
 }
 
+// The splits of a row put together: thread = (row, four elements). A split without keys has a maximum of -inf and takes no part.
+template <int D>
+__global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(PrefillParams p, int64_t rows) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, row = t / (D / 4);
+    const int d = 4 * (int)(t % (D / 4));
+    if (row >= rows) return;
+    const float2* ml = reinterpret_cast<const float2*>(p.ml) + row * p.splits;
+    float m = -INFINITY;
+    for (int i = 0; i < p.splits; ++i) m = fmaxf(m, ml[i].x);
+    const float ref = m == -INFINITY ? 0.f : m;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    float l = 0.f;
+    for (int i = 0; i < p.splits; ++i) {
+        const float2 s = ml[i];
+        const float c = __builtin_amdgcn_exp2f(s.x - ref);                  // -inf: 0
+        const float4 v = *reinterpret_cast<const float4*>(p.part + (row * p.splits + i) * D + d);
+        o.x = fmaf(c, v.x, o.x); o.y = fmaf(c, v.y, o.y); o.z = fmaf(c, v.z, o.z); o.w = fmaf(c, v.w, o.w);
+        l = fmaf(c, s.y, l);
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    int64_t to = row;
+    if (p.out_rows) {
+        const int64_t qi = row % p.seq_q, bh = row / p.seq_q;
+        to = (bh / p.heads * p.seq_q + qi) * p.heads + bh % p.heads;
+    }
+    *reinterpret_cast<float4*>(p.out + to * D + d) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+}
+
 void* kernel_workspace(size_t bytes);   // shim.hip: per-thread scratch, grown on demand
 
 static std::atomic<int> g_prefill_mfma{1};
 void set_sdpa_prefill_mfma(int v) { g_prefill_mfma = v; }
+static std::atomic<int> g_prefill_splits{0};  // 0: chosen from the shape
+void set_sdpa_prefill_splits(int v) { if (v >= 0 && v <= 32) g_prefill_splits = v; }
 static std::atomic<int> g_prefill_teams{0};   // 0: chosen from the grid, 1: one query group per workgroup, 2: paired groups
 void set_sdpa_prefill_teams(int v) { if (v >= 0 && v <= 2) g_prefill_teams = v; }
+
+// How many workgroups share a query group's keys, where one group per workgroup leaves CUs idle: a chunk of a long prompt, few
+// heads. Estimates in us, fitted to 22 shapes of 1 to 64 heads, 16 to 3000 queries, 64 to 5000 keys at 1 to 32 splits: a block of
+// 64 keys takes a workgroup 1.8 (D 128) or 1.15 (D 64), half as much again with two workgroups on a CU; splitting costs the
+// merging launch and the partial outputs, written and read at 6 bytes per ps. Measured with one and with the chosen number: 32
+// heads over 8, 64 queries on 2048 keys 67.2 -> 26.4 us, 128 on 2176 69.6 -> 30.2; 8 heads, 1024 on 1024 40.6 -> 26.8; one head, 3000 on
+// 3000 85.3 -> 29.1; 32 heads, 300 on 300 stays (19.2, 22.9 with two).
+static int prefill_splits(int64_t wgs, int64_t rows, int head_dim, int seq_kv, int q_per_group, int window, int right_context, int batch) {
+    const int64_t keys = window > 0 ? min((int64_t)seq_kv, (int64_t)window + right_context + q_per_group) : seq_kv;
+    const int blocks = (int)((keys + PF_KB - 1) / PF_KB);
+    const int most = (int)min(min((int64_t)32, 2 * (int64_t)num_cus() / wgs), (int64_t)min(blocks, 65535 / batch));
+    if (g_prefill_splits.load() > 0) return max(1, min(most, g_prefill_splits.load()));
+    const double block_us = head_dim == 64 ? 1.15 : 1.8;
+    int splits = 1;
+    double best = 0.95 * block_us * blocks;
+    for (int n = 2; n <= most; ++n) {
+        const double t = block_us * ((blocks + n - 1) / n) * (wgs * n > num_cus() ? 1.5 : 1.0) + 8.0 + 8.0 * rows * n * (head_dim + 2) / 6e6;
+        if (t < best) { best = t; splits = n; }
+    }
+    return splits;
+}
 
 template <int D>
 static int launch_prefill_d(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
@@ -390,22 +466,25 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
                             const int32_t* lengths, const float* mask, int mask_b, int mask_h, int mask_q, int mask_k, int out_rows) {
     const int spad = (seq_kv + PF_KB - 1) / PF_KB * PF_KB;
     const size_t elems = (size_t)batch * kv_heads * spad * D;
-    __bf16* ws = static_cast<__bf16*>(kernel_workspace(2 * elems * sizeof(__bf16)));
-    if (!ws) return -1;
-    __bf16 *kb = ws, *vt = ws + elems;
     hipStream_t s = current_stream();
-    kv_to_bf16_kernel<D><<<dim3(spad / PF_KB, kv_heads, batch), dim3(256), 0, s>>>(k, v, kb, vt, kv_heads, seq_kv, kv_capacity, spad);
-    SKH_CHECK(hipGetLastError());
     const int per_kv = heads / kv_heads;
     const int hpw = per_kv % 4 == 0 ? 4 : (per_kv % 2 == 0 ? 2 : 1);
     const int q_per_group = (4 / hpw) * PF_QW;
     const int ngroups = (seq_q + q_per_group - 1) / q_per_group;
-    PrefillParams p{q, kb, vt, out, heads, kv_heads, seq_q, seq_kv, spad, scale * 1.4426950408889634f, causal, window, right_context, lengths, hpw,
-                    mask, mask_b, mask_h, mask_q, mask_k, out_rows};
     // paired query groups where that still gives every CU a workgroup, else one group per (smaller) workgroup
     const int64_t paired_wgs = (int64_t)((ngroups + 1) / 2) * kv_heads * (per_kv / hpw) * batch;
     const bool paired = g_prefill_teams.load() == 0 ? paired_wgs >= num_cus() : g_prefill_teams.load() == 2;
-    const dim3 grid(paired ? (ngroups + 1) / 2 : ngroups, kv_heads * (per_kv / hpw), batch);
+    const size_t rows = (size_t)batch * heads * seq_q;
+    const int splits = paired ? 1 : prefill_splits((int64_t)ngroups * kv_heads * (per_kv / hpw) * batch, (int64_t)rows, D, seq_kv, q_per_group, window, right_context, batch);
+    uint8_t* ws = static_cast<uint8_t*>(kernel_workspace(2 * elems * sizeof(__bf16) + (splits > 1 ? rows * splits * (D + 2) * sizeof(float) : 0)));
+    if (!ws) return -1;
+    __bf16 *kb = reinterpret_cast<__bf16*>(ws), *vt = kb + elems;
+    float* part = reinterpret_cast<float*>(vt + elems);
+    kv_to_bf16_kernel<D><<<dim3(spad / PF_KB, kv_heads, batch), dim3(256), 0, s>>>(k, v, kb, vt, kv_heads, seq_kv, kv_capacity, spad);
+    SKH_CHECK(hipGetLastError());
+    PrefillParams p{q, kb, vt, out, heads, kv_heads, seq_q, seq_kv, spad, scale * 1.4426950408889634f, causal, window, right_context, lengths, hpw,
+                    mask, mask_b, mask_h, mask_q, mask_k, splits, part, part + rows * splits * D, out_rows};
+    const dim3 grid(paired ? (ngroups + 1) / 2 : ngroups, kv_heads * (per_kv / hpw), batch * splits);
     constexpr size_t smem = sizeof(__bf16) * (2 * PF_KB * (D + 8) + 2 * D * (PF_KB + 8));
     note_kernel("sdpa_prefill_kernel");
     if (paired) {
@@ -416,6 +495,10 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
         sdpa_prefill_kernel<D, 1><<<grid, dim3(256), smem, s>>>(p);
     }
     SKH_CHECK(hipGetLastError());
+    if (splits > 1) {
+        sdpa_prefill_merge_kernel<D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0, s>>>(p, (int64_t)rows);
+        SKH_CHECK(hipGetLastError());
+    }
     return 1;
 }
 

@@ -576,3 +576,45 @@ def test_thread_release_frees_and_regrows_scratch(hip_backend, torch_cuda):
     assert np.array_equal(results["before"][0], results["after"][0])
     assert np.array_equal(results["before"][1], results["after"][1])
     assert results["freed"] >= 64 << 20, results["freed"]
+
+
+@pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv,causal,window,rc,lengths,mask_dims", [
+    (1, 8, 2, 128, 17, 700, True, 0, 0, None, None),                  # a chunk of a long prompt: one ragged query group
+    (1, 2, 2, 64, 300, 300, True, 0, 0, None, None),                  # early groups have fewer blocks than there are splits
+    (2, 6, 3, 64, 64, 513, False, 0, 0, [513, 70], None),             # one key in the last block; a sequence whose keys end in the first split
+    (1, 4, 1, 128, 40, 640, True, 100, 3, None, None),                # a window inside two or three blocks
+    (3, 4, 4, 64, 130, 130, True, 50, 0, [130, 40, 0], None),         # queries without a key: every key equally, over all splits
+    (2, 4, 2, 128, 33, 260, True, 0, 0, [260, 0], (2, 4, 33, 260)),   # an additive mask, -1e30 + mask where no key is left
+])
+def test_attention_prefill_with_the_keys_split_over_workgroups(hip_backend, torch_cuda, batch, heads, kv_heads, d, sq, skv, causal, window,
+                                                               rc, lengths, mask_dims):
+    """Several workgroups share a query group's keys and a second launch merges their outputs: 2, 3 and as many splits as there
+    are blocks, against the oracle at the bounds of the unsplit kernel, and as token rows against the same call unsplit (weights
+    are rounded to bf16 against another running maximum: 2^-8 of a convex combination of values, at most the largest one)."""
+    rng = np.random.default_rng(sq * skv + d)
+    q = rng.standard_normal((batch, heads, sq, d)).astype(np.float32)
+    k = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
+    v = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
+    scale = float(1 / np.sqrt(d))
+    ln = None if lengths is None else np.asarray(lengths, np.int32)
+    mask = None if mask_dims is None else (rng.standard_normal(mask_dims) * 2).astype(np.float32)
+    want = L.sdpa(q, k, v, scale, causal, window, rc, ln, mask)
+    try:
+        hip_backend.set_tuning("sdpa_prefill_teams", 1)
+        for splits in (1, 2, 3, 32):
+            hip_backend.set_tuning("sdpa_prefill_splits", splits)
+            got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, scale, causal, window, rc, ln, mask)
+            assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+            assert np.isfinite(got).all()
+            assert normalized_err(got, want, eps=1.0) <= 2e-2
+            assert np.sqrt(np.mean((got - want) ** 2)) <= 5e-3 * np.abs(want).max()
+            ones = gpu_sdpa(hip_backend, torch_cuda, q, k, np.ones_like(v), scale, causal, window, rc, ln, mask)
+            assert np.abs(ones - 1.0).max() <= 1e-2
+            if ln is None and mask is None and rc == 0 and batch == 1:
+                t = [dev(torch_cuda, a) for a in (q, k, v)]
+                rows = torch_cuda.full((sq, heads, d), float("nan"), device="cuda")
+                hip_backend.sdpa_cache_rows_dev(*t, rows, 1, heads, kv_heads, sq, skv, skv, d, scale, causal, window)
+                assert np.array_equal(rows.cpu().numpy(), got[0].transpose(1, 0, 2))
+    finally:
+        hip_backend.set_tuning("sdpa_prefill_teams", 0)
+        hip_backend.set_tuning("sdpa_prefill_splits", 0)
