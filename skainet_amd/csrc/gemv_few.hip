@@ -9,12 +9,11 @@
 //   * v_mfma_f32_4x4x1 (16 blocks of 4 x 4, exact fp32 products) multiplies: lane l = 4 blk + j holds weights of row j of a
 //     quad of weight rows and the activations of batch row j, both of K slot blk; one instruction takes 64 weights times
 //     four batch rows in 4.2 ns (a vector instruction: 0.96), and the two kinds do not overlap.
-
 //   * A slot is the 64 weights that one lane decodes (packed_lane64.h). Its activations (64 floats per four batch rows) stay
 //     in registers while the wave walks the workgroup's rows; 16 slots are a pass of 1024 elements of K and the waves of a
 //     workgroup share the passes. R quads of weight rows are requested ahead.
 //   * One and two rows would leave the instruction half empty: the vector unit multiplies, same lanes and loads (Q8_0
-//     2 x 10000 x 4096 13.9 us on the row kernel, 12 on the matrix instruction, 10.7 here).
+//     2 x 10000 x 4096 13.9 us on the row kernel, 10.7 here; 2 x 4096 x 11008 16.5 on the matrix instruction, 13.0 at n 4000 here).
 //   * The 16 blocks' sums fold inside a DPP row; the four DPP rows and the waves meet in LDS once, summed in a fixed order.
 #include "packed_lane64.h"
 
@@ -254,10 +253,10 @@ void set_gemv_few(int v) { g_gemv_few = v; }
 // rows, rows of few kilobytes, K that leaves their waves unequal shares (more than 8192, 4096 to 5120). They hold their own with
 // few products on full waves, and where K takes this kernel a second round that few waves share (6144 to 8192).
 //   32-element blocks, 3 to 8 rows: everywhere (Q8_0 4 x 4096 x 11008 26.1 -> 14.6, 8 x 32000 x 4096 111 -> 41)
-//     2 rows: Q4_0 everywhere (4000 x 4096 7.2 -> 5.3), the others outside 6144 < K <= 8192 (Q8_0 10000 x 4096 13.9 -> 10.7, x
-//     7168 16.2 -> 17.2)
+//     2 rows: outside 6144 < K <= 8192 (Q4_0 4000 x 4096 7.2 -> 5.3, Q8_0 10000 x 4096 13.9 -> 10.7, x 7168 16.2 -> 17.2)
 //     1 row: many weight rows (Q5_0 30000 x 4096 27.7 -> 20.7; Q8_0 has the integer kernel at multiples of 1024), and for formats of
-//     4 and 5 bits a K beyond the streaming kernel's (Q4_0 4000 x 11008 11.7 -> 9.9, Q5_0 10000 x 8192 15.2 -> 15.8)
+//     4 and 5 bits a K beyond the streaming kernel's (Q4_0 4000 x 11008 11.7 -> 9.9; Q5_0 10000 x 8192 15.2 -> 15.8, Q5_1 31331 x
+//     14080 73 -> 85)
 //   Q6_K, Q5_K: their decode costs more, so 5 to 8 rows (Q6_K 8 x 4096 x 11008 53 -> 24; 5 x 1500 x 7168 13.2 -> 15.0), 3 and 4 of Q5_K,
 //     and below that rows that leave the row kernel's lanes idle (Q6_K 1 x 30000 x 768 18.0 -> 10.0, 2 x 10000 x 11008 36.6 -> 25.6;
 //     4 x 14336 x 4096 15.9 -> 16.8)
