@@ -54,8 +54,10 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
 }
 
 // MQ: several queries per sequence (a draft of a few tokens). The rows that share a KV head are then its query heads times
-// the queries, GS of them to a workgroup: each has a key range of its own (causal and window move with the query), the
-// workgroup walks the union and a key outside a row's range scores -inf for that row.
+// the queries, GS of them to a workgroup: each has a key range of its own (causal and window move with the query) and the
+// workgroup walks the union. A key outside a row's range takes no part in that row: it scores -inf and its V is replaced by
+// zeros, since a weight of zero times an infinite or undefined element (a later token's, or the padding of a cache) is not
+// zero. Passes whose keys lie in every row's range, nearly all of them, skip both.
 template <int GS, int DPL, bool MQ>
 __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     constexpr int D = 16 * DPL;
@@ -77,7 +79,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     int64_t row_of[GS];
     int first_of[GS], end_of[GS];
     bool uniform_of[GS];
-    int first = 0x7FFFFFFF, end = 0;
+    int first = 0x7FFFFFFF, end = 0;           // the union of the rows' ranges, and the keys that all rows share
+    int common_first = 0, common_end = 0x7FFFFFFF;
 #pragma unroll
     for (int g = 0; g < GS; ++g) {
         const int r = MQ ? min(r0 + g, rows_kv - 1) : r0 + g;
@@ -97,6 +100,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         if (uniform_of[g]) { f = 0; e = p.seq_kv; }
         first_of[g] = f; end_of[g] = e;
         first = min(first, f); end = max(end, e);
+        common_first = max(common_first, f); common_end = min(common_end, e);
     }
     const bool uniform = uniform_of[0];        // one query: the same for all rows of the workgroup
     const int chunk = ((end - first + p.splits - 1) / p.splits + 15) & ~15;
@@ -143,14 +147,16 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
             }
         }
     };
-    auto consume = [&](const float (&kr)[U][DPL], const float (&vr)[U][DPL], int k0) {
+    // cut: some row's range leaves out a key of this pass (MQ only, wave-uniform)
+    auto consume = [&](const float (&kr)[U][DPL], const float (&vr)[U][DPL], int k0, auto cut_c) __attribute__((always_inline)) {
+        constexpr bool CUT = MQ && decltype(cut_c)::value;
         bool valid[U][MQ ? GS : 1];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int key = k0 + 16 * u + kg;
 #pragma unroll
             for (int g = 0; g < (MQ ? GS : 1); ++g)
-                valid[u][g] = MQ ? key < min(hi, end_of[g]) && key >= first_of[g] : key < hi;
+                valid[u][g] = !MQ ? key < hi : CUT ? key < min(hi, end_of[g]) && key >= first_of[g] : true;
         }
         // Branch-free from here to the end of the body: the U x GS score chains (dot product, row reduction, exponentials)
         // are independent and the compiler interleaves them; behind a per-key branch each ran on its own, one
@@ -187,7 +193,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
             for (int d = 0; d < DPL; ++d) {
                 float a = acc[g][d] * alpha;
 #pragma unroll
-                for (int u = 0; u < U; ++u) a = fmaf(pr[u], vr[u][d], a);
+                for (int u = 0; u < U; ++u) a = fmaf(pr[u], CUT && !valid[u][g] ? 0.f : vr[u][d], a);
                 acc[g][d] = a;
             }
             m[g] = m_new;
@@ -200,14 +206,22 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     float ka[U][DPL], va[U][DPL], kb2[U][DPL], vb2[U][DPL];
     const int k_first = lo + wave * 4;
     if (k_first < hi) request(ka, va, k_first);                 // wave-uniform
-    for (int k0 = k_first; k0 < hi; k0 += 2 * STEP) {
+    auto pair = [&](int k0, auto cut) __attribute__((always_inline)) {
         request(kb2, vb2, k0 + STEP);                           // past the range: clamped re-reads of the last row
         __builtin_amdgcn_sched_barrier(0);                      // requests are issued where they are written, ahead of the arithmetic
-        consume(ka, va, k0);
+        consume(ka, va, k0, cut);
         request(ka, va, k0 + 2 * STEP);
         __builtin_amdgcn_sched_barrier(0);
-        consume(kb2, vb2, k0 + STEP);
+        consume(kb2, vb2, k0 + STEP, cut);
+    };
+    int k0 = k_first;
+    if constexpr (MQ) {
+        // a pair of passes whose keys all rows attend; a loop of each kind, not a branch inside one (199 instead of 158 registers)
+        auto whole = [&] { return k0 >= common_first && k0 + STEP + 16 * (U - 1) + 4 <= min(hi, common_end); };
+        for (; k0 < hi && !whole(); k0 += 2 * STEP) pair(k0, std::true_type{});
+        for (; whole(); k0 += 2 * STEP) pair(k0, std::false_type{});
     }
+    for (; k0 < hi; k0 += 2 * STEP) pair(k0, std::true_type{});
 
     // Merge the 16 running states of the workgroup (4 lane groups x 4 waves) through LDS: every lane parks its slice,
     // one 16-lane row per head works out the 16 weights 2^(m_s - max) and the weighted sum of the l_s, then each thread

@@ -150,6 +150,41 @@ def test_attention_of_a_few_queries_over_a_cache(hip_backend, torch_cuda, batch,
         hip_backend.set_tuning("sdpa_decode_one_launch", 1)
 
 
+@pytest.mark.parametrize("one_launch", [1, 0])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("heads,kv_heads,d,sq,skv", [(8, 2, 128, 2, 65), (6, 2, 64, 3, 300), (3, 1, 64, 15, 700), (2, 1, 256, 5, 129), (4, 4, 128, 5, 1500),
+                                                     (1, 1, 64, 2, 40)])
+def test_a_draft_query_takes_nothing_from_keys_that_are_hidden_from_it(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv, bad, one_launch):
+    """Rows with different key ranges share a workgroup that walks the union of the ranges. Infinite or undefined K and V at
+    keys that some rows attend and others do not: the later tokens of the draft, the first query's oldest window key, the
+    padding past a short length beside a row that the window and the length leave no key (that row weighs every key). Rows
+    that do not attend the bad keys give the oracle's result on finite values there."""
+    rng = np.random.default_rng(heads * d + skv + sq)
+    q = rng.standard_normal((1, heads, sq, d)).astype(np.float32)
+    k = rng.standard_normal((1, kv_heads, skv, d)).astype(np.float32)
+    v = rng.standard_normal((1, kv_heads, skv, d)).astype(np.float32)
+    scale = float(1 / np.sqrt(d))
+    pos, key = np.arange(skv - sq, skv)[:, None], np.arange(skv)[None, :]
+    win = min(3, sq)
+    hip_backend.set_tuning("sdpa_decode_one_launch", one_launch)
+    try:
+        # (window, length, bad keys): the last token, every later token than the first query's, the first query's oldest key, padding
+        for w, length, keys in ((0, None, [skv - 1]), (0, None, range(skv - sq + 1, skv)), (win, None, [skv - sq - win + 1]),
+                                (win, skv - win, range(skv - win, skv))):
+            lens = None if length is None else np.array([length], np.int32)
+            attended = (key <= pos) & (key > pos - w if w else True) & (key < (skv if length is None else length))
+            attended[~attended.any(1)] = True
+            kb, vb = k.copy(), v.copy()
+            kb[:, :, list(keys)], vb[:, :, list(keys)] = bad, bad
+            clean = ~attended[:, list(keys)].any(1)
+            assert 0 < clean.sum() < sq
+            got = gpu_sdpa(hip_backend, torch_cuda, q, kb, vb, scale, True, w, 0, lens)
+            assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+            close(got[:, :, clean], L.sdpa(q, k, v, scale, True, w, 0, lens)[:, :, clean], rel=2e-5, abs_=2e-6)
+    finally:
+        hip_backend.set_tuning("sdpa_decode_one_launch", 1)
+
+
 def test_attention_prefill_config_against_torch_fp32(hip_backend, torch_cuda):
     """Prefill: seq 2048 causal, 32 / 8 heads, head_dim 128. The oracle checks a 256-long prefix problem exactly;
     the full size is compared with torch's fp32 attention on the same device (textbook softmax(QK^T)V)."""
