@@ -375,7 +375,9 @@ static bool host_memory(const void* p) {
     if (hipPointerGetAttributes(&at, p) != hipSuccess) { (void)hipGetLastError(); return true; }      // unknown to the runtime: pageable
     return at.type == hipMemoryTypeUnregistered || at.type == hipMemoryTypeHost;
 }
+// (a null pointer is refused here: host_memory takes it for pageable memory, which the host side of the copy reads or writes)
 static int copy_h2d(void* dst, const void* src, size_t bytes) {
+    if (!dst || !src) return set_error("memcpy h2d: null pointer");
     if (!copy_kernel_fits(bytes) || !device_range(dst, bytes) || !host_memory(src)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
@@ -384,6 +386,7 @@ static int copy_h2d(void* dst, const void* src, size_t bytes) {
     return pin ? copy_up(dst, src, pin, bytes, true) : -1;
 }
 static int copy_d2h(void* dst, const void* src, size_t bytes) {
+    if (!dst || !src) return set_error("memcpy d2h: null pointer");
     if (!copy_kernel_fits(bytes) || !device_range(src, bytes) || !host_memory(dst)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");

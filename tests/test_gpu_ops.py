@@ -220,3 +220,26 @@ def test_host_copies_past_an_allocation_are_refused(hip_backend, nbytes):
         assert np.array_equal(back, host[:256])
     finally:
         lib.skainet_hip_free(p)
+
+
+@pytest.mark.parametrize("nbytes", [1, 4096, 1 << 20, (1 << 20) + 1])
+def test_host_copies_refuse_a_null_pointer(hip_backend, nbytes):
+    """On either side, in both directions, through the copy kernel's sizes and past them: an error, not a crash. The copy out
+    of a host-pointer entry is the same one."""
+    from skainet_amd import _lib
+    lib = _lib.hip()
+    host = np.arange(nbytes, dtype=np.uint32).astype(np.uint8)
+    p = lib.skainet_hip_malloc(nbytes)
+    try:
+        for call in (lambda: lib.skainet_hip_memcpy_h2d(p, None, nbytes), lambda: lib.skainet_hip_memcpy_h2d(None, host.ctypes.data, nbytes),
+                     lambda: lib.skainet_hip_memcpy_d2h(None, p, nbytes), lambda: lib.skainet_hip_memcpy_d2h(host.ctypes.data, None, nbytes)):
+            assert call() != 0 and "null pointer" in _lib.last_error()
+        assert lib.skainet_hip_memcpy_h2d(None, None, 0) == 0 and lib.skainet_hip_memcpy_d2h(None, None, 0) == 0
+        x, gain = np.ones(64, np.float32), np.ones(64, np.float32)
+        lib.skainet_hip_f32_rms_norm(x.ctypes.data, gain.ctypes.data, None, 1, 64, 1e-5)
+        assert "null pointer" in _lib.last_error()
+        back = np.empty_like(host)                                               # and the thread goes on
+        assert lib.skainet_hip_memcpy_h2d(p, host.ctypes.data, nbytes) == 0 and lib.skainet_hip_memcpy_d2h(back.ctypes.data, p, nbytes) == 0
+        assert np.array_equal(back, host)
+    finally:
+        lib.skainet_hip_free(p)
