@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         for (int e = 0; e < EPT; ++e) {
             const int d = i0 + e;                                   // a state's layout in LDS is the row's own element order
             if (!p.part) {
-                p.out[row * D + d] = ls > 0.f ? o[e] / ls : 0.f;
+                p.out[row * D + d] = ls == 0.f ? 0.f : o[e] / ls;   // an undefined score leaves an undefined sum: no zero for it
             } else {
                 p.part[(row * p.splits + split) * D + d] = o[e];
                 if (d == 0) *reinterpret_cast<float2*>(p.ml + (row * p.splits + split) * 2) = make_float2(mm, ls);
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(4 * D) void sdpa_decode_combine_kernel(const float*
         for (int off = 32; off > 0; off >>= 1) mm = fmaxf(mm, __shfl_xor(mm, off, 64));
         const float w = exp_diff(m, mm);
         const float ls = wave_sum(l * w);
-        if (sp < SDPA_DECODE_MAX_SPLITS) sw[sp] = ls > 0.f ? w / ls : 0.f;
+        if (sp < SDPA_DECODE_MAX_SPLITS) sw[sp] = ls == 0.f ? 0.f : w / ls;
     }
     __syncthreads();
     float o = 0.f;

@@ -185,6 +185,27 @@ def test_a_draft_query_takes_nothing_from_keys_that_are_hidden_from_it(hip_backe
         hip_backend.set_tuning("sdpa_decode_one_launch", 1)
 
 
+@pytest.mark.parametrize("one_launch", [1, 0])
+@pytest.mark.parametrize("heads,kv_heads,d,sq,skv", [(8, 2, 128, 1, 40), (8, 2, 128, 1, 200), (4, 1, 64, 1, 1000), (6, 2, 64, 3, 200), (2, 1, 256, 5, 129), (4, 4, 128, 4, 900)])
+def test_an_undefined_score_makes_the_output_undefined(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv, one_launch):
+    """A NaN in the K row of an attended key reaches every query that attends it, with one split of the keys and with several:
+    no zeros in its place. V is finite."""
+    rng = np.random.default_rng(heads * d + skv + sq)
+    q = rng.standard_normal((1, heads, sq, d)).astype(np.float32)
+    k = rng.standard_normal((1, kv_heads, skv, d)).astype(np.float32)
+    v = rng.standard_normal((1, kv_heads, skv, d)).astype(np.float32)
+    hip_backend.set_tuning("sdpa_decode_one_launch", one_launch)
+    try:
+        for key in (0, skv // 2, skv - sq):
+            kb = k.copy()
+            kb[:, :, key, 1] = np.nan
+            got = gpu_sdpa(hip_backend, torch_cuda, q, kb, v, float(1 / np.sqrt(d)), True)
+            assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+            assert np.isnan(got).all()
+    finally:
+        hip_backend.set_tuning("sdpa_decode_one_launch", 1)
+
+
 def test_attention_prefill_config_against_torch_fp32(hip_backend, torch_cuda):
     """Prefill: seq 2048 causal, 32 / 8 heads, head_dim 128. The oracle checks a 256-long prefix problem exactly;
     the full size is compared with torch's fp32 attention on the same device (textbook softmax(QK^T)V)."""
