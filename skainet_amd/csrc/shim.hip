@@ -285,9 +285,10 @@ static int staged_h2d(void* dst, const uint8_t* src, size_t bytes) {
 // and the host polls a page-locked flag that the kernel's last workgroup sets. A launch costs 2.8 us here, a launch with
 // hipStreamSynchronize behind it 11.3, a launch that sets a flag the host polls 6.5 (a kernel with nothing to do). Both
 // directions still return only when the bytes are where they belong. More than COPY_CHUNK bytes go in pieces, the host
-// filling (or emptying) one piece of staging while the kernel of another is on the bus. Measured against the runtime's copy
-// and wait, up / down: 4 KB 15.3 / 21.8 -> 8.6 / 7.9 us, 16 KB 14.2 / 21.2 -> 9.0 / 8.8, 128 KB 87 (an array
-// the runtime pins for the call) -> 14.5 up, 1 MB 40.8 / 59.8 -> 42 / 43. Above COPY_KERNEL_MAX the
+// filling (or emptying) one piece of staging while the kernel of another is on the bus. Pageable arrays against the runtime's
+// copy and wait, up / down: alone 4 KB 14 / 21 -> 8 / 7 us, 16 KB 13 / 20 -> 8.6 / 8.3, 128 KB 12 / 14 -> 13 / 13, 1 MB 38 to 65 / 57 to
+// 67 -> 40 to 43 / 41 to 46 (the first figure: one array again and again); with a kernel behind / two in front 128 KB 28 / 28 -> 25 /
+// 20, 512 KB 39 to 46 / 44 to 48 -> 42 / 36. A request of 32 x 1024 floats against a dense network: 155 -> 119. Above COPY_KERNEL_MAX the
 // copy engine's rate counts for more than its hand-over; where the bytes pass through page-locked staging anyway (a product
 // on host arrays) the pieces hide the bus behind the host's memcpy up to STAGED_KERNEL_MAX.
 constexpr size_t COPY_KERNEL_MAX = 1u << 20, STAGED_KERNEL_MAX = 8u << 20, COPY_CHUNK = 128u << 10;
@@ -370,15 +371,20 @@ static bool device_range(const void* p, size_t bytes) {
     const size_t off = (size_t)(static_cast<const uint8_t*>(p) - static_cast<const uint8_t*>(base));
     return at.type == hipMemoryTypeDevice && at.device == g_device && off <= size && bytes <= size - off;
 }
-static bool host_memory(const void* p) {
+// Page-locked memory of the caller's goes through staging as well up to one piece: what that copy costs is less than the
+// hand-over to a copy engine, as soon as a kernel runs before or behind it (up and then a kernel, two kernels and then down, us,
+// runtime's one transfer and staged: 4 KB 24.1 / 17.2 and 19.4 / 12.6, 64 KB 25.0 / 24.4 and 23.8 / 17.4, 128 KB 26.3 / 25.6 and
+// 24.8 / 20.4; alone, 128 KB 10.9 / 10.9 and 12.6 / 13.5). More than that is one transfer from where it lies: 256 KB 28.2 / 27.7
+// against 30.2 / 25.7, alone 13.2 / 13.2 against 17.6 / 18.3; 1 MB 42 / 43 against 54 / 50, alone 27 against 43 / 41.
+static bool staged_host_memory(const void* p, size_t bytes) {
     hipPointerAttribute_t at;
     if (hipPointerGetAttributes(&at, p) != hipSuccess) { (void)hipGetLastError(); return true; }      // unknown to the runtime: pageable
-    return at.type == hipMemoryTypeUnregistered || at.type == hipMemoryTypeHost;
+    return at.type == hipMemoryTypeUnregistered || (at.type == hipMemoryTypeHost && bytes <= COPY_CHUNK);
 }
-// (a null pointer is refused here: host_memory takes it for pageable memory, which the host side of the copy reads or writes)
+// (a null pointer is refused here: staged_host_memory takes it for pageable memory, which the host side of the copy reads or writes)
 static int copy_h2d(void* dst, const void* src, size_t bytes) {
     if (!dst || !src) return set_error("memcpy h2d: null pointer");
-    if (!copy_kernel_fits(bytes) || !device_range(dst, bytes) || !host_memory(src)) {
+    if (!copy_kernel_fits(bytes) || !device_range(dst, bytes) || !staged_host_memory(src, bytes)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t_stream), "hipMemcpy h2d") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }
@@ -387,7 +393,7 @@ static int copy_h2d(void* dst, const void* src, size_t bytes) {
 }
 static int copy_d2h(void* dst, const void* src, size_t bytes) {
     if (!dst || !src) return set_error("memcpy d2h: null pointer");
-    if (!copy_kernel_fits(bytes) || !device_range(src, bytes) || !host_memory(dst)) {
+    if (!copy_kernel_fits(bytes) || !device_range(src, bytes) || !staged_host_memory(dst, bytes)) {
         if (check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, t_stream), "hipMemcpy d2h") != 0) return -1;
         return check_hip(hipStreamSynchronize(t_stream), "hipStreamSynchronize");
     }

@@ -204,6 +204,36 @@ def test_host_copies_of_every_size_and_alignment_are_byte_exact(hip_backend, nby
         lib.skainet_hip_free(p)
 
 
+@pytest.mark.parametrize("offset", [0, 4, 1])
+@pytest.mark.parametrize("nbytes", [17, 16384, 131072, 131073, 300001])
+def test_host_copies_of_page_locked_memory_are_byte_exact(hip_backend, nbytes, offset):
+    """Memory of skainet_hip_host_alloc goes through staging up to 128 KB and as one transfer from there: either way bytes equal
+    and neighbours untouched, on the device and in the caller's buffer."""
+    import ctypes
+    from skainet_amd import _lib
+    lib = _lib.hip()
+    size = nbytes + 64
+    p, h = lib.skainet_hip_malloc(size), lib.skainet_hip_host_alloc(size)
+    try:
+        host = np.ctypeslib.as_array(ctypes.cast(h, ctypes.POINTER(ctypes.c_uint8)), (size,))
+        src = np.random.default_rng(nbytes + offset).integers(0, 256, nbytes, dtype=np.uint8)
+        want = np.full(size, 0xA5, np.uint8)
+        host[:] = want
+        assert lib.skainet_hip_memcpy_h2d(p, h, size) == 0
+        want[16 + offset:16 + offset + nbytes] = src
+        host[:] = 0
+        host[offset:offset + nbytes] = src
+        assert lib.skainet_hip_memcpy_h2d(p + 16 + offset, h + offset, nbytes) == 0
+        host[:] = 0x5A
+        assert lib.skainet_hip_memcpy_d2h(h + 32, p + 16 + offset, nbytes) == 0
+        assert np.array_equal(host[32:32 + nbytes], src) and (host[:32] == 0x5A).all() and (host[32 + nbytes:] == 0x5A).all()
+        assert lib.skainet_hip_memcpy_d2h(h, p, size) == 0
+        assert np.array_equal(host, want)
+    finally:
+        lib.skainet_hip_free(p)
+        lib.skainet_hip_host_free(h)
+
+
 @pytest.mark.parametrize("nbytes", [300, 5000, 70000])
 def test_host_copies_past_an_allocation_are_refused(hip_backend, nbytes):
     """A run that leaves its allocation returns an error, as the runtime's copy does: it never reaches the copy kernel."""
