@@ -434,11 +434,13 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * 2 wherever they fit), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
  * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2), "gemm_wide" (1 / 0: force the 256-column / 128-column tile, -1 = chosen from the shape), "gemm_rows" (2 / 4: 128 / 256
  * activation rows per tile, 0 = chosen from the shape), "gemm_ksw" (the Q4_K kernel that splits K over the
- * waves of a workgroup: 0 never, 1 where the launcher's estimate favours it, 2 wherever it fits), "gemm_ksw_teams" (teams
+ * waves of a workgroup: 0 never, 1 where "gemm_frag" is 0 and the launcher's estimate favours it -- the fragment-order kernel
+ * is the faster one wherever both fit -- 2 wherever it fits; 0 keeps Q4_K from "gemm_frag" and "gemm_skinny" by rule as well:
+ * the tile kernel is left), "gemm_ksw_teams" (teams
  * of four waves per workgroup of that kernel, each with its own share of K: 1 or 2, default 2; rows with an odd number
  * of 256-element super-blocks always run one team), "gemm_ksw_stages" (activation tiles the one-team form keeps in LDS: 3 to 7,
- * default 5), "gemm_frag" (the Q4_K kernel that reads its activations in matrix-fragment order: 0 never, 1 where the
- * launcher's estimate favours it, 2 wherever it fits), "gemm_frag_waves" (waves per workgroup of that kernel: 8 = one
+ * default 5), "gemm_frag" (the Q4_K kernel that reads its activations in matrix-fragment order: 0 never, nor "gemm_skinny" by rule
+ * for Q4_K, 1 where the launcher's estimate favours it, 2 wherever it fits), "gemm_frag_waves" (waves per workgroup of that kernel: 8 = one
  * workgroup per CU, 4 = two, 0 = eight for one round of tiles and four for more), "gemm_frag_gm" (row tiles per group of
  * its tile order, 0 = by the launcher's traffic estimate), "gemm_frag_touch" (0: the pass in front of it does not touch the
  * weight's lines), "gemm_frag_pieces" (64-element groups a workgroup of that pass takes: 1, 2 or 4),

@@ -826,7 +826,10 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     const double frag_estimate = frag_by_rule ? gemm_frag_us(m, n, k) : tile_estimate;
     // Few rows: the kernel without a row tile to fill. (The epilogue plays no part in the choice: a product takes one
     // kernel, and sums in one order, whatever is done to it on the way out.)
-    const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 && gemm_ksw_enabled() && gemm_frag_enabled();
+    // A forced tile or split keeps it out, and so does either of the two Q4_K kernels switched off, for Q4_K alone: that
+    // leaves the format to the kernels before them.
+    const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 &&
+                         (enc != ENC_Q4_K || (gemm_ksw_enabled() && gemm_frag_enabled()));
     if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k) &&
         gemm_skinny_estimate(enc, m, n, k) < 0.95 * fmin(tile_estimate, frag_estimate))
         return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);

@@ -233,3 +233,20 @@ def test_gemm_of_few_rows(hip_backend, torch_cuda, enc, m, n, k):
             assert normalized_err(half.cpu().numpy(), p[:, 0::2] / (1 + np.exp(-p[:, 0::2])) * p[:, 1::2], eps=1.0) <= 4e-3
     finally:
         kx.set_tuning("gemm_skinny", 1)
+
+
+@pytest.mark.parametrize("knob", ["gemm_frag", "gemm_ksw"])
+def test_the_q4k_gemm_knobs_leave_other_formats_alone(hip_backend, torch_cuda, knob):
+    """Either Q4_K kernel switched off: a product of few rows in another format takes the kernel it takes by rule, Q4_K one
+    of those before the switched-off one."""
+    m, n, k = 24, 4096, 4096
+    x = np.random.default_rng(24).standard_normal((m, k)).astype(np.float32)
+    try:
+        hip_backend.set_tuning(knob, 0)
+        for enc in ALL_ENCS:
+            packed = gaussian_weight(hip_backend, enc, n, k, 24)
+            got = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
+            assert (hip_backend.last_kernel() == "packed_gemm_skinny_kernel") == (enc != "Q4_K")
+            check(got[:2], L.gemv(enc, x[:2], packed, n))
+    finally:
+        hip_backend.set_tuning(knob, 1)
