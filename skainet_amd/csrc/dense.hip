@@ -318,7 +318,7 @@ int launch_fp32_matmul(const float* a, int64_t a_stride, const float* b, int64_t
     const int64_t tiles64 = (int64_t)((n + MT - 1) / MT) * ((m + 63) / 64);
     // (B read along its rows at an odd alignment and 64 rows or more: the LDS tile kernel, whose loads do not mind)
     if (g_dense_mfma && k >= 1 && tiles64 < num_cus() && (b_transposed || aligned || m < 64)) {
-        note_kernel("sgemm_mfma_kernel");
+        note_kernel("sgemm_mfma_skinny_kernel");
         if (b_transposed) launch_skinny_rows<true>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
         else launch_skinny_rows<false>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
         SKH_CHECK(hipGetLastError());

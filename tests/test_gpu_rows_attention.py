@@ -480,12 +480,14 @@ def test_dense_matmuls(hip_backend, torch_cuda):
 
 
 @pytest.mark.parametrize("m,n,k,wt", [(512, 1024, 768, False), (200, 300, 260, False), (64, 32, 4, True), (130, 4096, 516, True),
-                                      (1000, 132, 2048, False), (65, 257, 100, True)])
+                                      (1000, 132, 2048, False), (65, 257, 100, True), (1030, 2052, 100, True), (1030, 2052, 36, False),
+                                      (2100, 2100, 20, True), (2100, 2100, 132, False)])
 def test_dense_fp32_matmul_on_the_matrix_cores(hip_backend, torch_cuda, m, n, k, wt):
     """fp32 operands on the fp32 matrix instruction (exact products, fp32 accumulation in the instruction's order):
     resident operands through the device entries, ragged tiles in every direction, K from one instruction step to many
-    slices, both layouts of B; against fp64 and against the tile kernel that takes the same call when the matrix-core
-    one is switched off. Products whose strides or alignment the matrix-core kernel does not read stay on the tile
+    slices, both layouts of B: shapes whose 64 x 128 tiles leave CUs idle run the kernel that splits K over waves, the others
+    64- or 128-row tiles; against fp64 and against the tile kernel that takes the same call when the matrix-core
+    ones are switched off. Products whose strides or alignment the matrix-core kernel does not read stay on the tile
     kernel."""
     torch = torch_cuda
     rng = np.random.default_rng(m + n + k)
@@ -502,7 +504,8 @@ def test_dense_fp32_matmul_on_the_matrix_cores(hip_backend, torch_cuda, m, n, k,
         return out.cpu().numpy()
 
     got = run()
-    assert hip_backend.last_kernel() == "sgemm_mfma_kernel"
+    few = -(-m // 64) * -(-n // 128) < torch.cuda.get_device_properties(0).multi_processor_count
+    assert hip_backend.last_kernel() == ("sgemm_mfma_skinny_kernel" if few else "sgemm_mfma_kernel")
     close(got, want, rel=1e-5, abs_=2e-6 * np.sqrt(k) * 16)
     try:
         hip_backend.set_tuning("dense_mfma", 0)
@@ -540,7 +543,7 @@ def test_dense_fp32_products_with_k_split_over_waves(hip_backend, torch_cuda, m,
     else:
         hip_backend.fp32_matmul_dev(dev(torch, a), 0, k, dev(torch, b), 0, n, out, 0, n, m, n, k)
     if wt or m < 64:                                    # unaligned rows of B at 64 rows and more stay on the tile kernel
-        assert hip_backend.last_kernel() == "sgemm_mfma_kernel"
+        assert hip_backend.last_kernel() == "sgemm_mfma_skinny_kernel"
     got = out.cpu().numpy()
     assert np.isnan(got[m]).all()                       # nothing past the last row
     assert np.abs(got[:m] - want).max() <= max(1, k / 4) * 2.0 ** -24 * 0.64 * k + 1e-6
