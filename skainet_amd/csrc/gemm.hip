@@ -698,44 +698,54 @@ void set_gemm_wide(int v) { g_gemm_wide = v; }
 static std::atomic<int> g_gemm_rows{0};     // 0 = choose from the shape, 2 / 4 = 128 / 256 activation rows per tile
 void set_gemm_rows(int v) { if (v == 0 || v == 2 || v == 4) g_gemm_rows = v; }
 
-// What a product takes on the tile kernel, in us, the pass in front and both launches (5.5) included. A round is one
-// workgroup per CU; a step of 64 elements of K costs more the fuller the round (clocks and memory are shared): the two
-// numbers per format and tile are for 64 and for 256 tiles, measured at K 2048 and 4096, and a round spends 3 us outside its
-// loop. Two of the 128 x 128 workgroups fit a CU: two rounds of them take 1.42 (half of the second full) to 1.67 of one.
-static double gemm_round_us(const double (&step)[2], double tiles, double steps) {
-    const double fill = tiles <= 64 ? 0.0 : tiles >= 256 ? 1.0 : (tiles - 64) / 192;
-    return 3.0 + (step[0] + (step[1] - step[0]) * fill) * steps;
-}
-static double gemm_tile_us(int enc, int wtm, int wtn, double tiles, double steps) {
+// What a product takes on the tile kernel, in us: its launches, what it moves outside the loop, and per round of 256 tiles a part
+// outside the K loop and a step of 64 elements of K. Fitted to 145 000 timings of 73 000 random products (9 to 1024 rows, n 512 to
+// 32000, K 512 to 14336, every format, tile and split), which it meets within 4 to 5 % (rms). A step takes longer the fuller the
+// round (clocks and memory are shared): the two numbers per format are for 64 and for 256 tiles. Two of the 128 x 128 workgroups
+// fit a CU: two rounds of them take 1.43 (the second barely begun) to 1.6 of one. The launch that sums splits has its own
+// cost and (splits + 1) m n floats to move; splits that would get no K are not counted.
+static double gemm_tile_us(int enc, int wtm, int wtn, int m, int n, int k, int ks) {
     // [128 x 128, 128 x 256, 256 x 128, 256 x 256][64 tiles, 256 tiles]
-    static const double q4k[4][2] = {{0.586, 0.739}, {0.99, 1.29}, {0.825, 1.10}, {1.44, 1.99}}, q5k[4][2] = {{0.623, 0.783}, {1.14, 1.42}, {0.872, 1.19}, {1.58, 2.17}};
-    static const double q6k[4][2] = {{0.68, 0.805}, {1.25, 1.51}, {0.908, 1.23}, {1.69, 2.35}}, q80[4][2] = {{0.803, 0.894}, {1.39, 1.96}, {1.03, 1.29}, {1.83, 2.68}};
-    static const double q40[4][2] = {{0.539, 0.705}, {0.994, 1.24}, {0.806, 1.08}, {1.38, 1.95}}, q50[4][2] = {{0.628, 0.764}, {1.22, 1.43}, {0.853, 1.15}, {1.63, 2.17}};
-    static const double q51[4][2] = {{0.602, 0.764}, {1.14, 1.46}, {0.84, 1.17}, {1.57, 2.26}};
+    static const double q4k[4][2] = {{0.603, 0.701}, {0.921, 1.18}, {0.781, 0.988}, {1.33, 1.81}}, q5k[4][2] = {{0.647, 0.748}, {1.03, 1.32}, {0.816, 1.03}, {1.43, 1.92}};
+    static const double q6k[4][2] = {{0.722, 0.828}, {1.26, 1.47}, {0.881, 1.09}, {1.61, 2.08}}, q80[4][2] = {{0.762, 0.835}, {1.27, 1.53}, {1.09, 1.18}, {1.58, 2.11}};
+    static const double q40[4][2] = {{0.573, 0.672}, {0.877, 1.13}, {0.759, 0.942}, {1.26, 1.69}}, q50[4][2] = {{0.621, 0.728}, {1.14, 1.34}, {0.794, 0.988}, {1.49, 1.90}};
+    static const double q51[4][2] = {{0.631, 0.712}, {1.06, 1.26}, {0.807, 0.955}, {1.43, 1.82}};
+    static const double outside[4] = {2.4, 5.6, 5.5, 9.0};
     const double (*table)[2] = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
                              : enc == ENC_Q5_1 ? q51 : q80;
     const int shape = (wtm == 4 ? 2 : 0) + (wtn == 4 ? 1 : 0);
-    const double cus = num_cus(), one = gemm_round_us(table[shape], 256, steps);
-    tiles *= 256 / cus;                                          // the measurements are for 256 CUs
-    double t = 5.5;
+    const int kgroups = (k + 255) / 256, per = (kgroups + ks - 1) / ks, splits = (kgroups + per - 1) / per;
+    const double steps = per * (256 / GK);
+    // the measurements are for 256 CUs
+    double tiles = (double)((m + gemm_gm(wtm) - 1) / gemm_gm(wtm)) * ((n + gemm_gn(wtn) - 1) / gemm_gn(wtn)) * splits * 256 / num_cus();
+    auto round = [&](double t) {                                 // one round of t <= 256 tiles
+        const double fill = t <= 64 ? 0.0 : (t - 64) / 192;
+        return outside[shape] + (table[shape][0] + (table[shape][1] - table[shape][0]) * fill) * steps;
+    };
+    double t = 4.0 + 1.0e-6 * m * k + 5.2e-7 * m * n;
+    if (splits > 1) t += 3.9 + 6.4e-7 * (splits + 1) * m * n;
     if (shape == 0) {
         const double pairs = floor(tiles / 512);
-        t += pairs * 1.67 * one;
+        t += pairs * 1.6 * round(256);
         tiles -= 512 * pairs;
-        if (tiles > 256) return t + one * (tiles <= 384 ? 1.42 : 1.42 + 0.5 * (tiles - 384) / 256);
+        if (tiles > 256) return t + round(256) * (1.43 + 0.17 * (tiles - 256) / 256);
     } else {
         const double rounds = floor(tiles / 256);
-        t += rounds * one;
+        t += rounds * round(256);
         tiles -= 256 * rounds;
     }
-    return tiles > 0 ? t + gemm_round_us(table[shape], tiles, steps) : t;
+    return tiles > 0 ? t + round(tiles) : t;
 }
-// The same for the fragment-order kernel (Q4_K, 128 x 64 tiles), measured at 64 to 1024 tiles, K 1024 to 14336.
+// The same for the fragment-order kernel (Q4_K, 128 x 64 tiles), 14 000 timings within 5 %. Up to a tile per CU its eight waves
+// share K by super-blocks: a started round of four costs about half of a whole one at once. Above, two workgroups of four waves on
+// a CU: the first of a pair takes a third of what both take, a pair on every second CU four fifths.
 static double gemm_frag_us(int m, int n, int k) {
-    const double tiles = (double)((m + 127) / 128) * ((n + 63) / 64) * 256 / num_cus(), steps = k / GK;
-    if (tiles <= 128) return 8.8 + 0.19 * steps;
-    if (tiles <= 256) return 8.8 + 0.7 * (tiles - 128) / 128 + (0.19 + 0.085 * (tiles - 128) / 128) * steps;
-    return 8.5 + tiles / 256 + (0.2575 * tiles / 256 + (tiles < 512 ? 0.06 : 0.0)) * steps;
+    const double tiles = (double)((m + 127) / 128) * ((n + 63) / 64) * 256 / num_cus(), steps = k / GK, whole = 16 * ((k + 1023) / 1024);
+    const double t = 8.4 + 1.69e-6 * m * k + 1.14e-6 * m * n;
+    if (tiles <= 256) return t + (0.175 + 0.055 * (tiles <= 64 ? 0.0 : (tiles - 64) / 192)) * (0.52 * steps + 0.48 * whole);
+    const double pairs = ceil(tiles / 512) - 1, rest = tiles - 512 * pairs;
+    const double share = rest <= 256 ? 0.323 + 0.456 * rest / 256 : 0.779 + 0.221 * (rest - 256) / 256;
+    return t + 0.476 * (0.74 * steps + 0.26 * whole) * (pairs + share);
 }
 
 // y = epilogue(prologue(x) . W^T): gain != null normalises every activation row first (RMSNorm, folded into the pass that
@@ -796,11 +806,11 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     if (frag_ok && gemm_frag_forced()) return run_frag();
     if (ksw_ok && gemm_ksw_forced()) return run_ksw();
     // The tile shape and the number of K splits with the least estimate. K chunks are whole 256-element groups so every
-    // encoding's blocks stay intact; the launch that sums the splits takes 5 us and (splits + 1) m n floats at 8 bytes per ns.
-    // The estimates are good to about 7 %, so the tile that fits most shapes -- 256 rows (128 where there are no more), the
-    // wide one where it fills three quarters of the chip in a round -- gives way only to one 5 % below it, and the tile kernel
-    // to the fragment-order kernel only 8 % below (167 random shapes of 129 to 1024 rows: the least estimate alone left 16 of
-    // them 3 to 15 % slower than that tile, Q6_K 593 x 10514 x 14080 272 -> 312 us).
+    // encoding's blocks stay intact. An estimate is off by 5 to 10 % now and then, and what was the better choice by less than
+    // that is kept: the tile that fits most shapes -- 256 rows (128 where there are no more), the wide one where it fills three
+    // quarters of the chip in a round -- gives way only to one 5 % below it, a split more has to save 1 %, the few-rows kernel
+    // 5 %; the fragment-order kernel stays up to 2 % above. On 9300 other random products, against one tile shape
+    // by the row count: geometric mean 1.44x, 36 of them more than 3 % slower, 4 more than 10 %, the worst 15 %.
     const int kgroups = (k + 255) / 256;
     const int usual_tm = m <= 128 ? 2 : 4;
     const bool usual_wide = 4 * (int64_t)((m + gemm_gm(usual_tm) - 1) / gemm_gm(usual_tm)) * ((n + gemm_gn(4) - 1) / gemm_gn(4)) >= 3 * num_cus();
@@ -811,12 +821,10 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
         if (g_gemm_rows.load() != 0 && tm != g_gemm_rows.load()) continue;
         for (int tn = 2; tn <= 4; tn += 2) {
             if (g_gemm_wide.load() >= 0 && (tn == 4) != (g_gemm_wide.load() != 0)) continue;
-            const double tiles = (double)((m + gemm_gm(tm) - 1) / gemm_gm(tm)) * ((n + gemm_gn(tn) - 1) / gemm_gn(tn));
             for (int ks = 1; ks <= 8 && ks <= kgroups; ++ks) {
                 if (g_gemm_ksplit.load() > 0 && ks != (g_gemm_ksplit.load() < kgroups ? g_gemm_ksplit.load() : kgroups)) continue;
-                double t = gemm_tile_us(enc, tm, tn, tiles * ks, ((kgroups + ks - 1) / ks) * (256 / GK));
-                if (ks > 1) t += 5.0 + (double)(ks + 1) * m * n * 4.0 / 8.0e6;
-                const double rank = tm == usual_tm && (tn == 4) == usual_wide ? 0.95 * t : t;
+                const double t = gemm_tile_us(enc, tm, tn, m, n, k, ks);
+                const double rank = t * (1 + 0.01 * (ks - 1)) * (tm == usual_tm && (tn == 4) == usual_wide ? 0.95 : 1.0);
                 if (least == 0.0 || rank < least) { least = rank; tile_estimate = t; wtm = tm; wtn = tn; ksplit = ks; }
             }
         }
@@ -833,7 +841,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k) &&
         gemm_skinny_estimate(enc, m, n, k) < 0.95 * fmin(tile_estimate, frag_estimate))
         return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
-    if (frag_by_rule && frag_estimate < 0.92 * tile_estimate) return run_frag();
+    if (frag_by_rule && frag_estimate < 1.02 * tile_estimate) return run_frag();
     if (ksw_ok && gemm_ksw_enabled() && !gemm_frag_enabled() && g_gemm_ksplit.load() <= 0) {
         // with the fragment-order kernel switched off, its predecessor where it would beat the tile kernel (0.31 us per 64
         // elements of K, 6.5 us per round outside the loop)

@@ -236,27 +236,34 @@ static int launch_skinny_tile(const uint8_t* a, const uint8_t* w, float* c, cons
     return 0;
 }
 
-// The tile of a shape and what it is estimated to take, in us. A wave's time for one super-block of its tile, measured per
-// format on 4096 x 4096, 4096 x 14336 and 14336 x 4096 (time of the call without its two launches' 5.5 us, per super-block
-// of a wave and round of one workgroup per CU): columns are tiles of 16 MT rows x 16 NT columns.
+// The tile of a shape and what it is estimated to take, in us: the two launches, what both move, and what the workgroups of a CU
+// take: the first one and each further one for a share of K of one super-block per wave (2048 elements). Fitted to 142 000
+// timings of random products (9 to 1024 rows, n 512 to 32000, K 512 to 14336, every format and tile), which it meets within 5
+// to 6 % (rms). The last, partial round of a CU costs a share `whole` of a full one whatever there is in it, the last, partial
+// share of K of the taller tiles a third.
 struct SknTile { int mt, nt; double us; };
 SknTile gemm_skinny_tile(int enc, int m, int n, int k) {
-    static const int shapes[6][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 2}, {2, 2}, {4, 2}};
-    static const double q4k[6] = {1.3, 2.2, 3.8, 2.2, 2.95, 4.4}, q5k[6] = {1.7, 2.3, 4.0, 3.4, 4.0, 5.7}, q6k[6] = {2.1, 2.8, 4.2, 4.3, 5.0, 6.7};
-    static const double q80[6] = {2.1, 3.0, 5.3, 3.8, 4.7, 6.4}, q40[6] = {1.3, 2.0, 3.6, 2.2, 3.0, 4.7}, q50[6] = {1.5, 2.1, 4.0, 2.7, 3.4, 5.0};
-    static const double q51[6] = {1.6, 2.2, 4.1, 2.8, 3.7, 5.3};
-    const double* cost = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
-                       : enc == ENC_Q5_1 ? q51 : q80;
-    const int mtiles = (m + 15) / 16, iters = ((k >> 8) + SKN_WAVES - 1) / SKN_WAVES;
-    // weights that do not stay in the 256 MB memory-side cache between calls were measured a fifth slower
-    const double slow = (double)n * (k / block_elems(enc)) * block_bytes(enc) > 64e6 ? 1.2 : 1.0;
+    static const int shapes[6][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 2}, {2, 2}, {4, 2}};     // tiles of 16 mt rows x 16 nt columns
+    static const double q4k[6][2] = {{1.15, 1.24}, {2.37, 1.83}, {3.80, 3.86}, {2.17, 1.94}, {2.80, 2.37}, {3.58, 3.81}};
+    static const double q5k[6][2] = {{1.63, 1.40}, {2.18, 1.98}, {3.97, 3.80}, {3.17, 2.71}, {3.68, 2.97}, {4.96, 5.02}};
+    static const double q6k[6][2] = {{2.16, 2.08}, {2.76, 2.55}, {3.89, 4.14}, {4.31, 4.90}, {4.63, 5.67}, {6.04, 6.26}};
+    static const double q80[6][2] = {{1.67, 2.01}, {2.63, 2.33}, {5.23, 3.44}, {3.07, 3.85}, {4.08, 4.03}, {4.98, 5.31}};
+    static const double q40[6][2] = {{1.18, 1.29}, {2.02, 1.82}, {3.42, 2.46}, {2.03, 2.11}, {2.87, 2.44}, {3.81, 3.94}};
+    static const double q50[6][2] = {{1.32, 1.36}, {2.06, 1.81}, {3.82, 2.60}, {2.65, 2.53}, {3.26, 2.81}, {4.07, 4.44}};
+    static const double q51[6][2] = {{1.48, 1.37}, {2.01, 1.97}, {3.95, 2.57}, {2.76, 2.53}, {3.63, 2.94}, {4.69, 4.92}};
+    static const double whole[6] = {0.86, 0.75, 0.78, 0.81, 0.82, 0.96}, whole_k[6] = {0.0, 0.06, 0.32, 0.04, 0.08, 0.32};
+    const double (*cost)[2] = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
+                            : enc == ENC_Q5_1 ? q51 : q80;
+    const int mtiles = (m + 15) / 16;
+    const double shares = k / (256.0 * SKN_WAVES);
     SknTile best{1, 1, 0.0};
     for (int i = 0; i < 6; ++i) {
         const int mt = shapes[i][0], nt = shapes[i][1];
         if (mt > 1 && mt >= 2 * mtiles) continue;                         // more rows than there are
         const double groups = (double)((mtiles + mt - 1) / mt) * ((n + 16 * nt - 1) / (16 * nt)) / num_cus();
-        const double rounds = groups <= 1.0 ? 1.0 : mt * nt >= 4 ? ceil(groups) : groups;     // the large tiles run one workgroup per CU
-        const double us = 5.5 + iters * rounds * cost[i] * slow;
+        const double further = groups <= 1.0 ? 0.0 : whole[i] * ceil(groups) + (1 - whole[i]) * groups - 1;
+        const double us = 3.9 + 2.06e-6 * m * k + 3.55e-6 * m * n +
+                          (cost[i][0] + cost[i][1] * further) * ((1 - whole_k[i]) * shares + whole_k[i] * ceil(shares));
         if (best.us == 0.0 || us < best.us) best = SknTile{mt, nt, us};
     }
     return best;
