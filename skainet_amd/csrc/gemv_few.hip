@@ -262,6 +262,11 @@ void set_gemv_few(int v) { g_gemv_few = v; }
 //     4 x 14336 x 4096 15.9 -> 16.8)
 //   Q4_K has batched kernels of its own: rows shorter than a wave's share there (8 x 30000 x 512 35.5 -> 12.6) and few long ones (4 x 2048
 //     x 14336 15.3 -> 10.9; 4 x 10000 x 14336 27.3 -> 28.3).
+// Where it is a little slower it stays, for its error against float64 is a third of the row kernel's (1.1e-7 against 3e-7 to 5e-7) and
+// a fortieth of the bf16 quads' (4e-6): Q5_K 3 and 4 rows, K 7168 to 8192, n just above 16384 (18600 x 8192 35.1 -> 37.6 us),
+// 32-element blocks 2 rows, n 1024 to 1200, K 8192 to 10240 (7.9 -> 8.4), Q5_1 1 row 12288 to 13300 x 1536 (8.0 -> 8.6), Q4_K 3 and 4 rows
+// below 1024 x 2048 (4.5 -> 4.7 to 5.4). Of 16800 random products of 1 to 8 rows 18 are more than 3 % slower than without it, none more than
+// 10 %.
 // Besides: rows go in fours per workgroup, so a little more than 16 per CU costs a quarter (Q6_K 4 x 4147 x 6144 13.6 -> 16.2, x 4000
 // 12.1 -> 12.2), and products of 4 us are as long as their launch on either side (within 0.3 us).
 static bool few_by_rule(int enc, int m, int n, int k) {
