@@ -141,9 +141,11 @@ __device__ __forceinline__ void pf_store_block(const pf_u32x4 (&kreg)[PF_KB * (D
 // TEAMS 2: the paired form described above. TEAMS 1: one query group per workgroup of four waves (two workgroups per
 // CU), for calls whose paired grid would leave CUs without a workgroup; where that leaves CUs idle too, several workgroups
 // share a group's keys (splits) and sdpa_prefill_merge_kernel puts their outputs together: what bounds such a call is the
-// chain of blocks a workgroup walks.
-template <int D, int TEAMS>
+// chain of blocks a workgroup walks. SPLIT is a form of its own: with the division of the grid and the second way out in it,
+// calls without splits took 1 to 2 % longer up to 300 keys (0.15 us of 9).
+template <int D, int TEAMS, bool SPLIT>
 __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_kernel(PrefillParams p) {
+    static_assert(!SPLIT || TEAMS == 1, "keys are split in the form with one query group per workgroup");
     constexpr int PF_THREADS = 256 * TEAMS;
     constexpr int KP = D + 8;          // K tile row pitch (bf16): 16-byte aligned rows, 16 lanes of a b128 read on distinct banks
     constexpr int VP = PF_KB + 8;      // V^T tile row pitch (bf16)
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
     const int head_groups = per_kv / hpw;
     const int kvh = blockIdx.y / head_groups;
     const int head = kvh * per_kv + (blockIdx.y % head_groups) * hpw + wave % hpw;
-    const int b = TEAMS == 1 ? blockIdx.z / p.splits : blockIdx.z;
+    const int b = SPLIT ? blockIdx.z / p.splits : blockIdx.z;
     // query groups (a team's share of the query positions). Causal over the whole prefix: team 0 takes group G - 1 - i,
     // team 1 group i (equal work in every workgroup). Under a sliding window, or without the causal rule, every group
     // has about the same work and neighbours share most of their key blocks: groups 2 i + 1 and 2 i. With an odd number
@@ -212,8 +214,8 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
     const int l_beg = first_of(group_first(g_late)) / PF_KB, l_end = (end_of(group_last(g_late)) + PF_KB - 1) / PF_KB;
     int blk_begin = all_keys ? 0 : min(e_beg, l_beg);
     int nblocks = all_keys ? (p.seq_kv + PF_KB - 1) / PF_KB : max(max(e_end, l_end), blk_begin);
-    const int split = TEAMS == 1 ? blockIdx.z % p.splits : 0;
-    if (TEAMS == 1 && p.splits > 1) {                                       // this workgroup's share of the group's blocks (may be none)
+    const int split = SPLIT ? blockIdx.z % p.splits : 0;
+    if (SPLIT) {                                                            // this workgroup's share of the group's blocks (may be none)
         const int share = (nblocks - blk_begin + p.splits - 1) / p.splits;
         blk_begin += split * share;
         nblocks = min(nblocks, blk_begin + share);
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
 
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    if (TEAMS == 1 && p.splits > 1) {
+    if (SPLIT) {
         if (my_q < p.seq_q) {
             const int64_t at = (((int64_t)b * p.heads + head) * p.seq_q + my_q) * p.splits + split;
             float* op = p.part + at * D;
@@ -488,11 +490,14 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
     constexpr size_t smem = sizeof(__bf16) * (2 * PF_KB * (D + 8) + 2 * D * (PF_KB + 8));
     note_kernel("sdpa_prefill_kernel");
     if (paired) {
-        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 2>), smem);
-        sdpa_prefill_kernel<D, 2><<<grid, dim3(512), smem, s>>>(p);
+        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 2, false>), smem);
+        sdpa_prefill_kernel<D, 2, false><<<grid, dim3(512), smem, s>>>(p);
+    } else if (splits > 1) {
+        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 1, true>), smem);
+        sdpa_prefill_kernel<D, 1, true><<<grid, dim3(256), smem, s>>>(p);
     } else {
-        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 1>), smem);
-        sdpa_prefill_kernel<D, 1><<<grid, dim3(256), smem, s>>>(p);
+        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 1, false>), smem);
+        sdpa_prefill_kernel<D, 1, false><<<grid, dim3(256), smem, s>>>(p);
     }
     SKH_CHECK(hipGetLastError());
     if (splits > 1) {
