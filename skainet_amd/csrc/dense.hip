@@ -316,8 +316,13 @@ int launch_fp32_matmul(const float* a, int64_t a_stride, const float* b, int64_t
     // 64 x 128 tiles that do not fill the CUs leave the product to the kernel that splits K over waves; where they fill
     // them the tile kernel reads each operand less often
     const int64_t tiles64 = (int64_t)((n + MT - 1) / MT) * ((m + 63) / 64);
-    // (B read along its rows at an odd alignment and 64 rows or more: the LDS tile kernel, whose loads do not mind)
-    if (g_dense_mfma && k >= 1 && tiles64 < num_cus() && (b_transposed || aligned || m < 64)) {
+    // (B read along its rows at an odd alignment and 64 rows or more: the LDS tile kernel, whose loads do not mind). A K of one
+    // step of a wave has nothing to split: from a quarter of the CUs (half of them for a whole step) the tile kernel is faster
+    // at the same error (232 x 7124 x 20 9.7 -> 6.2 us, 8.3e-8 of float64 either way; 301 x 4660 x 24 7.9 -> 6.0). At larger K
+    // it is, too, above three quarters (712 x 2600 x 84 17.4 and 9.7 us, 468 x 3684 x 416 31.8 and 26.4; none from K 1024 on), but one
+    // chain of K is up to twice as far from float64 as K in shares (1.7e-7 and 1.1e-7 at 84, 4.1e-7 and 2.1e-7 at 512): that stays.
+    const bool shallow = aligned && m >= 64 && n >= 32 && k >= 4 && k <= 32 && tiles64 * (k < 32 ? 4 : 2) >= num_cus();
+    if (g_dense_mfma && k >= 1 && tiles64 < num_cus() && !shallow && (b_transposed || aligned || m < 64)) {
         note_kernel("sgemm_mfma_skinny_kernel");
         if (b_transposed) launch_skinny_rows<true>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
         else launch_skinny_rows<false>(a, a_stride, b, b_stride, c, c_stride, m, n, k);

@@ -481,7 +481,8 @@ def test_dense_matmuls(hip_backend, torch_cuda):
 
 @pytest.mark.parametrize("m,n,k,wt", [(512, 1024, 768, False), (200, 300, 260, False), (64, 32, 4, True), (130, 4096, 516, True),
                                       (1000, 132, 2048, False), (65, 257, 100, True), (1030, 2052, 100, True), (1030, 2052, 36, False),
-                                      (2100, 2100, 20, True), (2100, 2100, 132, False)])
+                                      (2100, 2100, 20, True), (2100, 2100, 132, False), (232, 7124, 20, True), (232, 7124, 36, True), (948, 1164, 32, False), (500, 1284, 28, False),
+                                      (948, 1164, 36, False)])
 def test_dense_fp32_matmul_on_the_matrix_cores(hip_backend, torch_cuda, m, n, k, wt):
     """fp32 operands on the fp32 matrix instruction (exact products, fp32 accumulation in the instruction's order):
     resident operands through the device entries, ragged tiles in every direction, K from one instruction step to many
@@ -504,7 +505,8 @@ def test_dense_fp32_matmul_on_the_matrix_cores(hip_backend, torch_cuda, m, n, k,
         return out.cpu().numpy()
 
     got = run()
-    few = -(-m // 64) * -(-n // 128) < torch.cuda.get_device_properties(0).multi_processor_count
+    tiles, cus = -(-m // 64) * -(-n // 128), torch.cuda.get_device_properties(0).multi_processor_count
+    few = tiles < cus and not (k <= 32 and tiles * (4 if k < 32 else 2) >= cus)          # a K of one step is not split
     assert hip_backend.last_kernel() == ("sgemm_mfma_skinny_kernel" if few else "sgemm_mfma_kernel")
     close(got, want, rel=1e-5, abs_=2e-6 * np.sqrt(k) * 16)
     try:
