@@ -380,38 +380,48 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     // keys that a query can attend: a window bounds them whatever the cache holds
     const int keys = window > 0 ? (int)min((int64_t)seq_kv, (int64_t)window + right_context + seq_q - 1) : seq_kv;
     // One split, no merge behind it: the merge is a second launch (2.8 us of a host's time, and about that between two
-    // dependent kernels on the device), which buys the parallelism of the splits. The choice is the least of an estimate in us.
-    // Measured, 32 heads over 8, D 128, one sequence: 128 keys 7.1 -> 4.6 us, 512 keys 6.8 -> 6.0; 8100 random calls (1 to 16 sequences,
-    // 1 to 64 heads, 1 to 8 queries, 65 to 2400 keys, D 64 and 128) take 0.77 of their time with splits, 8 of them more than 5 %
-    // longer. A key count on the device (a decode step over a growing cache)
+    // dependent kernels on the device), which buys the parallelism of the splits -- and shorter sums: with one split the error
+    // against float64 is up to a third larger (950 keys 1.6e-7 and 2.1e-7). So two estimates in us both have to say that it pays.
+    // Measured, 32 heads over 8, D 128, one sequence: 128 keys 7.1 -> 4.6 us, 512 keys 6.8 -> 6.0; 16 sequences at 1024 keys 25.1 -> 20.6;
+    // 8950 random calls of 1 to 8 queries take 0.785 of their time with splits, 8 of them more than 5 % longer (by the first estimate
+    // alone 0.785 and 107 of 15 500). A key count on the device (a decode step over a growing cache)
     // stays with splits above 256: `keys` is then only a bound, and between a layer's products the cache comes from memory,
     // where a chain of passes waits longer (19 layers at 430 keys: 608 us per step with splits, 664 with one).
     bool single = false;
     const int cols = draft ? per_kv * seq_q : per_kv;           // rows that share a KV head
     if (g_sdpa_decode_one_launch && !leave && g_sdpa_decode_gs.load() == 0 && keys > g_sdpa_decode_split_keys &&
         keys <= (lengths ? 256 : 2048)) {
-        // What bounds a workgroup per 64 keys, fitted to 15 500 such calls with splits (within 5 %) and with one at 1, 2 and 4
-        // rows: a chain of loads and arithmetic, longer with more rows and, at 1 and 2, where the loads miss the L2s (32 MB
-        // together; a group of rows per die keeps a copy of its own); or its share of the traffic, whole workgroups to a CU.
-        static const double hit[2][3] = {{0.235, 0.40, 0.75}, {0.395, 0.60, 1.07}}, miss[2][3] = {{0.44, 0.51, 0.75}, {0.64, 0.68, 1.08}};   // [D 64, 128][1, 2, 4 rows]
         const double once = 8e-6 * batch * kv_heads * keys * head_dim, cus = num_cus();       // MB of K and V
+        const int gs_most = gs, wide = head_dim > 64, slot[5] = {0, 0, 1, 0, 2};              // slot: 1, 2, 4 rows per workgroup
         auto groups_of = [&](int g) { return (double)((cols + g - 1) / g); };
+        auto takes = [&](int g) { return draft ? g == 1 || cols > g / 2 : per_kv % g == 0; };
+        // The first: passes of 32 keys (a chain of loads and arithmetic, longer with more rows per workgroup) or the traffic, every
+        // group of rows that shares a KV head reading it for itself; with splits the traffic alone.
+        static const double pass[2][3] = {{0.137, 0.21, 0.32}, {0.21, 0.30, 0.54}};           // [D 64, 128][slot]
+        bool pays = false;
+        for (int g = 1; g <= gs_most && takes(g); g *= 2) {
+            const double wgs = groups_of(g) * batch * kv_heads, rate = wgs >= 128 ? 7.5 : 6.3 * fmin(1.0, sqrt(wgs / 64));
+            const double one = fmax(4.4, 2.7 + fmax((keys + 31) / 32 * pass[wide][slot[g]] * (head_dim == 256 ? 2 : 1), once * groups_of(g) / rate));
+            pays |= one < 0.95 * fmax(6.8, 4.9 + once * groups_of(gs_most) / 6.9);
+        }
+        // The second, fitted to 15 500 random calls with splits (within 5 %) and with one, counts what the first does not: loads of 1
+        // and 2 rows that miss the L2s (32 MB together; a group of rows per die keeps a copy of its own), workgroups that leave the CUs
+        // uneven shares or crowd the memory from half of them, and the partial outputs. The chains are per 64 keys.
+        static const double hit[2][3] = {{0.235, 0.40, 0.75}, {0.395, 0.60, 1.07}}, miss[2][3] = {{0.44, 0.51, 0.75}, {0.64, 0.68, 1.08}};
         auto misses = [&](int g) { return once * fmin(groups_of(g), 8) > 32; };
-        auto chain = [&](int g) { return (misses(g) ? miss : hit)[head_dim > 64][g == 4 ? 2 : g - 1] * (head_dim == 256 ? 2 : 1); };
+        auto chain = [&](int g) { return (misses(g) ? miss : hit)[wide][slot[g]] * (head_dim == 256 ? 2 : 1); };
         auto uneven = [&](double wgs) { return wgs > cus ? ceil(wgs / cus) * cus / wgs : 1.0; };
         const int gs_split = gs == 4 && !draft && batch * kv_heads * (per_kv / 4) * fmin(SDPA_DECODE_MAX_SPLITS, (keys + 63) / 64) < cus ? 2 : gs;     // as below
         const double groups_split = groups_of(gs_split) * batch * kv_heads, rows = (double)batch * heads * seq_q;
         const int splits_est = (int)fmin(fmin(SDPA_DECODE_MAX_SPLITS, (keys + 63) / 64), ceil(2 * cus / groups_split));
-        const int passes = ((keys + splits_est - 1) / splits_est + 63) / 64;
-        const double wgs_split = groups_split * splits_est;
+        const double passes = ((keys + splits_est - 1) / splits_est + 63) / 64, wgs_split = groups_split * splits_est;
         double best = 0.95 * fmax(8.0, 4.9 + fmax(1.26 * chain(gs_split) * passes * ceil(wgs_split / cus),
                                                   once * groups_of(gs_split) * uneven(wgs_split) / (misses(gs_split) ? 9.5 : 34)) +
                                        8.4e-6 * rows * head_dim * splits_est + 8e-4 * rows);
-        const int most = gs;
-        for (int g = 1; g <= most; g *= 2) {
-            if (draft ? g > 1 && cols <= g / 2 : per_kv % g != 0) break;
-            const double traffic = once * groups_of(g) * uneven(groups_of(g) * batch * kv_heads) / (misses(g) ? 7.5 : 20);
-            const double t = fmax(4.4, 3.7 + fmax((keys + 63) / 64 * chain(g), traffic));
+        for (int g = 1; pays && g <= gs_most && takes(g); g *= 2) {
+            const double wgs = groups_of(g) * batch * kv_heads, traffic = once * groups_of(g) * uneven(wgs) / (misses(g) ? 7.5 : 20);
+            const double crowded = wide && misses(g) && 2 * wgs > cus ? 1.4 : 1.0;
+            const double t = fmax(4.4, 3.7 + fmax((keys + 63) / 64 * chain(g) * crowded, traffic));
             if (t < best) { best = t; gs = g; single = true; }
         }
     }
