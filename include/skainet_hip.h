@@ -449,8 +449,8 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * one-row Q8_0 products stay off the integer matrix cores), "q8_0_mfma_per_cu" (workgroups per CU of that kernel: 1, 2
  * or 4, default 2),
  * "sdpa_prefill_mfma" (0: prompt-shape attention on the fp32 kernel), "sdpa_prefill_teams" (query groups per workgroup of
- * the matrix-core prompt kernel: 1, 2 = a late and an early group paired, 0 = paired where that still fills the chip),
- * "sdpa_prefill_splits" (workgroups that share the keys of an unpaired query group: 1 to 32, 0 = chosen from the shape), "sdpa_decode_split_keys" (least keys per split of
+ * the matrix-core prompt kernel: 1, 2 = two, one after the other, 0 = as many as leave one workgroup per CU),
+ * "sdpa_prefill_splits" (workgroups that share the keys of a query group that has workgroups of its own: 1 to 32, 0 = chosen from the shape), "sdpa_decode_split_keys" (least keys per split of
  * decode-shape attention, default 64), "sdpa_decode_one_launch" (0: short contexts are split over workgroups and merged by a
  * second launch too), "sdpa_decode_gs" (query heads per workgroup of decode-shape attention: 1, 2 or 4, 0 = chosen from
  * the shape), "attn_merge_enable" (0: skainet_hip_attn_out_proj_dev always merges the key

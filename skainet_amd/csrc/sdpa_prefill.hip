@@ -14,26 +14,37 @@
 // plus its mask value (the mask is added to every score), so no key block is skipped.
 //
 // Two launches (three where keys are split over workgroups, see the kernel):
-//   1. kv_to_bf16_kernel: K -> bf16 [kv head][key][D], V -> bf16 transposed [kv head][D][key], keys padded with
-//      zeros to a multiple of 64. (The PV product contracts over keys, and an MFMA operand wants 8 consecutive
-//      contraction values per lane: V has to be read along keys, hence the transpose, done once per call.)
-//   2. sdpa_prefill_kernel: one workgroup = two teams of 4 waves; a team = up to 4 query heads that share a KV head x
-//      32 query positions (fewer heads per KV head: more query blocks per team). The teams of workgroup i take query
-//      group G - 1 - i and query group i of the same KV head (groups 2 i + 1 and 2 i under a sliding window or without
-//      the causal rule, where neighbours share their key blocks): under the causal rule a late group (many keys) and an
-//      early one (few), so every workgroup carries the same work and one workgroup per CU keeps its SIMDs busy from
-//      start to end (with one group per workgroup, which two groups shared a CU was the dispatcher's choice: two late
-//      groups on one CU set the kernel's time). Keys in blocks of 64: the K and V^T tiles of a block go
-//      global -> registers -> LDS (double-buffered, one barrier per block) and are shared by the 8 waves; a block no
-//      wave of either team needs is never loaded. Per wave and block:
+//   1. kv_to_fragments_kernel: K and V -> bf16 in the order the matrix instructions read them, one run of 2 x 64 x D values
+//      per 64-key block (keys padded with zeros). An operand of v_mfma_f32_32x32x16_bf16 is then 1 KB of consecutive bytes
+//      per wave: a block is copied into LDS as it lies (loads that write LDS directly, no registers, no rows to pad) and
+//      read with one conflict-free 16-byte access per lane and instruction. (The PV product contracts over keys, and an
+//      MFMA operand wants 8 consecutive contraction values per lane: V is read along keys, hence the pass in front.)
+//   2. sdpa_prefill_kernel: one workgroup per CU, two teams of 4 waves; a wave = one of up to 4 query heads that share a KV
+//      head x 32 query positions (fewer heads per KV head: more query blocks). Both teams hold the SAME queries; team t
+//      takes key blocks 2 s + t of the group's range in step s and the two states meet in LDS at the end, so the chain of
+//      blocks a wave walks is half the keys and every SIMD has two waves at work until the last step. (With the teams on a late
+//      and an early query group, the workgroup with the latest group ran 32 blocks with one wave per SIMD.) A workgroup takes its
+//      query groups one after the other, a late one and an early one under the causal rule: the same work everywhere, and the
+//      next group's queries and first blocks arrive while the one before is put together and stored.
+//      Measured, 32 heads over 8, D 128, causal, both launches, before and after: 2048 x 2048 67.1 and 50.2 us, 300 x 300 19.1 and
+//      14.9, 1000 x 1000 40.9 and 27.4, 3000 x 3000 152 and 98, a window of 512 keys on 2048 43.0 and 39.1; 64 heads over 8, D 64,
+//      3000 on 5000 286 and 226.
+//      Per wave and block of 64 keys:
 //        S^T[key][query] = K_tile . Q^T           16 MFMAs (Q lives in registers, pre-multiplied by scale * log2 e)
 //        online softmax per query: a query is one accumulator COLUMN, so its 32 scores per 32-key tile sit in
 //          one lane pair (l, l ^ 32): the row statistics need a single cross-lane step
 //        O^T[d][query] += V^T_tile . P            16 MFMAs; P is the S^T accumulator converted in place: the MFMA
 //          contraction index is a free permutation, so the keys a lane holds (4h + {0..3}, 8 + 4h + {0..3} of each
-//          16) are simply declared to be its 8 k-slots and V^T is read in the same order.
+//          16) are simply declared to be its 8 k-slots and V^T is laid out in the same order.
 //      Blocks wholly above the diagonal are skipped, only blocks that cross it (or the end of the keys) mask.
+//      What bounds it: a step of 128 keys takes a CU 1.5 to 1.9 us. Its matrix instructions alone take 0.95 (64 per SIMD of 32
+//      cycles), the LDS reads they need the same (256 KB at 128 B/clk) next to the 64 KB written, the softmax 0.4 to 0.5 per wave pair
+//      of vector time of which little hides behind matrix instructions: measured by taking one kind out at a time, 0.28 us without
+//      the softmax, 0.32 without the loads, 0.18 without the LDS reads. Besides the steps: kv_to_fragments_kernel 6 to 7 us, the first
+//      round trip 4, two to five for a group's end (the second pass over that code takes a third of the first: instruction cache).
 #include "common.h"
+
+#include <type_traits>
 
 namespace skh {
 
@@ -44,149 +55,137 @@ typedef uint32_t pf_u32x4 __attribute__((ext_vector_type(4)));   // a native 16-
 
 constexpr int PF_KB = 64;          // keys per block
 constexpr int PF_QW = 32;          // query positions per wave
+constexpr int PF_THREADS = 512;    // two teams of four waves
+template <int D> constexpr int pf_block_bytes() { return 2 * PF_KB * D * (int)sizeof(__bf16); }   // K, then V, of one block
 
-// K [b][kvh][kv_capacity][D] fp32 -> kb [b*kvh][spad][D] bf16;  V -> vt [b*kvh][D][spad] bf16. One workgroup per
-// (64-key block, kv head, batch); keys >= seq_kv are written as zeros.
+// K, V [b][kvh][kv_capacity][D] fp32 -> [b * kvh][block of 64 keys][K | V] bf16, each of the two in operand order:
+//   K: [32-key tile][step of 16 d][lane = (key of the tile, half h)][d 8 h .. 8 h + 7 of the step]
+//   V: [32-key tile][16 keys][32-row tile of d][lane = (d of the tile, half h)][keys 4 h .. 4 h + 3, 8 + 4 h .. 8 + 4 h + 3 of the 16]
+// One workgroup per (32-key tile, kv head, batch), built in LDS and written out as consecutive kilobytes; keys >= seq_kv are
+// zeros. Bound by latency: a round trip for the loads, one for the stores (2048 keys x 8 heads are 512 workgroups of 48 KB).
 template <int D>
-__global__ __launch_bounds__(256) void kv_to_bf16_kernel(const float* __restrict__ k, const float* __restrict__ v,
-                                                         __bf16* __restrict__ kb, __bf16* __restrict__ vt, int kv_heads,
-                                                         int seq_kv, int kv_capacity, int spad) {
-    __shared__ float tile[PF_KB][D + 1];
-    const int k0 = blockIdx.x * PF_KB;
+__global__ __launch_bounds__(256) void kv_to_fragments_kernel(const float* __restrict__ k, const float* __restrict__ v,
+                                                              __bf16* __restrict__ frag, int kv_heads, int seq_kv, int kv_capacity, int spad) {
+    __shared__ __attribute__((aligned(16))) __bf16 kimg[32 * D];
+    __shared__ __attribute__((aligned(16))) __bf16 vimg[32 * D];
+    const int tile = blockIdx.x, k0 = 32 * tile, tid = threadIdx.x;
     const int64_t head = (int64_t)blockIdx.z * kv_heads + blockIdx.y;
     const float* ksrc = k + head * kv_capacity * D;
     const float* vsrc = v + head * kv_capacity * D;
-    // K: straight conversion, 4 floats per thread-step; every load of the workgroup's 64 KB is requested before the
-    // first value is used (keys past the sequence: a clamped address, zeroed afterwards)
-    constexpr int STEPS = PF_KB * D / 4 / 256;
-    float4 xs[STEPS], ys[STEPS];
+    constexpr int KT = 32 * D / 8 / 256;                     // K: thread-step = 8 consecutive d of a key
+    constexpr int VN = 8 * (D / 4);                          // V: threads with a task of 4 consecutive keys x 4 consecutive d
+    float4 kx[KT][2], vx[4];
 #pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        const int t = threadIdx.x + 256 * i, key = t / (D / 4), d4 = t % (D / 4);
-        const int64_t off = (int64_t)min(k0 + key, seq_kv - 1) * D + 4 * d4;
-        xs[i] = *reinterpret_cast<const float4*>(ksrc + off);
-        ys[i] = *reinterpret_cast<const float4*>(vsrc + off);
+    for (int i = 0; i < KT; ++i) {
+        const int t = tid + 256 * i, key = t / (D / 8), c = t % (D / 8);
+        const float* p = ksrc + (int64_t)min(k0 + key, seq_kv - 1) * D + 8 * c;
+        kx[i][0] = *reinterpret_cast<const float4*>(p);
+        kx[i][1] = *reinterpret_cast<const float4*>(p + 4);
     }
+    const int d4 = tid % (D / 4), kq = tid / (D / 4);
+    if (VN == 256 || tid < VN)
 #pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        const int t = threadIdx.x + 256 * i, key = t / (D / 4), d4 = t % (D / 4);
+        for (int j = 0; j < 4; ++j) vx[j] = *reinterpret_cast<const float4*>(vsrc + (int64_t)min(k0 + 4 * kq + j, seq_kv - 1) * D + 4 * d4);
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+        const int t = tid + 256 * i, key = t / (D / 8), c = t % (D / 8);
         const float keep = k0 + key < seq_kv ? 1.0f : 0.0f;
-        const float4 x = xs[i], y = ys[i];
-        pf_bf16x4 o;
-        o[0] = (__bf16)(x.x * keep); o[1] = (__bf16)(x.y * keep); o[2] = (__bf16)(x.z * keep); o[3] = (__bf16)(x.w * keep);
-        *reinterpret_cast<pf_bf16x4*>(kb + (head * spad + k0 + key) * D + 4 * d4) = o;
-        tile[key][4 * d4] = y.x * keep; tile[key][4 * d4 + 1] = y.y * keep; tile[key][4 * d4 + 2] = y.z * keep; tile[key][4 * d4 + 3] = y.w * keep;
+        const float4 a = kx[i][0], b = kx[i][1];
+        *reinterpret_cast<pf_bf16x8*>(kimg + (c >> 1) * 512 + ((c & 1) * 32 + key) * 8) =
+            pf_bf16x8{(__bf16)(a.x * keep), (__bf16)(a.y * keep), (__bf16)(a.z * keep), (__bf16)(a.w * keep),
+                      (__bf16)(b.x * keep), (__bf16)(b.y * keep), (__bf16)(b.z * keep), (__bf16)(b.w * keep)};
+    }
+    if (VN == 256 || tid < VN) {
+        // keys 4 kq .. + 3 of the tile: 16-key group kq / 4, of which quad kq % 4 = 2 (slot half) + h
+        const int g = kq >> 2, r = kq & 3, h = r & 1, half = r >> 1;
+        float e[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float keep = k0 + 4 * kq + j < seq_kv ? 1.0f : 0.0f;
+            e[j][0] = vx[j].x * keep; e[j][1] = vx[j].y * keep; e[j][2] = vx[j].z * keep; e[j][3] = vx[j].w * keep;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = 4 * d4 + i;
+            *reinterpret_cast<pf_bf16x4*>(vimg + (g * (D / 32) + (d >> 5)) * 512 + (h * 32 + (d & 31)) * 8 + 4 * half) =
+                pf_bf16x4{(__bf16)e[0][i], (__bf16)e[1][i], (__bf16)e[2][i], (__bf16)e[3][i]};
+        }
     }
     __syncthreads();
-    // V^T: thread-step = (d, 8 consecutive keys)
-    for (int t = threadIdx.x; t < D * PF_KB / 8; t += 256) {
-        const int d = t / (PF_KB / 8), kc = t % (PF_KB / 8);
-        pf_bf16x8 o;
+    // tile `tile` is half (tile % 2) of its block's K part and of its V part
+    __bf16* dst = frag + (head * spad + (k0 & ~(PF_KB - 1))) * 2 * D + (tile & 1) * 32 * D;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = (__bf16)tile[8 * kc + j][d];
-        *reinterpret_cast<pf_bf16x8*>(vt + (head * D + d) * spad + k0 + 8 * kc) = o;
+    for (int i = 0; i < 32 * D / 8 / 256; ++i) {
+        const int c = 8 * (tid + 256 * i);
+        *reinterpret_cast<pf_u32x4*>(dst + c) = *reinterpret_cast<const pf_u32x4*>(kimg + c);
+        *reinterpret_cast<pf_u32x4*>(dst + PF_KB * D + c) = *reinterpret_cast<const pf_u32x4*>(vimg + c);
     }
 }
 
 struct PrefillParams {
     const float* q;
-    const __bf16 *kb, *vt;
+    const __bf16* frag;        // kv_to_fragments_kernel's output
     float* out;
     int heads, kv_heads, seq_q, seq_kv, spad;
     float scale_log2e;
     int causal, window, right_context;
     const int32_t* lengths;    // per-sequence key counts on the device, or null
-    int heads_per_wg;      // 1, 2 or 4 query heads of one KV head per workgroup
+    int heads_per_wg;          // 1, 2 or 4 query heads of one KV head per workgroup
+    int head_groups;           // workgroups' worth of query heads per KV head
+    int ngroups;               // query groups of 128 / heads_per_wg positions
     const float* mask;         // additive mask or null; dims 1 or the full extent (heads: 1, kv_heads or heads)
     int mask_b, mask_h, mask_q, mask_k;
-    int splits;                // workgroups that share a query group's keys (one team only)
+    int places;                // workgroups that share the query groups of a KV head's heads
+    int splits;                // workgroups that share a query group's keys (one group per workgroup only)
     float* part;               // [row][splits][D] unnormalised outputs, row = (b, head, query); splits > 1 only
     float* ml;                 // [row][splits][2] running maximum (in units of ln 2) and sum
     int out_rows;              // 0: out is [batch, heads, seq_q, D]; 1: [batch, seq_q, heads, D], token rows of a projection's input
 };
 
-// One 64-key block of the bf16 K and V^T copies: global -> registers, and registers -> the LDS tiles.
-// PF_THREADS threads of a workgroup (one or two teams of four waves) stage a block together
-template <int D, int PF_THREADS>
-__device__ __forceinline__ void pf_load_block(pf_u32x4 (&kreg)[PF_KB * (D / 8) / PF_THREADS], pf_u32x4 (&vreg)[D * (PF_KB / 8) / PF_THREADS],
-                                              const __bf16* kbase, const __bf16* vbase, int spad, int k0, int tid) {
-    constexpr int KCH = D / 8;
-#pragma unroll
-    for (int j = 0; j < PF_KB * KCH / PF_THREADS; ++j) {
-        const int c = tid + PF_THREADS * j, key = c / KCH, ch = c % KCH;
-        kreg[j] = *reinterpret_cast<const pf_u32x4*>(kbase + (int64_t)(k0 + key) * D + 8 * ch);
-    }
-#pragma unroll
-    for (int j = 0; j < D * (PF_KB / 8) / PF_THREADS; ++j) {
-        const int c = tid + PF_THREADS * j, d = c / (PF_KB / 8), ch = c % (PF_KB / 8);
-        vreg[j] = *reinterpret_cast<const pf_u32x4*>(vbase + (int64_t)d * spad + k0 + 8 * ch);
-    }
+// 16 bytes per lane from base + off into LDS at lds_addr + 16 * lane (M0 carries the LDS address). Nothing but
+// pf_wait_loads waits for it.
+__device__ __forceinline__ void pf_load_to_lds(uint32_t lds_addr, uint32_t off, const uint8_t* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory");
 }
-template <int D, int PF_THREADS>
-__device__ __forceinline__ void pf_store_block(const pf_u32x4 (&kreg)[PF_KB * (D / 8) / PF_THREADS], const pf_u32x4 (&vreg)[D * (PF_KB / 8) / PF_THREADS],
-                                               __bf16* kt, __bf16* vt, int tid) {
-    constexpr int KCH = D / 8, KP = D + 8, VP = PF_KB + 8;
-#pragma unroll
-    for (int j = 0; j < PF_KB * KCH / PF_THREADS; ++j) {
-        const int c = tid + PF_THREADS * j, key = c / KCH, ch = c % KCH;
-        *reinterpret_cast<pf_u32x4*>(kt + key * KP + 8 * ch) = kreg[j];
-    }
-#pragma unroll
-    for (int j = 0; j < D * (PF_KB / 8) / PF_THREADS; ++j) {
-        const int c = tid + PF_THREADS * j, d = c / (PF_KB / 8), ch = c % (PF_KB / 8);
-        *reinterpret_cast<pf_u32x4*>(vt + d * VP + 8 * ch) = vreg[j];
-    }
+// max(v of this lane, v of the lane 32 away)
+__device__ __forceinline__ float pf_max_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+// A barrier for what the waves exchange through LDS. (__syncthreads also waits for every global load and store in flight: the next
+// group's queries, the outputs of the one before.)
+__device__ __forceinline__ void pf_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void pf_wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// TEAMS 2: the paired form described above. TEAMS 1: one query group per workgroup of four waves (two workgroups per
-// CU), for calls whose paired grid would leave CUs without a workgroup; where that leaves CUs idle too, several workgroups
-// share a group's keys (splits) and sdpa_prefill_merge_kernel puts their outputs together: what bounds such a call is the
-// chain of blocks a workgroup walks. SPLIT is a form of its own: with the division of the grid and the second way out in it,
-// calls without splits took 1 to 2 % longer up to 300 keys (0.15 us of 9).
-template <int D, int TEAMS, bool SPLIT>
-__global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_kernel(PrefillParams p) {
-    static_assert(!SPLIT || TEAMS == 1, "keys are split in the form with one query group per workgroup");
-    constexpr int PF_THREADS = 256 * TEAMS;
-    constexpr int KP = D + 8;          // K tile row pitch (bf16): 16-byte aligned rows, 16 lanes of a b128 read on distinct banks
-    constexpr int VP = PF_KB + 8;      // V^T tile row pitch (bf16)
+// SPLIT: several workgroups share a group's keys, where one group per workgroup leaves CUs idle, and
+// sdpa_prefill_merge_kernel puts their outputs together: what bounds such a call is the chain of blocks a workgroup walks.
+template <int D, bool SPLIT, bool MASKED>
+__global__ __launch_bounds__(PF_THREADS, 2) void sdpa_prefill_kernel(PrefillParams p) {
     constexpr int NT = D / 16;         // MFMA steps along head_dim for S
     constexpr int ND = D / 32;         // 32-row tiles of O^T
-    constexpr int KCH = D / 8;         // 16-byte chunks per K row
-    constexpr int K_LOADS = PF_KB * KCH / PF_THREADS;       // 16-byte loads per thread for the K tile
-    constexpr int V_LOADS = D * (PF_KB / 8) / PF_THREADS;   // and for the V^T tile
-    extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];       // 2 K tiles, then 2 V^T tiles
-    __bf16* const ktile0 = reinterpret_cast<__bf16*>(pf_smem);
-    __bf16* const vtile0 = ktile0 + 2 * PF_KB * KP;
+    constexpr int BLK = pf_block_bytes<D>();
+    constexpr int SHARE = BLK / 4;     // bytes of a block that each of a team's four waves loads
+    // two buffers of two blocks (one per team); the teams' states meet in whichever is not being read, and in pf_ml
+    extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+    float2* const pf_ml = reinterpret_cast<float2*>(pf_smem + 4 * BLK);     // [team][wave][lane]
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), team = TEAMS == 2 ? wave_all >> 2 : 0, wave = wave_all & 3;
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), team = wave_all >> 2, wave = wave_all & 3;
     const int col = lane & 31, h = lane >> 5;
-    const int per_kv = p.heads / p.kv_heads;
-    const int hpw = p.heads_per_wg;
-    const int qblocks_per_wg = 4 / hpw;
-    const int head_groups = per_kv / hpw;
-    const int kvh = blockIdx.y / head_groups;
-    const int head = kvh * per_kv + (blockIdx.y % head_groups) * hpw + wave % hpw;
+    const int hpw = p.heads_per_wg;               // 1, 2 or 4
+    const int q_per_group = 4 * PF_QW >> (hpw >> 1);
+    // heads run fastest over the grid: workgroups that read the same keys land on the same die where there are 8 KV heads
+    const int place = blockIdx.y;
+    const int head = blockIdx.x * hpw + (wave & (hpw - 1));
+    const int kvh = p.head_groups == 1 ? blockIdx.x : blockIdx.x / p.head_groups;
+    const int qblock = wave >> (hpw >> 1);        // this wave's 32 queries of a group
     const int b = SPLIT ? blockIdx.z / p.splits : blockIdx.z;
-    // query groups (a team's share of the query positions). Causal over the whole prefix: team 0 takes group G - 1 - i,
-    // team 1 group i (equal work in every workgroup). Under a sliding window, or without the causal rule, every group
-    // has about the same work and neighbours share most of their key blocks: groups 2 i + 1 and 2 i. With an odd number
-    // of groups one group is team 0's alone.
-    const int q_per_group = qblocks_per_wg * PF_QW;
-    const int ngroups = (p.seq_q + q_per_group - 1) / q_per_group;
-    const bool adjacent = p.window > 0 || !p.causal;
-    int g_early, g_late;
-    if (TEAMS == 2) {
-        g_early = adjacent ? 2 * (int)blockIdx.x : (int)blockIdx.x;
-        g_late = adjacent ? min(g_early + 1, ngroups - 1) : ngroups - 1 - (int)blockIdx.x;
-    } else {
-        g_late = g_early = p.causal ? ngroups - 1 - (int)blockIdx.x : (int)blockIdx.x;   // the groups with the most keys start first
-    }
-    const int my_group = team ? g_early : g_late;
-    const bool team_active = TEAMS == 1 || !(team == 1 && g_early == g_late);
-    const int q0 = my_group * q_per_group + (wave / hpw) * PF_QW;          // first query position of this wave
-    auto group_first = [&](int g) { return g * q_per_group; };
-    auto group_last = [&](int g) { return min(p.seq_q, (g + 1) * q_per_group) - 1; };
+    // the workgroup's groups, those with the most keys first: of every 2 p.places groups the one at its place and the one at its
+    // place from the end
+    auto group_of = [&](int turn) {
+        const int rank = turn * p.places + ((turn & 1) ? p.places - 1 - place : place);
+        return rank >= p.ngroups ? -1 : p.causal ? p.ngroups - 1 - rank : rank;
+    };
     const int shift = p.seq_kv - p.seq_q;                                   // absolute position of query 0
     const int len = p.lengths ? p.lengths[b] : p.seq_kv;
     // attended keys [first, end) of a query position: both bounds grow with the position
@@ -197,210 +196,326 @@ __global__ __launch_bounds__(256 * TEAMS, TEAMS == 1 ? 2 : 1) void sdpa_prefill_
         if (p.causal) e = min(e, qi + shift + 1);
         return max(min(e, len), 0);
     };
-    const int my_q = q0 + col;
-    const int my_qc = min(my_q, p.seq_q - 1);
-    const bool masked = p.mask != nullptr;                                  // uniform
-    const int real_first = first_of(my_qc), real_last = end_of(my_qc) - 1;  // the rules' own range (may be empty)
-    // no key left: every key of the sequence, equally (with a mask the -1e30 scores do that by themselves)
-    const bool my_uniform = !masked && first_of(my_qc) >= end_of(my_qc);
-    const int my_first_key = my_uniform ? 0 : first_of(my_qc);
-    const int my_last_key = my_uniform ? p.seq_kv - 1 : end_of(my_qc) - 1;
-    const bool wave_uniform = __ballot(my_uniform) != 0;
-    const bool wg_uniform = __syncthreads_or(my_uniform) != 0;
-    // keys any wave of this workgroup needs: the two teams' ranges (both bounds grow with the query position), whole
-    // blocks; between the early team's last block and the late team's first (a sliding window) lie blocks nobody needs
-    const bool all_keys = wg_uniform || masked;
-    const int e_beg = first_of(group_first(g_early)) / PF_KB, e_end = (end_of(group_last(g_early)) + PF_KB - 1) / PF_KB;
-    const int l_beg = first_of(group_first(g_late)) / PF_KB, l_end = (end_of(group_last(g_late)) + PF_KB - 1) / PF_KB;
-    int blk_begin = all_keys ? 0 : min(e_beg, l_beg);
-    int nblocks = all_keys ? (p.seq_kv + PF_KB - 1) / PF_KB : max(max(e_end, l_end), blk_begin);
-    const int split = SPLIT ? blockIdx.z % p.splits : 0;
-    if (SPLIT) {                                                            // this workgroup's share of the group's blocks (may be none)
-        const int share = (nblocks - blk_begin + p.splits - 1) / p.splits;
-        blk_begin += split * share;
-        nblocks = min(nblocks, blk_begin + share);
-    }
-    auto needed = [&](int blk) { return all_keys || (blk >= e_beg && blk < e_end) || (blk >= l_beg && blk < l_end); };
-    auto next_needed = [&](int blk) { int nb = blk + 1; while (nb < nblocks && !needed(nb)) ++nb; return nb; };
-    // this wave's 32 positions: the keys any of them attends, and the keys all of them attend
-    const int q_wave_last = min(q0 + PF_QW - 1, p.seq_q - 1), q_wave_first = min(q0, p.seq_q - 1);
-    const int wave_first_key = (wave_uniform || masked) ? 0 : first_of(q_wave_first);
-    const int wave_last_key = !team_active ? -1 : (wave_uniform || masked) ? p.seq_kv - 1 : end_of(q_wave_last) - 1;
-    const int wave_common_first = first_of(q_wave_last), wave_common_last = end_of(q_wave_first) - 1;
-
-    // Q fragment: lane (query col, half h) holds q[16 t + 8 h .. + 7] for every t, times scale * log2(e)
-    pf_bf16x8 qf[NT];
-    {
-        const int qrow = min(my_q, p.seq_q - 1);
-        const float* qp = p.q + (((int64_t)b * p.heads + head) * p.seq_q + qrow) * D + 8 * h;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const float4 a = *reinterpret_cast<const float4*>(qp + 16 * t);
-            const float4 c = *reinterpret_cast<const float4*>(qp + 16 * t + 4);
-            const float f = p.scale_log2e;
-            qf[t] = pf_bf16x8{(__bf16)(a.x * f), (__bf16)(a.y * f), (__bf16)(a.z * f), (__bf16)(a.w * f),
-                              (__bf16)(c.x * f), (__bf16)(c.y * f), (__bf16)(c.z * f), (__bf16)(c.w * f)};
-        }
-    }
-
-    // this lane's row of the mask (one query position; the key index is added per score), in units of ln 2 later
-    const float* mrow = nullptr;
-    if (masked) {
-        const int bi = p.mask_b == 1 ? 0 : b;
-        const int hi = p.mask_h == 1 ? 0 : (p.mask_h == p.heads ? head : kvh);
-        mrow = p.mask + (((int64_t)bi * p.mask_h + hi) * p.mask_q + (p.mask_q == 1 ? 0 : my_qc)) * p.mask_k;
-    }
+    constexpr bool masked = MASKED;
     const int64_t kvhead = (int64_t)b * p.kv_heads + kvh;
-    const __bf16* kbase = p.kb + kvhead * p.spad * D;
-    const __bf16* vbase = p.vt + kvhead * D * p.spad;
-    pf_u32x4 kreg[K_LOADS], vreg[V_LOADS];
-    pf_f32x16 oacc[ND];
+    const uint8_t* const frag = reinterpret_cast<const uint8_t*>(p.frag) + kvhead * p.spad * (4 * D) + wave * SHARE;
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)pf_smem + team * BLK + wave * SHARE;
+    const uint32_t lane_off = 16u * lane;
+    // this wave's share of block blk into its team's place in buffer buf
+    auto load_block = [&](int blk, int buf) {
+        const uint8_t* src = frag + (int64_t)__builtin_amdgcn_readfirstlane(blk) * BLK;
+        const uint32_t dst = lds0 + __builtin_amdgcn_readfirstlane(buf) * (2 * BLK);
 #pragma unroll
-    for (int i = 0; i < ND; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) oacc[i][e] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;     // per query (column); l_run is this lane's half of the keys
+        for (int u = 0; u < SHARE / 1024; ++u) pf_load_to_lds(dst + u * 1024, lane_off, src + u * 1024);
+    };
 
-    int blk = blk_begin;
-    while (blk < nblocks && !needed(blk)) ++blk;
-    if (blk < nblocks) {
-        pf_load_block<D, PF_THREADS>(kreg, vreg, kbase, vbase, p.spad, blk * PF_KB, tid);
-        pf_store_block<D, PF_THREADS>(kreg, vreg, ktile0, vtile0, tid);
-    }
-    __syncthreads();
+    const int split = SPLIT ? blockIdx.z % p.splits : 0;
+    // does a group hold a query that the rules leave no key? Such a query weighs every key of the sequence equally (with a mask
+    // the -1e30 scores do that by themselves), so its group walks all of them. The same answer in every wave.
+    auto walks_all = [&](int group) {
+        if (masked) return true;
+        const int qa = min(group * q_per_group + min(lane, q_per_group - 1), p.seq_q - 1);
+        const int qb = min(group * q_per_group + min(lane + 64, q_per_group - 1), p.seq_q - 1);
+        return __ballot(first_of(qa) >= end_of(qa) || first_of(qb) >= end_of(qb)) != 0;
+    };
+    // the key blocks [blk0, blk1) a group walks (under SPLIT this workgroup's share of them, which may be none)
+    auto blocks_of = [&](int group, int& blk0, int& blk1) {
+        const bool all_keys = walks_all(group);
+        blk0 = all_keys ? 0 : first_of(group * q_per_group) / PF_KB;
+        blk1 = ((all_keys ? p.seq_kv : end_of(min(p.seq_q, (group + 1) * q_per_group) - 1)) + PF_KB - 1) / PF_KB;
+        if (SPLIT) {
+            const int share = (blk1 - blk0 + p.splits - 1) / p.splits;
+            blk0 += split * share;
+            blk1 = min(blk1, blk0 + share);
+        }
+        blk1 = max(blk1, blk0);
+    };
+    // Half of a wave's 32 x D queries (the other half is its partner's in the other team): 16 rows x 64 bytes per load
+    float4 qraw[NT];
+    auto load_q = [&](int group) {
+        int at = lane;
+        asm volatile("" : "+v"(at));              // see the end of a group
+        const int row = min(group * q_per_group + qblock * PF_QW + 16 * team + (at & 15), p.seq_q - 1);
+        const float* qp = p.q + (((int64_t)b * p.heads + head) * p.seq_q + row) * D + 4 * (at >> 4);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) qraw[t] = *reinterpret_cast<const float4*>(qp + 16 * t);
+    };
+    int blk0, blk1, par = 0;                                                // step st of a group reads buffer (par + st) % 2
+    int group = group_of(0);
+    blocks_of(group, blk0, blk1);
+    if (blk0 + team < blk1) load_block(blk0 + team, par);
+    load_q(group);
 
-    for (int buf = 0; blk < nblocks; buf ^= 1) {
-        const int k0 = blk * PF_KB;
-        const int nblk = next_needed(blk);
-        if (nblk < nblocks) pf_load_block<D, PF_THREADS>(kreg, vreg, kbase, vbase, p.spad, nblk * PF_KB, tid);
-        if (k0 <= wave_last_key && k0 + PF_KB > wave_first_key) {     // wave-uniform: this wave has keys in the block
-            // S^T tiles: s[j] covers keys k0 + 32 j .. + 31 (rows) x this wave's 32 queries (columns)
-            pf_f32x16 s[2];
+    for (int turn = 1; group >= 0; ++turn) {
+        const int q0 = group * q_per_group + qblock * PF_QW;          // first query position of this wave
+        const int my_q = q0 + col, my_qc = min(my_q, p.seq_q - 1);
+        const int real_first = first_of(my_qc), real_last = end_of(my_qc) - 1;  // the rules' own range (may be empty)
+        const bool my_uniform = !masked && first_of(my_qc) >= end_of(my_qc);
+        const int my_first_key = my_uniform ? 0 : real_first;
+        const int my_last_key = my_uniform ? p.seq_kv - 1 : real_last;
+        const bool wave_uniform = __ballot(my_uniform) != 0;
+        const int steps = (blk1 - blk0 + 1) >> 1;
+        // this wave's 32 positions: the keys any of them attends, and the keys all of them attend
+        const int q_wave_last = min(q0 + PF_QW - 1, p.seq_q - 1), q_wave_first = min(q0, p.seq_q - 1);
+        const int wave_first_key = (wave_uniform || masked) ? 0 : first_of(q_wave_first);
+        const int wave_last_key = (wave_uniform || masked) ? p.seq_kv - 1 : end_of(q_wave_last) - 1;
+        const int wave_common_first = first_of(q_wave_last), wave_common_last = end_of(q_wave_first) - 1;
+
+        // Q fragment: lane (query col, half h) holds q[16 t + 8 h .. + 7] for every t, times scale * log2(e). The two halves meet in the
+        // buffer that the first step does not read (loading the fragment as it is held would touch 32 rows with every load,
+        // in both teams: 512 pieces of 32 bytes per wave where this takes 128 of 64).
+        pf_bf16x8 qf[NT];
+        {
+            __bf16* const qs = reinterpret_cast<__bf16*>(pf_smem + (par ^ 1) * (2 * BLK)) + wave * (32 * D);
+            pf_lds_barrier();                      // the group before has left that buffer
+            const float f = p.scale_log2e;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int t = 0; t < NT; ++t)
+                *reinterpret_cast<pf_bf16x4*>(qs + t * 512 + ((lane >> 5) * 32 + 16 * team + (lane & 15)) * 8 + 4 * ((lane >> 4) & 1)) =
+                    pf_bf16x4{(__bf16)(qraw[t].x * f), (__bf16)(qraw[t].y * f), (__bf16)(qraw[t].z * f), (__bf16)(qraw[t].w * f)};
+            pf_lds_barrier();
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s[j][e] = 0.f;
-                const __bf16* kt = ktile0 + buf * (PF_KB * KP) + (32 * j + col) * KP + 8 * h;
+            for (int t = 0; t < NT; ++t) qf[t] = *reinterpret_cast<const pf_bf16x8*>(qs + t * 512 + lane * 8);
+        }
+        // this lane's row of the mask (one query position; the key index is added per score), in units of ln 2 later
+        const float* mrow = nullptr;
+        if (masked) {
+            const int bi = p.mask_b == 1 ? 0 : b;
+            const int hi = p.mask_h == 1 ? 0 : (p.mask_h == p.heads ? head : kvh);
+            mrow = p.mask + (((int64_t)bi * p.mask_h + hi) * p.mask_q + (p.mask_q == 1 ? 0 : my_qc)) * p.mask_k;
+        }
+        // O^T; accumulator i is d tile (i + team ND / 2) % ND, so the first half of them is what this team finishes
+        pf_f32x16 oacc[ND];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const pf_bf16x8 kf = *reinterpret_cast<const pf_bf16x8*>(kt + 16 * t);
-                    s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[t], s[j], 0, 0, 0);
-                }
-            }
-            if (masked) {
-                // the reference's arithmetic: an excluded key scores -1e30, the mask is added to every score; keys past
-                // the sequence (padding of the last block) take no part. Four adjacent keys per 16-byte mask load.
-                constexpr float LOG2E = 1.4426950408889634f;
+        for (int i = 0; i < ND; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int e = 0; e < 16; ++e) oacc[i][e] = 0.f;
+        float m_run = -INFINITY, l_run = 0.f;     // per query (column); l_run is this lane's half of the keys
+        // Scores come out of the matrix instructions with the reference of their exponentials taken off: it is what the accumulators
+        // start from. Large references (where a score near zero would lose digits to it) and masked calls take it off in settle().
+        pf_f32x16 minus_ref;
+        bool explicit_ref = false;                // wave-uniform
+        auto set_reference = [&]() {
+            const float m = m_run == -INFINITY ? 0.f : m_run;
+            explicit_ref = masked || __ballot(!(fabsf(m) <= 1024.0f)) != 0;
 #pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const int key4 = k0 + 32 * j + 8 * e4 + 4 * h;
-                        float4 mv;
-                        if (p.mask_k == 1) { const float m1 = mrow[0]; mv = make_float4(m1, m1, m1, m1); }
-                        else mv = *reinterpret_cast<const float4*>(mrow + min(key4, p.seq_kv - 4));     // seq_kv is a multiple of 4 here
-                        const float m4[4] = {mv.x, mv.y, mv.z, mv.w};
+            for (int e = 0; e < 16; ++e) minus_ref[e] = explicit_ref ? 0.f : -m;
+        };
+        set_reference();
+
+                    // The reference starts as the maximum over the group's first block, for both teams (weights rounded against two references would
+        // differ by bf16's rounding from those of one): step -1 is team 0's scores of that block and no more.
+        if (team == 0) pf_ml[wave * 64 + lane].x = -INFINITY;
+        for (int st = steps ? -1 : 0; st < steps; ++st) {
+            const int blk = st < 0 ? blk0 : blk0 + 2 * st + team, k0 = blk * PF_KB;
+            if (st != 0) pf_wait_loads();         // this wave's share of the step's block (of step 0 with step -1) ...
+            pf_lds_barrier();                     // ... and everybody's; the other buffer has been read by all
+            const int ahead = st < 0 ? 1 : st + 1;
+            if (st != 0 && blk0 + 2 * ahead + team < blk1) load_block(blk0 + 2 * ahead + team, (par + ahead) & 1);
+            if (st == 0) { m_run = pf_ml[wave * 64 + lane].x; set_reference(); }
+            if ((st < 0 && team) || blk >= blk1 || k0 > wave_last_key || k0 + PF_KB <= wave_first_key) continue;      // wave-uniform: no keys in the block
+            // The block in two halves of 32 keys, a and b: S of a; S of b with the softmax of a between its matrix instructions;
+            // O += V^T . P of a with the softmax of b in between; O += V^T . P of b. The order is pinned (sched_barrier) and
+            // AHEAD operand reads are in flight throughout: left alone, the compiler waits out the latency of every read and puts the
+            // vector work behind the matrix work.
+            const uint8_t* const tile = pf_smem + (2 * ((par + max(st, 0)) & 1) + team) * BLK + lane_off;
+            constexpr int AHEAD = 3, OPS = 2 * NT + 4 * ND;       // K's operands, then V's, as they lie
+            pf_bf16x8 fr[AHEAD];
+            // (V's d tiles in this team's order: team 1 starts with the second half of them)
+            const uint8_t* const first_v = tile + team * (ND / 2) * 1024;
+            const uint8_t* const second_v = tile - team * (ND / 2) * 1024;
+            auto read = [&](int n) {
+                const uint8_t* from = n < 2 * NT ? tile : n % ND < ND / 2 ? first_v : second_v;
+                if (n < OPS) fr[n % AHEAD] = *reinterpret_cast<const pf_bf16x8*>(from + n * 1024);
+            };
+            pf_f32x16 s[2];                       // s[j]: keys k0 + 32 j .. + 31 (rows) x this wave's 32 queries (columns)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int key = key4 + i;
-                            float sc = (key > real_last || key < real_first) ? -1.0e30f * LOG2E : s[j][4 * e4 + i];
-                            sc = fmaf(m4[i], LOG2E, sc);
-                            s[j][4 * e4 + i] = key < p.seq_kv ? sc : -INFINITY;
-                        }
-                    }
-            } else
-            // keys outside this query's range score -inf (they take no part); a query without a range scores every key 0
-            if (wave_uniform || k0 < wave_common_first || k0 + PF_KB - 1 > wave_common_last) {   // wave-uniform: the block crosses a boundary
+            for (int n = 0; n < AHEAD; ++n) read(n);
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int e = 0; e < 16; ++e) s[0][e] = s[1][e] = minus_ref[e];
+            auto qk = [&](int n) {
+                __builtin_amdgcn_sched_barrier(0);
+                s[n / NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[n % AHEAD], qf[n % NT], s[n / NT], 0, 0, 0);
+                read(n + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto hide = [&](int j) {              // the mask and the range rules on the scores of half j
+                            if (masked) {
+                                // the reference's arithmetic: an excluded key scores -1e30, the mask is added to every score; keys past
+                                // the sequence (padding of the last block) take no part. Four adjacent keys per 16-byte mask load.
+                                constexpr float LOG2E = 1.4426950408889634f;
+                                const int lo = real_first - k0 - 4 * h, hi = real_last - k0 - 4 * h, end = p.seq_kv - k0 - 4 * h;
+            #pragma unroll
+                                for (int e4 = 0; e4 < 4; ++e4) {
+                                    const int key4 = k0 + 32 * j + 8 * e4 + 4 * h;
+                                    float4 mv;
+                                    if (p.mask_k == 1) { const float m1 = mrow[0]; mv = make_float4(m1, m1, m1, m1); }
+                                    else mv = *reinterpret_cast<const float4*>(mrow + min(key4, p.seq_kv - 4));     // seq_kv is a multiple of 4 here
+                                    const float m4[4] = {mv.x, mv.y, mv.z, mv.w};
+            #pragma unroll
+                                    for (int i = 0; i < 4; ++i) {
+                                        const int key = 32 * j + 8 * e4 + i;                          // relative to k0 + 4 h
+                                        float sc = (key > hi || key < lo) ? -1.0e30f * LOG2E : s[j][4 * e4 + i];
+                                        sc = fmaf(m4[i], LOG2E, sc);
+                                        s[j][4 * e4 + i] = key < end ? sc : -INFINITY;
+                                    }
+                                }
+                            } else
+                            // keys outside this query's range score -inf (they take no part); a query without a range scores every key 0
+                            if (wave_uniform || k0 < wave_common_first || k0 + PF_KB - 1 > wave_common_last) {   // wave-uniform: the block crosses a boundary
+                                const int lo = my_first_key - k0 - 4 * h, hi = my_last_key - k0 - 4 * h;
+            #pragma unroll
+                                for (int e = 0; e < 16; ++e) {
+                                    const int key = 32 * j + 8 * (e >> 2) + (e & 3);                  // relative to k0 + 4 h
+                                    if (my_uniform) s[j][e] = minus_ref[0];
+                                    if (key > hi || key < lo) s[j][e] = -INFINITY;
+                                }
+                            }
+                        };
+            // Four weights: scores 4 c .. 4 c + 3 of half j
+            float psum[2];
+            auto exps = [&](int j, int c, pf_bf16x8 (&to)[2]) {
+                const float p0 = __builtin_amdgcn_exp2f(s[j][4 * c]), p1 = __builtin_amdgcn_exp2f(s[j][4 * c + 1]);
+                const float p2 = __builtin_amdgcn_exp2f(s[j][4 * c + 2]), p3 = __builtin_amdgcn_exp2f(s[j][4 * c + 3]);
+                psum[0] += p0 + p1; psum[1] += p2 + p3;
+                const int at = 4 * (c & 1);
+                to[c >> 1][at] = (__bf16)p0; to[c >> 1][at + 1] = (__bf16)p1; to[c >> 1][at + 2] = (__bf16)p2; to[c >> 1][at + 3] = (__bf16)p3;
+            };
+            // The reference point of a query's exponentials is lazy: it stays as long as the weights of a half sum to at most 2^8 per
+            // lane (far inside bf16 and fp32 range; the final division by the sum takes the common factor out), so neither the
+            // maximum of a block nor the rescaling of the output accumulators is computed but where some query of the wave needs a
+            // new reference -- for most waves the first half of the first block only. A sum that is no number comes here too.
+            auto settle = [&](int j, pf_bf16x8 (&to)[2]) {
+                if (!explicit_ref && __ballot(!(psum[0] + psum[1] <= 256.0f) || m_run == -INFINITY) == 0) return;      // wave-uniform
+                const float off = -minus_ref[0];                              // what the scores are already less
+                float mx = s[j][0];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const int key = k0 + 32 * j + 8 * (e >> 2) + 4 * h + (e & 3);
-                        if (my_uniform) s[j][e] = 0.f;
-                        if (key > my_last_key || key < my_first_key) s[j][e] = -INFINITY;
-                    }
-            }
-            float mx = s[0][0];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[j][e]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            // The reference point of the exponentials follows the running maximum lazily: it moves only when a block's
-            // maximum exceeds it by more than 8 (in units of ln 2; weights then stay below 2^8, far inside bf16 and fp32
-            // range, and the final division by the sum takes the common factor out). So the 64 output accumulators are
-            // rescaled in the few blocks where some query of the wave moves its reference -- for most waves the first
-            // block only -- instead of in every block.
-            const bool move = mx > m_run + 8.0f;                                      // also the first block (m_run = -inf) with any finite score
-            const float m_new = move ? mx : m_run;
-            // a query of a padded row past seq_q, or a block wholly past a query's keys, can leave m_new at -inf
-            const float m_use = m_new == -INFINITY ? 0.f : m_new;
-            float psum = 0.f;
-            pf_bf16x8 pf[4];                                         // pf[2 j + g]: keys 16 g .. of tile j, this lane's 8 slots
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float pr[16];
-#pragma unroll
-                for (int e = 0; e < 16; ++e) { pr[e] = __builtin_amdgcn_exp2f(s[j][e] - m_use); psum += pr[e]; }
-                pf[2 * j] = pf_bf16x8{(__bf16)pr[0], (__bf16)pr[1], (__bf16)pr[2], (__bf16)pr[3],
-                                      (__bf16)pr[4], (__bf16)pr[5], (__bf16)pr[6], (__bf16)pr[7]};
-                pf[2 * j + 1] = pf_bf16x8{(__bf16)pr[8], (__bf16)pr[9], (__bf16)pr[10], (__bf16)pr[11],
-                                          (__bf16)pr[12], (__bf16)pr[13], (__bf16)pr[14], (__bf16)pr[15]};
-            }
-            if (__ballot(move) != 0) {                                               // wave-uniform
-                const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_use) : 1.0f;   // m_run = -inf -> 0
+                for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[j][e]);
+                mx = pf_max_halves(mx) + off;
+                const bool move = mx > m_run + (explicit_ref ? 8.0f : 0.0f);  // no reference yet (-inf): with any finite score
+                const float m_new = move ? mx : m_run, use = m_new == -INFINITY ? 0.f : m_new;      // keys wholly past a query's range leave it at -inf
+                const float alpha = move ? __builtin_amdgcn_exp2f(m_run - use) : 1.0f;              // m_run = -inf -> 0
+                m_run = m_new;
                 l_run *= alpha;
 #pragma unroll
                 for (int i = 0; i < ND; ++i)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) oacc[i][e] *= alpha;
-            }
-            l_run += psum;
-            m_run = m_new;
+                set_reference();
+#pragma unroll
+                for (int e = 0; e < 16; ++e) { s[j][e] -= use - off; if (j == 0) s[1][e] += off + minus_ref[0]; }
+                psum[0] = psum[1] = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) exps(j, c, to);
+            };
+            pf_bf16x8 pf[2], pg[2];               // weights of the two halves: keys 16 g .. of a half, this lane's 8 slots
             // O^T += V^T . P : A = V^T rows d, this lane's k-slots are keys 16 g + 4 h + {0..3} and 16 g + 8 + 4 h + {0..3}
+            auto pv = [&](int n, pf_bf16x8 (&from)[2]) {
+                __builtin_amdgcn_sched_barrier(0);
+                oacc[n % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[(2 * NT + n) % AHEAD], from[(n / ND) & 1], oacc[n % ND], 0, 0, 0);
+                read(2 * NT + n + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+            };
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
+            for (int n = 0; n < NT + NT / 4; ++n) qk(n);
+            hide(0);
+            psum[0] = psum[1] = 0.f;
 #pragma unroll
-                for (int i = 0; i < ND; ++i) {
-                    const __bf16* vp = vtile0 + buf * (D * VP) + (32 * i + col) * VP + 16 * g + 4 * h;
-                    const pf_bf16x4 lo = *reinterpret_cast<const pf_bf16x4*>(vp);
-                    const pf_bf16x4 hi = *reinterpret_cast<const pf_bf16x4*>(vp + 8);
-                    const pf_bf16x8 vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    oacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[g], oacc[i], 0, 0, 0);
-                }
+            for (int n = NT + NT / 4; n < 2 * NT; ++n) {
+                qk(n);
+                if (n >= 2 * NT - 4 && NT >= 8) exps(0, n - (2 * NT - 4), pf);
             }
+            if (NT < 8)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) exps(0, c, pf);
+            hide(1);
+            if (st < 0) {
+                float mx = s[0][0];
+#pragma unroll
+                for (int e = 1; e < 32; ++e) mx = fmaxf(mx, s[e >> 4][e & 15]);
+                pf_ml[wave * 64 + lane].x = pf_max_halves(mx);
+                continue;
+            }
+            settle(0, pf);
+            l_run += psum[0] + psum[1];
+            psum[0] = psum[1] = 0.f;
+#pragma unroll
+            for (int n = 0; n < 2 * ND; ++n) {
+                pv(n, pf);
+                if (n >= 2 * ND - 4) exps(1, n - (2 * ND - 4), pg);
+            }
+            settle(1, pg);
+            l_run += psum[0] + psum[1];
+#pragma unroll
+            for (int n = 2 * ND; n < 4 * ND; ++n) pv(n, pg);
         }
-        if (nblk < nblocks) pf_store_block<D, PF_THREADS>(kreg, vreg, ktile0 + (buf ^ 1) * (PF_KB * KP), vtile0 + (buf ^ 1) * (D * VP), tid);
-        __syncthreads();
-        blk = nblk;
-    }
 
-    const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    if (SPLIT) {
-        if (my_q < p.seq_q) {
-            const int64_t at = (((int64_t)b * p.heads + head) * p.seq_q + my_q) * p.splits + split;
-            float* op = p.part + at * D;
+        // The two teams' states of a query put together. Team t finishes d tiles t * ND / 2 .. and hands the others over, through the
+        // buffer that nobody reads any more (the last step read the other one). A team without keys has a maximum of -inf and
+        // takes no part. The next group's queries and first blocks are on their way meanwhile.
+        // (its addresses are formed here, not ahead of the loop: held through it they would not fit the registers, and the reload waits
+        // for everything in flight)
+        int at = lane;
+        asm volatile("" : "+v"(at));
+        const int next_group = group_of(turn);                             // uniform; negative: none
+        if (next_group >= 0) load_q(next_group);
+        const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+        constexpr int HALF = ND / 2, CH = 8 * HALF;                         // 16-byte chunks of an output row's half
+        float4* const xch = reinterpret_cast<float4*>(pf_smem + ((par + steps) & 1) * (2 * BLK));          // [team][wave][4 HALF][lane]
+        float4* const mine_at = xch + (team * 4 + wave) * (4 * HALF * 64);
+        const float4* const theirs_at = xch + ((team ^ 1) * 4 + wave) * (4 * HALF * 64);
+        pf_ml[(team * 4 + wave) * 64 + at] = make_float2(m_run, l_tot);
 #pragma unroll
-            for (int i = 0; i < ND; ++i)
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4)
-                    *reinterpret_cast<float4*>(op + 32 * i + 8 * e4 + 4 * h) =
-                        make_float4(oacc[i][4 * e4], oacc[i][4 * e4 + 1], oacc[i][4 * e4 + 2], oacc[i][4 * e4 + 3]);
-            if (h == 0) *reinterpret_cast<float2*>(p.ml + 2 * at) = make_float2(m_run, l_tot);
-        }
-        return;
-    }
-    if (my_q < p.seq_q && team_active) {
-        float* op = p.out + (p.out_rows ? (((int64_t)b * p.seq_q + my_q) * p.heads + head) : (((int64_t)b * p.heads + head) * p.seq_q + my_q)) * D;
-#pragma unroll
-        for (int i = 0; i < ND; ++i)
+        for (int i = 0; i < HALF; ++i)
 #pragma unroll
             for (int e4 = 0; e4 < 4; ++e4) {
-                const int d = 32 * i + 8 * e4 + 4 * h;
-                *reinterpret_cast<float4*>(op + d) = make_float4(oacc[i][4 * e4] * inv, oacc[i][4 * e4 + 1] * inv,
-                                                                 oacc[i][4 * e4 + 2] * inv, oacc[i][4 * e4 + 3] * inv);
+                const pf_f32x16& o = oacc[HALF + i];
+                mine_at[(4 * i + e4) * 64 + at] = make_float4(o[4 * e4], o[4 * e4 + 1], o[4 * e4 + 2], o[4 * e4 + 3]);
             }
+        pf_lds_barrier();
+        par = (par + steps + 1) & 1;
+        if (next_group >= 0) {
+            blocks_of(next_group, blk0, blk1);
+            if (blk0 + team < blk1) load_block(blk0 + team, par);
+        }
+        const float2 other = pf_ml[((team ^ 1) * 4 + wave) * 64 + at];
+        const float m_all = fmaxf(m_run, other.x), m_ref = m_all == -INFINITY ? 0.f : m_all;
+        float mine = __builtin_amdgcn_exp2f(m_run - m_ref), theirs = __builtin_amdgcn_exp2f(other.x - m_ref);
+        const float l_all = fmaf(mine, l_tot, theirs * other.y);
+        const int64_t row0 = ((int64_t)b * p.heads + head) * p.seq_q;
+        if (SPLIT) {
+            if (team == 0 && at < 32 && q0 + (at & 31) < p.seq_q)
+                *reinterpret_cast<float2*>(p.ml + 2 * ((row0 + q0 + (at & 31)) * p.splits + split)) = make_float2(m_all, l_all);
+        } else {
+            const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
+            mine *= inv; theirs *= inv;
+        }
+#pragma unroll
+        for (int i = 0; i < HALF; ++i)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                pf_f32x16& o = oacc[i];
+                const float4 t = theirs_at[(4 * i + e4) * 64 + at];
+                o[4 * e4] = fmaf(mine, o[4 * e4], theirs * t.x); o[4 * e4 + 1] = fmaf(mine, o[4 * e4 + 1], theirs * t.y);
+                o[4 * e4 + 2] = fmaf(mine, o[4 * e4 + 2], theirs * t.z); o[4 * e4 + 3] = fmaf(mine, o[4 * e4 + 3], theirs * t.w);
+            }
+        pf_lds_barrier();                         // what this wave handed over has been read: its place turns the outputs into rows
+#pragma unroll
+        for (int c = 0; c < 4 * HALF; ++c) {
+            const pf_f32x16& o = oacc[c / 4];
+            mine_at[(at & 31) * CH + ((2 * c + (at >> 5)) ^ (at & (CH - 1)))] = make_float4(o[4 * (c % 4)], o[4 * (c % 4) + 1], o[4 * (c % 4) + 2], o[4 * (c % 4) + 3]);
+        }
+        float* const out0 = SPLIT ? p.part + (row0 * p.splits + split) * D : p.out + (p.out_rows ? (int64_t)b * p.seq_q * p.heads + head : row0) * D;
+        const int64_t pitch = (SPLIT ? p.splits : p.out_rows ? p.heads : 1) * D;
+        const int r0 = at / CH, c0 = at & (CH - 1);
+        float* op = out0 + (q0 + r0) * pitch + 32 * team * HALF + 4 * c0;
+#pragma unroll
+        for (int i = 0; i < 32 * CH / 64; ++i, op += (64 / CH) * pitch) {
+            const int r = (64 / CH) * i + r0;
+            const float4 v = mine_at[r * CH + (c0 ^ (r & (CH - 1)))];
+            if (q0 + r < p.seq_q) *reinterpret_cast<float4*>(op) = v;
+        }
+        group = next_group;
     }
 }
 
@@ -438,28 +553,34 @@ static std::atomic<int> g_prefill_mfma{1};
 void set_sdpa_prefill_mfma(int v) { g_prefill_mfma = v; }
 static std::atomic<int> g_prefill_splits{0};  // 0: chosen from the shape
 void set_sdpa_prefill_splits(int v) { if (v >= 0 && v <= 32) g_prefill_splits = v; }
-static std::atomic<int> g_prefill_teams{0};   // 0: chosen from the grid, 1: one query group per workgroup, 2: paired groups
+static std::atomic<int> g_prefill_teams{0};   // 0: chosen from the grid, 1: one query group per workgroup, 2: two, one after the other
 void set_sdpa_prefill_teams(int v) { if (v >= 0 && v <= 2) g_prefill_teams = v; }
 
 // How many workgroups share a query group's keys, where one group per workgroup leaves CUs idle: a chunk of a long prompt, few
-// heads. Estimates in us, fitted to 22 shapes of 1 to 64 heads, 16 to 3000 queries, 64 to 5000 keys at 1 to 32 splits: a block of
-// 64 keys takes a workgroup 1.8 (D 128) or 1.15 (D 64), half as much again with two workgroups on a CU; splitting costs the
-// merging launch and the partial outputs, written and read at 6 bytes per ps. Measured with one and with the chosen number: 32
-// heads over 8, 64 queries on 2048 keys 67.2 -> 26.4 us, 128 on 2176 69.6 -> 30.2; 8 heads, 1024 on 1024 40.6 -> 26.8; one head, 3000 on
-// 3000 85.3 -> 29.1; 32 heads, 300 on 300 stays (19.2, 22.9 with two).
+// heads. Estimates in us, read off 40 shapes of 1 to 64 heads, 16 to 2500 queries, 20 to 2500 keys at 1 to 32 splits (within 8 % of
+// most of them): launches, prologue and output 9.5; a step of 128 keys 1.65 (D 128) or 1.0 (D 64); splitting costs the merging launch,
+// 3.3, and the partial outputs, written and read at 3 bytes per ps. Measured with one and with the chosen number: 8 heads over 4, 143
+// queries on 1214 keys 26.2 -> 20.4; 4 heads over 2, 73 on 1865, D 64, 23.0 -> 15.5; 8 heads over 4, 1519 on 1519 stays (30.6, 31.1 with two).
 static int prefill_splits(int64_t wgs, int64_t rows, int head_dim, int seq_kv, int q_per_group, int window, int right_context, int batch) {
     const int64_t keys = window > 0 ? min((int64_t)seq_kv, (int64_t)window + right_context + q_per_group) : seq_kv;
     const int blocks = (int)((keys + PF_KB - 1) / PF_KB);
-    const int most = (int)min(min((int64_t)32, 2 * (int64_t)num_cus() / wgs), (int64_t)min(blocks, 65535 / batch));
-    if (g_prefill_splits.load() > 0) return max(1, min(most, g_prefill_splits.load()));
-    const double block_us = head_dim == 64 ? 1.15 : 1.8;
+    const int room = (int)min((int64_t)32, (int64_t)min(blocks, 65535 / batch));
+    if (g_prefill_splits.load() > 0) return max(1, min((int)min((int64_t)room, 2 * (int64_t)num_cus() / wgs), g_prefill_splits.load()));
+    const double step_us = head_dim == 64 ? 1.0 : 1.65;
     int splits = 1;
-    double best = 0.95 * block_us * blocks;
-    for (int n = 2; n <= most; ++n) {
-        const double t = block_us * ((blocks + n - 1) / n) * (wgs * n > num_cus() ? 1.5 : 1.0) + 8.0 + 8.0 * rows * n * (head_dim + 2) / 6e6;
+    double best = 0.97 * (9.5 + step_us * ((blocks + 1) / 2));
+    for (int n = 2; n <= room && n * wgs <= num_cus(); ++n) {
+        const double t = 9.5 + step_us * (((blocks + n - 1) / n + 1) / 2) + 3.3 + 8.0 * rows * n * (head_dim + 2) / 3e6;
         if (t < best) { best = t; splits = n; }
     }
     return splits;
+}
+
+template <int D, bool SPLIT, bool MASKED>
+static int launch_prefill_kernel(dim3 grid, size_t smem, hipStream_t s, const PrefillParams& p) {
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, SPLIT, MASKED>), smem);
+    sdpa_prefill_kernel<D, SPLIT, MASKED><<<grid, dim3(PF_THREADS), smem, s>>>(p);
+    return 0;
 }
 
 template <int D>
@@ -473,32 +594,30 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
     const int hpw = per_kv % 4 == 0 ? 4 : (per_kv % 2 == 0 ? 2 : 1);
     const int q_per_group = (4 / hpw) * PF_QW;
     const int ngroups = (seq_q + q_per_group - 1) / q_per_group;
-    // paired query groups where that still gives every CU a workgroup, else one group per (smaller) workgroup
-    const int64_t paired_wgs = (int64_t)((ngroups + 1) / 2) * kv_heads * (per_kv / hpw) * batch;
-    const bool paired = g_prefill_teams.load() == 0 ? paired_wgs >= num_cus() : g_prefill_teams.load() == 2;
+    const int64_t heads_wgs = (int64_t)kv_heads * (per_kv / hpw) * batch;
+    // One workgroup per CU that takes its share of the query groups one after the other, where such workgroups fill the chip: the next
+    // group's first loads then run under the end of the one before
+    const int share = (int)(num_cus() / heads_wgs);
+    const int teams = g_prefill_teams.load();
+    const int places = min(65535, teams == 1 ? ngroups : teams == 2 ? (ngroups + 1) / 2
+                     : share >= 1 && share < ngroups && share * heads_wgs * 10 >= 9 * (int64_t)num_cus() ? share : ngroups);
+    const bool paired = places < ngroups;
     const size_t rows = (size_t)batch * heads * seq_q;
     const int splits = paired ? 1 : prefill_splits((int64_t)ngroups * kv_heads * (per_kv / hpw) * batch, (int64_t)rows, D, seq_kv, q_per_group, window, right_context, batch);
     uint8_t* ws = static_cast<uint8_t*>(kernel_workspace(2 * elems * sizeof(__bf16) + (splits > 1 ? rows * splits * (D + 2) * sizeof(float) : 0)));
     if (!ws) return -1;
-    __bf16 *kb = reinterpret_cast<__bf16*>(ws), *vt = kb + elems;
-    float* part = reinterpret_cast<float*>(vt + elems);
-    kv_to_bf16_kernel<D><<<dim3(spad / PF_KB, kv_heads, batch), dim3(256), 0, s>>>(k, v, kb, vt, kv_heads, seq_kv, kv_capacity, spad);
+    __bf16* frag = reinterpret_cast<__bf16*>(ws);
+    float* part = reinterpret_cast<float*>(frag + 2 * elems);
+    kv_to_fragments_kernel<D><<<dim3(spad / 32, kv_heads, batch), dim3(256), 0, s>>>(k, v, frag, kv_heads, seq_kv, kv_capacity, spad);
     SKH_CHECK(hipGetLastError());
-    PrefillParams p{q, kb, vt, out, heads, kv_heads, seq_q, seq_kv, spad, scale * 1.4426950408889634f, causal, window, right_context, lengths, hpw,
-                    mask, mask_b, mask_h, mask_q, mask_k, splits, part, part + rows * splits * D, out_rows};
-    const dim3 grid(paired ? (ngroups + 1) / 2 : ngroups, kv_heads * (per_kv / hpw), batch * splits);
-    constexpr size_t smem = sizeof(__bf16) * (2 * PF_KB * (D + 8) + 2 * D * (PF_KB + 8));
+    PrefillParams p{q, frag, out, heads, kv_heads, seq_q, seq_kv, spad, scale * 1.4426950408889634f, causal, window, right_context, lengths, hpw, per_kv / hpw, ngroups,
+                    mask, mask_b, mask_h, mask_q, mask_k, places, splits, part, part + rows * splits * D, out_rows};
+    const dim3 grid(kv_heads * (per_kv / hpw), places, batch * splits);
+    constexpr size_t smem = 4 * pf_block_bytes<D>() + 2 * 4 * 64 * sizeof(float2);
     note_kernel("sdpa_prefill_kernel");
-    if (paired) {
-        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 2, false>), smem);
-        sdpa_prefill_kernel<D, 2, false><<<grid, dim3(512), smem, s>>>(p);
-    } else if (splits > 1) {
-        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 1, true>), smem);
-        sdpa_prefill_kernel<D, 1, true><<<grid, dim3(256), smem, s>>>(p);
-    } else {
-        SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sdpa_prefill_kernel<D, 1, false>), smem);
-        sdpa_prefill_kernel<D, 1, false><<<grid, dim3(256), smem, s>>>(p);
-    }
+    const int rc = splits > 1 ? (mask ? launch_prefill_kernel<D, true, true>(grid, smem, s, p) : launch_prefill_kernel<D, true, false>(grid, smem, s, p))
+                              : (mask ? launch_prefill_kernel<D, false, true>(grid, smem, s, p) : launch_prefill_kernel<D, false, false>(grid, smem, s, p));
+    if (rc != 0) return rc;
     SKH_CHECK(hipGetLastError());
     if (splits > 1) {
         sdpa_prefill_merge_kernel<D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0, s>>>(p, (int64_t)rows);

@@ -679,3 +679,45 @@ def test_attention_prefill_with_the_keys_split_over_workgroups(hip_backend, torc
     finally:
         hip_backend.set_tuning("sdpa_prefill_teams", 0)
         hip_backend.set_tuning("sdpa_prefill_splits", 0)
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,sq,skv,slope,splits", [
+    (4, 1, 128, 96, 96, 100.0, 1), (4, 1, 128, 96, 96, -100.0, 1), (2, 1, 64, 70, 90, 8.0, 1), (1, 1, 64, 70, 90, -100.0, 1), (4, 2, 128, 40, 90, 100.0, 2)])
+def test_attention_prefill_reference_point_moves(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv, slope, splits):
+    """Scores that rise or fall by `slope` from key to key, into the thousands: the reference point of the exponentials moves in every
+    half block (rising), is large (taken off behind the products, not inside them) or stays at the first key's (falling), and the two
+    teams' states and the splits differ by thousands. A query's weight is all on its last (first) key but for e^-7.9 at the smallest
+    slope (multiples of 8 up to 712 are bf16 values, the factor log2 e is rounded by at most 2^-8 for all keys alike; at 100 the keys'
+    rounding, 2^-9 of 9600, leaves a gap of more than 60), so the output is that key's V: bound 2^-8 for bf16's rounding of V and P,
+    plus e^-7.9 / (1 - e^-7.9) of the largest difference of two values."""
+    rng = np.random.default_rng(skv)
+    q = np.zeros((1, heads, sq, d), np.float32)
+    q[..., 0] = 1.0
+    k = np.zeros((1, kv_heads, skv, d), np.float32)
+    k[..., 0] = slope * np.arange(skv)
+    v = rng.standard_normal((1, kv_heads, skv, d)).astype(np.float32)
+    try:
+        hip_backend.set_tuning("sdpa_prefill_teams", 1)
+        hip_backend.set_tuning("sdpa_prefill_splits", splits)
+        got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, 1.0, True)
+        assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+    finally:
+        hip_backend.set_tuning("sdpa_prefill_teams", 0)
+        hip_backend.set_tuning("sdpa_prefill_splits", 0)
+    at = np.arange(sq) + skv - sq if slope > 0 else np.zeros(sq, np.int64)
+    want = np.repeat(v[:, :, at], heads // kv_heads, axis=1)
+    bound = 2.0 ** -8 + (0.0 if abs(slope) > 50 else 2 * np.exp(-7.9) / (1 - np.exp(-7.9)))
+    assert np.abs(got - want).max() <= bound * np.abs(v).max()
+
+
+def test_attention_prefill_workgroup_with_three_query_groups(hip_backend, torch_cuda):
+    """As many workgroups as CUs, each with its share of the query groups one after the other: three turns at the most, the last
+    of them for one workgroup of two only, rows past the end in the last group."""
+    rng = np.random.default_rng(3)
+    b, h, sq, d = 16, 8, 520, 64
+    q, k, v = (rng.standard_normal((b, h, sq, d)).astype(np.float32) for _ in range(3))
+    got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, 0.125, True)
+    assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+    want = L.sdpa(q, k, v, 0.125, True)
+    assert normalized_err(got, want, eps=1.0) <= 2e-2
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 5e-3 * np.abs(want).max()
