@@ -279,29 +279,173 @@ __global__ __launch_bounds__(64 * NW) void sgemm_mfma_skinny_kernel(const float*
     }
 }
 
+// The same product (BT) with the operands brought in through LDS, in loads of W = 4 floats a lane where both operands' rows are 16-byte
+// aligned, of one where they are not. What bounds the kernel above
+// is the address unit: the 16 lanes that one pass of a load serves sit in 16 rows, 16 bytes of a cache line each, and a CU takes in 16 to
+// 18 bytes a cycle (the number of steps in flight, 2 to 4, made no difference). Here a load covers 8 rows (W 1: 2) of 128 consecutive
+// bytes and writes LDS directly; the lanes then read their operands from there. Piece c of row r lies at position c ^ (r % 8) of the
+// row's eight, which the loading lanes arrange by picking their address, so that the reads of 16 rows spread over the banks. STAGES steps of 32
+// elements per wave are in LDS, the same waves take the same steps in the same order as above: the sums have the same bits.
+// Measured (us, above / here): 32 x 4096 x 4096 25.9 / 16.6 (a read of its weight 15), 32 x 1000 x 4096 18.0 / 8.3, 32 x 4096 x 1024
+// 9.2 / 5.9, 32 x 1001 x 4097 18.1 / 10.6, 256 x 4096 x 4096 101 / 77, 32 x 10 x 8192 26.2 / 10.8.
+template <int W>
+__device__ __forceinline__ void dense_load_to_lds(uint32_t lds_addr, uint32_t off, const float* base) {
+    if constexpr (W == 4) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(off), "s"(base) : "memory");
+}
+template <int MTILES, int NT, int NW, int STAGES, int W>
+__global__ __launch_bounds__(64 * NW) void sgemm_mfma_skinny_lds_kernel(const float* __restrict__ a, int64_t a_stride, const float* __restrict__ b,
+                                                                        int64_t b_stride, float* __restrict__ c, int64_t c_stride, int m, int n, int k) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int TILES = MTILES + NT, STAGE_BYTES = TILES * 2048, PER_TILE = 8 / W, LOADS = PER_TILE * TILES;
+    static_assert((STAGES - 1) * LOADS <= 63, "loads in flight must fit the wave's counter");
+    extern __shared__ __attribute__((aligned(16))) uint8_t dense_smem[];      // [wave][stage][tile][16 rows][8 pieces of 16 bytes]; at the end the partial tiles
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int j0 = blockIdx.x * (16 * NT), i0 = blockIdx.y * (16 * MTILES);
+    uint8_t* const mine = dense_smem + wave * (STAGES * STAGE_BYTES);
+    const uint32_t mine_addr = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)mine;
+    // byte offset of what this lane loads of tile t, rows 2 W u .. 2 W u + 2 W - 1 (rows past the end are copies of the last one)
+    uint32_t off[TILES][PER_TILE];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int u = 0; u < PER_TILE; ++u) {
+            const int flt = 64 * W * u + W * lane, row = flt >> 5, piece = ((flt >> 2) & 7) ^ (row & 7);
+            const int at = t < MTILES ? min(i0 + 16 * t + row, m - 1) : min(j0 + 16 * (t - MTILES) + row, n - 1);
+            off[t][u] = (uint32_t)(at * (t < MTILES ? a_stride : b_stride) * 4) + 16u * piece + 4u * (flt & 3);
+        }
+    auto issue = [&](int stage, int step) {
+        const int64_t p = (int64_t)(wave + NW * step) * 32;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int u = 0; u < PER_TILE; ++u)
+                dense_load_to_lds<W>(mine_addr + stage * STAGE_BYTES + t * 2048 + u * (256 * W), off[t][u], (t < MTILES ? a : b) + p);
+    };
+    f32x4 acc[MTILES][NT];
+#pragma unroll
+    for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float sa[MTILES][8], sb[NT][8];
+    auto multiply = [&]() {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[t][e], sb[u][e], acc[t][u], 0, 0, 0);
+    };
+    const int full = k >> 5;                       // whole steps; wave w takes w, w + NW, ...
+    const int steps = full > wave ? (full - wave + NW - 1) / NW : 0;
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s)
+        if (s < steps) issue(s, s);
+    const uint32_t at0 = (uint32_t)(r * 128 + ((q ^ (r & 7)) << 4)), at1 = (uint32_t)(r * 128 + (((q + 4) ^ (r & 7)) << 4));
+    int stage = 0;
+    for (int st = 0; st < steps; ++st) {
+        if (st + STAGES <= steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const uint8_t* const from = mine + stage * STAGE_BYTES;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const float4 x = *reinterpret_cast<const float4*>(from + t * 2048 + at0), y = *reinterpret_cast<const float4*>(from + t * 2048 + at1);
+            float (&s)[8] = t < MTILES ? sa[t < MTILES ? t : 0] : sb[t < MTILES ? 0 : t - MTILES];
+            s[0] = x.x; s[1] = x.y; s[2] = x.z; s[3] = x.w; s[4] = y.x; s[5] = y.y; s[6] = y.z; s[7] = y.w;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the stage has been read: it may be filled again
+        if (st + STAGES < steps) issue(stage, st + STAGES);
+        multiply();
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+    if ((k & 31) && wave == full % NW) {           // the last, partial step: elements past K are zeros on both sides
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t at = (int64_t)full * 32 + 4 * q + (e < 4 ? e : 12 + e);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sb[t][e] = at < k ? b[(int64_t)min(j0 + 16 * t + r, n - 1) * b_stride + at] : 0.f;
+#pragma unroll
+            for (int t = 0; t < MTILES; ++t) sa[t][e] = at < k ? a[(int64_t)min(i0 + 16 * t + r, m - 1) * a_stride + at] : 0.f;
+        }
+        multiply();
+    }
+    __syncthreads();                               // every wave is through with its stages
+    float* const part = reinterpret_cast<float*>(dense_smem);      // [wave][tile][256]
+    // accumulator element e of lane (r, q): row 4 q + e, column r of the tile
+#pragma unroll
+    for (int t = 0; t < MTILES; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[(wave * (MTILES * NT) + t * NT + u) * 256 + (4 * q + e) * 16 + r] = acc[t][u][e];
+    __syncthreads();
+    for (int at = threadIdx.x; at < MTILES * NT * 256; at += 64 * NW) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += part[w * (MTILES * NT * 256) + at];
+        const int tile = at >> 8;
+        const int row = i0 + 16 * (tile / NT) + ((at >> 4) & 15), cc = j0 + 16 * (tile % NT) + (at & 15);
+        if (row < m && cc < n) c[(int64_t)row * c_stride + cc] = sum;
+    }
+}
+template <int MTILES, int NT, int NW, int W>
+static int launch_skinny_lds_w(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride, int m, int n, int k, dim3 grid) {
+    // as many stages as 160 KB of LDS and the wave's load counter hold, two to four
+    constexpr int STAGE = (MTILES + NT) * 2048 * NW, LOADS = (MTILES + NT) * 8 / W;
+    constexpr int STAGES = 4 * STAGE <= 160 * 1024 && 3 * LOADS <= 63 ? 4 : 3 * STAGE <= 160 * 1024 && 2 * LOADS <= 63 ? 3 : 2;
+    constexpr size_t smem = (size_t)STAGES * STAGE > (size_t)NW * MTILES * NT * 1024 ? (size_t)STAGES * STAGE : (size_t)NW * MTILES * NT * 1024;
+    static_assert(smem <= 160 * 1024, "stages and partial tiles fit the CU's LDS");
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&sgemm_mfma_skinny_lds_kernel<MTILES, NT, NW, STAGES, W>), smem);
+    sgemm_mfma_skinny_lds_kernel<MTILES, NT, NW, STAGES, W><<<grid, dim3(64 * NW), smem, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    return 0;
+}
+template <int MTILES, int NT, int NW>
+static int launch_skinny_lds(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride, int m, int n, int k, dim3 grid) {
+    const bool rows16 = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && (a_stride & 3) == 0 && (b_stride & 3) == 0;
+    return rows16 ? launch_skinny_lds_w<MTILES, NT, NW, 4>(a, a_stride, b, b_stride, c, c_stride, m, n, k, grid)
+                  : launch_skinny_lds_w<MTILES, NT, NW, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k, grid);
+}
+
 template <bool BT, int MTILES, int NT>
-static void launch_skinny(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
+static int launch_skinny(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
                           int m, int n, int k) {
     const dim3 grid((n + 16 * NT - 1) / (16 * NT), (m + 16 * MTILES - 1) / (16 * MTILES));
     // waves per workgroup: enough for eight waves per CU over the whole grid, as long as every wave has a step of K
     const int64_t groups = (int64_t)grid.x * grid.y;
     int nw = 4;
     while (nw < 16 / NT && groups * nw < 8 * (int64_t)num_cus() && 32 * nw < k) nw *= 2;
+    // Through LDS from a few steps per wave on: with fewer, what the loads cost to set up is not earned back (us, straight / through LDS,
+    // 16-byte rows: 36 x 4109 x 676, 2.6 steps, 12.0 / 13.0; 32 x 4096 x 1024, 4 steps, 9.2 / 5.9; rows at 4 bytes and the eight-tile
+    // form, whose loads are four times as many or whose matrix instructions hide more, a few steps later: 239 x 4789 x 692,
+    // 5.4 steps, 35.8 / 37.7; 131 x 476 x 774, 3 steps, 6.1 / 7.0). Sixteen waves, grids of less than half the CUs, always: from 1.8
+    // steps on 1.07 to 2.0 times faster. Offsets are 32 bits wide.
+    if constexpr (BT) {
+        const bool rows16 = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && (a_stride & 3) == 0 && (b_stride & 3) == 0;
+        const int least = nw == 16 ? 1 : rows16 && MTILES * NT < 8 ? 4 : 8;
+        if (k >= 32 * nw * least && (uint64_t)m * (uint64_t)a_stride < ((uint64_t)1 << 30) && (uint64_t)n * (uint64_t)b_stride < ((uint64_t)1 << 30)) {
+            // (two stages of more tiles and waves than these do not fit the LDS)
+            if constexpr (MTILES * NT == 1) if (nw == 16) return launch_skinny_lds<1, 1, 16>(a, a_stride, b, b_stride, c, c_stride, m, n, k, grid);
+            if constexpr (NT == 1) if (nw == 8) return launch_skinny_lds<MTILES, 1, 8>(a, a_stride, b, b_stride, c, c_stride, m, n, k, grid);
+            if (nw == 4 || NT == 2) return launch_skinny_lds<MTILES, NT, 4>(a, a_stride, b, b_stride, c, c_stride, m, n, k, grid);
+        }
+    }
     if (NT == 1 && nw == 16) sgemm_mfma_skinny_kernel<BT, MTILES, 1, 16><<<grid, dim3(1024), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
     else if (nw == 8) sgemm_mfma_skinny_kernel<BT, MTILES, NT, 8><<<grid, dim3(512), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
     else sgemm_mfma_skinny_kernel<BT, MTILES, NT, 4><<<grid, dim3(256), 0, current_stream()>>>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    return 0;
 }
 // The largest tile whose grid still gives every CU a workgroup (a larger tile reads its operands less often, an idle CU
 // costs more than that), and no more rows than the product has.
 template <bool BT>
-static void launch_skinny_rows(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
+static int launch_skinny_rows(const float* a, int64_t a_stride, const float* b, int64_t b_stride, float* c, int64_t c_stride,
                                int m, int n, int k) {
     auto groups = [&](int mt, int nt) { return (int64_t)((n + 16 * nt - 1) / (16 * nt)) * ((m + 16 * mt - 1) / (16 * mt)); };
     const int cus = num_cus();
-    if (m > 32 && groups(4, 2) >= cus) launch_skinny<BT, 4, 2>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
-    else if (m > 32 && groups(4, 1) >= cus) launch_skinny<BT, 4, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
-    else if (m > 16 && groups(2, 1) >= cus) launch_skinny<BT, 2, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
-    else launch_skinny<BT, 1, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    if (m > 32 && groups(4, 2) >= cus) return launch_skinny<BT, 4, 2>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    if (m > 32 && groups(4, 1) >= cus) return launch_skinny<BT, 4, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    if (m > 16 && groups(2, 1) >= cus) return launch_skinny<BT, 2, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+    return launch_skinny<BT, 1, 1>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
 }
 
 static std::atomic<int> g_dense_mfma{1};
@@ -324,8 +468,9 @@ int launch_fp32_matmul(const float* a, int64_t a_stride, const float* b, int64_t
     const bool shallow = aligned && m >= 64 && n >= 32 && k >= 4 && k <= 32 && tiles64 * (k < 32 ? 4 : 2) >= num_cus();
     if (g_dense_mfma && k >= 1 && tiles64 < num_cus() && !shallow && (b_transposed || aligned || m < 64)) {
         note_kernel("sgemm_mfma_skinny_kernel");
-        if (b_transposed) launch_skinny_rows<true>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
-        else launch_skinny_rows<false>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+        const int rc = b_transposed ? launch_skinny_rows<true>(a, a_stride, b, b_stride, c, c_stride, m, n, k)
+                                    : launch_skinny_rows<false>(a, a_stride, b, b_stride, c, c_stride, m, n, k);
+        if (rc != 0) return rc;
         SKH_CHECK(hipGetLastError());
         return 0;
     }

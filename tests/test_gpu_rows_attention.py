@@ -721,3 +721,25 @@ def test_attention_prefill_workgroup_with_three_query_groups(hip_backend, torch_
     want = L.sdpa(q, k, v, 0.125, True)
     assert normalized_err(got, want, eps=1.0) <= 2e-2
     assert np.sqrt(np.mean((got - want) ** 2)) <= 5e-3 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("m,n,k,offset", [
+    (1, 20, 512, 0), (3, 33, 545, 0), (16, 16, 8192, 0), (5, 1000, 1500, 3),            # sixteen waves: one step each, a tail, many, an odd base
+    (20, 4100, 1028, 0), (18, 4099, 2053, 0), (2, 4200, 1028, 0), (2, 4200, 2047, 0),   # eight waves, two row tiles and one
+    (1, 8200, 516, 0), (33, 4160, 2052, 0), (64, 8200, 2080, 0), (70, 8210, 2051, 0)])  # four waves; four row tiles, one and two column tiles
+def test_dense_fp32_products_staged_through_lds(hip_backend, torch_cuda, m, n, k, offset):
+    """Few rows with enough K per wave: operands come in through LDS, 16 or 4 bytes a lane by their alignment, in two to four stages,
+    with partial last steps, rows and columns past the end and a row of another buffer behind the last. Bound as above."""
+    torch = torch_cuda
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64).T
+    flat = np.full(offset + n * k + k, np.nan, np.float32)
+    flat[offset:offset + n * k] = b.reshape(-1)
+    out = torch.full((m + 1, n), float("nan"), dtype=torch.float32, device="cuda")
+    hip_backend.fp32_matmul_wt_dev(dev(torch, a), 0, dev(torch, flat), offset, out, 0, m, n, k)
+    assert hip_backend.last_kernel() == "sgemm_mfma_skinny_kernel"
+    got = out.cpu().numpy()
+    assert np.isnan(got[m]).all()
+    assert np.abs(got[:m] - want).max() <= k / 4 * 2.0 ** -24 * 0.64 * k + 1e-6
