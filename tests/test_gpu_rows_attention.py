@@ -743,3 +743,41 @@ def test_dense_fp32_products_staged_through_lds(hip_backend, torch_cuda, m, n, k
     got = out.cpu().numpy()
     assert np.isnan(got[m]).all()
     assert np.abs(got[:m] - want).max() <= k / 4 * 2.0 ** -24 * 0.64 * k + 1e-6
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 1), (2, 3), (5, 4), (1, 1023), (2, 1024), (1, 1025), (3, 4095), (2, 4096), (1, 8191), (2, 8192), (1, 8193)])
+def test_layer_norm_and_softmax_row_shapes(hip_backend, torch_cuda, rows, cols):
+    """Every form of the kernels that keep a row in registers (4, 16 and 32 elements per thread, float4s and single floats) and the looping
+    ones behind them, at the edges of their ranges, with and without gamma and beta, a row of -inf but for one element, log form:
+    against float64 (a sum of cols fp32 terms in a tree: within 16 * 2^-24 of the magnitudes that enter it)."""
+    torch, kx = torch_cuda, hip_backend
+    rng = np.random.default_rng(cols)
+    x = (rng.standard_normal((rows, cols)) * 2 + 0.5).astype(np.float32)
+    g, b = (rng.standard_normal(cols).astype(np.float32) for _ in range(2))
+    xd = x.astype(np.float64)
+    mu, var = xd.mean(1, keepdims=True), xd.var(1, keepdims=True)
+    norm = (xd - mu) / np.sqrt(var + 1e-5)
+    out = torch.full((rows + 1, cols), float("nan"), device="cuda")
+    for gamma, beta in ((g, b), (None, b), (g, None), (None, None)):
+        kx.layer_norm_dev(dev(torch, x), None if gamma is None else dev(torch, gamma), None if beta is None else dev(torch, beta), out, rows, cols, 1e-5)
+        want = norm * (1 if gamma is None else gamma) + (0 if beta is None else beta)
+        got = out.cpu().numpy()
+        # the difference x - mean carries 2^-24 of |x| and of the mean, scaled up where a row's values lie close together
+        assert np.abs(got[:rows] - want).max() <= 16 * 2.0 ** -24 * (np.abs(x).max() / np.sqrt(var.min() + 1e-5) + 1) * 8
+        assert np.isnan(got[rows]).all()
+    x[0, :] = -np.inf
+    x[0, cols // 2] = 3.0
+    xd = x.astype(np.float64)
+    e = np.exp(xd - xd.max(1, keepdims=True))
+    for log in (False, True):
+        out.fill_(float("nan"))
+        kx.softmax_rows_dev(dev(torch, x), out, rows, cols, log)
+        got = out.cpu().numpy()
+        assert np.isnan(got[rows]).all()
+        if log:
+            want = xd - (np.log(e.sum(1, keepdims=True)) + xd.max(1, keepdims=True))
+            assert np.array_equal(np.isneginf(got[:rows]), np.isneginf(want))
+            fin = np.isfinite(want)
+            close(got[:rows][fin], want[fin], rel=1e-5, abs_=1e-5)
+        else:
+            close(got[:rows], e / e.sum(1, keepdims=True), rel=1e-5, abs_=1e-7)
