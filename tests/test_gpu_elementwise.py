@@ -64,6 +64,24 @@ def test_binary_ops_and_operand_modes(hip_backend, torch_cuda, n, inner):
     kx.binary_dev("add", out, out, out, 0)                              # nothing to do is not an error
 
 
+@pytest.mark.parametrize("n,inner,shift", [(3 * (1 << 20) + 4, 1000, 0), (3 * (1 << 20), 12, 0), (600004, 6, 0), (4096, 64, 1), (1022, 8, 0), (64, 4096, 0), (5, 1, 0)])
+def test_binary_bias_and_scalar_walks(hip_backend, torch_cuda, n, inner, shift):
+    """Four outputs at a time and one at a time, walks longer than one stride of the grid, a bias longer than the result, operands
+    `shift` elements off 16 bytes; the sum of two floats is one rounding, so the results are the same bits."""
+    torch, kx = torch_cuda, hip_backend
+    rng = np.random.default_rng(n + inner)
+    base = {0: rng.standard_normal(n).astype(np.float32), 1: rng.standard_normal(1).astype(np.float32), 2: rng.standard_normal(inner).astype(np.float32)}
+    idx = {0: np.arange(n), 1: np.zeros(n, np.int64), 2: np.arange(n) % inner}
+    for a_mode, b_mode in ((0, 2), (2, 0), (0, 1), (2, 1), (2, 2)):
+        a, b = (torch.cat([torch.zeros(shift), torch.from_numpy(base[m])]).cuda()[shift:] for m in (a_mode, b_mode))
+        out = torch.full((n + shift + 4,), 7.0, dtype=torch.float32, device="cuda")
+        kx.binary_dev("add", a, b, out[shift:], n, a_mode, b_mode, inner)
+        kx.sync()
+        got = out.cpu().numpy()
+        assert np.array_equal(got[shift:shift + n].view(np.uint32), (base[a_mode][idx[a_mode]] + base[b_mode][idx[b_mode]]).view(np.uint32)), (a_mode, b_mode)
+        assert (got[:shift] == 7.0).all() and (got[shift + n:] == 7.0).all()
+
+
 def test_unary_activations(hip_backend, torch_cuda):
     import math
     torch, kx = torch_cuda, hip_backend
