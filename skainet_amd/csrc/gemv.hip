@@ -117,18 +117,37 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void gemv_kernel(
     }
 }
 
+// Weight rows of a workgroup of `nwaves` waves: even contiguous shares over whole workgroups per CU, as many as fit a budget of
+// waves_per_cu, and whole rounds of them where the shares pass GEMV_MAX_ROWS. A share counted in waves (2.67 workgroups of three
+// waves for a budget of eight, 1.14 of seven) leaves some CUs twice the rows of the others: one row of Q5_K 4096 x 14336 19.0 us
+// so, 11.8 with one workgroup per CU; Q8_0 11008 x 5120 16.1 -> 12.9, x 11008 30.0 -> 26.1; two rows of Q6_K 2048 x 11008 14.4 -> 8.9.
+// A workgroup has at least the rows that keep its loads in flight (two rows of Q6_K 2048 x 1024 in ones 6.0 us, in fours 4.7). Of
+// few rows one row of Q6_K over two waves goes in three workgroups per CU instead of four where that is no more rows per CU, each share rounded up
+// (4523 x 4864 in four fives 9.2, in three sixes 8.5; Q5_K loses by it, 2544 x 2816 4.9 -> 5.5). From three waves on, a second workgroup per CU pays only from some rows each (Q6_K 2048 x 14336 8.4 us with one, 9.1
+// with two; 4096 x 14336 12.6 and 12.3; Q4_0 2048 x 5120 5.5 and 6.9). `four`: Q5_K's three waves, the last of them part empty, go on
+// to four workgroups, of which a CU starts one when one ends (20000 x 5120 22.6 us with two, 17.0).
+static int gemv_rows_per_wg(int n, int nwaves, int waves_per_cu, int batch, int ahead, bool four) {
+    const int64_t cus = num_cus();
+    int64_t per_cu = waves_per_cu / nwaves > 1 ? waves_per_cu / nwaves : 1;
+    if (nwaves >= 3 && n <= (nwaves > 3 ? 5 : ahead < 8 ? 2 : 7) * cus * per_cu) per_cu = 1;
+    else if (nwaves == 3 && per_cu == 2 && four) per_cu = 4;
+    auto rows_of = [&](int64_t wgs) {                                     // of a workgroup, with wgs of them per CU at a time
+        const int64_t rounds = (n + cus * wgs * GEMV_MAX_ROWS - 1) / (cus * wgs * GEMV_MAX_ROWS);
+        return (n + cus * wgs * rounds - 1) / (cus * wgs * rounds);
+    };
+    int64_t rows = rows_of(per_cu);
+    if (nwaves == 2 && per_cu == 4 && batch == 1 && ahead == 2 && rows <= 6 && 3 * rows_of(3) <= 4 * rows) rows = rows_of(3);
+    const int least = batch == 4 || ahead < 4 ? ahead : 4;
+    return rows < least ? least : (int)rows;
+}
+
 template <class F, int B, int R>
 static int launch_one(const uint8_t* w, const float* x, float* y, int k, int n, int batch, int waves_per_cu) {
     const int nslots = k / F::SLOT_ELEMS;
     const int nseg = (nslots + 63) / 64;
     const int nwaves = nseg < GEMV_MAX_WAVES ? nseg : GEMV_MAX_WAVES;
     const int64_t row_bytes = (int64_t)(k / (F::SLOT_ELEMS * F::SLOTS_PER_BLOCK)) * F::BLOCK_BYTES;
-    // Even contiguous row shares: about waves_per_cu resident waves on every CU.
-    int target_wgs = (num_cus() * waves_per_cu) / nwaves;
-    if (target_wgs < 1) target_wgs = 1;
-    int rows_per_wg = (n + target_wgs - 1) / target_wgs;
-    if (rows_per_wg < 1) rows_per_wg = 1;
-    if (rows_per_wg > GEMV_MAX_ROWS) rows_per_wg = GEMV_MAX_ROWS;
+    const int rows_per_wg = gemv_rows_per_wg(n, nwaves, waves_per_cu, B, R, std::is_same<F, Q5KSlot>::value && B == 1);
     const int grid = (n + rows_per_wg - 1) / rows_per_wg;
     note_kernel("gemv_kernel");
     gemv_kernel<F, B, R><<<dim3(grid), dim3(64 * nwaves), 0, current_stream()>>>(w, x, y, k, n, batch, row_bytes, rows_per_wg);
@@ -143,16 +162,20 @@ template <> struct RowsInFlight<Q80Slot> { static constexpr int B1 = 3; };
 template <> struct RowsInFlight<Q6KSlot> { static constexpr int B1 = 2; };
 template <> struct RowsInFlight<Q5KSlot> { static constexpr int B1 = 3; };
 
-static std::atomic<int> g_gemv_waves_per_cu{0};   // 0: per encoding (measured best: Q8_0 4, Q6_K at batch 1 6, the others 8)
+static std::atomic<int> g_gemv_waves_per_cu{0};   // 0: per encoding (measured best: 32-element blocks 4, of three waves 6; the others 8)
 static std::atomic<int> g_q6k_slot64{1};   // 0: Q6_K at batch 1 stays on the 32-weight slot
 
 template <class F>
 static int launch_format(const uint8_t* w, const float* x, float* y, int k, int n, int batch, int waves_per_cu) {
     if (batch == 1) {
-        // Q6_K: the 64-weight slot, 2 rows in flight, 6 waves per CU unless the caller set a count (measured on 32000 x 4096
-        // over 1 .. 4 rows and 5 .. 16 waves: 23.1 us against 25.5 us for the 32-weight slot at its best, 2 rows and 8 waves)
-        if (std::is_same<F, Q6KSlot>::value && g_q6k_slot64)
-            return launch_one<Q6KSlot64, 1, 2>(w, x, y, k, n, batch, g_gemv_waves_per_cu.load() > 0 ? g_gemv_waves_per_cu.load() : 6);
+        // Q6_K: the 64-weight slot, 2 rows in flight (32000 x 4096: 23.1 us against 25.5 us for the 32-weight slot at its best).
+        // Eight waves per CU; four where a row is one wave and eight of them would have few rows each (four and eight waves:
+        // 4096 x 4096 6.1 and 7.0 us, 11008 x 4096 10.1 and 10.2, 32000 x 4096 20.9 and 19.2); six where two waves share a row and fill
+        // it (8192 x 8192 14.8 us, with eight 15.3) or have few rows (2048 x 7168 6.6 and 6.9; 8192 x 6144 12.9 and 11.7).
+        if (std::is_same<F, Q6KSlot>::value && g_q6k_slot64) {
+            const int auto_waves = k <= 4096 ? (n < 48 * num_cus() ? 4 : 8) : k <= 8192 && (k > 7168 || n <= 8 * num_cus()) ? 6 : 8;
+            return launch_one<Q6KSlot64, 1, 2>(w, x, y, k, n, batch, g_gemv_waves_per_cu.load() > 0 ? g_gemv_waves_per_cu.load() : auto_waves);
+        }
         return launch_one<F, 1, RowsInFlight<F>::B1>(w, x, y, k, n, batch, waves_per_cu);
     }
     if (batch == 2) return launch_one<F, 2, 4>(w, x, y, k, n, batch, waves_per_cu);
@@ -250,7 +273,7 @@ int launch_gemv(int enc, const uint8_t* w, const float* x, int m, int k, int n, 
     if (!is_packed(enc)) return set_error("gemv: unsupported encoding %d", enc);
     if (k <= 0 || k % block_elems(enc) != 0)
         return set_error("gemv: inputDim must be a positive multiple of %d; got %d", block_elems(enc), k);
-    const int waves_per_cu = g_gemv_waves_per_cu.load() > 0 ? g_gemv_waves_per_cu.load() : (block_elems(enc) == 32 ? 4 : 8);
+    const int waves_per_cu = g_gemv_waves_per_cu.load() > 0 ? g_gemv_waves_per_cu.load() : (block_elems(enc) == 32 ? (k > 4096 && k <= 6144 ? 6 : 4) : 8);
     for (int b0 = 0; b0 < m;) {
         const int left = m - b0;
         const float* xb = x + (int64_t)b0 * k;

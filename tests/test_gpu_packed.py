@@ -630,3 +630,29 @@ def test_products_of_one_to_eight_rows_by_lanes_that_decode_64_weights(hip_backe
         assert normalized_err(gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0), want) <= GEMV_TOL
     finally:
         kx.set_tuning("gemv_few", 1)
+
+
+@pytest.mark.parametrize("enc,n,k,m", [("Q6_K", 1, 256, 1), ("Q6_K", 2441, 4096, 1), ("Q6_K", 12300, 1024, 1), ("Q6_K", 2753, 4352, 1), ("Q6_K", 1030, 7424, 1),
+                                       ("Q6_K", 517, 9216, 1), ("Q6_K", 1800, 9472, 1), ("Q6_K", 1281, 14336, 1), ("Q6_K", 3, 33024, 1), ("Q5_K", 2049, 5120, 1),
+                                       ("Q5_K", 515, 5376, 1), ("Q5_K", 16500, 9216, 1), ("Q8_0", 2049, 5152, 1), ("Q4_0", 17000, 8224, 2),
+                                       ("Q6_K", 1025, 11008, 2), ("Q5_K", 2049, 1024, 4), ("Q6_K", 1540, 14592, 4)])
+def test_row_kernel_shares_of_rows(hip_backend, torch_cuda, enc, n, k, m):
+    """The row kernel's split of the weight rows: one, two, three, four and eight workgroups per CU of one to eight waves, shares
+    that the last workgroup has only part of, several rounds, two passes of K per wave. Against float64 sums of the oracle's decoded
+    weights, on rows from every part of the result: a lane's chain is at most 64 products per pass and of a format's 2 or 4 partial
+    sums, the fold 6 and the waves 8 more: fewer than 192 fp32 roundings, each at most 2^-24 of the sum of magnitudes (of the codes
+    with their bias apart: 32 or less against codes of 63, so three times the magnitudes)."""
+    kx, bs = hip_backend, G.PACKED[enc][0]
+    packed = gaussian_weight(kx, enc, n, k, 300 + n)
+    x = np.random.default_rng(n + k).standard_normal((m, k)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(min(n, 70)), np.arange(max(0, n - 70), n), np.random.default_rng(n).integers(0, n, 200)]))
+    w = L.dequant(enc, packed.reshape(n, -1)[rows].reshape(-1)).reshape(rows.size, k).astype(np.float64)
+    biased = np.abs(w) + 64 * np.abs(w).max(axis=1, keepdims=True) / 31
+    try:
+        kx.set_tuning("gemv_few", 0)
+        got = gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0)
+        assert kx.last_kernel() == "gemv_kernel"
+    finally:
+        kx.set_tuning("gemv_few", 1)
+    assert not np.isnan(got).any()
+    assert (np.abs(got[:, rows] - x.astype(np.float64) @ w.T) <= 192 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ biased.T)).all()
