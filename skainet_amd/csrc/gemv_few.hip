@@ -248,50 +248,73 @@ static int launch_few(const uint8_t* w, const float* x, float* y, int m, int n, 
 static std::atomic<int> g_gemv_few{1};      // 0 never, 1 by rule, 2 wherever it fits
 void set_gemv_few(int v) { g_gemv_few = v; }
 
-// Where this kernel is faster than the ones behind it (row kernel, for one row of 32-element blocks the streaming kernel), measured
-// over n 1500 to 30000, K 512 to 14336 in us, theirs -> this one's. It is where they multiply much or load badly: many activation
-// rows, rows of few kilobytes, K that leaves their waves unequal shares (more than 8192, 4096 to 5120). They hold their own with
-// few products on full waves, and where K takes this kernel a second round that few waves share (6144 to 8192).
+// Where this kernel is faster than the ones behind it (row kernel; for one row of 32-element blocks the streaming kernel and Q8_0's
+// integer kernel; Q4_K's own kernels), from 91 000 random products of n 512 to 32000, K 512 to 15360, in us, theirs -> this one's. It is
+// where they multiply much or load badly: many activation rows, rows of few kilobytes, K that leaves their waves unequal shares. They
+// hold their own with few products on full waves, and where K takes this kernel a second round that few waves share (5120 to 7168).
 //   32-element blocks, 3 to 8 rows: everywhere (Q8_0 4 x 4096 x 11008 26.1 -> 14.6, 8 x 32000 x 4096 111 -> 41)
-//     2 rows: outside 6144 < K <= 8192 (Q4_0 4000 x 4096 7.2 -> 5.3, Q8_0 10000 x 4096 13.9 -> 10.7, x 7168 16.2 -> 17.2)
-//     1 row: many weight rows (Q5_0 30000 x 4096 27.7 -> 20.7; Q8_0 has the integer kernel at multiples of 1024), and for formats of
-//     4 and 5 bits a K beyond the streaming kernel's (Q4_0 4000 x 11008 11.7 -> 9.9; Q5_0 10000 x 8192 15.2 -> 15.8, Q5_1 31331 x
-//     14080 73 -> 85)
-//   Q6_K, Q5_K: their decode costs more, so 5 to 8 rows (Q6_K 8 x 4096 x 11008 53 -> 24; 5 x 1500 x 7168 13.2 -> 15.0), 3 and 4 of Q5_K,
-//     and below that rows that leave the row kernel's lanes idle (Q6_K 1 x 30000 x 768 18.0 -> 10.0, 2 x 10000 x 11008 36.6 -> 25.6;
-//     4 x 14336 x 4096 15.9 -> 16.8)
-//   Q4_K has batched kernels of its own: rows shorter than a wave's share there (8 x 30000 x 512 35.5 -> 12.6) and few long ones (4 x 2048
-//     x 14336 15.3 -> 10.9; 4 x 10000 x 14336 27.3 -> 28.3).
-// Where it is a little slower it stays, for its error against float64 is a third of the row kernel's (1.1e-7 against 3e-7 to 5e-7) and
-// a fortieth of the bf16 quads' (4e-6): Q5_K 3 and 4 rows, K 7168 to 8192, n just above 16384 (18600 x 8192 35.1 -> 37.6 us),
-// 32-element blocks 2 rows, n 1024 to 1200, K 8192 to 10240 (7.9 -> 8.4), Q5_1 1 row 12288 to 13300 x 1536 (8.0 -> 8.6), Q4_K 3 and 4 rows
-// below 1024 x 2048 (4.5 -> 4.7 to 5.4). Of 16800 random products of 1 to 8 rows 18 are more than 3 % slower than without it, none more than
-// 10 %.
+//     2 rows: outside 6144 < K <= 7168 (Q4_0 4000 x 4096 7.2 -> 5.3, 4000 x 8192 9.6 -> 8.0, Q8_0 10000 x 4096 13.9 -> 10.7, x 7168 16.2 ->
+//     17.2)
+//     1 row, formats of 4 and 5 bits: K up to 4096 (Q5_0 6800 x 768 6.9 -> 4.5, 1780 x 3072 5.6 -> 4.6, 30000 x 4096 27.7 -> 20.7), and beyond
+//     the streaming kernel's K (Q5_0 620 x 15100 9.6 -> 6.5; Q4_0 4000 x 11008 11.7 -> 9.9; Q5_1 31331 x 14080 73 -> 85). Rows of 4096
+//     and 8192 fill the waves of the kernels behind: those stay there up to 48 rows per CU (Q4_0 4096 x 4096 5.9, here 5.1)
+//     1 row of Q8_0: many short rows and between the integer kernel's K (30000 x 768 10.5 -> 7.3, 12170 x 2560 12.7 -> 10.5)
+//   Q6_K, Q5_K: their decode costs more, so 5 to 8 rows (Q6_K 8 x 4096 x 11008 53 -> 24, Q5_K 8 x 3000 x 13312 30.6 -> 20.6; Q6_K 5 x 1500 x 7168
+//     13.2 -> 15.0), 3 and 4 of Q5_K, and below that rows that leave the row kernel's lanes idle (Q6_K 1 x 30000 x 768 18.0 -> 10.0, Q5_K 2 x
+//     30800 x 1024 13.0 -> 8.9, 2 x 10000 x 11008 36.6 -> 25.6; 4 x 14336 x 4096 15.9 -> 16.8)
+//   Q4_K: rows shorter than a wave's share there (1 x 31600 x 512 12.2 -> 7.0, 8 x 30000 x 512 35.5 -> 12.6), long ones (4 x 2048 x 14336 15.3 ->
+//     10.9, 5 x 13000 x 9216 61.6 -> 36.1; 4 x 10000 x 14336 27.3 -> 28.3), and more rows than their workgroups take in whole rounds (8 x 15000 x
+//     3328 28 -> 21). K = 4096 has kernels for its four full slices (8 x 15000 x 4096 13.5 -> 21.8).
+// Where it is slower it stays, for its error against float64 is a third of the row kernel's (1.1e-7 against 3e-7 to 5e-7) and
+// a fortieth of the bf16 quads' (4e-6): Q5_K 1 row, Q6_K 2 to 4 rows, 32-element blocks 1 and 2 rows, K above 8192 (Q5_K 3500 x 10240 10.4 ->
+// 15.8, Q6_K 2 x 3300 x 12800 12.3 -> 17.9, Q5_1 7300 x 14848 18.3 -> 24.2), Q4_K 3 and 4 rows below 1024 x 2048 (4.5 -> 4.7 to 5.4).
 // Besides: rows go in fours per workgroup, so a little more than 16 per CU costs a quarter (Q6_K 4 x 4147 x 6144 13.6 -> 16.2, x 4000
 // 12.1 -> 12.2), and products of 4 us are as long as their launch on either side (within 0.3 us).
 static bool few_by_rule(int enc, int m, int n, int k) {
     const int cus = num_cus();
     const bool many = n >= 12 * cus, lots = n >= 48 * cus, uneven = n > 16 * cus && n < 24 * cus;
     if (enc == ENC_Q4_K) {
-        if (m == 1) return false;
-        if (m == 2 && k <= 4096) return many && k <= 2048;
-        return k <= 2048 || (k > 4096 && (k <= 5120 || (n < 16 * cus && (k > 7168 || (m == 2 && k <= 6144)))));
+        const bool third = n > 48 * cus && n <= 64 * cus;                 // a third round of the kernels behind, the first one here
+        if (m == 1) {
+            if (k <= 1024) return n >= (k <= 768 ? 24 : 32) * cus;
+            return k % 1024 != 0 && (k <= 2048 ? n >= 24 * cus : k > 4096 && k <= 5120 && n > 64 * cus);      // K % 1024 = 0: the integer kernel
+        }
+        if (k <= 2048) return m > 2 || many;
+        if (k <= 4096) return k < 4096 && (m > 4 ? third || (k <= 3072 && lots) : m > 2 && n <= 8 * cus);
+        if (k <= 5120) return true;
+        if (k <= 6144) return m == 2 || n <= 16 * cus || n > 48 * cus;
+        if (k <= 7168) return m > 2 && (n <= (m <= 4 ? 8 : 4) * cus || third);
+        if (n < 24 * cus || (m > 2 && third && k <= 11264)) return true;
+        const int most = m == 2 ? 64 : k <= 9216 && m <= 4 ? 64 : 32;
+        return k > 8192 && k <= 10240 && n <= most * cus;
     }
     if (block_elems(enc) == 32) {
         if (m >= 3) return true;
         if (m == 2) {
             if (k <= 1024) return many;
             if (enc == ENC_Q8_0 && k <= 2048) return !lots;
-            return k <= 4096 || (n >= 4 * cus && (k <= 6144 || (k > 8192 && (k <= 12288 || !lots))));
+            if (k > 7168 && k <= 8192) return n <= (enc == ENC_Q8_0 ? 12 : 64) * cus;
+            return k <= 4096 || (n >= 4 * cus && k <= 6144) || (k > 8192 && (k <= 12288 || !lots));
         }
-        if (k <= 4096) return lots && (enc != ENC_Q8_0 || (k % 1024 != 0 && (k < 1024 || k > 2048)));
-        return many && !lots && enc != ENC_Q8_0 && (k <= 6144 || k > 8192);
+        if (enc == ENC_Q8_0) return k % 1024 != 0 && (k <= 768 ? n >= 32 * cus : k <= 1536 ? n > 64 * cus : k > 2048 && k <= 4096 && many);
+        if (k <= 2048) return n >= (enc == ENC_Q5_0 && k > 1024 ? 16 : 24) * cus;
+        if (k <= 4096) return n >= (k == 4096 ? 48 : 5) * cus;
+        if (k > 7168 && k < 8192) return enc == ENC_Q4_0 ? n <= 64 * cus : !many;
+        if (k > 8192 && enc != ENC_Q5_1 && (many ? k <= 10240 : k > 10240 || n <= 4 * cus || n > 6 * cus)) return true;
+        return many && !lots && (k <= 6144 || k > 8192);
     }
-    if (m >= 5) return many || k <= 4096 || (k > 7168 && k <= 11264);
-    if (m >= 3 && enc == ENC_Q5_K) return k <= 4096 || (many && !(uneven && k <= 8192));
-    if (!many) return m >= 2 && k <= 768 && n >= 4 * cus;
-    if (m == 1) return enc == ENC_Q6_K ? k <= 768 || (k <= 1792 && n >= 32 * cus) : k > 8192 && k <= 12288 && !lots;
-    return k <= 768 || (k > 8192 && (k <= 12288 || !lots)) || (k > 4096 && k <= (m == 2 ? 5120 : 6144) && !uneven);
+    if (m >= 5) {
+        if (enc == ENC_Q5_K && (m >= 6 || k <= 12288 || n >= 6 * cus)) return true;
+        if (enc == ENC_Q6_K && m >= 7 && !(k > 6144 && k <= 7168)) return true;
+        return many || k <= 4096 || (k > 7168 && k <= 11264);
+    }
+    if (m >= 3 && enc == ENC_Q5_K) return k <= 4096 || (k > 7168 && k <= 8192) || (many && !(uneven && k <= 8192));
+    const bool q5k_3072 = enc == ENC_Q5_K && k > 2048 && k <= 3072;       // the row kernel's second wave half empty
+    if (!many) return m >= 2 && (k <= 1024 || q5k_3072) && n >= 4 * cus;
+    if (m == 1 && enc == ENC_Q6_K) return k <= 768 || (k <= 1792 && n >= 32 * cus);
+    if (m == 1) return k <= 1024 ? n >= 32 * cus : k > 8192 && k <= 12288 && (!lots || k <= 10240);
+    if (m == 2 && q5k_3072 && n <= 24 * cus) return true;
+    return k <= 1024 || (k > 8192 && (k <= 12288 || !lots)) || (k > 4096 && k <= (m == 2 ? 5120 : 6144) && !uneven);
 }
 
 // Returns 1 when this kernel took the product, 0 when the row kernel is the faster one or the shape is outside its range, -1 on

@@ -656,3 +656,28 @@ def test_row_kernel_shares_of_rows(hip_backend, torch_cuda, enc, n, k, m):
         kx.set_tuning("gemv_few", 1)
     assert not np.isnan(got).any()
     assert (np.abs(got[:, rows] - x.astype(np.float64) @ w.T) <= 192 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ biased.T)).all()
+
+
+@pytest.mark.parametrize("enc,n,k,m", [("Q4_K", 6144, 768, 1), ("Q4_K", 8192, 1024, 1), ("Q4_K", 6144, 1536, 1), ("Q4_K", 2048, 3328, 4), ("Q4_K", 12300, 2816, 8),
+                                       ("Q4_K", 1024, 6912, 5), ("Q4_K", 6100, 8192, 2), ("Q5_0", 1280, 3072, 1), ("Q4_0", 900, 7936, 1), ("Q4_0", 600, 15104, 1),
+                                       ("Q8_0", 16400, 1280, 1), ("Q8_0", 3072, 2560, 1), ("Q5_1", 700, 8448, 2), ("Q5_K", 1100, 1024, 2), ("Q5_K", 70, 6656, 6),
+                                       ("Q5_K", 8200, 512, 1), ("Q6_K", 70, 5120, 8)])
+def test_products_that_the_few_rows_kernel_takes_by_its_rule(hip_backend, torch_cuda, enc, n, k, m):
+    """Sizes at the edges of the rule, against float64 sums of the oracle's decoded weights on rows from every part of the result
+    (fewer than 96 fp32 roundings per product, as above); the kernel behind is held to the product's own bound at the same size."""
+    kx, bs = hip_backend, G.PACKED[enc][0]
+    packed = gaussian_weight(kx, enc, n, k, 500 + n)
+    x = np.random.default_rng(n + k).standard_normal((m, k)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(min(n, 70)), np.arange(max(0, n - 70), n), np.random.default_rng(n).integers(0, n, 200)]))
+    w = L.dequant(enc, packed.reshape(n, -1)[rows].reshape(-1)).reshape(rows.size, k).astype(np.float64)
+    want, magnitude = x.astype(np.float64) @ w.T, np.abs(x).astype(np.float64) @ np.abs(w).T
+    got = gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0)
+    assert kx.last_kernel() == "packed_gemv_few_kernel"
+    assert not np.isnan(got).any() and (np.abs(got[:, rows] - want) <= 96 * 2.0 ** -24 * magnitude).all()
+    try:
+        kx.set_tuning("gemv_few", 0)
+        behind = gpu_matmul(kx, torch_cuda, enc, packed, n, k, x, kind=0)
+        assert kx.last_kernel() != "packed_gemv_few_kernel"
+    finally:
+        kx.set_tuning("gemv_few", 1)
+    assert normalized_err(behind[:, rows], want) <= GEMV_TOL
