@@ -323,8 +323,9 @@ __global__ __launch_bounds__(64 * NW * T, (PRO == 2 || NW * T == 8) ? 1 : 2) voi
     // shared by its two waves, behind the rings.
     const uint32_t ring_bytes = T == 1 ? mfma_ring_bytes(nli_max, W) : (uint32_t)(W + 1) * nli_max * 1024u;
     uint8_t* ring = smem + wave_all * ring_bytes;
+    const int with_slice = T == 1 ? min(NW, nsl) : NW;         // waves that have a slice, and a ring
     uint8_t* xa_stage = T == 1 ? ring + (uint32_t)W * (uint32_t)nli_max * 1024u : smem + NW * T * ring_bytes + wave * MFMA_XA_BYTES;
-    float* partials_all = reinterpret_cast<float*>(smem + NW * T * ring_bytes + (T == 1 ? 0 : NW * MFMA_XA_BYTES));   // [NW slices of K][qt][64]
+    float* partials_all = reinterpret_cast<float*>(smem + with_slice * T * ring_bytes + (T == 1 ? 0 : NW * MFMA_XA_BYTES));   // [NW slices of K][qt][64]
     float* ssq_lds = partials_all + NW * qt * 64;
     float* partials = partials_all + wave * qt * 64;
     const int r0 = blockIdx.x * (4 * qt);
@@ -440,7 +441,7 @@ static int mfma_window(int k) { return (((k >> 10) + 3) >> 2) >= 3 ? 2 : 3; }
 static size_t mfma_smem_bytes(int k, int qt, int window, int nw, int teams) {
     const int ns_max = ((k >> 10) + nw - 1) / nw;
     const int nli_max = (144 * ns_max + 63) / 64;
-    const size_t rings = teams == 1 ? (size_t)nw * mfma_ring_bytes(nli_max, window)
+    const size_t rings = teams == 1 ? (size_t)min(nw, k >> 10) * mfma_ring_bytes(nli_max, window)
                                     : (size_t)nw * teams * (window + 1) * nli_max * 1024 + (size_t)nw * MFMA_XA_BYTES;
     return rings + (size_t)nw * qt * 64 * sizeof(float) + 32;
 }
@@ -513,11 +514,14 @@ int launch_q4k_gemv_mfma(const uint8_t* w, const float* x, float* y, int k, int 
     }
     if (epilogue >= EPI_SWIGLU && (n & 1)) return 0;
     if (epilogue == EPI_RESIDUAL && (!residual || (reinterpret_cast<uintptr_t>(residual) & 3))) return 0;
-    // one round of workgroups over the chip: a workgroup's quads are consecutive rows, the last workgroup may own fewer
+    // Whole rounds of workgroups over the chip: a workgroup's quads are consecutive rows, the last workgroup may own fewer (shares of
+    // the largest size ran one workgroup too many in a round of its own: 33000 x 4096 21.0 us, 14.8 in two even rounds). K below
+    // 4096 leaves waves of a workgroup without a slice: more workgroups per CU then, whose LDS is that of the waves that have one
+    // (32000 x 1024, 2048, 3072: with one per CU 11.0, 11.7, 12.2 us, with these 6.1, 8.5, 11.0; twice as many 7.7, 8.3, 12.1).
     const int quads = (n + 3) / 4;
-    int qt = (quads + num_cus() - 1) / num_cus();
-    if (qt > MFMA_MAX_QUADS) qt = MFMA_MAX_QUADS;
-    if (qt < 1) qt = 1;
+    const int per_cu = merge || k >= 4096 ? 1 : k == 1024 ? 4 : k == 2048 ? 3 : 2, most = per_cu > 1 ? MFMA_MAX_QUADS / 2 : MFMA_MAX_QUADS;
+    const int at_once = num_cus() * per_cu, rounds = (quads + at_once * most - 1) / (at_once * most);      // at least one: n is
+    const int qt = (quads + at_once * rounds - 1) / (at_once * rounds);
     const int grid = (quads + qt - 1) / qt;
     // measured on 11008 x 4096 with two / three / four quads in flight: 7.06 / 6.52 / 6.68 us; in a Llama-3-8B decode
     // step (every Q4_K product) 1.617 / 1.564 / 1.568 / 1.578 ms per token with two / three / four / five

@@ -43,7 +43,7 @@ constexpr int Q8M_QUAD = 4 * Q8M_SLICE;                // 4352 bytes = 272 piece
 constexpr int Q8M_NLI = 5;
 constexpr int Q8M_XROW = 20;                           // dwords per (group, plane) row of 16 operand dwords, padded against bank conflicts
 constexpr int Q8M_XA_BYTES = 16 * 4 * Q8M_XROW * 4 + 16 * 4;   // operand planes of 16 groups + a scale per group
-constexpr int Q8M_MAX_QUADS = 32;                      // row quads per workgroup
+constexpr int Q8M_MAX_QUADS = 24;                      // row quads per workgroup: two workgroups with two quads in flight fit a CU's LDS
 __host__ __device__ constexpr uint32_t q8m_ring_bytes(int window) { return (uint32_t)window * Q8M_QUAD + Q8M_XA_BYTES; }   // the planes' staging area behind the W slots
 
 // W: quads in flight per wave (the ring has W slots: a slot is refilled once its quad is used up)
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256, W == 1 ? 4 : W == 2 ? 2 : 1) void q8_0_gemv_mf
     const int nsl = k >> 10;                                   // slices of 1024 elements, at most 4
     uint8_t* ring = q8m_smem + wave * q8m_ring_bytes(W);
     uint8_t* xa_stage = ring + W * Q8M_QUAD;
-    float* partials_all = reinterpret_cast<float*>(q8m_smem + 4 * q8m_ring_bytes(W));   // [4 slices of K][qt][64]
+    float* partials_all = reinterpret_cast<float*>(q8m_smem + nsl * q8m_ring_bytes(W));   // [4 slices of K][qt][64]
     float* partials = partials_all + wave * qt * 64;
     const int r0 = blockIdx.x * (4 * qt);
     const int nq = min(qt, (n - r0 + 3) / 4);                  // this workgroup's quads (uniform, at least one)
@@ -188,7 +188,7 @@ void set_q8_0_mfma_per_cu(int v) { if (v >= 1 && v <= 4) g_q8_0_mfma_per_cu = v;
 
 template <int W>
 static int launch_q8m(int grid, int qt, hipStream_t s, const uint8_t* w, const float* x, float* y, int k, int n) {
-    const size_t smem = (size_t)4 * q8m_ring_bytes(W) + (size_t)4 * qt * 64 * sizeof(float);
+    const size_t smem = (size_t)(k >> 10) * q8m_ring_bytes(W) + (size_t)4 * qt * 64 * sizeof(float);
     SKH_SET_MAX_DYNAMIC_LDS_ONCE((&q8_0_gemv_mfma_kernel<W>), 160 * 1024);
     if (smem > 160 * 1024) return 0;
     note_kernel("q8_0_gemv_mfma_kernel");
@@ -205,11 +205,16 @@ int launch_q8_0_gemv_mfma(const uint8_t* w, const float* x, float* y, int k, int
     if ((reinterpret_cast<uintptr_t>(w) & 15) || (reinterpret_cast<uintptr_t>(x) & 15)) return 0;
     const int quads = (n + 3) / 4;
     const int per_cu = g_q8_0_mfma_per_cu.load();
-    int qt = (quads + per_cu * num_cus() - 1) / (per_cu * num_cus());
-    if (qt > Q8M_MAX_QUADS) qt = Q8M_MAX_QUADS;
+    // Whole rounds of workgroups on every CU. Two of them keep two quads in flight at every size: with four from nine quads per
+    // workgroup on, one workgroup filled the LDS and the grid ran in two rounds (18000 x 4096 14.9 -> 13.4 us, x 3072 12.5 -> 10.5). K
+    // below 3072 leaves half or more of a workgroup's waves without a slice and a ring: three or four workgroups per CU (32000 x
+    // 2048 15.5 -> 12.3, x 1024 14.7 -> 7.6; six and eight there: the same).
+    const int64_t at_once = (int64_t)(per_cu == 2 && k < 3072 ? (k == 1024 ? 4 : 3) : per_cu) * num_cus();
+    const int64_t rounds = (quads + at_once * Q8M_MAX_QUADS - 1) / (at_once * Q8M_MAX_QUADS);
+    const int qt = (int)((quads + at_once * rounds - 1) / (at_once * rounds));
     const int grid = (quads + qt - 1) / qt;
     if (per_cu >= 3 && qt <= 4) return launch_q8m<1>(grid, qt, current_stream(), w, x, y, k, n);
-    if (per_cu == 2 && qt <= 8) return launch_q8m<2>(grid, qt, current_stream(), w, x, y, k, n);
+    if (per_cu == 2) return launch_q8m<2>(grid, qt, current_stream(), w, x, y, k, n);
     return launch_q8m<4>(grid, qt, current_stream(), w, x, y, k, n);
 }
 

@@ -681,3 +681,23 @@ def test_products_that_the_few_rows_kernel_takes_by_its_rule(hip_backend, torch_
     finally:
         kx.set_tuning("gemv_few", 1)
     assert normalized_err(behind[:, rows], want) <= GEMV_TOL
+
+
+@pytest.mark.parametrize("enc,n,k", [("Q4_K", 33000, 4096), ("Q4_K", 66000, 1024), ("Q4_K", 24600, 2048), ("Q4_K", 4100, 3072), ("Q8_0", 98400, 1024), ("Q8_0", 18000, 2048),
+                                     ("Q8_0", 16500, 4096), ("Q8_0", 49300, 3072)])
+def test_one_row_integer_kernels_in_whole_rounds(hip_backend, torch_cuda, enc, n, k):
+    """More quads than one round of workgroups takes, and several workgroups per CU where K leaves waves without a slice: against
+    float64 sums of the oracle's decoded weights, on rows from every part of the result."""
+    kx = hip_backend
+    packed = gaussian_weight(kx, enc, n, k, 700 + n)
+    x = np.random.default_rng(n + k).standard_normal((1, k)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(140), np.arange(n - 140, n), np.random.default_rng(n).integers(0, n, 600)]))
+    w = L.dequant(enc, packed.reshape(n, -1)[rows].reshape(-1)).reshape(rows.size, k).astype(np.float64)
+    try:
+        kx.set_tuning("gemv_few", 0)
+        got = gpu_matmul(kx, torch_cuda, enc, packed, n, k, x)
+        assert kx.last_kernel() == ("q4k_gemv_mfma_kernel" if enc == "Q4_K" else "q8_0_gemv_mfma_kernel")
+    finally:
+        kx.set_tuning("gemv_few", 1)
+    assert not np.isnan(got).any()
+    assert normalized_err(got[:, rows], x.astype(np.float64) @ w.T) <= GEMV_TOL
