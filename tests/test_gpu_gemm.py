@@ -250,3 +250,18 @@ def test_the_q4k_gemm_knobs_leave_other_formats_alone(hip_backend, torch_cuda, k
             check(got[:2], L.gemv(enc, x[:2], packed, n))
     finally:
         hip_backend.set_tuning(knob, 1)
+
+
+@pytest.mark.parametrize("enc,m,n,k", [("Q8_0", 129, 907, 13312), ("Q6_K", 229, 581, 14336), ("Q4_0", 256, 700, 9472), ("Q8_0", 500, 513, 6400), ("Q5_K", 385, 513, 14336)])
+def test_gemm_of_few_tiles_with_more_than_eight_splits(hip_backend, torch_cuda, enc, m, n, k):
+    """Few tiles over a long K: 9 to 24 splits, the last of them shorter than the rest or none at all, summed in split order."""
+    packed = gaussian_weight(hip_backend, enc, n, k, 210 + n)
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    try:
+        hip_backend.set_tuning("gemm_skinny", 0)
+        got = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
+    finally:
+        hip_backend.set_tuning("gemm_skinny", 1)
+    assert hip_backend.last_kernel() == "dequant_gemm_kernel"
+    assert not np.isnan(got).any()
+    check_exact(torch_cuda, enc, got, x, packed, n)
