@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void gemv_kernel(
 static int gemv_rows_per_wg(int n, int nwaves, int waves_per_cu, int batch, int ahead, bool four) {
     const int64_t cus = num_cus();
     int64_t per_cu = waves_per_cu / nwaves > 1 ? waves_per_cu / nwaves : 1;
-    if (nwaves >= 3 && n <= (nwaves > 3 ? 5 : ahead < 8 ? 2 : 7) * cus * per_cu) per_cu = 1;
+    if (nwaves >= 3 && n <= (nwaves > 3 ? 4 : ahead < 8 ? 2 : 7) * cus * per_cu) per_cu = 1;
     else if (nwaves == 3 && per_cu == 2 && four) per_cu = 4;
     auto rows_of = [&](int64_t wgs) {                                     // of a workgroup, with wgs of them per CU at a time
         const int64_t rounds = (n + cus * wgs * GEMV_MAX_ROWS - 1) / (cus * wgs * GEMV_MAX_ROWS);
@@ -137,8 +137,8 @@ static int gemv_rows_per_wg(int n, int nwaves, int waves_per_cu, int batch, int 
     };
     int64_t rows = rows_of(per_cu);
     if (nwaves == 2 && per_cu == 4 && batch == 1 && ahead == 2 && rows <= 6 && 3 * rows_of(3) <= 4 * rows) rows = rows_of(3);
-    const int least = batch == 4 || ahead < 4 ? ahead : 4;
-    return rows < least ? least : (int)rows;
+    const int64_t least = std::min<int64_t>(batch == 4 || ahead < 4 ? ahead : 4, rows_of(1));      // no CU is left without one for it
+    return (int)(rows < least ? least : rows);
 }
 
 template <class F, int B, int R>
