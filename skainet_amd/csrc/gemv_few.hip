@@ -30,8 +30,8 @@ constexpr int FEW_STAGE_FLOATS = 2 * 16 * 68;      // two batch rows x 16 slots 
 
 // ROWS: batch rows computed (4 or 8 on the matrix instruction; 1 or 2 on the vector unit, every lane with the rows' activations of
 // its slot), R: quads in flight.
-template <class F, int ROWS, int R>
-__global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+template <class F, int ROWS, int R, int WAVES = FEW_MAX_WAVES>
+__global__ __launch_bounds__(64 * WAVES) void packed_gemv_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                                              float* __restrict__ y, int m, int n, int k, int rows_per_wg) {
     constexpr bool VECTOR = ROWS <= 2;
     constexpr int MB = VECTOR ? 1 : ROWS / 4, NX = VECTOR ? ROWS : MB;    // batch rows in fours; sets of 64 activations in a lane
@@ -221,19 +221,29 @@ __global__ __launch_bounds__(64 * FEW_MAX_WAVES) void packed_gemv_few_kernel(con
     }
 }
 
-template <class F, int ROWS, int R>
+template <class F, int ROWS, int R, int WAVES = FEW_MAX_WAVES>
 static int launch_few_rows(const uint8_t* w, const float* x, float* y, int m, int n, int k) {
     const int passes = (k / 256 + 3) / 4;
-    // a wave per pass up to four and for eight; else rounds of four or eight and a shared rest, so that the SIMDs get the same
-    const int nwaves = passes <= 4 ? passes : passes < 8 ? 4 : FEW_MAX_WAVES;
+    const int cus = num_cus();
+    // 9 to 12 passes: as many waves, in the registers of three per SIMD (two quads ahead instead of three or four), so that no wave has to
+    // load activations a second time (Q8_0 4 x 4096 x 11008 15.1 -> 13.0 us, Q4_K 4 x 8000 x 12288 20.3 -> 18.7). Eight batch rows and Q6_K
+    // do not fit there; nine passes leave three SIMDs of four two waves, which costs more than it saves from 24 rows per CU on.
+    if constexpr ((ROWS == 4 || ROWS == 1) && WAVES == FEW_MAX_WAVES && !F::Q6) {
+        if (passes > 8 && passes <= 12 && (passes > 9 || n <= 24 * cus)) return launch_few_rows<F, ROWS, 2, 12>(w, x, y, m, n, k);
+    }
+    // A wave per pass up to four and for eight. Five to seven: one workgroup per CU with a wave per pass while the one round of activations
+    // outweighs the SIMDs with one wave of two (five, six and seven passes up to 16, 32 and 64 rows per CU: Q6_K 2 x 3000 x 6144 0.77 of its time,
+    // 8 x 2000 x 7168 0.76); else two of four, the second round shared. From there on rounds of eight and a shared rest.
+    const bool one_round = passes == 5 ? n <= 16 * cus : passes == 6 ? n <= 32 * cus : n <= 64 * cus;
+    const int nwaves = WAVES == 12 || passes <= 4 || (passes < 8 && one_round) ? passes : passes < 8 ? 4 : FEW_MAX_WAVES;
     // whole rounds of workgroups over the chip, eight waves on a CU at a time, rows in fours
-    const int resident = num_cus() * (FEW_MAX_WAVES / nwaves);
+    const int resident = cus * (WAVES / nwaves);
     const int turns = (int)(((int64_t)n + (int64_t)resident * FEW_MAX_ROWS - 1) / ((int64_t)resident * FEW_MAX_ROWS));
     const int rows = (int)(((int64_t)n + (int64_t)resident * turns - 1) / ((int64_t)resident * turns) + 3) & ~3;      // at most FEW_MAX_ROWS
     const size_t smem = (size_t)nwaves * (FEW_STAGE_FLOATS + rows * 4 * ROWS) * sizeof(float);
-    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&packed_gemv_few_kernel<F, ROWS, R>), (size_t)FEW_MAX_WAVES * (FEW_STAGE_FLOATS + FEW_MAX_ROWS * 4 * ROWS) * sizeof(float));
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&packed_gemv_few_kernel<F, ROWS, R, WAVES>), (size_t)WAVES * (FEW_STAGE_FLOATS + FEW_MAX_ROWS * 4 * ROWS) * sizeof(float));
     note_kernel("packed_gemv_few_kernel");
-    packed_gemv_few_kernel<F, ROWS, R><<<dim3((n + rows - 1) / rows), dim3(64 * nwaves), smem, current_stream()>>>(w, x, y, m, n, k, rows);
+    packed_gemv_few_kernel<F, ROWS, R, WAVES><<<dim3((n + rows - 1) / rows), dim3(64 * nwaves), smem, current_stream()>>>(w, x, y, m, n, k, rows);
     SKH_CHECK(hipGetLastError());
     return 1;
 }

@@ -701,3 +701,10 @@ def test_one_row_integer_kernels_in_whole_rounds(hip_backend, torch_cuda, enc, n
         kx.set_tuning("gemv_few", 1)
     assert not np.isnan(got).any()
     assert normalized_err(got[:, rows], x.astype(np.float64) @ w.T) <= GEMV_TOL
+
+
+@pytest.mark.parametrize("enc", ENCS + MORE_ENCS)
+@pytest.mark.parametrize("n,k,m", [(1030, 8448, 3), (517, 11008, 4), (7, 12288, 1), (6200, 9216, 1), (4100, 4352, 2), (4100, 5120, 8), (8200, 6144, 2), (16500, 6912, 1)])
+def test_few_rows_kernel_with_a_wave_per_pass(hip_backend, torch_cuda, enc, n, k, m):
+    """9 to 12 passes of K in one round of as many waves, 5 to 7 in one workgroup per CU, and the sizes just past both: the bound above."""
+    test_products_of_one_to_eight_rows_by_lanes_that_decode_64_weights(hip_backend, torch_cuda, enc, n, k, m)
