@@ -168,6 +168,9 @@ __global__ __launch_bounds__(PF_THREADS, 2) void sdpa_prefill_kernel(PrefillPara
     // two buffers of two blocks (one per team); the teams' states meet in whichever is not being read, and in pf_ml
     extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
     float2* const pf_ml = reinterpret_cast<float2*>(pf_smem + 4 * BLK);     // [team][wave][lane]
+    // [wave][lane]: team 0's first reference for both. Not in pf_ml: over one step there is no barrier between team 1 reading it and
+    // team 0 writing its state
+    float* const pf_ref = reinterpret_cast<float*>(pf_ml + 2 * 4 * 64);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), team = wave_all >> 2, wave = wave_all & 3;
@@ -303,16 +306,16 @@ __global__ __launch_bounds__(PF_THREADS, 2) void sdpa_prefill_kernel(PrefillPara
         };
         set_reference();
 
-                    // The reference starts as the maximum over the group's first block, for both teams (weights rounded against two references would
+        // The reference starts as the maximum over the group's first block, for both teams (weights rounded against two references would
         // differ by bf16's rounding from those of one): step -1 is team 0's scores of that block and no more.
-        if (team == 0) pf_ml[wave * 64 + lane].x = -INFINITY;
+        if (team == 0) pf_ref[wave * 64 + lane] = -INFINITY;
         for (int st = steps ? -1 : 0; st < steps; ++st) {
             const int blk = st < 0 ? blk0 : blk0 + 2 * st + team, k0 = blk * PF_KB;
             if (st != 0) pf_wait_loads();         // this wave's share of the step's block (of step 0 with step -1) ...
             pf_lds_barrier();                     // ... and everybody's; the other buffer has been read by all
             const int ahead = st < 0 ? 1 : st + 1;
             if (st != 0 && blk0 + 2 * ahead + team < blk1) load_block(blk0 + 2 * ahead + team, (par + ahead) & 1);
-            if (st == 0) { m_run = pf_ml[wave * 64 + lane].x; set_reference(); }
+            if (st == 0) { m_run = pf_ref[wave * 64 + lane]; set_reference(); }
             if ((st < 0 && team) || blk >= blk1 || k0 > wave_last_key || k0 + PF_KB <= wave_first_key) continue;      // wave-uniform: no keys in the block
             // The block in two halves of 32 keys, a and b: S of a; S of b with the softmax of a between its matrix instructions;
             // O += V^T . P of a with the softmax of b in between; O += V^T . P of b. The order is pinned (sched_barrier) and
@@ -340,38 +343,38 @@ __global__ __launch_bounds__(PF_THREADS, 2) void sdpa_prefill_kernel(PrefillPara
                 __builtin_amdgcn_sched_barrier(0);
             };
             auto hide = [&](int j) {              // the mask and the range rules on the scores of half j
-                            if (masked) {
-                                // the reference's arithmetic: an excluded key scores -1e30, the mask is added to every score; keys past
-                                // the sequence (padding of the last block) take no part. Four adjacent keys per 16-byte mask load.
-                                constexpr float LOG2E = 1.4426950408889634f;
-                                const int lo = real_first - k0 - 4 * h, hi = real_last - k0 - 4 * h, end = p.seq_kv - k0 - 4 * h;
-            #pragma unroll
-                                for (int e4 = 0; e4 < 4; ++e4) {
-                                    const int key4 = k0 + 32 * j + 8 * e4 + 4 * h;
-                                    float4 mv;
-                                    if (p.mask_k == 1) { const float m1 = mrow[0]; mv = make_float4(m1, m1, m1, m1); }
-                                    else mv = *reinterpret_cast<const float4*>(mrow + min(key4, p.seq_kv - 4));     // seq_kv is a multiple of 4 here
-                                    const float m4[4] = {mv.x, mv.y, mv.z, mv.w};
-            #pragma unroll
-                                    for (int i = 0; i < 4; ++i) {
-                                        const int key = 32 * j + 8 * e4 + i;                          // relative to k0 + 4 h
-                                        float sc = (key > hi || key < lo) ? -1.0e30f * LOG2E : s[j][4 * e4 + i];
-                                        sc = fmaf(m4[i], LOG2E, sc);
-                                        s[j][4 * e4 + i] = key < end ? sc : -INFINITY;
-                                    }
-                                }
-                            } else
-                            // keys outside this query's range score -inf (they take no part); a query without a range scores every key 0
-                            if (wave_uniform || k0 < wave_common_first || k0 + PF_KB - 1 > wave_common_last) {   // wave-uniform: the block crosses a boundary
-                                const int lo = my_first_key - k0 - 4 * h, hi = my_last_key - k0 - 4 * h;
-            #pragma unroll
-                                for (int e = 0; e < 16; ++e) {
-                                    const int key = 32 * j + 8 * (e >> 2) + (e & 3);                  // relative to k0 + 4 h
-                                    if (my_uniform) s[j][e] = minus_ref[0];
-                                    if (key > hi || key < lo) s[j][e] = -INFINITY;
-                                }
-                            }
-                        };
+                if (masked) {
+                    // the reference's arithmetic: an excluded key scores -1e30, the mask is added to every score; keys past
+                    // the sequence (padding of the last block) take no part. Four adjacent keys per 16-byte mask load.
+                    constexpr float LOG2E = 1.4426950408889634f;
+                    const int lo = real_first - k0 - 4 * h, hi = real_last - k0 - 4 * h, end = p.seq_kv - k0 - 4 * h;
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; ++e4) {
+                        const int key4 = k0 + 32 * j + 8 * e4 + 4 * h;
+                        float4 mv;
+                        if (p.mask_k == 1) { const float m1 = mrow[0]; mv = make_float4(m1, m1, m1, m1); }
+                        else mv = *reinterpret_cast<const float4*>(mrow + min(key4, p.seq_kv - 4));     // seq_kv is a multiple of 4 here
+                        const float m4[4] = {mv.x, mv.y, mv.z, mv.w};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int key = 32 * j + 8 * e4 + i;                          // relative to k0 + 4 h
+                            float sc = (key > hi || key < lo) ? -1.0e30f * LOG2E : s[j][4 * e4 + i];
+                            sc = fmaf(m4[i], LOG2E, sc);
+                            s[j][4 * e4 + i] = key < end ? sc : -INFINITY;
+                        }
+                    }
+                } else
+                // keys outside this query's range score -inf (they take no part); a query without a range scores every key 0
+                if (wave_uniform || k0 < wave_common_first || k0 + PF_KB - 1 > wave_common_last) {   // wave-uniform: the block crosses a boundary
+                    const int lo = my_first_key - k0 - 4 * h, hi = my_last_key - k0 - 4 * h;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int key = 32 * j + 8 * (e >> 2) + (e & 3);                  // relative to k0 + 4 h
+                        if (my_uniform) s[j][e] = minus_ref[0];
+                        if (key > hi || key < lo) s[j][e] = -INFINITY;
+                    }
+                }
+            };
             // Four weights: scores 4 c .. 4 c + 3 of half j
             float psum[2];
             auto exps = [&](int j, int c, pf_bf16x8 (&to)[2]) {
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void sdpa_prefill_kernel(PrefillPara
                 float mx = s[0][0];
 #pragma unroll
                 for (int e = 1; e < 32; ++e) mx = fmaxf(mx, s[e >> 4][e & 15]);
-                pf_ml[wave * 64 + lane].x = pf_max_halves(mx);
+                pf_ref[wave * 64 + lane] = pf_max_halves(mx);
                 continue;
             }
             settle(0, pf);
@@ -613,7 +616,7 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
     PrefillParams p{q, frag, out, heads, kv_heads, seq_q, seq_kv, spad, scale * 1.4426950408889634f, causal, window, right_context, lengths, hpw, per_kv / hpw, ngroups,
                     mask, mask_b, mask_h, mask_q, mask_k, places, splits, part, part + rows * splits * D, out_rows};
     const dim3 grid(kv_heads * (per_kv / hpw), places, batch * splits);
-    constexpr size_t smem = 4 * pf_block_bytes<D>() + 2 * 4 * 64 * sizeof(float2);
+    constexpr size_t smem = 4 * pf_block_bytes<D>() + 2 * 4 * 64 * sizeof(float2) + 4 * 64 * sizeof(float);
     note_kernel("sdpa_prefill_kernel");
     const int rc = splits > 1 ? (mask ? launch_prefill_kernel<D, true, true>(grid, smem, s, p) : launch_prefill_kernel<D, true, false>(grid, smem, s, p))
                               : (mask ? launch_prefill_kernel<D, false, true>(grid, smem, s, p) : launch_prefill_kernel<D, false, false>(grid, smem, s, p));
