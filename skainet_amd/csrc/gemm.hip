@@ -849,7 +849,6 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
         const int rounds = (((m + 127) / 128) * ((n + 63) / 64) + num_cus() - 1) / num_cus();
         if (rounds * (6.5 + 0.31 * (k / GK)) + 5.5 < tile_estimate) return run_ksw();
     }
-    const int tiles_m = (m + gemm_gm(wtm) - 1) / gemm_gm(wtm), tiles_n = (n + gemm_gn(wtn) - 1) / gemm_gn(wtn);
     // Few tiles over a long K want more than the eight splits that the choice above is made with, up to a tile per CU (Q8_0 129 x 907 x
     // 13312 37.6 us with 8, 28.9 with 16; Q6_K 229 x 581 x 14336 35.8 and 29.1). Not offered to that choice: the estimates of many
     // splits are 5 to 10 % low there, and the few-rows kernel lost products to them that it is 30 % faster on.
@@ -860,6 +859,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
             if (tiles * ks <= num_cus() && t < tile_estimate) { tile_estimate = t; wtm = 2; wtn = 2; ksplit = ks; }
         }
     }
+    const int tiles_m = (m + gemm_gm(wtm) - 1) / gemm_gm(wtm), tiles_n = (n + gemm_gn(wtn) - 1) / gemm_gn(wtn);
     if (ksplit > kgroups) ksplit = kgroups;
     const int k_chunk = ((kgroups + ksplit - 1) / ksplit) * 256;
     ksplit = (k + k_chunk - 1) / k_chunk;
