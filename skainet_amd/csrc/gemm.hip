@@ -689,6 +689,8 @@ int launch_gemm_skinny(int enc, const uint8_t* w, const float* x, int m, int k, 
                        const float* residual, int epilogue, bool x_pairs);                                       // gemm_skinny.hip
 bool gemm_skinny_fits(int enc, int m, int n, int k);
 double gemm_skinny_estimate(int enc, int m, int n, int k);
+int launch_gemm_skinny_direct(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* c, const float* residual, int epilogue);
+double gemm_skinny_direct_estimate(int enc, int m, int n, int k);
 int gemm_skinny_mode();
 
 constexpr int GEMM_MAX_SPLITS = 24;
@@ -771,7 +773,12 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
         (gain && ((reinterpret_cast<uintptr_t>(gain) & 15) || k > 256 * 4 * 16)) || (epilogue == GEMM_EPI_SWIGLU && (n & 1)) ||
         (epilogue != GEMM_EPI_NONE && !tmp))
         return fused ? 1 : launch_gemv(enc, w, x, m, k, n, y);
-    if (gemm_skinny_mode() >= 2 && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
+    // The one-launch form takes plain activations, and rows that no workgroup overwrites while another one reads them.
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    const bool direct_ok = !gain && !x_pairs && (x0 + sizeof(float) * (size_t)m * k <= y0 || y0 + sizeof(float) * (size_t)m * n <= x0);
+    const int skinny_mode = gemm_skinny_mode();
+    if (skinny_mode >= 100 && direct_ok && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);
+    if (skinny_mode != 3 && skinny_mode >= 2 && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     hipStream_t s = current_stream();
     auto round_activations = [&](__bf16* a) -> int {            // fp32 -> bf16, with the RMSNorm of a fused call folded in
         const int64_t n4 = (int64_t)m * k / 4;                  // k is a multiple of 64
@@ -839,9 +846,16 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     // leaves the format to the kernels before them.
     const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 &&
                          (enc != ENC_Q4_K || (gemm_ksw_enabled() && gemm_frag_enabled()));
-    if (by_rule && gemm_skinny_mode() == 1 && gemm_skinny_fits(enc, m, n, k) &&
-        gemm_skinny_estimate(enc, m, n, k) < 0.95 * fmin(tile_estimate, frag_estimate))
-        return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
+    if (by_rule && (skinny_mode == 1 || skinny_mode == 3) && gemm_skinny_fits(enc, m, n, k)) {
+        const double others = fmin(tile_estimate, frag_estimate), two = gemm_skinny_estimate(enc, m, n, k);
+        // One launch: 3 % below the others' estimate up to 5 us, 20 % of what is above that. Of 4 750 random products (9 to 300 rows) a quarter
+        // takes it, 1.26x on the device and 1.5x back to back from the host, where the second launch was 2.4 us; 15 of them are more than 3 % slower on
+        // the device. 3 % throughout would take 1 680 of them, 250 slower, by up to 30 %.
+        const double least_of_two = fmin(others, two);
+        if (skinny_mode == 1 && direct_ok && gemm_skinny_direct_estimate(enc, m, n, k) < (least_of_two <= 5.0 ? 0.97 * least_of_two : 4.85 + 0.8 * (least_of_two - 5.0)))
+            return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);
+        if (two < 0.95 * others) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
+    }
     if (frag_by_rule && frag_estimate < 1.02 * tile_estimate) return run_frag();
     if (ksw_ok && gemm_ksw_enabled() && !gemm_frag_enabled() && g_gemm_ksplit.load() <= 0) {
         // with the fragment-order kernel switched off, its predecessor where it would beat the tile kernel (0.31 us per 64

@@ -12,7 +12,8 @@
 //   * Lane (c, q) = (l % 16, l / 16) of a wave holds, of each of its NT weight rows c, the 64 weights of the super-block
 //     that its own B operands need: it loads their bytes straight from memory (48 to 80 bytes in 16-byte loads; the four
 //     lanes of a row read one consecutive run), decodes eight of them per matrix instruction, and no weight passes
-//     through LDS. The next super-block's bytes are requested before the current one is decoded.
+//     through LDS. The compiler moves the request for the next super-block down to its use; held in front of the current
+//     one it takes 200 registers instead of 120, two waves per SIMD instead of four: 24 x 14336 x 4096 15.4 -> 20.5 us.
 //   * The contraction index is a free permutation as long as both operands agree: step u (0..7) of a super-block takes,
 //     from lane q, elements 64 q + 8 u .. + 7 (a lane owns 64 consecutive elements), or for Q6_K, whose bytes interleave
 //     quarters, 128 (q / 2) + 32 (u / 2) + 16 (q % 2) + 8 (u % 2) .. + 7. The pass in front writes the activations in that
@@ -106,6 +107,41 @@ __global__ __launch_bounds__(256) void skinny_prepass_rmsnorm_kernel(const float
 
 // ---------------------------------------------------------------------------------------------- the product
 constexpr int SKN_WAVES = 8;      // one wave of a workgroup per super-block in turn (four waves measured the same or up to 10 % slower)
+// The waves' partial tiles meet in LDS and are summed in wave order; residual or SwiGLU are applied where the sums are stored.
+template <int MT, int NT>
+__device__ __forceinline__ void skinny_finish(float* skn_part, const skn_f32x4 (&acc)[MT][NT], int lane, int wave, int m0, int n0, float* c,
+                                              const float* residual, int m, int n, int epilogue) {
+    constexpr int NW = SKN_WAVES;
+    const int col = lane & 15, q = lane >> 4;
+    // accumulator element e of lane (col, q): row 4 q + e, column col of its 16 x 16 tile
+    float* mine = skn_part + (size_t)wave * (MT * NT * 256);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine[(i * NT + t) * 256 + (4 * q + e) * 16 + col] = acc[i][t][e];
+    __syncthreads();
+    for (int p = threadIdx.x; p < MT * NT * 128; p += 64 * NW) {          // two adjacent columns each
+        float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            const float2 t = *reinterpret_cast<const float2*>(skn_part + (size_t)v * (MT * NT * 256) + 2 * p);
+            s.x += t.x; s.y += t.y;
+        }
+        const int tile = p >> 7, gr = m0 + 16 * (tile / NT) + ((p >> 3) & 15), gc = n0 + 16 * (tile % NT) + 2 * (p & 7);
+        if (gr >= m || gc >= n) continue;
+        if (epilogue == SKN_EPI_SWIGLU) {                                 // n is even: (gate, up) pairs
+            c[(int64_t)gr * (n >> 1) + (gc >> 1)] = skn_silu(s.x) * s.y;
+            continue;
+        }
+        const int64_t o = (int64_t)gr * n + gc;
+        if (epilogue == SKN_EPI_RESIDUAL) { s.x += residual[o]; if (gc + 1 < n) s.y += residual[o + 1]; }
+        c[o] = s.x;
+        if (gc + 1 < n) c[o + 1] = s.y;
+    }
+}
+
 template <class F, int MT, int NT>
 __global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, float* c,
                                                                      const float* residual, int m, int n, int k, int epilogue) {
@@ -180,7 +216,243 @@ __global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_kernel(cons
             body(std::integral_constant<int, 1>{}, second, third < nsb ? third : second);
         }
     }
-    // accumulator element e of lane (col, q): row 4 q + e, column col of its 16 x 16 tile
+    skinny_finish<MT, NT>(skn_part, acc, lane, wave, 16 * mt0, n0, c, residual, m, n, epilogue);
+}
+
+// ---------------------------------------------------------------------------------------------- the product, in one launch
+// Small products spend more on the pass in front than it saves: a launch (2.3 us of the host, 1.3 behind another one on the device) and the trip of
+// its result through memory. Here the activations come straight from their fp32 rows, twice the bytes per workgroup, which is what ends it:
+// from about 10 us on the pass pays (gemm.hip has the rule). Back to back from the host (device alone in brackets): Q4_0 18 x 924 x 1024 6.7 ->
+// 4.3 us (4.4 -> 3.0), Q5_K 43 x 515 x 768 6.6 -> 4.3, Q6_K 15 x 589 x 3072 7.1 -> 5.9, Q4_0 46 x 11272 x 1280 10.2 as before.
+//
+// Two forms. `direct`: the tiles, waves and sums of the kernel above; a wave's super-block of 16 MT rows comes in four stages of two
+// steps, loaded in runs of 64 bytes, rounded to bf16 and put into LDS of the wave's own in fragment order, from where a step's A operand
+// is one 16-byte read per lane. Nothing is shared between waves, so nothing waits before the partial tiles meet.
+//   * LDS of a (row tile, stage): piece (r, q) of step u at UB u + QB q + 16 r bytes. A wave writes 4 rows x 4 q x 2 u x 2 halves of eight
+//     bytes at once: QB of 320 bytes spreads them evenly over the banks. (Stages of four steps: 5 to 10 % slower, for their registers.)
+constexpr int SKN_STAGE_STEPS = 2;
+template <bool Q6, int MT>
+struct SknStage {
+    static constexpr int S = SKN_STAGE_STEPS, LOADS = 2 * S * MT, RPL = 8 / S;      // 16-byte loads per lane, rows of one load
+    static constexpr int QB = 320, UB = 4 * QB, BYTES = MT * S * UB;
+    static constexpr int STRIDE = Q6 ? 16 * S : 8 * S;                      // elements from one stage to the next
+    // lane -> row of a load, first element of stage 0 inside the super-block, LDS offset of its eight bytes (the inverse of skn_elem)
+    static __device__ __forceinline__ int row(int lane) { return lane / (8 * S); }
+    static __device__ __forceinline__ int elem(int lane) {
+        const int f = lane & (8 * S - 1);
+        return Q6 ? 128 * (f / (4 * S)) + 4 * (f & (4 * S - 1)) : 64 * (f / (2 * S)) + 4 * (f & (2 * S - 1));
+    }
+    static __device__ __forceinline__ int lds(int lane) {
+        const int f = lane & (8 * S - 1);
+        const int q = Q6 ? 2 * (f / (4 * S)) + ((f >> 2) & 1) : f / (2 * S);
+        const int u = Q6 ? 2 * ((f & (4 * S - 1)) >> 3) + ((f >> 1) & 1) : (f & (2 * S - 1)) >> 1;
+        return u * UB + q * QB + 16 * row(lane) + 8 * (f & 1);
+    }
+};
+template <class F, int MT, int NT>
+__global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_direct_kernel(const float* __restrict__ x, const uint8_t* __restrict__ w, float* c,
+                                                                            const float* residual, int m, int n, int k, int epilogue) {
+    constexpr int NW = SKN_WAVES, S = SKN_STAGE_STEPS, STAGES = 8 / S;
+    using St = SknStage<F::Q6, MT>;
+    extern __shared__ __attribute__((aligned(16))) float skn_part[];       // [NW][stage of activations], then [NW][MT * NT][256]
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+    const int nsb = k >> 8;
+    const uint32_t row_bytes = (uint32_t)nsb * F::BYTES;
+    uint32_t row[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) row[t] = (uint32_t)min(n0 + 16 * t + col, n - 1) * row_bytes;    // rows past N: a valid copy, never stored
+    skn_f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = skn_f32x4{0.f, 0.f, 0.f, 0.f};
+
+    if (wave < nsb) {
+        uint8_t* const mine = reinterpret_cast<uint8_t*>(skn_part) + (size_t)wave * St::BYTES;
+        uint8_t* const put = mine + St::lds(lane);
+        const uint8_t* const get = mine + q * St::QB + 16 * col;
+        const int srow = m0 + St::row(lane), selem = St::elem(lane);
+        float4 xs[St::LOADS];
+        auto load_x = [&](int sb, int stage) __attribute__((always_inline)) {     // rows past m: copies of the last, never stored
+#pragma unroll
+            for (int i = 0; i < St::LOADS; ++i)
+                xs[i] = *reinterpret_cast<const float4*>(x + (int64_t)min(srow + St::RPL * i, m - 1) * k + (256 * sb + St::STRIDE * stage + selem));
+        };
+        auto store_x = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");        // wave-private: LDS serves a wave's accesses in order
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < St::LOADS; ++i) {                         // load i: rows RPL i .. of tile i / (2 S)
+                uint2* dst = reinterpret_cast<uint2*>(put + (i / (2 * S)) * (S * St::UB) + 16 * St::RPL * (i % (2 * S)));
+                *dst = make_uint2(skn_pack(xs[i].x, xs[i].y), skn_pack(xs[i].z, xs[i].w));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        typename F::Raw raw[2][NT];
+        auto load_w = [&](int set, int sb) __attribute__((always_inline)) {
+            const uint8_t* base = w + (int64_t)sb * F::BYTES;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) F::load(raw[set][t], base + row[t], q);
+        };
+        // one super-block: `set` holds its bytes, LDS its first stage; `next` and `after` are this wave's super-blocks behind it (its last, where
+        // there is none)
+        auto body = [&](auto set_c, int sb, int next, int after) __attribute__((always_inline)) {
+            constexpr int SET = decltype(set_c)::value;
+            typename F::Scales sc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sc[t] = F::scales(raw[SET][t], q);
+            auto step = [&](auto uc) __attribute__((always_inline)) {
+                constexpr int U = decltype(uc)::value;
+                if constexpr (U % S == 0) {
+                    if constexpr (U / S + 1 < STAGES) load_x(sb, U / S + 1);
+                    else load_x(next, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                skn_bf16x8 af[MT];
+#pragma unroll
+                for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const skn_bf16x8*>(get + i * (S * St::UB) + (U % S) * St::UB);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    SknBf16 o;
+                    F::template decode<U>(raw[SET][t], sc[t], o);
+                    const skn_bf16x8 b = __builtin_bit_cast(skn_bf16x8, uint4{o.o[0], o.o[1], o.o[2], o.o[3]});
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], b, acc[i][t], 0, 0, 0);
+                }
+                if constexpr (U == 7) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_w(SET, after);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (U % S == S - 1) store_x();
+            };
+            step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{}); step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 4>{}); step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 6>{}); step(std::integral_constant<int, 7>{});
+        };
+        const int last = wave + (nsb - 1 - wave) / NW * NW;               // this wave's last super-block
+        load_x(wave, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(0, wave);
+        load_w(1, min(wave + NW, last));
+        __builtin_amdgcn_sched_barrier(0);
+        store_x();
+        for (int sb = wave; sb < nsb; sb += 2 * NW) {
+            const int second = min(sb + NW, last), third = min(sb + 2 * NW, last), fourth = min(sb + 3 * NW, last);
+            body(std::integral_constant<int, 0>{}, sb, second, third);
+            if (sb + NW >= nsb) break;
+            body(std::integral_constant<int, 1>{}, second, third, fourth);
+        }
+    }
+    __syncthreads();                                                      // the partial tiles go where the activations were
+    skinny_finish<MT, NT>(skn_part, acc, lane, wave, m0, n0, c, residual, m, n, epilogue);
+}
+
+// `shared`: four waves on neighbouring columns take a share of K together, the two shares a super-block each in turn: the workgroup reads its
+// fp32 rows once for 64 NT columns (16 NT above), rounds them and leaves them in LDS in fragment order, two rounds deep. For many columns
+// of short rows: Q4_0 46 x 3830 x 1024 6.4 -> 5.2 us on the device, Q5_K 91 x 8978 x 512 10.7 -> 7.8.
+// LDS of a (share, row tile, round): piece (r, q) of step u at 1088 u + 272 q + 16 r bytes, which spreads the 64 halves of a row that a wave
+// writes at once evenly over the banks.
+constexpr int SKN_QB = 272, SKN_UB = 4 * SKN_QB, SKN_TILE_BYTES = 8 * SKN_UB, SKN_WN = 4;
+template <class F, int MT, int NT>
+__global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_shared_kernel(const float* __restrict__ x, const uint8_t* __restrict__ w, float* c,
+                                                                            const float* residual, int m, int n, int k, int epilogue) {
+    constexpr int NW = SKN_WAVES, WN = SKN_WN, WK = NW / WN, LOADS = 16 * MT * WK / NW;
+    extern __shared__ __attribute__((aligned(16))) float skn_part[];       // [2][WK][MT] tiles of activations, then [WK][WN][MT * NT][256]
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave / WN, wn = wave % WN;
+    const int col = lane & 15, q = lane >> 4;
+    const int n0 = (blockIdx.x * WN + wn) * (16 * NT), m0 = blockIdx.y * (16 * MT);
+    const int nsb = k >> 8;
+    const uint32_t row_bytes = (uint32_t)nsb * F::BYTES;
+    uint32_t row[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) row[t] = (uint32_t)min(n0 + 16 * t + col, n - 1) * row_bytes;    // rows past N: a valid copy, never stored
+    skn_f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = skn_f32x4{0.f, 0.f, 0.f, 0.f};
+
+    uint8_t* const smem = reinterpret_cast<uint8_t*>(skn_part);
+    // wave w stages rows w LOADS .. of the [WK][16 MT] rows of a round: all of one share and row tile
+    static_assert(16 % LOADS == 0 || LOADS % 16 == 0, "a wave's rows");
+    const int srow = wave * LOADS, skg = srow / (16 * MT), sr = srow % (16 * MT);
+    const int f = lane;
+    const int fq = F::Q6 ? 2 * (f >> 5) + ((f >> 2) & 1) : f >> 4, fu = F::Q6 ? 2 * ((f >> 3) & 3) + ((f >> 1) & 1) : (f & 15) >> 1;
+    uint8_t* const put = smem + (skg * MT + (sr >> 4)) * SKN_TILE_BYTES + (sr & 15) * 16 + fu * SKN_UB + fq * SKN_QB + 8 * (f & 1);
+    const uint8_t* const get = smem + kg * MT * SKN_TILE_BYTES + q * SKN_QB + 16 * col;
+    constexpr int ROUND_BYTES = WK * MT * SKN_TILE_BYTES;
+    float4 xs[LOADS];
+    auto load_x = [&](int round) __attribute__((always_inline)) {         // rows past m and super-blocks past the last: copies, not used
+        const int sb = min(round * WK + skg, nsb - 1);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) xs[i] = *reinterpret_cast<const float4*>(x + (int64_t)min(m0 + sr + i, m - 1) * k + (256 * sb + 4 * lane));
+    };
+    auto store_x = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            *reinterpret_cast<uint2*>(put + buf * ROUND_BYTES + (i >> 4) * SKN_TILE_BYTES + 16 * (i & 15)) = make_uint2(skn_pack(xs[i].x, xs[i].y), skn_pack(xs[i].z, xs[i].w));
+    };
+    typename F::Raw raw[2][NT];
+    auto load_w = [&](int set, int round) __attribute__((always_inline)) {
+        const uint8_t* base = w + (int64_t)min(round * WK + kg, nsb - 1) * F::BYTES;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) F::load(raw[set][t], base + row[t], q);
+    };
+    const int rounds = (nsb + WK - 1) / WK;
+    auto body = [&](auto set_c, int round) __attribute__((always_inline)) {
+        constexpr int SET = decltype(set_c)::value;
+        if (round * WK + kg < nsb) {
+            typename F::Scales sc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sc[t] = F::scales(raw[SET][t], q);
+            auto step = [&](auto uc) __attribute__((always_inline)) {
+                constexpr int U = decltype(uc)::value;
+                skn_bf16x8 af[MT];
+#pragma unroll
+                for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const skn_bf16x8*>(get + SET * ROUND_BYTES + i * SKN_TILE_BYTES + U * SKN_UB);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    SknBf16 o;
+                    F::template decode<U>(raw[SET][t], sc[t], o);
+                    const skn_bf16x8 b = __builtin_bit_cast(skn_bf16x8, uint4{o.o[0], o.o[1], o.o[2], o.o[3]});
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], b, acc[i][t], 0, 0, 0);
+                }
+            };
+            step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{}); step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 4>{}); step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 6>{}); step(std::integral_constant<int, 7>{});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(SET, round + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        store_x(SET ^ 1);
+        load_x(round + 2);
+        __syncthreads();
+    };
+    load_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(0, 0);
+    load_w(1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    store_x(0);
+    load_x(1);
+    __syncthreads();
+    for (int round = 0; round < rounds; round += 2) {
+        body(std::integral_constant<int, 0>{}, round);
+        if (round + 1 >= rounds) break;
+        body(std::integral_constant<int, 1>{}, round + 1);
+    }
+    // the shares' partial tiles meet where the activations were
     float* mine = skn_part + (size_t)wave * (MT * NT * 256);
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -189,14 +461,16 @@ __global__ __launch_bounds__(64 * SKN_WAVES) void packed_gemm_skinny_kernel(cons
 #pragma unroll
             for (int e = 0; e < 4; ++e) mine[(i * NT + t) * 256 + (4 * q + e) * 16 + col] = acc[i][t][e];
     __syncthreads();
-    for (int p = threadIdx.x; p < MT * NT * 128; p += 64 * NW) {          // two adjacent columns each
+    for (int p = threadIdx.x; p < WN * MT * NT * 128; p += 64 * NW) {
+        const int g = p / (MT * NT * 128), pt = p % (MT * NT * 128);
         float2 s = make_float2(0.f, 0.f);
 #pragma unroll
-        for (int v = 0; v < NW; ++v) {
-            const float2 t = *reinterpret_cast<const float2*>(skn_part + (size_t)v * (MT * NT * 256) + 2 * p);
+        for (int v = 0; v < WK; ++v) {
+            const float2 t = *reinterpret_cast<const float2*>(skn_part + (size_t)(v * WN + g) * (MT * NT * 256) + 2 * pt);
             s.x += t.x; s.y += t.y;
         }
-        const int tile = p >> 7, gr = 16 * (mt0 + tile / NT) + ((p >> 3) & 15), gc = n0 + 16 * (tile % NT) + 2 * (p & 7);
+        const int tile = pt >> 7, gr = m0 + 16 * (tile / NT) + ((pt >> 3) & 15);
+        const int gc = (blockIdx.x * WN + g) * (16 * NT) + 16 * (tile % NT) + 2 * (pt & 7);
         if (gr >= m || gc >= n) continue;
         if (epilogue == SKN_EPI_SWIGLU) {                                 // n is even: (gate, up) pairs
             c[(int64_t)gr * (n >> 1) + (gc >> 1)] = skn_silu(s.x) * s.y;
@@ -215,6 +489,18 @@ bool gemm_skinny_fits(int enc, int m, int n, int k) {
     return k % 256 == 0 && (uint64_t)n * (uint64_t)(k / block_elems(enc)) * block_bytes(enc) < ((uint64_t)1 << 32) && (m + 15) / 16 <= 65535;
 }
 
+template <class F, int MT, int NT, bool SHARED>
+static int launch_skinny_direct_tile(const float* x, const uint8_t* w, float* c, const float* residual, int m, int n, int k, int epilogue, hipStream_t s) {
+    constexpr size_t stage = SHARED ? 2 * (SKN_WAVES / SKN_WN) * MT * SKN_TILE_BYTES : SKN_WAVES * SknStage<F::Q6, MT>::BYTES;
+    constexpr size_t tile = SKN_WAVES * MT * NT * 256 * sizeof(float), smem = stage > tile ? stage : tile;
+    constexpr int columns = 16 * NT * (SHARED ? SKN_WN : 1);
+    constexpr auto kernel = SHARED ? &packed_gemm_skinny_shared_kernel<F, MT, NT> : &packed_gemm_skinny_direct_kernel<F, MT, NT>;
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE(kernel, smem);
+    note_kernel(SHARED ? "packed_gemm_skinny_shared_kernel" : "packed_gemm_skinny_direct_kernel");
+    kernel<<<dim3((n + columns - 1) / columns, (m + 16 * MT - 1) / (16 * MT)), dim3(64 * SKN_WAVES), smem, s>>>(x, w, c, residual, m, n, k, epilogue);
+    SKH_CHECK(hipGetLastError());
+    return 0;
+}
 template <bool Q6>
 static int skinny_prepass(const float* x, const float* gain, float eps, uint8_t* a, int m, int k, bool pairs, hipStream_t s) {
     const int mtiles = (m + 15) / 16;
@@ -241,7 +527,7 @@ static int launch_skinny_tile(const uint8_t* a, const uint8_t* w, float* c, cons
 // timings of random products (9 to 1024 rows, n 512 to 32000, K 512 to 14336, every format and tile), which it meets within 5
 // to 6 % (rms). The last, partial round of a CU costs a share `whole` of a full one whatever there is in it, the last, partial
 // share of K of the taller tiles a third.
-struct SknTile { int mt, nt; double us; };
+struct SknTile { int mt, nt, wn; double us; };      // wn: waves that share activations in the one-launch forms (1: none)
 SknTile gemm_skinny_tile(int enc, int m, int n, int k) {
     static const int shapes[6][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 2}, {2, 2}, {4, 2}};     // tiles of 16 mt rows x 16 nt columns
     static const double q4k[6][2] = {{1.15, 1.24}, {2.37, 1.83}, {3.80, 3.86}, {2.17, 1.94}, {2.80, 2.37}, {3.58, 3.81}};
@@ -256,7 +542,7 @@ SknTile gemm_skinny_tile(int enc, int m, int n, int k) {
                             : enc == ENC_Q5_1 ? q51 : q80;
     const int mtiles = (m + 15) / 16;
     const double shares = k / (256.0 * SKN_WAVES);
-    SknTile best{1, 1, 0.0};
+    SknTile best{1, 1, 0, 0.0};
     for (int i = 0; i < 6; ++i) {
         const int mt = shapes[i][0], nt = shapes[i][1];
         if (mt > 1 && mt >= 2 * mtiles) continue;                         // more rows than there are
@@ -264,13 +550,46 @@ SknTile gemm_skinny_tile(int enc, int m, int n, int k) {
         const double further = groups <= 1.0 ? 0.0 : whole[i] * ceil(groups) + (1 - whole[i]) * groups - 1;
         const double us = 3.9 + 2.06e-6 * m * k + 3.55e-6 * m * n +
                           (cost[i][0] + cost[i][1] * further) * ((1 - whole_k[i]) * shares + whole_k[i] * ceil(shares));
-        if (best.us == 0.0 || us < best.us) best = SknTile{mt, nt, us};
+        if (best.us == 0.0 || us < best.us) best = SknTile{mt, nt, 0, us};
     }
     return best;
 }
 double gemm_skinny_estimate(int enc, int m, int n, int k) { return gemm_skinny_tile(enc, m, n, k).us; }
 
-static std::atomic<int> g_gemm_skinny{1};   // 0 never, 1 where the estimate favours it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits
+// The one-launch form of a shape and what it is estimated to take, in us, or mt = 0: outside its range. Terms as above: the launch, the result, the
+// workgroups of a CU for their shares of K. Fitted to 2 560 random products (9 to 200 rows, m n k up to 1.2e9, every format), which it meets
+// within 4 to 7 % (rms); 20 to 30 % off, and low, for few columns of more than 6144, which are left out.
+SknTile gemm_skinny_direct_tile(int enc, int m, int n, int k) {
+    struct Form { int mt, nt, wn; double launch, result, whole, whole_k, cost[7][2]; };          // formats: Q4_K, Q5_K, Q6_K, Q8_0, Q4_0, Q5_0, Q5_1
+    static const Form forms[4] = {
+        {1, 1, 1, 2.16, 6.98e-06, 0.84, 0.00, {{1.69, 2.41}, {2.36, 2.64}, {3.47, 4.51}, {2.30, 3.08}, {1.85, 2.48}, {1.95, 2.52}, {2.08, 2.70}}},
+        {1, 2, 1, 2.39, 4.43e-06, 0.86, 0.03, {{2.64, 4.09}, {3.92, 5.83}, {7.05, 9.79}, {4.02, 5.82}, {2.85, 2.90}, {3.21, 3.02}, {3.58, 3.52}}},
+        {1, 1, 4, 2.46, 2.10e-06, 0.75, 0.47, {{1.10, 1.15}, {1.54, 1.59}, {2.65, 3.06}, {1.69, 1.71}, {1.12, 1.20}, {1.30, 1.24}, {1.35, 1.44}}},
+        {2, 2, 4, 3.40, 1.21e-06, 0.75, 0.46, {{2.59, 4.99}, {3.41, 5.97}, {5.94, 8.48}, {3.63, 6.63}, {2.44, 4.65}, {2.79, 3.10}, {2.93, 3.57}}},
+    };
+    SknTile best{0, 0, 0, 0.0};
+    if (k > 6144) return best;
+    const int format = enc == ENC_Q4_K ? 0 : enc == ENC_Q5_K ? 1 : enc == ENC_Q6_K ? 2 : enc == ENC_Q8_0 ? 3 : enc == ENC_Q4_0 ? 4 : enc == ENC_Q5_0 ? 5 : 6;
+    const int mtiles = (m + 15) / 16;
+    for (const Form& f : forms) {
+        if (f.mt > 1 && f.mt >= 2 * mtiles) continue;                     // more rows than there are
+        const double shares = k / (256.0 * (SKN_WAVES / f.wn));
+        const double groups = (double)((mtiles + f.mt - 1) / f.mt) * ((n + 16 * f.nt * f.wn - 1) / (16 * f.nt * f.wn)) / num_cus();
+        const double further = groups <= 1.0 ? 0.0 : f.whole * ceil(groups) + (1 - f.whole) * groups - 1;
+        const double us = f.launch + f.result * m * n + (f.cost[format][0] + f.cost[format][1] * further) * ((1 - f.whole_k) * shares + f.whole_k * ceil(shares));
+        if (best.mt == 0 || us < best.us) best = SknTile{f.mt, f.nt, f.wn, us};
+    }
+    if (k % 2048 == 0) best.us *= 1.08;      // rows of 2^n KB meet in the same channels of the L2
+    return best;
+}
+double gemm_skinny_direct_estimate(int enc, int m, int n, int k) {
+    const SknTile t = gemm_skinny_direct_tile(enc, m, n, k);
+    return t.mt ? t.us : 1e30;
+}
+
+// 0 never, 1 where the estimates favour it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits; 100 wn + 10 mt + nt: that
+// one-launch form (111, 112, 411, 422), wherever it fits; 3: as 1 without the one-launch forms
+static std::atomic<int> g_gemm_skinny{1};
 void set_gemm_skinny(int v) { g_gemm_skinny = v; }
 int gemm_skinny_mode() { return g_gemm_skinny.load(); }
 
@@ -279,7 +598,7 @@ static int launch_skinny_format(int enc, const float* x, const float* gain, floa
                                 const float* residual, int m, int n, int k, int epilogue, hipStream_t s) {
     if (skinny_prepass<F::Q6>(x, gain, eps, a, m, k, pairs, s) != 0) return -1;
     SknTile t = gemm_skinny_tile(enc, m, n, k);
-    if (const int forced = g_gemm_skinny.load(); forced >= 11) { t.mt = forced / 10; t.nt = forced % 10; }
+    if (const int forced = g_gemm_skinny.load(); forced >= 11) { t.mt = forced / 10 % 10; t.nt = forced % 10; }
     note_kernel("packed_gemm_skinny_kernel");
     if (t.nt == 2) {
         if (t.mt == 4) return launch_skinny_tile<F, 4, 2>(a, w, c, residual, m, n, k, epilogue, s);
@@ -289,6 +608,31 @@ static int launch_skinny_format(int enc, const float* x, const float* gain, floa
     if (t.mt == 4) return launch_skinny_tile<F, 4, 1>(a, w, c, residual, m, n, k, epilogue, s);
     if (t.mt == 2) return launch_skinny_tile<F, 2, 1>(a, w, c, residual, m, n, k, epilogue, s);
     return launch_skinny_tile<F, 1, 1>(a, w, c, residual, m, n, k, epilogue, s);
+}
+
+template <class F>
+static int launch_skinny_direct_format(SknTile t, const float* x, const uint8_t* w, float* c, const float* residual, int m, int n, int k, int epilogue, hipStream_t s) {
+    if (t.wn > 1) {
+        if (t.mt == 2) return launch_skinny_direct_tile<F, 2, 2, true>(x, w, c, residual, m, n, k, epilogue, s);
+        return launch_skinny_direct_tile<F, 1, 1, true>(x, w, c, residual, m, n, k, epilogue, s);
+    }
+    if (t.nt == 2) return launch_skinny_direct_tile<F, 1, 2, false>(x, w, c, residual, m, n, k, epilogue, s);
+    return launch_skinny_direct_tile<F, 1, 1, false>(x, w, c, residual, m, n, k, epilogue, s);
+}
+// c = epilogue(x . W^T) in one launch, inside gemm_skinny_fits. Workgroups read x while others store c: the two must not overlap.
+int launch_gemm_skinny_direct(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* c, const float* residual, int epilogue) {
+    SknTile t = gemm_skinny_direct_tile(enc, m, n, k);
+    if (const int forced = g_gemm_skinny.load(); forced >= 100) { t.wn = forced / 100; t.mt = forced / 10 % 10; t.nt = forced % 10; }
+    hipStream_t s = current_stream();
+    switch (enc) {
+        case ENC_Q4_K: return launch_skinny_direct_format<SknQ4K>(t, x, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_K: return launch_skinny_direct_format<SknQ5K>(t, x, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q6_K: return launch_skinny_direct_format<SknQ6K>(t, x, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q4_0: return launch_skinny_direct_format<SknQ45<0>>(t, x, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_0: return launch_skinny_direct_format<SknQ45<1>>(t, x, w, c, residual, m, n, k, epilogue, s);
+        case ENC_Q5_1: return launch_skinny_direct_format<SknQ45<2>>(t, x, w, c, residual, m, n, k, epilogue, s);
+        default: return launch_skinny_direct_format<SknQ80>(t, x, w, c, residual, m, n, k, epilogue, s);
+    }
 }
 
 // c = epilogue(prologue(x) . W^T), all of it: the pass in front and the product. `c` is [m, n] ([m, n / 2] with SwiGLU).

@@ -235,6 +235,52 @@ def test_gemm_of_few_rows(hip_backend, torch_cuda, enc, m, n, k):
         kx.set_tuning("gemm_skinny", 1)
 
 
+@pytest.mark.parametrize("enc", ALL_ENCS)
+@pytest.mark.parametrize("m,n,k", [(9, 5, 256), (16, 64, 2048), (17, 65, 512), (33, 130, 768), (40, 129, 4352), (150, 40, 1280)])
+def test_gemm_of_few_rows_in_one_launch(hip_backend, torch_cuda, enc, m, n, k):
+    """The forms that read their fp32 rows themselves, forced at each tile: ragged rows, columns and rounds, waves without a
+    super-block, Q6_K rows on odd half words. `direct` has the tiles, operands and sums of the two-launch kernel: the same bits.
+    `shared` sums K in two shares instead of eight: the product of bf16-rounded operands (2e-4). With a residual, and with an output
+    that overlaps the rows, which is two launches again."""
+    torch, kx = torch_cuda, hip_backend
+    packed = gaussian_weight(kx, enc, n, k, 900 + n)
+    rng = np.random.default_rng(m * n + k)
+    x, res = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    w = kx.DeviceWeight.upload(enc, packed, n, k)
+    try:
+        for tile in (111, 112, 411, 422):
+            kx.set_tuning("gemm_skinny", tile)
+            got = gpu_gemm(kx, torch, enc, packed, n, k, x)
+            assert kx.last_kernel() == ("packed_gemm_skinny_shared_kernel" if tile > 400 else "packed_gemm_skinny_direct_kernel")
+            check_exact(torch, enc, got, x, packed, n)
+            out = torch.full((m, n), float("nan"), device="cuda")
+            w.matmul_fused(dev(torch, x), m, out, residual=dev(torch, res), epilogue=kx.EPI_RESIDUAL)
+            assert np.array_equal(out.cpu().numpy(), got + res)
+            if tile < 400:
+                kx.set_tuning("gemm_skinny", tile - 100)
+                assert np.array_equal(gpu_gemm(kx, torch, enc, packed, n, k, x), got)
+        kx.set_tuning("gemm_skinny", 111)
+        buf = torch.zeros(m * max(n, k), device="cuda")
+        buf[:m * k] = dev(torch, x).reshape(-1)
+        w.matmul(buf, m, buf)
+        assert kx.last_kernel() == "packed_gemm_skinny_kernel"
+        check_exact(torch, enc, buf[:m * n].cpu().numpy().reshape(m, n), x, packed, n)
+    finally:
+        kx.set_tuning("gemm_skinny", 1)
+
+
+@pytest.mark.parametrize("enc,m,n,k,kernel", [("Q4_0", 18, 924, 1024, "direct"), ("Q5_K", 91, 8978, 512, "shared"), ("Q8_0", 24, 4096, 4096, "kernel"),
+                                              ("Q4_0", 46, 1086, 9984, "kernel")])
+def test_small_products_of_few_rows_take_one_launch(hip_backend, torch_cuda, enc, m, n, k, kernel):
+    packed = gaussian_weight(hip_backend, enc, n, k, 31)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    got = []
+    ran = launches(torch_cuda, lambda: got.append(gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)))
+    ours = [name for name, _, _ in ran if "skinny" in name]
+    assert len(ours) == (2 if kernel == "kernel" else 1) and f"packed_gemm_skinny_{kernel}" in ours[-1], ran
+    check_exact(torch_cuda, enc, got[0], x, packed, n)
+
+
 @pytest.mark.parametrize("knob", ["gemm_frag", "gemm_ksw"])
 def test_the_q4k_gemm_knobs_leave_other_formats_alone(hip_backend, torch_cuda, knob):
     """Either Q4_K kernel switched off: a product of few rows in another format takes the kernel it takes by rule, Q4_K one
