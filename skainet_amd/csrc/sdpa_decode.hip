@@ -39,6 +39,7 @@ struct SdpaDecodeParams {
     int splits;
     float* part;          // [query rows][splits][D] unnormalised outputs; null: one split, the normalised result goes to out
     float* ml;            // [query rows][splits][2] running maximum (in units of ln 2) and sum of each split
+    int subs, tuples;     // workgroups that share a split's keys, and how many such (split, kv head, sequence) there are; tuples 0: a grid of three dimensions
     int seq_q, causal;    // queries per sequence (the last ones of its positions) and whether a later key is hidden from them
 };
 
@@ -69,12 +70,22 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform, and said so: the key loop's exits stay scalar branches
     const int sub = lane & 15, kg = lane >> 4;
-    const int split = blockIdx.x, b = blockIdx.z;
     const int per_kv = p.heads / p.kv_heads;
     const int rows_kv = MQ ? per_kv * p.seq_q : per_kv;        // query rows that share a KV head
-    const int subs = MQ ? (rows_kv + GS - 1) / GS : per_kv / GS;
-    const int kvh = blockIdx.y / subs;
-    const int r0 = (blockIdx.y % subs) * GS;
+    int split = blockIdx.x, b = blockIdx.z, kvh = blockIdx.y, sub_group = 0;
+    if (p.tuples) {
+        // workgroups go to the dies in turn: every eighth one takes the next group of rows of the same keys, so that one L2 has them
+        const int turn = blockIdx.x >> 3, tuple = turn / p.subs * 8 + (blockIdx.x & 7);
+        if (tuple >= p.tuples) return;
+        sub_group = turn % p.subs;
+        split = tuple % p.splits;
+        kvh = tuple / p.splits % p.kv_heads;
+        b = tuple / p.splits / p.kv_heads;
+    } else if (p.subs > 1) {
+        kvh = blockIdx.y / p.subs;
+        sub_group = blockIdx.y % p.subs;
+    }
+    const int r0 = sub_group * GS;
     // row g of the workgroup: its place among the [batch, heads, seq_q] query rows (rows past the last are copies of it)
     int64_t row_of[GS];
     int first_of[GS], end_of[GS];
@@ -333,7 +344,8 @@ template <int GS, int DPL, bool MQ>
 static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge) {
     constexpr int D = 16 * DPL;
     note_kernel("sdpa_decode_kernel");
-    sdpa_decode_kernel<GS, DPL, MQ><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
+    const dim3 grid = p.tuples ? dim3((unsigned)((p.tuples + 7) / 8 * 8 * subs)) : dim3(p.splits, p.kv_heads * subs, p.batch);
+    sdpa_decode_kernel<GS, DPL, MQ><<<grid, dim3(256), 0, current_stream()>>>(p);
     SKH_CHECK(hipGetLastError());
     if (merge) {
         sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits);
@@ -350,6 +362,8 @@ static int launch_decode_d(const SdpaDecodeParams& p, int gs, int subs, bool mer
 
 static std::atomic<int> g_sdpa_decode_gs{0};            // query heads per workgroup: 0 = chosen from the shape, else 1 / 2 / 4
 void set_sdpa_decode_gs(int v) { if (v == 0 || v == 1 || v == 2 || v == 4) g_sdpa_decode_gs = v; }
+static std::atomic<int> g_sdpa_decode_dies{1};
+void set_sdpa_decode_dies(int v) { g_sdpa_decode_dies = v != 0; }
 static std::atomic<int> g_sdpa_decode_one_launch{1};
 void set_sdpa_decode_one_launch(int v) { g_sdpa_decode_one_launch = v != 0; }
 static std::atomic<int> g_attn_merge_max_keys{176};    // most keys per split the unmerged form accepts (a multiple of 16)
@@ -438,7 +452,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     const int subs = (cols + gs - 1) / gs;
     if (batch > 65535 || (int64_t)kv_heads * subs > 65535) return 0;
     SdpaDecodeParams p{q, k, v, out, batch, heads, kv_heads, seq_kv, kv_capacity, scale, window, right_context, lengths, 1,
-                       nullptr, nullptr, seq_q, causal};
+                       nullptr, nullptr, subs, 0, seq_q, causal};
     // enough workgroups to put every CU on the cache, at least 64 keys per split (measured in the decoder at 500 to 650
     // keys: 32 or 48 keys per split 2.5 % slower per token, 96 and 128 keys the same as 64)
     const int64_t groups = (int64_t)batch * kv_heads * subs;
@@ -458,6 +472,14 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
         }
     }
     p.splits = splits;
+    // Workgroups that share keys on one die each, where the dies' own copies of them would not stay in the L2s (32 MB together): 8 queries,
+    // 8 heads over 2, three sequences at 3815 keys 37.7 -> 24.1 us, one query, 8 heads over 1, six at 6012 18.8 -> 14.0, 16 over 2, six at 4556,
+    // D 64, 18.5 -> 14.6. With less traffic the index arithmetic costs 0.1 to 0.2 us, and few groups leave the dies uneven shares (3 queries, 4 heads over
+    // 1, three at 1720 8.3 -> 9.3).
+    const int64_t tuples = (int64_t)batch * kv_heads * splits;
+    const double mb = 8e-6 * batch * kv_heads * keys * head_dim;
+    if (g_sdpa_decode_dies && mb * min(subs, 8) > 24 && subs > 1 && (tuples >= 24 || (tuples + 7) / 8 * subs <= num_cus() / 8) && (tuples + 7) / 8 * 8 * subs <= 0x7FFFFFFF)
+        p.tuples = (int)tuples;
     if (splits > 1 || leave) {
         const size_t rows = (size_t)batch * heads * seq_q;
         p.part = sdpa_workspace(sizeof(float) * rows * splits * (head_dim + 2));

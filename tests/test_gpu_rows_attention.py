@@ -858,3 +858,29 @@ def test_layer_norm_and_softmax_row_shapes(hip_backend, torch_cuda, rows, cols):
             close(got[:rows][fin], want[fin], rel=1e-5, abs_=1e-5)
         else:
             close(got[:rows], e / e.sum(1, keepdims=True), rel=1e-5, abs_=1e-7)
+
+
+@pytest.mark.parametrize("batch,heads,kv_heads,sq,skv,dim,window", [(3, 8, 2, 8, 3815, 128, 0), (5, 8, 1, 1, 2600, 128, 0), (6, 16, 2, 1, 4556, 64, 0), (7, 12, 3, 1, 1500, 256, 0),
+                                                                    (4, 10, 2, 3, 3591, 128, 0), (12, 64, 8, 1, 4775, 128, 360)])
+def test_attention_groups_of_one_die_give_the_same_bits(hip_backend, torch_cuda, batch, heads, kv_heads, sq, skv, dim, window):
+    """Where the workgroups that share keys are placed on one die each (enough traffic, several groups of rows per KV head): the
+    same splits by the same workgroups, so the outputs of the plain grid bit for bit, with a count of workgroups that eight does not
+    divide and with key counts on the device, one of them zero."""
+    torch, kx = torch_cuda, hip_backend
+    gen = torch.Generator(device="cuda").manual_seed(skv)
+    q, k, v = (torch.randn(s, generator=gen, device="cuda") for s in ((batch, heads, sq, dim), (batch, kv_heads, skv, dim), (batch, kv_heads, skv, dim)))
+    lengths = torch.tensor([skv - 7 * i if i != 2 else 0 for i in range(batch)], dtype=torch.int32, device="cuda")
+    got = {}
+    try:
+        for dies in (0, 1):
+            kx.set_tuning("sdpa_decode_dies", dies)
+            for keys in (None, lengths):
+                out = torch.full((batch, heads, sq, dim), float("nan"), device="cuda")
+                ran = launches(torch, lambda: kx.sdpa_cache_dev(q, k, v, out, batch, heads, kv_heads, sq, skv, skv, dim, dim ** -0.5, True, window, 0, keys))
+                grid = [g for name, g, _ in ran if "sdpa_decode_kernel" in name]
+                assert len(grid) == 1 and (grid[0][1] == 1 and grid[0][2] == 1) == (dies == 1), ran
+                got[dies, keys is None] = out
+    finally:
+        kx.set_tuning("sdpa_decode_dies", 1)
+    for keys in (False, True):
+        assert not torch.isnan(got[0, keys]).any() and torch.equal(got[0, keys], got[1, keys])
