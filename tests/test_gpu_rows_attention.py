@@ -884,3 +884,17 @@ def test_attention_groups_of_one_die_give_the_same_bits(hip_backend, torch_cuda,
         kx.set_tuning("sdpa_decode_dies", 1)
     for keys in (False, True):
         assert not torch.isnan(got[0, keys]).any() and torch.equal(got[0, keys], got[1, keys])
+
+
+@pytest.mark.parametrize("cols", [1, 255, 257, 4095, 4096, 4097, 15454, 16384, 65537])
+def test_argmax_at_the_edges_of_a_thread_s_walk(hip_backend, torch_cuda, cols):
+    """The maximum at the first and the last column, ties between a thread's own elements and between threads, rows of -inf."""
+    torch, kx = torch_cuda, hip_backend
+    lg = np.random.default_rng(cols).standard_normal((5, cols)).astype(np.float32)
+    lg[0, 0] = lg[1, cols - 1] = 9.0
+    lg[2, cols // 3] = lg[2, min(cols // 3 + 256, cols - 1)] = 9.0
+    lg[3, cols // 2:] = 9.0
+    lg[4, :] = -np.inf
+    idx = torch.full((5,), -1, dtype=torch.int32, device="cuda")
+    kx.argmax_rows_dev(dev(torch, lg), 5, cols, idx)
+    assert idx.cpu().tolist() == [int(r.argmax()) for r in lg]
