@@ -36,11 +36,17 @@ constexpr int G_WAVES_M = 2, G_WAVES_N = 2;
 constexpr int GK = 64;
 constexpr int G_THREADS = G_WAVES_M * G_WAVES_N * 64;
 constexpr int GSTRIDE = GK + 8;                               // bf16 elements per LDS row (144 bytes)
-// A wave owns WTM x WTN MFMA tiles of 32 x 32: WTM = 4 row tiles (workgroup tile 256 rows) for prompts, WTM = 2 (128 rows)
-// where at most 128 activation rows exist or where the taller tile would leave most of the chip idle.
+// A wave owns WTM x WTN MFMA tiles of 32 x 32, 2 to 4 of them each way (not 2 x 3): workgroup tiles of 128, 192 or 256 rows and columns, so that
+// what a product leaves of its last row of tiles and of the last round over the CUs is small. With 128 and 256 alone 300 rows took
+// three or four thirds of what they need and 1000 x 11008 left 84 of 256 CUs idle: Q6_K 1000 x 11008 x 4096 124.0 -> 112.6 us, Q8_0
+// 400 x 9000 x 3072 64 -> 55. Of 605 random products (100 to 1024 rows) 146 take one of the four tiles with a 192: 1.10x, 5 of all more than 3 % slower.
 constexpr int gemm_gm(int wtm) { return 32 * wtm * G_WAVES_M; }
 constexpr int gemm_gn(int wtn) { return 32 * wtn * G_WAVES_N; }
-constexpr size_t gemm_smem(int wtm, int wtn) { return 2 * (size_t)(gemm_gm(wtm) + gemm_gn(wtn)) * GSTRIDE * sizeof(__bf16); }   // two stages
+// Weight rows that a step decodes: two threads share a row, so whole multiples of 128. 192 columns (WTN = 3) decode 256, the last 64 of them
+// copies of the tile's last row that no wave reads: a third more decode per matrix instruction than the 256-column tile, and per
+// 32 x 32 outputs and step it takes the same time (Q4_K 0.113 us, Q6_K 0.127).
+constexpr int gemm_wrows(int wtn) { return (gemm_gn(wtn) + G_THREADS / 2 - 1) / (G_THREADS / 2) * (G_THREADS / 2); }
+constexpr size_t gemm_smem(int wtm, int wtn) { return 2 * (size_t)(gemm_gm(wtm) + gemm_wrows(wtn)) * GSTRIDE * sizeof(__bf16); }   // two stages
 
 void* kernel_workspace(size_t bytes);   // shim.hip
 int launch_gemv(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* y);   // gemv.hip
@@ -420,8 +426,8 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
     constexpr int G_WTN = WTN, GN = gemm_gn(WTN), GM = gemm_gm(WTM);
     constexpr int G_A_LOADS = GM * (GK / 8) / G_THREADS;      // 16-byte chunks of the activation tile per thread
     constexpr int G_A_ELEMS = GM * GSTRIDE;
-    constexpr int G_W_TASKS = GN * 2 / G_THREADS;             // 32-weight decode tasks per thread and step
-    constexpr int G_W_ELEMS = GN * GSTRIDE;
+    constexpr int G_W_TASKS = gemm_wrows(WTN) * 2 / G_THREADS;   // 32-weight decode tasks per thread and step
+    constexpr int G_W_ELEMS = gemm_wrows(WTN) * GSTRIDE;
     // Register slots of the activation ring. Narrow tile: two (requested two steps ahead, like the weights). Wide tile:
     // one -- the second slot's 32 registers are what the 256 accumulators leave no room for: a step parks the slot in
     // LDS at its end and requests the step after next into it right away, a full step ahead of its own parking.
@@ -443,8 +449,8 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
     const int wrow = tid >> 1, wsub = tid & 1;
     const uint8_t* wrow_ptr[G_W_TASKS];
 #pragma unroll
-    for (int t = 0; t < G_W_TASKS; ++t)   // rows past N decode a valid row, never stored
-        wrow_ptr[t] = w + (int64_t)min(n0 + wrow + (G_THREADS / 2) * t, n - 1) * row_bytes;
+    for (int t = 0; t < G_W_TASKS; ++t)   // rows past the tile or N decode a valid row, never stored
+        wrow_ptr[t] = w + (int64_t)min(n0 + min(wrow + (G_THREADS / 2) * t, GN - 1), n - 1) * row_bytes;
 
     // Staging registers: a two-slot ring of the activation tile chunks and of the raw weight bytes, requested two
     // steps ahead. One workgroup owns a CU (the double-buffered tiles fill its LDS), so the register file is there
@@ -666,6 +672,12 @@ static int launch_gemm_tile(const __bf16* a, const uint8_t* w, float* c, int m, 
 template <class Raw, int BE, int BB>
 static int launch_gemm_enc(int wtm, int wtn, const __bf16* a, const uint8_t* w, float* c, int m, int n, int k, dim3 grid, int k_chunk,
                            int64_t split_stride, hipStream_t s) {
+    if (wtm == 3) {
+        if (wtn == 4) return launch_gemm_tile<Raw, BE, BB, 3, 4>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+        if (wtn == 3) return launch_gemm_tile<Raw, BE, BB, 3, 3>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+        return launch_gemm_tile<Raw, BE, BB, 3, 2>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    }
+    if (wtn == 3) return launch_gemm_tile<Raw, BE, BB, 4, 3>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
     if (wtm == 2) {
         if (wtn == 4) return launch_gemm_tile<Raw, BE, BB, 2, 4>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
         return launch_gemm_tile<Raw, BE, BB, 2, 2>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
@@ -696,10 +708,10 @@ int gemm_skinny_mode();
 constexpr int GEMM_MAX_SPLITS = 24;
 static std::atomic<int> g_gemm_ksplit{0};   // 0 = choose from the tile count
 void set_gemm_ksplit(int v) { g_gemm_ksplit = v; }
-static std::atomic<int> g_gemm_wide{-1};    // -1 = choose from the shape, 0 / 1 = narrow / wide tile
+static std::atomic<int> g_gemm_wide{-1};    // -1 = choose from the shape, 0 / 1 / 2 = 128 / 256 / 192 columns per tile (192 with 128 rows: 256)
 void set_gemm_wide(int v) { g_gemm_wide = v; }
-static std::atomic<int> g_gemm_rows{0};     // 0 = choose from the shape, 2 / 4 = 128 / 256 activation rows per tile
-void set_gemm_rows(int v) { if (v == 0 || v == 2 || v == 4) g_gemm_rows = v; }
+static std::atomic<int> g_gemm_rows{0};     // 0 = choose from the shape, 2 / 3 / 4 = 128 / 192 / 256 activation rows per tile
+void set_gemm_rows(int v) { if (v == 0 || (v >= 2 && v <= 4)) g_gemm_rows = v; }
 
 // What a product takes on the tile kernel, in us: its launches, what it moves outside the loop, and per round of 256 tiles a part
 // outside the K loop and a step of 64 elements of K. Fitted to 145 000 timings of 73 000 random products (9 to 1024 rows, n 512 to
@@ -708,15 +720,19 @@ void set_gemm_rows(int v) { if (v == 0 || v == 2 || v == 4) g_gemm_rows = v; }
 // fit a CU: two rounds of them take 1.43 (the second barely begun) to 1.6 of one. The launch that sums splits has its own
 // cost and (splits + 1) m n floats to move; splits that would get no K are not counted.
 static double gemm_tile_us(int enc, int wtm, int wtn, int m, int n, int k, int ks) {
-    // [128 x 128, 128 x 256, 256 x 128, 256 x 256][64 tiles, 256 tiles]
-    static const double q4k[4][2] = {{0.603, 0.701}, {0.921, 1.18}, {0.781, 0.988}, {1.33, 1.81}}, q5k[4][2] = {{0.647, 0.748}, {1.03, 1.32}, {0.816, 1.03}, {1.43, 1.92}};
-    static const double q6k[4][2] = {{0.722, 0.828}, {1.26, 1.47}, {0.881, 1.09}, {1.61, 2.08}}, q80[4][2] = {{0.762, 0.835}, {1.27, 1.53}, {1.09, 1.18}, {1.58, 2.11}};
-    static const double q40[4][2] = {{0.573, 0.672}, {0.877, 1.13}, {0.759, 0.942}, {1.26, 1.69}}, q50[4][2] = {{0.621, 0.728}, {1.14, 1.34}, {0.794, 0.988}, {1.49, 1.90}};
-    static const double q51[4][2] = {{0.631, 0.712}, {1.06, 1.26}, {0.807, 0.955}, {1.43, 1.82}};
-    static const double outside[4] = {2.4, 5.6, 5.5, 9.0};
+    // [128 x 128, 128 x 256, 256 x 128, 256 x 256, 192 x 128, 192 x 192, 192 x 256, 256 x 192][64 tiles, 256 tiles]; the last four are timings of
+    // each tile at both counts and two K, brought to the scale of the others
+    static const double q4k[8][2] = {{0.603, 0.701}, {0.921, 1.18}, {0.781, 0.988}, {1.33, 1.81}, {0.662, 0.824}, {1.02, 1.25}, {1.08, 1.42}, {1.14, 1.46}};
+    static const double q5k[8][2] = {{0.647, 0.748}, {1.03, 1.32}, {0.816, 1.03}, {1.43, 1.92}, {0.700, 0.865}, {1.14, 1.34}, {1.21, 1.55}, {1.26, 1.58}};
+    static const double q6k[8][2] = {{0.722, 0.828}, {1.26, 1.47}, {0.881, 1.09}, {1.61, 2.08}, {0.771, 0.935}, {1.29, 1.46}, {1.37, 1.68}, {1.41, 1.70}};
+    static const double q80[8][2] = {{0.762, 0.835}, {1.27, 1.53}, {1.09, 1.18}, {1.58, 2.11}, {0.890, 1.02}, {1.37, 1.51}, {1.48, 1.73}, {1.49, 1.74}};
+    static const double q40[8][2] = {{0.573, 0.672}, {0.877, 1.13}, {0.759, 0.942}, {1.26, 1.69}, {0.645, 0.768}, {0.970, 1.15}, {1.03, 1.32}, {1.09, 1.35}};
+    static const double q50[8][2] = {{0.621, 0.728}, {1.14, 1.34}, {0.794, 0.988}, {1.49, 1.90}, {0.684, 0.830}, {1.21, 1.33}, {1.26, 1.55}, {1.31, 1.55}};
+    static const double q51[8][2] = {{0.631, 0.712}, {1.06, 1.26}, {0.807, 0.955}, {1.43, 1.82}, {0.684, 0.800}, {1.17, 1.25}, {1.22, 1.45}, {1.27, 1.47}};
+    static const double outside[8] = {2.4, 5.6, 5.5, 9.0, 5.0, 6.0, 7.2, 7.2};
     const double (*table)[2] = enc == ENC_Q4_K ? q4k : enc == ENC_Q5_K ? q5k : enc == ENC_Q6_K ? q6k : enc == ENC_Q4_0 ? q40 : enc == ENC_Q5_0 ? q50
                              : enc == ENC_Q5_1 ? q51 : q80;
-    const int shape = (wtm == 4 ? 2 : 0) + (wtn == 4 ? 1 : 0);
+    const int shape = wtm == 3 ? 2 + wtn : wtn == 3 ? 7 : (wtm == 4 ? 2 : 0) + (wtn == 4 ? 1 : 0);
     const int kgroups = (k + 255) / 256, per = (kgroups + ks - 1) / ks, splits = (kgroups + per - 1) / per;
     const double steps = per * (256 / GK);
     // the measurements are for 256 CUs
@@ -825,10 +841,13 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     double least = 0.0;
     int wtm = 2, wtn = 2, ksplit = 1;
     double tile_estimate = 0.0;
-    for (int tm = 2; tm <= 4; tm += 2) {
-        if (g_gemm_rows.load() != 0 && tm != g_gemm_rows.load()) continue;
-        for (int tn = 2; tn <= 4; tn += 2) {
-            if (g_gemm_wide.load() >= 0 && (tn == 4) != (g_gemm_wide.load() != 0)) continue;
+    const int forced_tm = g_gemm_rows.load(), wide = g_gemm_wide.load();
+    for (int tm = 2; tm <= 4; ++tm) {
+        if (forced_tm != 0 && tm != forced_tm) continue;
+        const int forced_tn = wide < 0 ? 0 : wide == 0 ? 2 : wide == 2 && tm > 2 ? 3 : 4;
+        for (int tn = 2; tn <= 4; ++tn) {
+            if (tm == 2 && tn == 3) continue;                    // not built: at most 2 % better than its neighbours, rarely
+            if (forced_tn != 0 && tn != forced_tn) continue;
             for (int ks = 1; ks <= 8 && ks <= kgroups; ++ks) {
                 if (g_gemm_ksplit.load() > 0 && ks != (g_gemm_ksplit.load() < kgroups ? g_gemm_ksplit.load() : kgroups)) continue;
                 const double t = gemm_tile_us(enc, tm, tn, m, n, k, ks);

@@ -96,6 +96,29 @@ def test_gemm_on_random_valid_blocks_and_forced_k_splits(hip_backend, torch_cuda
         hip_backend.set_tuning("gemm_rows", 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(192, 192, 256), (193, 385, 512), (385, 191, 768), (255, 257, 1024)])
+@pytest.mark.parametrize("enc", ALL_ENCS)
+def test_gemm_tiles_of_192_rows_or_columns_give_the_bits_of_the_others(hip_backend, torch_cuda, enc, m, n, k):
+    """An output is one chain of matrix instructions over K whatever tile it lies in, so every tile gives the same bits."""
+    packed = gaussian_weight(hip_backend, enc, n, k, 900 + n)
+    x = np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float32)
+    try:
+        hip_backend.set_tuning("gemm_ksplit", 1)
+        hip_backend.set_tuning("gemm_rows", 2)
+        hip_backend.set_tuning("gemm_wide", 0)
+        want = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
+        check_exact(torch_cuda, enc, want, x, packed, n)
+        for rows, wide in ((3, 0), (3, 2), (3, 1), (4, 2)):
+            hip_backend.set_tuning("gemm_rows", rows)
+            hip_backend.set_tuning("gemm_wide", wide)
+            got = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rows, wide)
+    finally:
+        hip_backend.set_tuning("gemm_ksplit", 0)
+        hip_backend.set_tuning("gemm_wide", -1)
+        hip_backend.set_tuning("gemm_rows", 0)
+
+
 @pytest.mark.parametrize("k", [96, 192, 320, 448])
 def test_gemm_q8_0_rows_that_are_not_whole_256_element_groups_fall_back_to_the_row_kernels(hip_backend, torch_cuda, k):
     """The tile kernel's K loop runs over whole 256-element groups; a Q8_0 row of 3, 6, 10 or 14 blocks takes the
