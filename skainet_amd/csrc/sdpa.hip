@@ -177,11 +177,32 @@ __global__ __launch_bounds__(256) void zero_kernel(float* out, int64_t n) {
 float* sdpa_workspace(size_t bytes);   // shim.hip: per-thread scratch, grown on demand
 int launch_sdpa_decode(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                        int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window,
-                       int right_context, const int32_t* lengths, AttnMergePrologue* leave);   // sdpa_decode.hip
+                       int right_context, const int32_t* lengths, AttnMergePrologue* leave, int out_rows);   // sdpa_decode.hip
+bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context);
+bool sdpa_prefill_by_rule();   // sdpa_prefill.hip
 int launch_sdpa_prefill(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                         int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window,
                         int right_context, const int32_t* lengths, const float* mask, int mask_b, int mask_h, int mask_q,
                         int mask_k, int out_rows);   // sdpa_prefill.hip
+
+// The calls that one of the two cache kernels carries, the output [batch, heads, seq_q, head_dim] or with out_rows [batch, seq_q, heads,
+// head_dim]: 1 taken, 0 neither carries it (nothing launched), -1 an error. Arguments as launch_sdpa has checked them.
+int launch_sdpa_cache(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
+                      int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window, int right_context,
+                      const int32_t* lengths, const float* mask, int mask_b, int mask_h, int mask_q, int mask_k, int out_rows) {
+    // decode and draft shapes, and the prompts that are shorter on it: the split-K cache-streaming kernel, when the head shape is one it carries
+    // (a forced form of the prompt kernel keeps its prompts)
+    if (!mask && (seq_q < 16 || (sdpa_prefill_by_rule() &&
+                                 sdpa_decode_takes_prompt(batch, heads, kv_heads, seq_q, seq_kv, head_dim, causal, window, right_context)))) {
+        const int r = launch_sdpa_decode(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal, window,
+                                         right_context, lengths, nullptr, out_rows);
+        if (r != 0) return r;
+    }
+    if (seq_q > 1)   // prompt shape: the matrix-core kernel, when it carries the shape (and the mask's layout)
+        return launch_sdpa_prefill(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal,
+                                   window, right_context, lengths, mask, mask_b, mask_h, mask_q, mask_k, out_rows);
+    return 0;
+}
 
 int launch_sdpa(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                 int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window, int right_context,
@@ -206,16 +227,9 @@ int launch_sdpa(const float* q, const float* k, const float* v, float* out, int 
         if (!ok) return set_error("sdpa: mask dims [%d,%d,%d,%d] do not broadcast over [%d,%d|%d,%d,%d]", mask_b, mask_h,
                                   mask_q, mask_k, batch, heads, kv_heads, seq_q, seq_kv);
     }
-    if (seq_q < 16 && !mask) {   // decode and draft shapes: the split-K cache-streaming kernel, when the head shape is one it carries
-        const int r = launch_sdpa_decode(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal, window,
-                                         right_context, lengths, nullptr);
-        if (r != 0) return r < 0 ? -1 : 0;
-    }
-    if (seq_q > 1) {   // prompt shape: the matrix-core kernel, when it carries the shape (and the mask's layout)
-        const int r = launch_sdpa_prefill(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal,
-                                          window, right_context, lengths, mask, mask_b, mask_h, mask_q, mask_k, 0);
-        if (r != 0) return r < 0 ? -1 : 0;
-    }
+    const int taken = launch_sdpa_cache(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal, window,
+                                        right_context, lengths, mask, mask_b, mask_h, mask_q, mask_k, 0);
+    if (taken != 0) return taken < 0 ? -1 : 0;
     SdpaParams p{q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, head_dim, kv_capacity, scale, causal, window, right_context,
                  lengths, mask, mask_b, mask_h, mask_q, mask_k, 1, 1, nullptr};
     const int per_kv = heads / kv_heads;

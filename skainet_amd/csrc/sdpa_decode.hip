@@ -1,4 +1,4 @@
-// Decode-shape attention (one query position per sequence, or the few of a draft) over a KV cache: bandwidth-bound split-K.
+// Decode-shape attention (one query position per sequence, the few of a draft, or a short prompt) over a KV cache: bandwidth-bound split-K.
 //
 // Same contract as the general kernel in sdpa.hip (reference: skainet_f32_sdpa,
 //   /root/reference/skainet-backends/skainet-backend-native-cpu/native/src/f32_fused.c:290-396, rules of
@@ -41,6 +41,7 @@ struct SdpaDecodeParams {
     float* ml;            // [query rows][splits][2] running maximum (in units of ln 2) and sum of each split
     int subs, tuples;     // workgroups that share a split's keys, and how many such (split, kv head, sequence) there are; tuples 0: a grid of three dimensions
     int seq_q, causal;    // queries per sequence (the last ones of its positions) and whether a later key is hidden from them
+    int out_rows;         // the output as [batch, seq_q, heads, D] instead of [batch, heads, seq_q, D]
 };
 
 // Scores are kept in units of ln 2 (the query is scaled by scale * log2(e) once), so every exponential of the softmax is
@@ -280,11 +281,13 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         int64_t row = row_of[0];
 #pragma unroll
         for (int e = 1; e < GS; ++e) row = g == e ? row_of[e] : row;
+        int64_t out_row = row;
+        if (MQ && p.out_rows) out_row = ((int64_t)b * p.seq_q + (r0 + g) % p.seq_q) * p.heads + kvh * per_kv + (r0 + g) / p.seq_q;
 #pragma unroll
         for (int e = 0; e < EPT; ++e) {
             const int d = i0 + e;                                   // a state's layout in LDS is the row's own element order
             if (!p.part) {
-                p.out[row * D + d] = ls == 0.f ? 0.f : o[e] / ls;   // an undefined score leaves an undefined sum: no zero for it
+                p.out[out_row * D + d] = ls == 0.f ? 0.f : o[e] / ls;   // an undefined score leaves an undefined sum: no zero for it
             } else {
                 p.part[(row * p.splits + split) * D + d] = o[e];
                 if (d == 0) *reinterpret_cast<float2*>(p.ml + (row * p.splits + split) * 2) = make_float2(mm, ls);
@@ -299,7 +302,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
 // lane, maximum and sum by wave reductions (splits <= 64), parked in LDS for everyone.
 template <int D>
 __global__ __launch_bounds__(4 * D) void sdpa_decode_combine_kernel(const float* __restrict__ part, const float* __restrict__ ml,
-                                                                    float* __restrict__ out, int splits) {
+                                                                    float* __restrict__ out, int splits, int heads, int seq_q, int out_rows) {
     __shared__ float sw[SDPA_DECODE_MAX_SPLITS];
     __shared__ float so[4][D];
     const float* src = part + (int64_t)blockIdx.x * splits * D;
@@ -332,7 +335,12 @@ __global__ __launch_bounds__(4 * D) void sdpa_decode_combine_kernel(const float*
     }
     so[j][d] = o;
     __syncthreads();
-    if (j == 0) out[(int64_t)blockIdx.x * D + d] = so[0][d] + so[1][d] + so[2][d] + so[3][d];
+    int64_t row = blockIdx.x;
+    if (out_rows) {
+        const int qi = blockIdx.x % seq_q, bh = blockIdx.x / seq_q;
+        row = ((int64_t)(bh / heads) * seq_q + qi) * heads + bh % heads;
+    }
+    if (j == 0) out[row * D + d] = so[0][d] + so[1][d] + so[2][d] + so[3][d];
 }
 
 float* sdpa_workspace(size_t bytes);   // shim.hip: per-thread scratch, grown on demand
@@ -348,7 +356,7 @@ static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge
     sdpa_decode_kernel<GS, DPL, MQ><<<grid, dim3(256), 0, current_stream()>>>(p);
     SKH_CHECK(hipGetLastError());
     if (merge) {
-        sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits);
+        sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits, p.heads, p.seq_q, p.out_rows);
         SKH_CHECK(hipGetLastError());
     }
     return 1;
@@ -374,13 +382,33 @@ void set_attn_merge_max_keys(int v) { if (v >= 16) g_attn_merge_max_keys = (v + 
 static std::atomic<int> g_attn_merge_splits{6};
 void set_attn_merge_splits(int v) { if (v >= 1 && v <= ATTN_MERGE_MAX_SPLITS) g_attn_merge_splits = v; }
 
+// Whether a prompt (16 queries and more, no mask) goes to this kernel instead of the matrix-core one, which lays K and V out in a launch of
+// its own and sets up a workgroup of eight waves for 32 queries: 8 to 11 us whatever little there is to do. Here a workgroup takes four rows
+// straight from the caller's memory, in one launch up to 256 keys and more, with fp32 operands (the other rounds them to bf16). What ends it is the
+// K and V that every four rows read for themselves. Both sides in us, back to back from the host, fitted to 7050 random prompts (16 to 400 queries,
+// up to 2048 earlier keys, 1 to 64 heads, D 64 and 128; 11 % and 5 % rms); this one has to be a sixth below. 0.62 of them take it, 1.75x, 6 more
+// than 3 % slower (9 % at most): 27 queries, one head, D 64 8.1 -> 4.9 us, 129 queries, 16 heads over 2, D 128 11.8 -> 6.9.
+bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context) {
+    if ((head_dim != 64 && head_dim != 128) || seq_q > seq_kv) return false;
+    const double groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
+    double keys = causal ? seq_kv - 0.5 * (seq_q - 1) : seq_kv, most = seq_kv;          // of a query, on average; of all queries together
+    if (window > 0) {
+        keys = fmin(keys, (double)window + right_context);
+        most = fmin(most, (double)window + right_context + seq_q - 1);
+    }
+    const double rounds = ceil(groups / num_cus()), walked = 1e-3 * groups * keys, kb = 1e-3 * batch * kv_heads * most;
+    const double here = head_dim == 64 ? fmax(5.6, 5.18 + 0.067 * walked + 0.36 * rounds) : fmax(5.6, 5.41 + 0.105 * walked + 0.74 * rounds);
+    const double there = head_dim == 64 ? 9.0 + 5.2e-3 * most + 0.228 * kb + 0.9e-3 * seq_q : 10.7 + 6.0e-3 * most + 0.453 * kb + 3.9e-3 * seq_q;
+    return 1.2 * here < there;
+}
+
 // Returns 1 when this kernel took the call, 0 when the shape is outside its range (the caller uses the general
 // kernel), -1 on error. With `leave` the per-split results are left unmerged for a consumer that folds the merge into
 // its own activation load (at most ATTN_MERGE_MAX_SPLITS splits, one sequence): `out` is not written, *leave describes
 // where the partials are; 0 when the key count would need more splits than that.
 int launch_sdpa_decode(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                        int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window, int right_context,
-                       const int32_t* lengths, AttnMergePrologue* leave) {
+                       const int32_t* lengths, AttnMergePrologue* leave, int out_rows) {
     if (seq_q > seq_kv) return 0;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return 0;
     if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) return 0;
@@ -452,7 +480,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     const int subs = (cols + gs - 1) / gs;
     if (batch > 65535 || (int64_t)kv_heads * subs > 65535) return 0;
     SdpaDecodeParams p{q, k, v, out, batch, heads, kv_heads, seq_kv, kv_capacity, scale, window, right_context, lengths, 1,
-                       nullptr, nullptr, subs, 0, seq_q, causal};
+                       nullptr, nullptr, subs, 0, seq_q, causal, out_rows && seq_q > 1};
     // enough workgroups to put every CU on the cache, at least 64 keys per split (measured in the decoder at 500 to 650
     // keys: 32 or 48 keys per split 2.5 % slower per token, 96 and 128 keys the same as 64)
     const int64_t groups = (int64_t)batch * kv_heads * subs;
@@ -515,7 +543,7 @@ int launch_attn_out_proj_q4k(const uint8_t* wo, int n, int k, const float* q, co
     if (residual && (reinterpret_cast<uintptr_t>(residual) & 3)) return 0;
     AttnMergePrologue am{};
     const int r = launch_sdpa_decode(q, k_cache, v_cache, nullptr, 1, heads, kv_heads, 1, seq_kv, kv_capacity, head_dim, scale, 1, window, 0,
-                                     lengths, &am);
+                                     lengths, &am, 0);
     if (r <= 0) return r;
     const int g = launch_q4k_gemv_mfma(wo, nullptr, out, k, n, nullptr, 0.f, residual, residual ? EPI_RESIDUAL : EPI_NONE, nullptr, &am);
     if (g == 0) return set_error("attn_out_proj: the projection refused a shape its checks had passed (n %d, k %d)", n, k);

@@ -668,6 +668,9 @@ static int launch_prefill_d(const float* q, const float* k, const float* v, floa
     return 1;
 }
 
+// No form of this kernel is forced and it is not switched off: the launcher may weigh it against others.
+bool sdpa_prefill_by_rule() { return g_prefill_mfma.load() && g_prefill_teams.load() == 0 && g_prefill_splits.load() == 0; }
+
 // Returns 1 when the MFMA path took the call, 0 when the shape is outside its range, -1 on error.
 int launch_sdpa_prefill(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                         int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window,

@@ -265,6 +265,41 @@ def test_attention_prefill_mfma_shapes(hip_backend, torch_cuda, batch, heads, kv
 
 
 @pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv,causal,window,rc,lengths", [
+    (1, 1, 1, 64, 16, 16, True, 0, 0, None), (1, 3, 1, 128, 17, 17, True, 0, 0, None),       # rows that are no multiple of a workgroup's four
+    (1, 8, 2, 128, 33, 97, True, 0, 0, None), (1, 2, 2, 64, 31, 400, True, 0, 0, None),      # a later chunk; keys split over workgroups
+    (2, 4, 2, 64, 40, 40, True, 0, 0, [40, 7]), (3, 4, 4, 64, 20, 30, True, 10, 0, [30, 9, 0]),   # key lengths, sequences without a key
+    (1, 6, 3, 128, 50, 50, False, 12, 5, None), (1, 4, 1, 64, 24, 64, False, 0, 0, None),
+    (1, 1, 1, 128, 100, 900, True, 128, 0, None), (2, 2, 1, 64, 90, 90, True, 0, 0, None)])
+def test_attention_short_prompts_stream_the_cache(hip_backend, torch_cuda, batch, heads, kv_heads, d, sq, skv, causal, window, rc, lengths):
+    """Prompts that the streaming kernel is the faster one for: fp32 operands, so the reference's own tolerance; as token rows the same bits;
+    values of excluded keys do not reach the output."""
+    torch = torch_cuda
+    rng = np.random.default_rng(sq * skv + d)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((batch, heads, sq, d), (batch, kv_heads, skv, d), (batch, kv_heads, skv, d)))
+    scale = float(1 / np.sqrt(d))
+    ln = None if lengths is None else np.asarray(lengths, np.int32)
+    got = gpu_sdpa(hip_backend, torch, q, k, v, scale, causal, window, rc, ln)
+    assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+    close(got, L.sdpa(q, k, v, scale, causal, window, rc, ln))
+    rows = torch.full((batch, sq, heads, d), float("nan"), device="cuda")
+    hip_backend.sdpa_cache_rows_dev(*(dev(torch, a) for a in (q, k, v)), rows, batch, heads, kv_heads, sq, skv, skv, d, scale, causal, window, rc,
+                                    None if ln is None else dev(torch, ln))
+    assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+    assert np.array_equal(rows.cpu().numpy(), got.transpose(0, 2, 1, 3))
+    if causal and window == 0 and ln is None:
+        v[:, :, -1] = np.nan                                        # the last key: only the last query's
+        late = gpu_sdpa(hip_backend, torch, q, k, v, scale, causal)
+        assert np.array_equal(late[:, :, :-1], got[:, :, :-1]) and np.isnan(late[:, :, -1]).all()
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,sq,skv", [(32, 8, 128, 512, 512), (8, 1, 64, 300, 2000)])
+def test_attention_long_prompts_stay_on_the_matrix_cores(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv):
+    q, k, v = (np.zeros(s, np.float32) for s in ((1, heads, sq, d), (1, kv_heads, skv, d), (1, kv_heads, skv, d)))
+    gpu_sdpa(hip_backend, torch_cuda, q, k, v, 1.0, True)
+    assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+
+
+@pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv,causal,window,rc,lengths", [
     (1, 8, 2, 128, 300, 300, True, 64, 0, None),            # sliding window shorter than a key block ... 
     (1, 8, 2, 128, 300, 300, True, 100, 0, None),           # ... and one that straddles blocks
     (2, 4, 2, 64, 200, 200, True, 0, 0, [200, 77]),         # key lengths: the second sequence ends inside a block
