@@ -433,7 +433,8 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * 0 = automatic), "gemv_few" (products of 1 to 8 rows by lanes that decode 64 weights at a time: 0 never, 1 where they are the faster ones,
  * 2 wherever they fit), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
  * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2), "gemm_wide" (0 / 1 / 2: force the tile of 128 / 256 / 192
- * columns, 192 with 128 rows being 256, -1 = chosen from the shape), "gemm_rows" (2 / 3 / 4: 128 / 192 / 256 activation rows per tile, 0 = chosen from the shape), "gemm_ksw" (the Q4_K kernel that splits K over the
+ * columns, 192 with 128 rows being 256, -1 = chosen from the shape), "gemm_rows" (2 / 3 / 4: 128 / 192 / 256 activation rows per tile, 0 = chosen from the shape),
+ * "gemm_f32" (the 128 x 128 tile on the fp32 rows instead of rounded copies: 0 never, 1 where the estimate favours it, 2 wherever that tile is taken), "gemm_ksw" (the Q4_K kernel that splits K over the
  * waves of a workgroup: 0 never, 1 where "gemm_frag" is 0 and the launcher's estimate favours it -- the fragment-order kernel
  * is the faster one wherever both fit -- 2 wherever it fits; 0 keeps Q4_K from "gemm_frag" and "gemm_skinny" by rule as well:
  * the tile kernel is left), "gemm_ksw_teams" (teams

@@ -20,6 +20,7 @@
 #include "common.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace skh {
 
@@ -419,11 +420,17 @@ __device__ __forceinline__ uint32_t decode_item_at(int h, const Raw& r, const Sb
     }
 }
 
-template <class Raw, int BLOCK_ELEMS, int BLOCK_BYTES, int WTM, int WTN>
-__global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* __restrict__ a, const uint8_t* __restrict__ w,
+// F32: `rows` are not the bf16 rows that the pass in front left but the caller's fp32 rows, rounded on their way into LDS (the same bits). That saves the
+// pass (a launch, and the rows once more through memory: 4 us and more) and doubles what a tile reads of them, so it is for products up to
+// about 20 us on 128 x 128 tiles: of 581 random ones (33 to 1024 rows) those below 12 us take 0.86 of their time there, 12 to 20 us 0.88, 30 to 50
+// us 1.01, longer ones 1.09 (256 x 128 tiles 0.95 at best, so those and the larger ones have no such form). Q6_K 932 x 773 x 1024 19.2 ->
+// 14.2 us, Q5_K 316 x 2181 x 3072 22.9 -> 19.1.
+template <class Raw, int BLOCK_ELEMS, int BLOCK_BYTES, int WTM, int WTN, bool F32>
+__global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const void* __restrict__ rows, const uint8_t* __restrict__ w,
                                                            float* __restrict__ c, int m, int n, int k, int k_chunk,
                                                            int64_t split_stride) {
     constexpr int G_WTN = WTN, GN = gemm_gn(WTN), GM = gemm_gm(WTM);
+    const auto* __restrict__ a = static_cast<const std::conditional_t<F32, float, __bf16>*>(rows);
     constexpr int G_A_LOADS = GM * (GK / 8) / G_THREADS;      // 16-byte chunks of the activation tile per thread
     constexpr int G_A_ELEMS = GM * GSTRIDE;
     constexpr int G_W_TASKS = gemm_wrows(WTN) * 2 / G_THREADS;   // 32-weight decode tasks per thread and step
@@ -458,7 +465,8 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     typedef typename DecOf<Raw>::type Dec;
     typedef typename SbOf<Raw>::type Sb;
-    u32x4 aring[A_SLOTS][G_A_LOADS];
+    constexpr int A_PIECES = F32 ? 2 : 1;                           // 16-byte loads of a chunk of eight elements
+    u32x4 aring[A_SLOTS][G_A_LOADS][A_PIECES];
     Raw wring[2][G_W_TASKS];
     // per-super-block constants of each task's row: those of the super-block being decoded, and those of the one after it,
     // requested in the second of a super-block's four steps and taken over behind the fourth
@@ -466,7 +474,9 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
     auto step_k = [&](int step) { return k_begin + min(step, nsteps - 1) * GK; };   // loads past the end re-read the last step
     auto load_a_chunk = [&](int slot, int step, int j) __attribute__((always_inline)) {
         const int p = tid + G_THREADS * j, row = p >> 3, kp = p & 7;
-        aring[slot][j] = *reinterpret_cast<const u32x4*>(a + (int64_t)min(m0 + row, m - 1) * k + step_k(step) + 8 * kp);
+        const u32x4* src = reinterpret_cast<const u32x4*>(a + (int64_t)min(m0 + row, m - 1) * k + step_k(step) + 8 * kp);
+#pragma unroll
+        for (int h = 0; h < A_PIECES; ++h) aring[slot][j][h] = src[h];
     };
     auto load_a = [&](int slot, int step) __attribute__((always_inline)) {
 #pragma unroll
@@ -481,7 +491,13 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
     };
     auto park_a = [&](int slot, int stage, int j) __attribute__((always_inline)) {      // chunk j of a step's activation tile -> LDS stage
         const int p = tid + G_THREADS * j, row = p >> 3, kp = p & 7;
-        *reinterpret_cast<u32x4*>(a_tile(stage) + row * GSTRIDE + 8 * kp) = aring[slot][j];
+        u32x4 v = aring[slot][j][0];
+        if constexpr (F32) {
+            typedef float f32x4 __attribute__((ext_vector_type(4)));
+            const f32x4 lo = __builtin_bit_cast(f32x4, aring[slot][j][0]), hi = __builtin_bit_cast(f32x4, aring[slot][j][1]);
+            v = __builtin_bit_cast(u32x4, bf16x8{(__bf16)lo.x, (__bf16)lo.y, (__bf16)lo.z, (__bf16)lo.w, (__bf16)hi.x, (__bf16)hi.y, (__bf16)hi.z, (__bf16)hi.w});
+        }
+        *reinterpret_cast<u32x4*>(a_tile(stage) + row * GSTRIDE + 8 * kp) = v;
     };
     uint32_t wp[G_W_TASKS][16];                                                         // packed bf16 pairs: weights 2 h, 2 h + 1
     auto park_w = [&](int stage, int t, int i) __attribute__((always_inline)) {         // weights 8 i .. 8 i + 7 of task t's 32
@@ -660,18 +676,19 @@ __global__ __launch_bounds__(G_THREADS) void dequant_gemm_kernel(const __bf16* _
         }
 }
 
-template <class Raw, int BE, int BB, int WTM, int WTN>
-static int launch_gemm_tile(const __bf16* a, const uint8_t* w, float* c, int m, int n, int k, dim3 grid, int k_chunk,
-                            int64_t split_stride, hipStream_t s) {
-    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&dequant_gemm_kernel<Raw, BE, BB, WTM, WTN>), gemm_smem(WTM, WTN));
+template <class Raw, int BE, int BB, int WTM, int WTN, bool F32 = false>
+static int launch_gemm_tile(const void* a, const uint8_t* w, float* c, int m, int n, int k, dim3 grid, int k_chunk, int64_t split_stride, hipStream_t s) {
+    SKH_SET_MAX_DYNAMIC_LDS_ONCE((&dequant_gemm_kernel<Raw, BE, BB, WTM, WTN, F32>), gemm_smem(WTM, WTN));
     note_kernel("dequant_gemm_kernel");
-    dequant_gemm_kernel<Raw, BE, BB, WTM, WTN><<<grid, dim3(G_THREADS), gemm_smem(WTM, WTN), s>>>(a, w, c, m, n, k, k_chunk, split_stride);
+    dequant_gemm_kernel<Raw, BE, BB, WTM, WTN, F32><<<grid, dim3(G_THREADS), gemm_smem(WTM, WTN), s>>>(a, w, c, m, n, k, k_chunk, split_stride);
     SKH_CHECK(hipGetLastError());
     return 0;
 }
+// x: fp32 rows for the 128 x 128 tile, where a is null
 template <class Raw, int BE, int BB>
-static int launch_gemm_enc(int wtm, int wtn, const __bf16* a, const uint8_t* w, float* c, int m, int n, int k, dim3 grid, int k_chunk,
+static int launch_gemm_enc(int wtm, int wtn, const float* x, const __bf16* a, const uint8_t* w, float* c, int m, int n, int k, dim3 grid, int k_chunk,
                            int64_t split_stride, hipStream_t s) {
+    if (!a) return launch_gemm_tile<Raw, BE, BB, 2, 2, true>(x, w, c, m, n, k, grid, k_chunk, split_stride, s);
     if (wtm == 3) {
         if (wtn == 4) return launch_gemm_tile<Raw, BE, BB, 3, 4>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
         if (wtn == 3) return launch_gemm_tile<Raw, BE, BB, 3, 3>(a, w, c, m, n, k, grid, k_chunk, split_stride, s);
@@ -710,6 +727,8 @@ static std::atomic<int> g_gemm_ksplit{0};   // 0 = choose from the tile count
 void set_gemm_ksplit(int v) { g_gemm_ksplit = v; }
 static std::atomic<int> g_gemm_wide{-1};    // -1 = choose from the shape, 0 / 1 / 2 = 128 / 256 / 192 columns per tile (192 with 128 rows: 256)
 void set_gemm_wide(int v) { g_gemm_wide = v; }
+static std::atomic<int> g_gemm_f32{1};      // the 128 x 128 tile on fp32 rows: 0 never, 1 where the estimate favours it, 2 wherever that tile is taken
+void set_gemm_f32(int v) { if (v >= 0 && v <= 2) g_gemm_f32 = v; }
 static std::atomic<int> g_gemm_rows{0};     // 0 = choose from the shape, 2 / 3 / 4 = 128 / 192 / 256 activation rows per tile
 void set_gemm_rows(int v) { if (v == 0 || (v >= 2 && v <= 4)) g_gemm_rows = v; }
 
@@ -755,6 +774,13 @@ static double gemm_tile_us(int enc, int wtm, int wtn, int m, int n, int k, int k
     }
     return tiles > 0 ? t + round(tiles) : t;
 }
+// What the 128 x 128 tile saves on the fp32 rows, in us: the pass, against a step's second half of the rows (fitted to the same 581
+// products on both forms, 4 % rms of the whole).
+static double gemm_f32_saves_us(int m, int n, int k, int ks) {
+    const int kgroups = (k + 255) / 256, per = (kgroups + ks - 1) / ks, splits = (kgroups + per - 1) / per;
+    const double tiles = (double)((m + gemm_gm(2) - 1) / gemm_gm(2)) * ((n + gemm_gn(2) - 1) / gemm_gn(2)) * splits / num_cus();
+    return 2.25 + 2.4e-7 * m * k - 0.068 * per * (256 / GK) * (tiles <= 1 ? 1 : 2 * ceil(tiles / 2));
+}
 // The same for the fragment-order kernel (Q4_K, 128 x 64 tiles), 14 000 timings within 5 %. Up to a tile per CU its eight waves
 // share K by super-blocks: a started round of four costs about half of a whole one at once. Above, two workgroups of four waves on
 // a CU: the first of a pair takes a third of what both take, a pair on every second CU four fifths.
@@ -789,7 +815,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
         (gain && ((reinterpret_cast<uintptr_t>(gain) & 15) || k > 256 * 4 * 16)) || (epilogue == GEMM_EPI_SWIGLU && (n & 1)) ||
         (epilogue != GEMM_EPI_NONE && !tmp))
         return fused ? 1 : launch_gemv(enc, w, x, m, k, n, y);
-    // The one-launch form takes plain activations, and rows that no workgroup overwrites while another one reads them.
+    // The forms on fp32 rows take plain activations, and rows that no workgroup overwrites while another one reads them.
     const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
     const bool direct_ok = !gain && !x_pairs && (x0 + sizeof(float) * (size_t)m * k <= y0 || y0 + sizeof(float) * (size_t)m * n <= x0);
     const int skinny_mode = gemm_skinny_mode();
@@ -892,28 +918,34 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
             if (tiles * ks <= num_cus() && t < tile_estimate) { tile_estimate = t; wtm = 2; wtn = 2; ksplit = ks; }
         }
     }
+    // The fp32 rows where that saves 2 %. It plays no part in the choices above: with its estimate among theirs, 102 of 1649 products went from
+    // the few-rows and fragment-order kernels to this one, most of them slower. Of 1280 others (24 to 1024 rows) 204 take it, 1.06x; the 8 of them
+    // that were more than 3 % slower had rows of more than 6144, which are left out.
+    const bool f32 = direct_ok && wtm == 2 && wtn == 2 && g_gemm_f32.load() != 0 &&
+                     (g_gemm_f32.load() == 2 || (k <= 6144 && gemm_f32_saves_us(m, n, k, ksplit) > 0.02 * tile_estimate));
     const int tiles_m = (m + gemm_gm(wtm) - 1) / gemm_gm(wtm), tiles_n = (n + gemm_gn(wtn) - 1) / gemm_gn(wtn);
     if (ksplit > kgroups) ksplit = kgroups;
     const int k_chunk = ((kgroups + ksplit - 1) / ksplit) * 256;
     ksplit = (k + k_chunk - 1) / k_chunk;
-    // workspace: the bf16 activations, then (split K) one partial product per split
-    const size_t a_bytes = (((size_t)m * k * sizeof(__bf16)) + 255) & ~(size_t)255;
+    // workspace: the bf16 activations unless the tile reads the fp32 rows, then (split K) one partial product per split
+    const size_t a_bytes = f32 ? 0 : (((size_t)m * k * sizeof(__bf16)) + 255) & ~(size_t)255;
     const int64_t split_stride = ksplit > 1 ? (((int64_t)m * n + 3) & ~(int64_t)3) : 0;
-    char* ws = static_cast<char*>(kernel_workspace(a_bytes + (size_t)split_stride * ksplit * sizeof(float)));
-    if (!ws) return -1;
-    __bf16* a = reinterpret_cast<__bf16*>(ws);
+    const size_t ws_bytes = a_bytes + (size_t)split_stride * ksplit * sizeof(float);
+    char* ws = ws_bytes ? static_cast<char*>(kernel_workspace(ws_bytes)) : nullptr;
+    if (ws_bytes && !ws) return -1;
+    __bf16* a = f32 ? nullptr : reinterpret_cast<__bf16*>(ws);
     float* part = reinterpret_cast<float*>(ws + a_bytes);
-    if (round_activations(a) != 0) return -1;
+    if (!f32 && round_activations(a) != 0) return -1;
     const dim3 grid(tiles_n, tiles_m, ksplit);
     float* c = ksplit > 1 ? part : (epilogue != GEMM_EPI_NONE ? tmp : y);
     int rc;
-    if (enc == ENC_Q4_K) rc = launch_gemm_enc<RawQ4K, QK_ELEMS, Q4K_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else if (enc == ENC_Q6_K) rc = launch_gemm_enc<RawQ6K, QK_ELEMS, Q6K_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else if (enc == ENC_Q5_K) rc = launch_gemm_enc<RawQ5K, QK_ELEMS, Q5K_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else if (enc == ENC_Q4_0) rc = launch_gemm_enc<RawQ45<0>, Q80_ELEMS, Q40_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else if (enc == ENC_Q5_0) rc = launch_gemm_enc<RawQ45<1>, Q80_ELEMS, Q50_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else if (enc == ENC_Q5_1) rc = launch_gemm_enc<RawQ45<2>, Q80_ELEMS, Q51_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
-    else rc = launch_gemm_enc<RawQ80, Q80_ELEMS, Q80_BYTES>(wtm, wtn, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    if (enc == ENC_Q4_K) rc = launch_gemm_enc<RawQ4K, QK_ELEMS, Q4K_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else if (enc == ENC_Q6_K) rc = launch_gemm_enc<RawQ6K, QK_ELEMS, Q6K_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else if (enc == ENC_Q5_K) rc = launch_gemm_enc<RawQ5K, QK_ELEMS, Q5K_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else if (enc == ENC_Q4_0) rc = launch_gemm_enc<RawQ45<0>, Q80_ELEMS, Q40_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else if (enc == ENC_Q5_0) rc = launch_gemm_enc<RawQ45<1>, Q80_ELEMS, Q50_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else if (enc == ENC_Q5_1) rc = launch_gemm_enc<RawQ45<2>, Q80_ELEMS, Q51_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
+    else rc = launch_gemm_enc<RawQ80, Q80_ELEMS, Q80_BYTES>(wtm, wtn, x, a, w, c, m, n, k, grid, k_chunk, split_stride, s);
     if (rc != 0) return rc;
     if (ksplit == 1) return finish();
     const int64_t total = (int64_t)m * n;

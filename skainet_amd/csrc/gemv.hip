@@ -190,6 +190,7 @@ void set_q4k_rows_waves_per_cu(int v);
 void set_gemm_wide(int v);
 void set_gemm_ksplit(int v);
 void set_gemm_rows(int v);
+void set_gemm_f32(int v);
 void set_gemm_ksw(int v);
 void set_gemm_skinny(int v);
 void set_gemm_ksw_teams(int v);
@@ -240,6 +241,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "gemm_wide")) { set_gemm_wide(value); return 0; }
     if (!strcmp(key, "q4k_rows_enable")) { g_q4k_rows_enable = value; return 0; }
     if (!strcmp(key, "gemm_ksplit")) { set_gemm_ksplit(value); return 0; }
+    if (!strcmp(key, "gemm_f32")) { set_gemm_f32(value); return 0; }
     if (!strcmp(key, "gemm_rows")) { set_gemm_rows(value); return 0; }
     if (!strcmp(key, "gemv_few")) { set_gemv_few(value); return 0; }
     if (!strcmp(key, "gemm_skinny")) { set_gemm_skinny(value); return 0; }

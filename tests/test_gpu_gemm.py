@@ -119,6 +119,33 @@ def test_gemm_tiles_of_192_rows_or_columns_give_the_bits_of_the_others(hip_backe
         hip_backend.set_tuning("gemm_rows", 0)
 
 
+@pytest.mark.parametrize("m,n,k,ks", [(128, 128, 256, 1), (129, 131, 512, 1), (33, 257, 1024, 3), (300, 127, 2304, 2), (16, 16, 256, 1)])
+@pytest.mark.parametrize("enc", ALL_ENCS)
+def test_gemm_tile_on_fp32_rows_gives_the_bits_of_the_rounded_rows(hip_backend, torch_cuda, enc, m, n, k, ks):
+    """The tile rounds the rows itself instead of a pass in front: the same values, so the same bits; also where the product lies over the
+    rows, which then go through the pass."""
+    torch = torch_cuda
+    w = hip_backend.DeviceWeight.upload(enc, gaussian_weight(hip_backend, enc, n, k, 700 + n), n, k)
+    x = torch.from_numpy(np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)).cuda()
+    got = {}
+    try:
+        for key, v in (("gemm_skinny", 0), ("gemm_frag", 0), ("gemm_ksw", 0), ("gemm_rows", 2), ("gemm_wide", 0), ("gemm_ksplit", ks)):
+            hip_backend.set_tuning(key, v)
+        for mode in (0, 2):
+            hip_backend.set_tuning("gemm_f32", mode)
+            both = torch.full((m * k + m * n,), float("nan"), device="cuda")
+            xs, apart, over = both[:m * k].reshape(m, k).copy_(x), both[m * k:], both[:m * n]
+            w.matmul(xs, m, apart, 1)
+            got[mode] = apart.clone()
+            if n <= k:
+                w.matmul(xs, m, over, 1)
+                assert torch.equal(over, got[mode])
+    finally:
+        for key, v in (("gemm_skinny", 1), ("gemm_frag", 1), ("gemm_ksw", 1), ("gemm_rows", 0), ("gemm_wide", -1), ("gemm_ksplit", 0), ("gemm_f32", 1)):
+            hip_backend.set_tuning(key, v)
+    assert not torch.isnan(got[0]).any() and torch.equal(got[0], got[2])
+
+
 @pytest.mark.parametrize("k", [96, 192, 320, 448])
 def test_gemm_q8_0_rows_that_are_not_whole_256_element_groups_fall_back_to_the_row_kernels(hip_backend, torch_cuda, k):
     """The tile kernel's K loop runs over whole 256-element groups; a Q8_0 row of 3, 6, 10 or 14 blocks takes the
