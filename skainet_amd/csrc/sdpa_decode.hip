@@ -386,8 +386,8 @@ void set_attn_merge_splits(int v) { if (v >= 1 && v <= ATTN_MERGE_MAX_SPLITS) g_
 // its own and sets up a workgroup of eight waves for 32 queries: 8 to 11 us whatever little there is to do. Here a workgroup takes four rows
 // straight from the caller's memory, in one launch up to 256 keys and more, with fp32 operands (the other rounds them to bf16). What ends it is the
 // K and V that every four rows read for themselves. Both sides in us, back to back from the host, fitted to 7050 random prompts (16 to 400 queries,
-// up to 2048 earlier keys, 1 to 64 heads, D 64 and 128; 11 % and 5 % rms); this one has to be a sixth below. 0.62 of them take it, 1.75x, 6 more
-// than 3 % slower (9 % at most): 27 queries, one head, D 64 8.1 -> 4.9 us, 129 queries, 16 heads over 2, D 128 11.8 -> 6.9.
+// up to 2048 earlier keys, 1 to 64 heads, D 64 and 128; 11 % and 5 % rms); this one has to be a sixth below. Of 8549 others 0.67 take it, 1.60x, 14
+// more than 3 % slower: 27 queries, one head, D 64 8.1 -> 4.9 us, 129 queries, 16 heads over 2, D 128 11.8 -> 6.9.
 bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context) {
     if ((head_dim != 64 && head_dim != 128) || seq_q > seq_kv) return false;
     const double groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
@@ -420,7 +420,8 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     // only not wider than the rows there are
     while (draft ? gs > 2 && per_kv * seq_q <= gs / 2 : per_kv % gs != 0) gs >>= 1;
     // keys that a query can attend: a window bounds them whatever the cache holds
-    const int keys = window > 0 ? (int)min((int64_t)seq_kv, (int64_t)window + right_context + seq_q - 1) : seq_kv;
+    // (a prompt: those of a workgroup's four queries; with all queries' 385 x 1828 under a window of 153 was split and took 21 us)
+    const int keys = window > 0 ? (int)min((int64_t)seq_kv, (int64_t)window + right_context + (seq_q < 16 ? seq_q - 1 : 3)) : seq_kv;
     // One split, no merge behind it: the merge is a second launch (2.8 us of a host's time, and about that between two
     // dependent kernels on the device), which buys the parallelism of the splits -- and shorter sums: with one split the error
     // against float64 is up to a third larger (950 keys 1.6e-7 and 2.1e-7). So two estimates in us both have to say that it pays.
