@@ -389,6 +389,13 @@ SKAINET_HIP_API int32_t skainet_hip_i32_increment_dev(int32_t* value, int32_t de
  * host reads the saturated position. */
 SKAINET_HIP_API int32_t skainet_hip_decode_advance_dev(int32_t* pos, int32_t* kv_len, const int32_t* token, int32_t* log,
     int32_t capacity);
+/* The same with the arg-max of `logits[cols]` in front, one launch: *token = arg-max (skainet_hip_f32_argmax_rows_dev), then the advance. */
+SKAINET_HIP_API int32_t skainet_hip_decode_end_dev(const float* logits, int32_t cols, int32_t* token, int32_t* pos, int32_t* kv_len,
+    int32_t* log, int32_t capacity);
+/* Start of a decode step: out[cols] = embedding row *token (skainet_hip_dequantize_rows_dev) and the rotation table of *pos_dev
+ * (skainet_hip_f32_rope_table_dev), one launch for Q4_K. */
+SKAINET_HIP_API int32_t skainet_hip_decode_begin_dev(const skainet_hip_weight* embedding, const int32_t* token, float* out,
+    const int32_t* pos_dev, float theta, int32_t head_dim, float* rope_table);
 SKAINET_HIP_API int32_t skainet_hip_i32_store_at_dev(int32_t* dst, const int32_t* index_dev, int32_t offset, const int32_t* src);
 
 /* HIP graphs (no reference counterpart; for launch-bound loops such as a decode step): graph_begin redirects this

@@ -98,6 +98,8 @@ SIGNATURES = {
     "skainet_hip_f32_argmax_rows_noalloc_dev": (_i32, [_vp, _i32, _i32, _vp]),
     "skainet_hip_f32_argmax_rows_noalloc_slot": (_i32, []),
     "skainet_hip_f32_rope_scatter_dev": (_i32, [_vp, _i64, _vp, _i32, _i32, _i32, _i32, _vp, _f32, _i32, _i64, _i32]),
+    "skainet_hip_decode_begin_dev": (_i32, [_vp, _vp, _vp, _vp, _f32, _i32, _vp]),
+    "skainet_hip_decode_end_dev": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _i32]),
     "skainet_hip_decode_advance_dev": (_i32, [_vp, _vp, _vp, _vp, _i32]),
     "skainet_hip_i32_store_at_dev": (_i32, [_vp, _vp, _i32, _vp]),
     "skainet_hip_f32_swiglu_pairs_dev": (_i32, [_vp, _vp, _i64]),

@@ -61,13 +61,8 @@ __device__ __forceinline__ void q4k_scale_min(const uint8_t* s, int j, int& sc, 
 
 // One thread per 8 output elements; 32 threads per Q4_K block. Thread u: sub-block sb = u / 4,
 // elements [8 * (u % 4), +8) of it, i.e. 8 consecutive bytes of 32-byte group sb / 2, low or high nibble.
-__global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t* __restrict__ w, float* __restrict__ out,
-                                                          int64_t nblocks, const int32_t* __restrict__ row_ids, int bpr, int rows) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t b = t >> 5;
-    if (b >= nblocks) return;
-    const int u = (int)(t & 31), sb = u >> 2, e0 = (u & 3) * 8;
-    const uint8_t* p = w + source_block(b, row_ids, bpr, rows) * Q4K_BYTES;
+__device__ __forceinline__ void dequant_q4k_part(const uint8_t* p, int u, float* out) {
+    const int sb = u >> 2, e0 = (u & 3) * 8;
     const uint32_t dd = *reinterpret_cast<const uint32_t*>(p);
     const float d = half_bits_to_float(dd & 0xFFFFu), dmin = half_bits_to_float(dd >> 16);
     int sc, mn;
@@ -82,9 +77,29 @@ __global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t* __restr
         v[i] = __fsub_rn(__fmul_rn((float)((q.x >> (8 * i + shift)) & 0xF), scale), offset);
         v[4 + i] = __fsub_rn(__fmul_rn((float)((q.y >> (8 * i + shift)) & 0xF), scale), offset);
     }
-    float4* o = reinterpret_cast<float4*>(out + b * QK_ELEMS + sb * 32 + e0);
+    float4* o = reinterpret_cast<float4*>(out + sb * 32 + e0);
     o[0] = make_float4(v[0], v[1], v[2], v[3]);
     o[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+__global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t* __restrict__ w, float* __restrict__ out,
+                                                          int64_t nblocks, const int32_t* __restrict__ row_ids, int bpr, int rows) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t b = t >> 5;
+    if (b >= nblocks) return;
+    dequant_q4k_part(w + source_block(b, row_ids, bpr, rows) * Q4K_BYTES, (int)(t & 31), out + b * QK_ELEMS);
+}
+// The start of a decode step in one launch: the embedding row of the token, and in the last workgroup the rotation table of its position
+// (together with the arg-max and the advance at the step's end: two launches less, 64.3 -> 60.9 us per step of two layers of 1024).
+__global__ __launch_bounds__(256) void decode_begin_q4k_kernel(const uint8_t* __restrict__ w, float* __restrict__ out, int bpr, int rows,
+                                                               const int32_t* __restrict__ token, const int32_t* __restrict__ pos, float theta,
+                                                               int head_dim, float2* __restrict__ table) {
+    if (blockIdx.x == gridDim.x - 1) {
+        for (int i = threadIdx.x; i < head_dim / 2; i += 256) table[i] = rope_cos_sin(pos[0], theta, i, head_dim);
+        return;
+    }
+    const int t = blockIdx.x * 256 + threadIdx.x, b = t >> 5;
+    if (b >= bpr) return;
+    dequant_q4k_part(w + source_block(b, token, bpr, rows) * Q4K_BYTES, t & 31, out + (int64_t)b * QK_ELEMS);
 }
 
 // One thread per 8 output elements; 32 threads per Q6_K block. Thread u: half = u / 16, quarter k = (u / 4) % 4
@@ -179,6 +194,17 @@ __global__ __launch_bounds__(256) void dequant_q5k_kernel(const uint8_t* __restr
     float4* o = reinterpret_cast<float4*>(out + b * QK_ELEMS + sb * 32 + e0);
     o[0] = make_float4(v[0], v[1], v[2], v[3]);
     o[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+
+int launch_rope_table(const int32_t* pos, float theta, int head_dim, float* table);   // rows.hip
+int launch_dequant(int enc, const uint8_t* w, int64_t nblocks, float* out, const int32_t* row_ids, int bpr, int rows);
+// out[cols] = row *token of the weight, table = the rotation table of *pos.
+int launch_decode_begin(int enc, const uint8_t* w, int bpr, int rows, const int32_t* token, float* out, const int32_t* pos, float theta, int head_dim, float* table) {
+    if (head_dim <= 0 || (head_dim & 1)) return set_error("decode_begin: head_dim must be positive and even; got %d", head_dim);
+    if (enc != ENC_Q4_K || bpr <= 0) return launch_dequant(enc, w, bpr, out, token, bpr, rows) != 0 ? -1 : launch_rope_table(pos, theta, head_dim, table);
+    decode_begin_q4k_kernel<<<dim3((bpr + 7) / 8 + 1), dim3(256), 0, current_stream()>>>(w, out, bpr, rows, token, pos, theta, head_dim, reinterpret_cast<float2*>(table));
+    SKH_CHECK(hipGetLastError());
+    return 0;
 }
 
 // Decodes `nblocks` consecutive output blocks; with `row_ids` (device int32) output row r is source row row_ids[r]

@@ -264,8 +264,21 @@ __device__ __forceinline__ void argmax_walk(const float* x, int lo, int hi, floa
     }
 }
 
+// What a greedy decode step does with its token: the position and the key count advance by one and the token is appended to the log at the new
+// position. The position saturates at `capacity` (the cache's row count, the log holds capacity + 1 entries): a step replayed past the end
+// writes nothing anywhere and the host sees pos == capacity. pos null: nothing to do.
+struct DecodeAdvance { int32_t *pos, *kv_len, *log; int32_t capacity; };
+__device__ __forceinline__ void decode_advance(const DecodeAdvance& a, int32_t token) {
+    if (!a.pos) return;
+    const int32_t p = a.pos[0] + 1;
+    if (p > a.capacity) return;
+    a.pos[0] = p;
+    a.kv_len[0] = min(a.kv_len[0] + 1, a.capacity);
+    a.log[p] = token;
+}
+
 // One workgroup per row; (value, index) pairs reduced with "larger value, then lower index" so ties keep the first.
-__global__ __launch_bounds__(ROW_THREADS) void argmax_rows_kernel(const float* __restrict__ in, int cols, int32_t* __restrict__ out) {
+__global__ __launch_bounds__(ROW_THREADS) void argmax_rows_kernel(const float* __restrict__ in, int cols, int32_t* out, DecodeAdvance advance) {
     __shared__ float rv[ROW_THREADS / 64];
     __shared__ int ri[ROW_THREADS / 64];
     const float* x = in + (int64_t)blockIdx.x * cols;
@@ -285,7 +298,9 @@ __global__ __launch_bounds__(ROW_THREADS) void argmax_rows_kernel(const float* _
         for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
             if (ri[w] != 0x7FFFFFFF && (bi == 0x7FFFFFFF || rv[w] > bv || (rv[w] == bv && ri[w] < bi))) { bv = rv[w]; bi = ri[w]; }
         }
-        out[blockIdx.x] = bi == 0x7FFFFFFF ? 0 : bi;
+        const int token = bi == 0x7FFFFFFF ? 0 : bi;
+        out[blockIdx.x] = token;
+        decode_advance(advance, token);
     }
 }
 
@@ -300,8 +315,8 @@ __device__ __forceinline__ void argmax_merge(float& bv, int& bi, float ov, int o
     if (oi != 0x7FFFFFFF && (bi == 0x7FFFFFFF || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
 }
 
-__global__ __launch_bounds__(ROW_THREADS) void argmax_split_kernel(const float* __restrict__ in, int cols, int32_t* __restrict__ out,
-                                                                   ArgmaxScratch* __restrict__ sc) {
+__global__ __launch_bounds__(ROW_THREADS) void argmax_split_kernel(const float* __restrict__ in, int cols, int32_t* out,
+                                                                   ArgmaxScratch* __restrict__ sc, DecodeAdvance advance) {
     __shared__ float rv[ROW_THREADS / 64];
     __shared__ int ri[ROW_THREADS / 64];
     __shared__ unsigned ticket;
@@ -331,7 +346,9 @@ __global__ __launch_bounds__(ROW_THREADS) void argmax_split_kernel(const float* 
 #pragma unroll
         for (int m = 32; m >= 1; m >>= 1) argmax_merge(bv, bi, __shfl_xor(bv, m, 64), __shfl_xor(bi, m, 64));
         if (threadIdx.x == 0) {
-            out[row] = bi == 0x7FFFFFFF ? 0 : bi;
+            const int token = bi == 0x7FFFFFFF ? 0 : bi;
+            out[row] = token;
+            decode_advance(advance, token);
             __hip_atomic_store(&sc->done[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -452,9 +469,7 @@ __global__ void i32_store_at_kernel(int32_t* dst, const int32_t* __restrict__ in
 __global__ void rope_table_kernel(const int32_t* __restrict__ pos, float theta, int head_dim, float2* __restrict__ table) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= head_dim / 2) return;
-    float sn, cs;
-    sincosf((float)pos[0] * powf(theta, -2.0f * (float)i / (float)head_dim), &sn, &cs);
-    table[i] = make_float2(cs, sn);
+    table[i] = rope_cos_sin(pos[0], theta, i, head_dim);
 }
 int launch_rope_table(const int32_t* pos, float theta, int head_dim, float* table) {
     if (head_dim <= 0 || (head_dim & 1)) return set_error("rope_table: head_dim must be positive and even; got %d", head_dim);
@@ -463,21 +478,13 @@ int launch_rope_table(const int32_t* pos, float theta, int head_dim, float* tabl
     return 0;
 }
 
-// End of a greedy decode step in one launch: the position and the key count advance by one and the token just
-// sampled is appended to the log at the new position. The position saturates at `capacity` (the cache's row count, the
-// log holds capacity + 1 entries): a step replayed past the end writes nothing anywhere and the host sees pos == capacity.
-__global__ void decode_advance_kernel(int32_t* pos, int32_t* kv_len, const int32_t* __restrict__ token, int32_t* log, int32_t capacity) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const int32_t p = pos[0] + 1;
-        if (p > capacity) return;
-        pos[0] = p;
-        kv_len[0] = min(kv_len[0] + 1, capacity);
-        log[p] = token[0];
-    }
+// End of a decode step whose token was sampled elsewhere.
+__global__ void decode_advance_kernel(DecodeAdvance advance, const int32_t* token) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) decode_advance(advance, token[0]);
 }
 int launch_decode_advance(int32_t* pos, int32_t* kv_len, const int32_t* token, int32_t* log, int32_t capacity) {
     if (capacity <= 0) return set_error("decode_advance: capacity must be positive; got %d", capacity);
-    decode_advance_kernel<<<dim3(1), dim3(64), 0, current_stream()>>>(pos, kv_len, token, log, capacity);
+    decode_advance_kernel<<<dim3(1), dim3(64), 0, current_stream()>>>(DecodeAdvance{pos, kv_len, log, capacity}, token);
     SKH_CHECK(hipGetLastError());
     return 0;
 }
@@ -615,18 +622,26 @@ int launch_add(const float* a, const float* b, float* out, int64_t n) {
     SKH_CHECK(hipGetLastError());
     return 0;
 }
-int launch_argmax_rows(const float* in, int rows, int cols, int32_t* out) {
-    if (rows <= 0 || cols <= 0) return 0;
+static int launch_argmax(const float* in, int rows, int cols, int32_t* out, const DecodeAdvance& advance) {
     if (rows <= ARGMAX_MAX_ROWS && cols >= 16384) {
         ArgmaxScratch* sc = static_cast<ArgmaxScratch*>(sync_scratch(sizeof(ArgmaxScratch)));
         if (!sc) return -1;
-        argmax_split_kernel<<<dim3(ARGMAX_SPLIT, rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out, sc);
+        argmax_split_kernel<<<dim3(ARGMAX_SPLIT, rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out, sc, advance);
         SKH_CHECK(hipGetLastError());
         return 0;
     }
-    argmax_rows_kernel<<<dim3(rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out);
+    argmax_rows_kernel<<<dim3(rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out, advance);
     SKH_CHECK(hipGetLastError());
     return 0;
+}
+int launch_argmax_rows(const float* in, int rows, int cols, int32_t* out) {
+    return rows <= 0 || cols <= 0 ? 0 : launch_argmax(in, rows, cols, out, DecodeAdvance{});
+}
+// The greedy token of one row of logits and what follows from it, one launch (decode_begin_q4k_kernel has what it saves).
+int launch_decode_end(const float* logits, int cols, int32_t* token, int32_t* pos, int32_t* kv_len, int32_t* log, int32_t capacity) {
+    if (cols <= 0) return set_error("decode_end: no logits");
+    if (capacity <= 0) return set_error("decode_end: capacity must be positive; got %d", capacity);
+    return launch_argmax(logits, 1, cols, token, DecodeAdvance{pos, kv_len, log, capacity});
 }
 // ---- arg-max for callers that cannot allocate ----
 // The same many-workgroups-per-row kernel, with its pairs and counters in a fixed array that is part of the loaded code
@@ -685,7 +700,7 @@ int launch_argmax_rows_noalloc(const float* in, int rows, int cols, int32_t* out
     // node, so the pair can be recorded into a graph)
     argmax_clear_kernel<<<dim3(1), dim3(ARGMAX_MAX_ROWS), 0, current_stream()>>>(sc, rows);
     SKH_CHECK(hipGetLastError());
-    argmax_split_kernel<<<dim3(ARGMAX_SPLIT, rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out, sc);
+    argmax_split_kernel<<<dim3(ARGMAX_SPLIT, rows), dim3(ROW_THREADS), 0, current_stream()>>>(in, cols, out, sc, DecodeAdvance{});
     SKH_CHECK(hipGetLastError());
     return 0;
 }

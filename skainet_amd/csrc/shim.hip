@@ -45,6 +45,8 @@ int launch_i32_store_at(int32_t* dst, const int32_t* index, int32_t offset, cons
 int launch_rope_table(const int32_t* pos, float theta, int head_dim, float* table);
 int launch_narrow_matmul(const float* a, int64_t a_stride, const uint8_t* b, int64_t b_byte_stride, float* c, int64_t c_stride,
                          int m, int n, int k, int fp16);
+int launch_decode_begin(int enc, const uint8_t* w, int bpr, int rows, const int32_t* token, float* out, const int32_t* pos, float theta, int head_dim, float* table);
+int launch_decode_end(const float* logits, int cols, int32_t* token, int32_t* pos, int32_t* kv_len, int32_t* log, int32_t capacity);
 int launch_decode_advance(int32_t* pos, int32_t* kv_len, const int32_t* token, int32_t* log, int32_t capacity);
 int launch_heads_to_rows(const float* in, float* out, int heads, int tokens, int head_dim);
 int launch_sdpa_cache(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads, int seq_q,
@@ -987,6 +989,19 @@ int32_t skainet_hip_f32_rope_table_dev(const int32_t* pos_dev, float theta, int3
     if (ensure_device() != 0) return -1;
     if (!pos_dev || !table) return set_error("rope_table: null argument");
     return launch_rope_table(pos_dev, theta, head_dim, table);
+}
+int32_t skainet_hip_decode_begin_dev(const skainet_hip_weight* embedding, const int32_t* token, float* out, const int32_t* pos_dev, float theta,
+                                     int32_t head_dim, float* rope_table) {
+    if (ensure_device() != 0) return -1;
+    if (!embedding || !token || !out || !pos_dev || !rope_table) return set_error("decode_begin: null pointer");
+    return launch_decode_begin(embedding->encoding, embedding->data, embedding->cols / block_elems(embedding->encoding), embedding->rows, token, out,
+                               pos_dev, theta, head_dim, rope_table);
+}
+int32_t skainet_hip_decode_end_dev(const float* logits, int32_t cols, int32_t* token, int32_t* pos, int32_t* kv_len, int32_t* log,
+                                   int32_t capacity) {
+    if (ensure_device() != 0) return -1;
+    if (!logits || !token || !pos || !kv_len || !log) return set_error("decode_end: null pointer");
+    return launch_decode_end(logits, cols, token, pos, kv_len, log, capacity);
 }
 int32_t skainet_hip_decode_advance_dev(int32_t* pos, int32_t* kv_len, const int32_t* token, int32_t* log, int32_t capacity) {
     if (ensure_device() != 0) return -1;

@@ -379,7 +379,6 @@ class LlamaDecoder:
         c = self.cfg
         kernels.rms_norm_dev(self.h.at(4 * row * c.hidden), self.w.out_norm, self.norm, 1, c.hidden, c.rms_eps)
         self.w.head.matmul(self.norm, 1, self.logits)
-        kernels.argmax_rows_dev(self.logits, 1, c.vocab, self.token)
 
     # ------------------------------------------------------------------ public API
     def prefill(self, token_ids) -> int:
@@ -398,6 +397,7 @@ class LlamaDecoder:
         for li in range(c.layers):
             self._block(li, rows, 0, None, rows, None)
         self._head(rows - 1)
+        kernels.argmax_rows_dev(self.logits, 1, c.vocab, self.token)
         kernels.sync()
         self.pos.upload(np.array([rows], np.int32))
         self.kv_len.upload(np.array([rows + 1], np.int32))
@@ -424,12 +424,12 @@ class LlamaDecoder:
         c = self.cfg
         if bound is None:
             bound = self._key_bound(self._host_pos + 1)
-        self.w.tok_embd.dequantize_rows(self.token, 1, self.h)
-        kernels.rope_table_dev(self.pos, c.rope_theta, c.head_dim, self.rope_table)     # once per token, shared by all layers
+        # the embedding row, and the rotation table that all layers share
+        kernels.decode_begin_dev(self.w.tok_embd, self.token, self.h, self.pos, c.rope_theta, c.head_dim, self.rope_table)
         for li in range(c.layers):
             self._block(li, 1, 0, self.pos, bound, self.kv_len)
         self._head(0)
-        kernels.decode_advance_dev(self.pos, self.kv_len, self.token, self.generated, c.ctx_max)
+        kernels.decode_end_dev(self.logits, c.vocab, self.token, self.pos, self.kv_len, self.generated, c.ctx_max)
 
     def _graph_step(self) -> None:
         """One decode step through the recorded graph; records it first (one eager step, then the recording, which runs

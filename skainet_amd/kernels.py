@@ -386,6 +386,16 @@ def decode_advance_dev(pos, kv_len, token, log, capacity: int) -> None:
     check(_lib.hip().skainet_hip_decode_advance_dev(_ptr(pos), _ptr(kv_len), _ptr(token), _ptr(log), capacity), "decode_advance")
 
 
+def decode_begin_dev(embedding, token, out, pos, theta: float, head_dim: int, table) -> None:
+    """A decode step's start: `out` = the packed embedding's row *token, `table` = rope_table_dev's of *pos."""
+    check(_lib.hip().skainet_hip_decode_begin_dev(embedding._h, _ptr(token), _ptr(out), _ptr(pos), theta, head_dim, _ptr(table)), "decode_begin")
+
+
+def decode_end_dev(logits, cols: int, token, pos, kv_len, log, capacity: int) -> None:
+    """A greedy decode step's end: *token = arg-max of the logits, then decode_advance_dev."""
+    check(_lib.hip().skainet_hip_decode_end_dev(_ptr(logits), cols, _ptr(token), _ptr(pos), _ptr(kv_len), _ptr(log), capacity), "decode_end")
+
+
 def i32_store_at_dev(dst, index_dev, offset: int, src) -> None:
     check(_lib.hip().skainet_hip_i32_store_at_dev(_ptr(dst), _ptr(index_dev), offset, _ptr(src)), "i32_store_at")
 

@@ -111,6 +111,32 @@ def test_heads_to_rows_and_swiglu_and_increment(hip_backend, torch_cuda):
     assert int(ctr.cpu()[0]) == 45
 
 
+@pytest.mark.parametrize("enc,cols,vocab", [("Q4_K", 256, 1), ("Q4_K", 2304, 1000), ("Q4_K", 4096, 16384), ("Q6_K", 512, 40001)])
+def test_decode_begin_and_end_are_the_launches_they_stand_for(hip_backend, torch_cuda, enc, cols, vocab):
+    """Embedding row + rotation table, and arg-max + advance, bit for bit as the separate calls, up to the cache's last position and past it."""
+    torch, kx = torch_cuda, hip_backend
+    rng = np.random.default_rng(cols + vocab)
+    w = kx.DeviceWeight.upload(enc, kx.quantize(enc, (rng.standard_normal((7, cols)) * 0.05).astype(np.float32)), 7, cols)
+    ints = lambda *v: dev(torch, np.array(v, np.int32))
+    logits = dev(torch, rng.integers(-3, 4, vocab).astype(np.float32))      # ties: the first one
+    for head_dim, at in ((64, 0), (128, 6), (1026, 41)):
+        row, table = [torch.full((cols,), 5.0, device="cuda") for _ in range(2)], [torch.zeros(head_dim, device="cuda") for _ in range(2)]
+        tok = ints(at % 7)
+        w.dequantize_rows(tok, 1, row[0])
+        kx.rope_table_dev(ints(at), 1e4, head_dim, table[0])
+        kx.decode_begin_dev(w, tok, row[1], ints(at), 1e4, head_dim, table[1])
+        kx.sync()
+        assert torch.equal(*row) and torch.equal(*table)
+    state = [[ints(0), ints(6), ints(7), ints(*[0] * 10)] for _ in range(2)]      # token, position, key count, log
+    for step in range(5):                                                   # three steps fit
+        (t0, p0, k0, l0), (t1, p1, k1, l1) = state
+        kx.argmax_rows_dev(logits, 1, vocab, t0)
+        kx.decode_advance_dev(p0, k0, t0, l0, 9)
+        kx.decode_end_dev(logits, vocab, t1, p1, k1, l1, 9)
+        kx.sync()
+        assert all(torch.equal(a, b) for a, b in zip(*state)) and int(p1.cpu()[0]) == min(9, 7 + step)
+
+
 def test_rope_qkv_equals_three_scatters(hip_backend, torch_cuda):
     torch, kx = torch_cuda, hip_backend
     rng = np.random.default_rng(31)
