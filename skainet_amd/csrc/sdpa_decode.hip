@@ -60,7 +60,8 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
 // workgroup walks the union. A key outside a row's range takes no part in that row: it scores -inf and its V is replaced by
 // zeros, since a weight of zero times an infinite or undefined element (a later token's, or the padding of a cache) is not
 // zero. Passes whose keys lie in every row's range, nearly all of them, skip both.
-template <int GS, int DPL, bool MQ>
+// DIES: a grid of one dimension, below. A template argument, since a run-time choice costs every call 0.03 to 0.1 us in front of its first load.
+template <int GS, int DPL, bool MQ, bool DIES>
 __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     constexpr int D = 16 * DPL;
     constexpr int U = 2;                       // groups of 4 keys a wave has in flight
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     const int per_kv = p.heads / p.kv_heads;
     const int rows_kv = MQ ? per_kv * p.seq_q : per_kv;        // query rows that share a KV head
     int split = blockIdx.x, b = blockIdx.z, kvh = blockIdx.y, sub_group = 0;
-    if (p.tuples) {
+    if constexpr (DIES) {
         // workgroups go to the dies in turn: every eighth one takes the next group of rows of the same keys, so that one L2 has them
         const int turn = blockIdx.x >> 3, tuple = turn / p.subs * 8 + (blockIdx.x & 7);
         if (tuple >= p.tuples) return;
@@ -82,9 +83,10 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         split = tuple % p.splits;
         kvh = tuple / p.splits % p.kv_heads;
         b = tuple / p.splits / p.kv_heads;
-    } else if (p.subs > 1) {
-        kvh = blockIdx.y / p.subs;
-        sub_group = blockIdx.y % p.subs;
+    } else {
+        const int subs = MQ ? (rows_kv + GS - 1) / GS : per_kv / GS;
+        kvh = blockIdx.y / subs;
+        sub_group = blockIdx.y % subs;
     }
     const int r0 = sub_group * GS;
     // row g of the workgroup: its place among the [batch, heads, seq_q] query rows (rows past the last are copies of it)
@@ -352,8 +354,8 @@ template <int GS, int DPL, bool MQ>
 static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge) {
     constexpr int D = 16 * DPL;
     note_kernel("sdpa_decode_kernel");
-    const dim3 grid = p.tuples ? dim3((unsigned)((p.tuples + 7) / 8 * 8 * subs)) : dim3(p.splits, p.kv_heads * subs, p.batch);
-    sdpa_decode_kernel<GS, DPL, MQ><<<grid, dim3(256), 0, current_stream()>>>(p);
+    if (p.tuples) sdpa_decode_kernel<GS, DPL, MQ, true><<<dim3((unsigned)((p.tuples + 7) / 8 * 8 * subs)), dim3(256), 0, current_stream()>>>(p);
+    else sdpa_decode_kernel<GS, DPL, MQ, false><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
     SKH_CHECK(hipGetLastError());
     if (merge) {
         sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits, p.heads, p.seq_q, p.out_rows);
@@ -503,11 +505,12 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     p.splits = splits;
     // Workgroups that share keys on one die each, where the dies' own copies of them would not stay in the L2s (32 MB together): 8 queries,
     // 8 heads over 2, three sequences at 3815 keys 37.7 -> 24.1 us, one query, 8 heads over 1, six at 6012 18.8 -> 14.0, 16 over 2, six at 4556,
-    // D 64, 18.5 -> 14.6. With less traffic the index arithmetic costs 0.1 to 0.2 us, and few groups leave the dies uneven shares (3 queries, 4 heads over
+    // D 64, 18.5 -> 14.6. Of 2616 random calls those with 24 to 32 MB together take 1.00 of their
+    // time, 32 to 40 0.96, 64 to 90 0.89, above 140 0.81. Few groups leave the dies uneven shares (3 queries, 4 heads over
     // 1, three at 1720 8.3 -> 9.3).
     const int64_t tuples = (int64_t)batch * kv_heads * splits;
     const double mb = 8e-6 * batch * kv_heads * keys * head_dim;
-    if (g_sdpa_decode_dies && mb * min(subs, 8) > 24 && subs > 1 && (tuples >= 24 || (tuples + 7) / 8 * subs <= num_cus() / 8) && (tuples + 7) / 8 * 8 * subs <= 0x7FFFFFFF)
+    if (g_sdpa_decode_dies && mb * min(subs, 8) > 34 && subs > 1 && (tuples >= 24 || (tuples + 7) / 8 * subs <= num_cus() / 8) && (tuples + 7) / 8 * 8 * subs <= 0x7FFFFFFF)
         p.tuples = (int)tuples;
     if (splits > 1 || leave) {
         const size_t rows = (size_t)batch * heads * seq_q;

@@ -895,7 +895,7 @@ def test_layer_norm_and_softmax_row_shapes(hip_backend, torch_cuda, rows, cols):
             close(got[:rows], e / e.sum(1, keepdims=True), rel=1e-5, abs_=1e-7)
 
 
-@pytest.mark.parametrize("batch,heads,kv_heads,sq,skv,dim,window", [(3, 8, 2, 8, 3815, 128, 0), (5, 8, 1, 1, 2600, 128, 0), (6, 16, 2, 1, 4556, 64, 0), (7, 12, 3, 1, 1500, 256, 0),
+@pytest.mark.parametrize("batch,heads,kv_heads,sq,skv,dim,window", [(3, 8, 2, 8, 3815, 128, 0), (7, 8, 1, 1, 2600, 128, 0), (6, 16, 2, 1, 4556, 64, 0), (7, 12, 3, 1, 1500, 256, 0),
                                                                     (4, 10, 2, 3, 3591, 128, 0), (12, 64, 8, 1, 4775, 128, 360)])
 def test_attention_groups_of_one_die_give_the_same_bits(hip_backend, torch_cuda, batch, heads, kv_heads, sq, skv, dim, window):
     """Where the workgroups that share keys are placed on one die each (enough traffic, several groups of rows per KV head): the
