@@ -9,7 +9,7 @@
 // The decode is the reference's block arithmetic (code * (d * sc) - dmin * m, (d * sc) * q, code * d) in fp32,
 // rounded to bf16 (nearest even) when it is parked in LDS.
 //
-// Tiling (MFMA-bound): workgroup tile 256 (M) x 128 (N), K step 64, 256 threads = 4 waves in a 2 x 2 grid, each wave
+// Tiling (MFMA-bound), for the workgroup tile of 256 (M) x 128 (N) (others below): K step 64, 256 threads = 4 waves in a 2 x 2 grid, each wave
 // owning a 128 x 64 patch = 4 x 2 MFMA tiles of 32 x 32 (128 accumulator registers per lane). Per K step a thread
 // decodes 32 consecutive weights of one row (one Q4_K sub-block / one Q6_K quarter / one Q8_0 block) and copies
 // 8 x 16 bytes of the bf16 activation tile; LDS rows are padded to 144 bytes so the 16-byte fragment reads of 32
@@ -27,12 +27,10 @@ namespace skh {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// The tile comes in two widths, WTN = 2 or 4 32-column MFMA tiles per wave along N (rows: always 4): 256 x 128 and
-// 256 x 256. Per K step a CU's LDS moves 144 KB for the narrow tile (1152 cycles at 128 B/clk against the 1024 cycles of
+// The tile comes in several sizes. Per K step a CU's LDS moves 144 KB for 256 x 128 (1152 cycles at 128 B/clk against the 1024 cycles of
 // its MFMAs; measured in isolation, 32 MFMAs take 505 ns, with the 24 fragment reads 688 ns, with the 12 tile stores
-// 820 ns: a wave that issues an LDS instruction is held while the LDS moves its 1 KB) and 192 KB for the wide tile with
-// twice the MFMAs, so the wide tile is the one that can keep the matrix cores busy; it needs 32 tiles per CU round
-// fewer to fill the chip, so it serves the wide weights (N >= 128 rows per CU) and the narrow one the rest.
+// 820 ns: a wave that issues an LDS instruction is held while the LDS moves its 1 KB) and 192 KB for 256 x 256 with
+// twice the MFMAs, so the larger the tile the busier the matrix cores, and the fewer tiles there are for the CUs.
 constexpr int G_WAVES_M = 2, G_WAVES_N = 2;
 constexpr int GK = 64;
 constexpr int G_THREADS = G_WAVES_M * G_WAVES_N * 64;

@@ -286,6 +286,12 @@ def test_attention_short_prompts_stream_the_cache(hip_backend, torch_cuda, batch
                                     None if ln is None else dev(torch, ln))
     assert hip_backend.last_kernel() == "sdpa_decode_kernel"
     assert np.array_equal(rows.cpu().numpy(), got.transpose(0, 2, 1, 3))
+    spare = [np.full((batch, kv_heads, skv + 5, d), np.nan, np.float32) for _ in range(2)]      # rows of a cache past its keys
+    spare[0][:, :, :skv], spare[1][:, :, :skv] = k, v
+    out = torch.full((batch, heads, sq, d), float("nan"), device="cuda")
+    hip_backend.sdpa_cache_dev(dev(torch, q), dev(torch, spare[0]), dev(torch, spare[1]), out, batch, heads, kv_heads, sq, skv, skv + 5, d, scale,
+                               causal, window, rc, None if ln is None else dev(torch, ln))
+    assert np.array_equal(out.cpu().numpy(), got)
     if causal and window == 0 and ln is None:
         v[:, :, -1] = np.nan                                        # the last key: only the last query's
         late = gpu_sdpa(hip_backend, torch, q, k, v, scale, causal)
