@@ -582,9 +582,11 @@ SknTile gemm_skinny_direct_tile(int enc, int m, int n, int k) {
     if (k % 2048 == 0) best.us *= 1.08;      // rows of 2^n KB meet in the same channels of the L2
     return best;
 }
+// From 8 us on the estimate is a tenth low for what only single waves share, for Q6_K and for one row tile of Q8_0: of 4 913 random products that took
+// these forms such ones took 1.05 of what two launches take (Q6_K 55 x 9274 x 768 11.3 -> 12.0 us, Q8_0 46 x 8548 x 768 8.2 -> 9.9), the others 0.87.
 double gemm_skinny_direct_estimate(int enc, int m, int n, int k) {
     const SknTile t = gemm_skinny_direct_tile(enc, m, n, k);
-    return t.mt ? t.us : 1e30;
+    return !t.mt || (t.us >= 8 && (t.wn == 1 || enc == ENC_Q6_K || (enc == ENC_Q8_0 && t.mt == 1))) ? 1e30 : t.us;
 }
 
 // 0 never, 1 where the estimates favour it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits; 100 wn + 10 mt + nt: that
