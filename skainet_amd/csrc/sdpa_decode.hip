@@ -389,7 +389,7 @@ void set_attn_merge_splits(int v) { if (v >= 1 && v <= ATTN_MERGE_MAX_SPLITS) g_
 // straight from the caller's memory, in one launch up to 256 keys and more, with fp32 operands (the other rounds them to bf16). What ends it is the
 // K and V that every four rows read for themselves. Both sides in us, back to back from the host, fitted to 7050 random prompts (16 to 400 queries,
 // up to 2048 earlier keys, 1 to 64 heads, D 64 and 128; 11 % and 5 % rms); this one has to be a sixth below. Of 8549 others 0.67 take it, 1.60x, 14
-// more than 3 % slower: 27 queries, one head, D 64 8.1 -> 4.9 us, 129 queries, 16 heads over 2, D 128 11.8 -> 6.9.
+// more than 3 % slower: 28 queries, one head, D 64 8.9 -> 5.6 us, 60 queries, 16 heads over 2, D 128 12.0 -> 5.7, 96 11.5 -> 8.4.
 bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context) {
     if ((head_dim != 64 && head_dim != 128) || seq_q > seq_kv) return false;
     const double groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
@@ -505,7 +505,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     p.splits = splits;
     // Workgroups that share keys on one die each, where the dies' own copies of them would not stay in the L2s (32 MB together): 8 queries,
     // 8 heads over 2, three sequences at 3815 keys 37.7 -> 24.1 us, one query, 8 heads over 1, six at 6012 18.8 -> 14.0, 16 over 2, six at 4556,
-    // D 64, 18.5 -> 14.6. Of 2616 random calls those with 24 to 32 MB together take 1.00 of their
+    // D 64, 18.5 -> 14.6. Of 4733 random calls those with 24 to 32 MB together take 1.00 of their
     // time, 32 to 40 0.96, 64 to 90 0.89, above 140 0.81. Few groups leave the dies uneven shares (3 queries, 4 heads over
     // 1, three at 1720 8.3 -> 9.3).
     const int64_t tuples = (int64_t)batch * kv_heads * splits;
