@@ -857,14 +857,14 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     // encoding's blocks stay intact. An estimate is off by 5 to 10 % now and then, and what was the better choice by less than
     // that is kept: the tile that fits most shapes -- 256 rows (128 where there are no more), the wide one where it fills three
     // quarters of the chip in a round -- gives way only to one 5 % below it, a split more has to save 1 %, the few-rows kernel
-    // 5 %; the fragment-order kernel stays up to 2 % above. On 9300 other random products, against one tile shape
+    // 5 %; the fragment-order kernel stays up to 2 % above the others, 5 % above a tile with a 192. On 9300 other random products, against one tile shape
     // by the row count: geometric mean 1.44x, 36 of them more than 3 % slower, 4 more than 10 %, the worst 15 %.
     const int kgroups = (k + 255) / 256;
     const int usual_tm = m <= 128 ? 2 : 4;
     const bool usual_wide = 4 * (int64_t)((m + gemm_gm(usual_tm) - 1) / gemm_gm(usual_tm)) * ((n + gemm_gn(4) - 1) / gemm_gn(4)) >= 3 * num_cus();
-    double least = 0.0;
+    double least = 0.0, least_even = 0.0;
     int wtm = 2, wtn = 2, ksplit = 1;
-    double tile_estimate = 0.0;
+    double tile_estimate = 0.0, even_estimate = 0.0;             // of all tiles, and of those without a 192
     const int forced_tm = g_gemm_rows.load(), wide = g_gemm_wide.load();
     for (int tm = 2; tm <= 4; ++tm) {
         if (forced_tm != 0 && tm != forced_tm) continue;
@@ -877,6 +877,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
                 const double t = gemm_tile_us(enc, tm, tn, m, n, k, ks);
                 const double rank = t * (1 + 0.01 * (ks - 1)) * (tm == usual_tm && (tn == 4) == usual_wide ? 0.95 : 1.0);
                 if (least == 0.0 || rank < least) { least = rank; tile_estimate = t; wtm = tm; wtn = tn; ksplit = ks; }
+                if (tm != 3 && tn != 3 && (least_even == 0.0 || rank < least_even)) { least_even = rank; even_estimate = t; }
             }
         }
     }
@@ -899,7 +900,10 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
             return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);
         if (two < 0.95 * others) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     }
-    if (frag_by_rule && frag_estimate < 1.02 * tile_estimate) return run_frag();
+    // The fragment-order kernel gives way to a tile with a 192 only where that is 5 % below it, as far as both estimates are good: its waves share K
+    // where a tile is one chain over it, so the choice shows in the sums. (By 2 % the gate / up product of a Llama-3-8B prompt of 300 rows changed
+    // kernels for 0.3 % of the prompt, and the logits behind 32 layers by 1 %.)
+    if (frag_by_rule && frag_estimate < 1.02 * even_estimate && frag_estimate < 1.05 * tile_estimate) return run_frag();
     if (ksw_ok && gemm_ksw_enabled() && !gemm_frag_enabled() && g_gemm_ksplit.load() <= 0) {
         // with the fragment-order kernel switched off, its predecessor where it would beat the tile kernel (0.31 us per 64
         // elements of K, 6.5 us per round outside the loop)

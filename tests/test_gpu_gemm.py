@@ -119,6 +119,20 @@ def test_gemm_tiles_of_192_rows_or_columns_give_the_bits_of_the_others(hip_backe
         hip_backend.set_tuning("gemm_rows", 0)
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [(300, 28672, 4096, "q4k_gemm_frag_kernel"), (300, 6144, 4096, "q4k_gemm_frag_kernel"),
+                                          (528, 21086, 6656, "3, 4, false>"), (260, 5954, 13824, "3, 4, false>")])
+def test_q4k_tiles_with_a_192_take_over_where_they_are_well_below(hip_backend, torch_cuda, m, n, k, kernel):
+    """The fragment-order kernel keeps products on which the new tiles' estimate is less than 5 % below its own (the first is 2 % off, the
+    second not below it): the choice changes the order of the sums. 23 and 15 % off, the tiles have them."""
+    torch = torch_cuda
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    packed = torch.randint(0, 120, (n * (k // 256) * 144,), generator=gen, dtype=torch.uint8, device="cuda")
+    w = hip_backend.DeviceWeight.wrap("Q4_K", packed, n, k)
+    x, got = torch.randn((m, k), generator=gen, device="cuda"), torch.empty((m, n), device="cuda")
+    ran = launches(torch, lambda: w.matmul(x, m, got, 1))
+    assert sum(kernel in name for name, _, _ in ran) == 1, ran
+
+
 @pytest.mark.parametrize("m,n,k,ks", [(128, 128, 256, 1), (129, 131, 512, 1), (33, 257, 1024, 3), (300, 127, 2304, 2), (16, 16, 256, 1)])
 @pytest.mark.parametrize("enc", ALL_ENCS)
 def test_gemm_tile_on_fp32_rows_gives_the_bits_of_the_rounded_rows(hip_backend, torch_cuda, enc, m, n, k, ks):
