@@ -42,6 +42,7 @@ struct SdpaDecodeParams {
     int subs, tuples;     // workgroups that share a split's keys, and how many such (split, kv head, sequence) there are; tuples 0: a grid of three dimensions
     int seq_q, causal;    // queries per sequence (the last ones of its positions) and whether a later key is hidden from them
     int out_rows;         // the output as [batch, seq_q, heads, D] instead of [batch, heads, seq_q, D]
+    int by_query;         // rows that share a KV head: query by query instead of head by head
 };
 
 // Scores are kept in units of ln 2 (the query is scaled by scale * log2(e) once), so every exponential of the softmax is
@@ -60,6 +61,9 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
 // workgroup walks the union. A key outside a row's range takes no part in that row: it scores -inf and its V is replaced by
 // zeros, since a weight of zero times an infinite or undefined element (a later token's, or the padding of a cache) is not
 // zero. Passes whose keys lie in every row's range, nearly all of them, skip both.
+// A draft's rows come head by head. A prompt's come query by query, so that a workgroup holds neighbouring queries, at most GS of them: head by head
+// some hold the last queries of one head and the first of the next, which share no key under a window (385 queries on 1828 keys under a
+// window of 153, 8 heads over 1: 537 keys walked by six of 770 workgroups, about 156 by the others).
 // DIES: a grid of one dimension, below. A template argument, since a run-time choice costs every call 0.03 to 0.1 us in front of its first load.
 template <int GS, int DPL, bool MQ, bool DIES>
 __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
@@ -89,6 +93,9 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         sub_group = blockIdx.y % subs;
     }
     const int r0 = sub_group * GS;
+    const int row_div = p.by_query ? per_kv : p.seq_q;
+    auto head_of = [&](int r) { return !MQ ? r : p.by_query ? r % row_div : r / row_div; };
+    auto query_of = [&](int r) { return !MQ ? 0 : p.by_query ? r / row_div : r % row_div; };
     // row g of the workgroup: its place among the [batch, heads, seq_q] query rows (rows past the last are copies of it)
     int64_t row_of[GS];
     int first_of[GS], end_of[GS];
@@ -98,7 +105,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
 #pragma unroll
     for (int g = 0; g < GS; ++g) {
         const int r = MQ ? min(r0 + g, rows_kv - 1) : r0 + g;
-        const int qi = MQ ? r % p.seq_q : 0, h = MQ ? r / p.seq_q : r;
+        const int qi = query_of(r), h = head_of(r);
         row_of[g] = MQ ? ((int64_t)b * p.heads + kvh * per_kv + h) * p.seq_q + qi : (int64_t)b * p.heads + kvh * per_kv + h;
         // attended key range of this row's query (one query: absolute position seq_kv - 1, so causal cuts nothing)
         const int pos = MQ ? p.seq_kv - p.seq_q + qi : p.seq_kv - 1;
@@ -284,7 +291,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
 #pragma unroll
         for (int e = 1; e < GS; ++e) row = g == e ? row_of[e] : row;
         int64_t out_row = row;
-        if (MQ && p.out_rows) out_row = ((int64_t)b * p.seq_q + (r0 + g) % p.seq_q) * p.heads + kvh * per_kv + (r0 + g) / p.seq_q;
+        if (MQ && p.out_rows) out_row = ((int64_t)b * p.seq_q + query_of(r0 + g)) * p.heads + kvh * per_kv + head_of(r0 + g);
 #pragma unroll
         for (int e = 0; e < EPT; ++e) {
             const int d = i0 + e;                                   // a state's layout in LDS is the row's own element order
@@ -422,7 +429,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     // only not wider than the rows there are
     while (draft ? gs > 2 && per_kv * seq_q <= gs / 2 : per_kv % gs != 0) gs >>= 1;
     // keys that a query can attend: a window bounds them whatever the cache holds
-    // (a prompt: those of a workgroup's four queries; with all queries' 385 x 1828 under a window of 153 was split and took 21 us)
+    // (a prompt: those of a workgroup's rows, at most four neighbouring queries; with all queries' 385 x 1828 under a window of 153 was split and took 21 us)
     const int keys = window > 0 ? (int)min((int64_t)seq_kv, (int64_t)window + right_context + (seq_q < 16 ? seq_q - 1 : 3)) : seq_kv;
     // One split, no merge behind it: the merge is a second launch (2.8 us of a host's time, and about that between two
     // dependent kernels on the device), which buys the parallelism of the splits -- and shorter sums: with one split the error
@@ -483,7 +490,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     const int subs = (cols + gs - 1) / gs;
     if (batch > 65535 || (int64_t)kv_heads * subs > 65535) return 0;
     SdpaDecodeParams p{q, k, v, out, batch, heads, kv_heads, seq_kv, kv_capacity, scale, window, right_context, lengths, 1,
-                       nullptr, nullptr, subs, 0, seq_q, causal, out_rows && seq_q > 1};
+                       nullptr, nullptr, subs, 0, seq_q, causal, out_rows && seq_q > 1, seq_q >= 16};
     // enough workgroups to put every CU on the cache, at least 64 keys per split (measured in the decoder at 500 to 650
     // keys: 32 or 48 keys per split 2.5 % slower per token, 96 and 128 keys the same as 64)
     const int64_t groups = (int64_t)batch * kv_heads * subs;

@@ -298,6 +298,20 @@ def test_attention_short_prompts_stream_the_cache(hip_backend, torch_cuda, batch
         assert np.array_equal(late[:, :, :-1], got[:, :, :-1]) and np.isnan(late[:, :, -1]).all()
 
 
+@pytest.mark.parametrize("heads,kv_heads,d,sq", [(4, 1, 64, 385), (8, 2, 128, 101), (8, 1, 128, 51)])
+def test_attention_short_prompt_rows_share_a_workgroup_with_their_own_query_only(hip_backend, torch_cuda, heads, kv_heads, d, sq):
+    """Four heads or more to a KV head: all rows of a workgroup belong to one query, so what it walks, and the order of a row's sums, do not depend on
+    how many queries the call has: the last 18 alone give the same bits. Head by head, with a count of queries that four does not divide, they
+    would share workgroups with other queries, and with the next head's first ones, which have no key in common with them under the window."""
+    q, k, v = sdpa_inputs(1, heads, kv_heads, sq, sq + 15, d, seed=sq)
+    got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, 0.1, True, 60)
+    assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+    last = gpu_sdpa(hip_backend, torch_cuda, q[:, :, -18:].copy(), k, v, 0.1, True, 60)
+    assert hip_backend.last_kernel() == "sdpa_decode_kernel"
+    assert np.array_equal(got[:, :, -18:], last)
+    close(got, L.sdpa(q, k, v, 0.1, True, 60))
+
+
 @pytest.mark.parametrize("heads,kv_heads,d,sq,skv", [(32, 8, 128, 512, 512), (8, 1, 64, 300, 2000)])
 def test_attention_long_prompts_stay_on_the_matrix_cores(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv):
     q, k, v = (np.zeros(s, np.float32) for s in ((1, heads, sq, d), (1, kv_heads, skv, d), (1, kv_heads, skv, d)))
