@@ -459,7 +459,8 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * "sdpa_prefill_mfma" (0: prompt-shape attention on the fp32 kernel), "sdpa_prefill_teams" (query groups per workgroup of
  * the matrix-core prompt kernel: 1, 2 = two, one after the other, 0 = as many as leave one workgroup per CU),
  * "sdpa_prefill_splits" (workgroups that share the keys of a query group that has workgroups of its own: 1 to 32, 0 = chosen from the shape), "sdpa_decode_split_keys" (least keys per split of
- * decode-shape attention, default 64), "sdpa_decode_one_launch" (0: short contexts are split over workgroups and merged by a
+ * decode-shape attention, default 64), "sdpa_decode_prompts" (prompts of 16 queries and more without a mask on the kernel for decode shapes:
+ * 0 never, 1 where the launcher's estimates of both favour it and no "sdpa_prefill_*" key is set, 2 wherever it fits unless one is), "sdpa_decode_one_launch" (0: short contexts are split over workgroups and merged by a
  * second launch too), "sdpa_decode_gs" (query heads per workgroup of decode-shape attention: 1, 2 or 4, 0 = chosen from
  * the shape), "attn_merge_enable" (0: skainet_hip_attn_out_proj_dev always merges the key
  * splits in a launch of its own), "attn_merge_max_keys" (most keys per split for which that entry leaves the merge to

@@ -215,6 +215,7 @@ void set_q4k_wide_min_batch(int v);
 void set_attn_merge_enable(int v);
 void set_sdpa_decode_gs(int v);
 void set_sdpa_decode_one_launch(int v);
+void set_sdpa_decode_prompts(int v);
 void set_sdpa_decode_dies(int v);
 void set_attn_merge_max_keys(int v);
 void set_attn_merge_splits(int v);
@@ -267,6 +268,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "sdpa_decode_split_keys")) { set_sdpa_decode_split_keys(value); return 0; }
     if (!strcmp(key, "attn_merge_enable")) { set_attn_merge_enable(value); return 0; }
     if (!strcmp(key, "sdpa_decode_one_launch")) { set_sdpa_decode_one_launch(value); return 0; }
+    if (!strcmp(key, "sdpa_decode_prompts")) { set_sdpa_decode_prompts(value); return 0; }
     if (!strcmp(key, "sdpa_decode_dies")) { set_sdpa_decode_dies(value); return 0; }
     if (!strcmp(key, "sdpa_decode_gs")) { set_sdpa_decode_gs(value); return 0; }
     if (!strcmp(key, "attn_merge_max_keys")) { set_attn_merge_max_keys(value); return 0; }

@@ -381,6 +381,8 @@ static std::atomic<int> g_sdpa_decode_gs{0};            // query heads per workg
 void set_sdpa_decode_gs(int v) { if (v == 0 || v == 1 || v == 2 || v == 4) g_sdpa_decode_gs = v; }
 static std::atomic<int> g_sdpa_decode_dies{1};
 void set_sdpa_decode_dies(int v) { g_sdpa_decode_dies = v != 0; }
+static std::atomic<int> g_sdpa_decode_prompts{1};       // prompts on this kernel: 0 never, 1 by rule, 2 wherever it fits
+void set_sdpa_decode_prompts(int v) { if (v >= 0 && v <= 2) g_sdpa_decode_prompts = v; }
 static std::atomic<int> g_sdpa_decode_one_launch{1};
 void set_sdpa_decode_one_launch(int v) { g_sdpa_decode_one_launch = v != 0; }
 static std::atomic<int> g_attn_merge_max_keys{176};    // most keys per split the unmerged form accepts (a multiple of 16)
@@ -391,24 +393,33 @@ void set_attn_merge_max_keys(int v) { if (v >= 16) g_attn_merge_max_keys = (v + 
 static std::atomic<int> g_attn_merge_splits{6};
 void set_attn_merge_splits(int v) { if (v >= 1 && v <= ATTN_MERGE_MAX_SPLITS) g_attn_merge_splits = v; }
 
+double sdpa_prefill_estimate(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context);   // sdpa_prefill.hip
+
 // Whether a prompt (16 queries and more, no mask) goes to this kernel instead of the matrix-core one, which lays K and V out in a launch of
 // its own and sets up a workgroup of eight waves for 32 queries: 8 to 11 us whatever little there is to do. Here a workgroup takes four rows
 // straight from the caller's memory, in one launch up to 256 keys and more, with fp32 operands (the other rounds them to bf16). What ends it is the
-// K and V that every four rows read for themselves. Both sides in us, back to back from the host, fitted to 7050 random prompts (16 to 400 queries,
-// up to 2048 earlier keys, 1 to 64 heads, D 64 and 128; 11 % and 5 % rms); this one has to be a sixth below. Of 8549 others 0.67 take it, 1.60x, 14
-// more than 3 % slower: 28 queries, one head, D 64 8.9 -> 5.6 us, 60 queries, 16 heads over 2, D 128 12.0 -> 5.7, 96 11.5 -> 8.4.
+// K and V that every four rows read for themselves. Both sides by what they do, in us back to back from the host: here the longest workgroup's
+// keys and all keys walked over the CUs (whichever is the longer, the fourth root of fourth powers between them), rounds of workgroups, and K and V once;
+// fitted to the 42 000 random prompts of the other estimate (12 % rms); this one has to be a sixth below. Of 23 384 other prompts of those ranges
+// 11 216 take it, 1.585x, 29 of them more than 5 % slower: 28 queries, one head, D 64 8.9 -> 5.6 us, 60 queries, 16 heads over 2, D 128 12.0 -> 5.7.
+// (Straight lines through the keys, fitted up to 2048 earlier ones, took 5 % more, 973 of 21 378 slower, by up to 3.3 times: beyond the fit they
+// did not know that the other kernel splits its keys, nor under a window what its workgroups walk.)
 bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context) {
+    if (g_sdpa_decode_prompts.load() != 1) return g_sdpa_decode_prompts.load() == 2;
     if ((head_dim != 64 && head_dim != 128) || seq_q > seq_kv) return false;
-    const double groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
-    double keys = causal ? seq_kv - 0.5 * (seq_q - 1) : seq_kv, most = seq_kv;          // of a query, on average; of all queries together
+    const double cus = num_cus(), groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
+    double keys = causal ? seq_kv - 0.5 * (seq_q - 1) : seq_kv, most = seq_kv, all = seq_kv;       // of a query on average, of a workgroup, of the call
     if (window > 0) {
         keys = fmin(keys, (double)window + right_context);
-        most = fmin(most, (double)window + right_context + seq_q - 1);
+        most = fmin(most, (double)window + right_context + 3);
+        all = fmin(all, (double)window + right_context + seq_q);
     }
-    const double rounds = ceil(groups / num_cus()), walked = 1e-3 * groups * keys, kb = 1e-3 * batch * kv_heads * most;
-    const double here = head_dim == 64 ? fmax(5.6, 5.18 + 0.067 * walked + 0.36 * rounds) : fmax(5.6, 5.41 + 0.105 * walked + 0.74 * rounds);
-    const double there = head_dim == 64 ? 9.0 + 5.2e-3 * most + 0.228 * kb + 0.9e-3 * seq_q : 10.7 + 6.0e-3 * most + 0.453 * kb + 3.9e-3 * seq_q;
-    return 1.2 * here < there;
+    const double splits = fmax(1.0, fmin(ceil(2 * cus / groups), fmin(SDPA_DECODE_MAX_SPLITS, ceil(most / 64)))), rounds = ceil(groups * splits / cus);
+    const double chain = most / 64 / splits, walked = groups * keys / 64 / cus, mb = 8e-6 * batch * kv_heads * all * head_dim;
+    auto longer = [](double a, double b) { return sqrt(sqrt(a * a * a * a + b * b * b * b)); };
+    const double here = head_dim == 64 ? fmax(6.58, 3.08 + longer(1.68 * chain, 0.78 * walked) + 0.98 * rounds + 0.318 * mb)
+                                       : fmax(5.83, 5.26 + longer(0.65 * chain, 1.35 * walked) + 0.875 * rounds + 0.095 * mb);
+    return 1.2 * here < sdpa_prefill_estimate(batch, heads, kv_heads, seq_q, seq_kv, head_dim, causal, window, right_context);
 }
 
 // Returns 1 when this kernel took the call, 0 when the shape is outside its range (the caller uses the general

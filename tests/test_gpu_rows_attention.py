@@ -319,6 +319,16 @@ def test_attention_long_prompts_stay_on_the_matrix_cores(hip_backend, torch_cuda
     assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
 
 
+@pytest.mark.parametrize("heads,kv_heads,d,sq,skv,window,streams", [
+    (8, 1, 128, 16, 8192, 0, False), (8, 1, 128, 16, 32768, 0, False), (1, 1, 128, 128, 16384, 0, False), (4, 1, 128, 23, 21041, 0, False),
+    (1, 1, 64, 8000, 8000, 128, False),                                   # a window: the prompt kernel walks a query group's keys, not all queries'
+    (1, 1, 128, 16, 8192, 0, True), (8, 1, 64, 40, 20000, 300, True), (16, 2, 128, 60, 60, 0, True)])
+def test_attention_prompts_over_long_caches_take_the_shorter_kernel(hip_backend, torch_cuda, heads, kv_heads, d, sq, skv, window, streams):
+    q, k, v = (torch_cuda.zeros(s, device="cuda") for s in ((1, heads, sq, d), (1, kv_heads, skv, d), (1, kv_heads, skv, d)))
+    hip_backend.sdpa_dev(q, k, v, torch_cuda.empty_like(q), 1, heads, kv_heads, sq, skv, d, 1.0, True, window)
+    assert hip_backend.last_kernel() == ("sdpa_decode_kernel" if streams else "sdpa_prefill_kernel")
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv,causal,window,rc,lengths", [
     (1, 8, 2, 128, 300, 300, True, 64, 0, None),            # sliding window shorter than a key block ... 
     (1, 8, 2, 128, 300, 300, True, 100, 0, None),           # ... and one that straddles blocks
