@@ -293,7 +293,8 @@ SKAINET_HIP_API int32_t skainet_hip_f32_sdpa_cache_dev(const float* q, const flo
     float scale, int32_t causal, int32_t window, int32_t right_context, const int32_t* lengths);
 /* The same with the output laid out [batch, seq_q, heads, head_dim] -- token rows, which is what the output projection
  * multiplies -- so a prompt pass needs no transposing launch between attention and projection. No reference counterpart
- * (the reference's attention output is head-major, f32_fused.c:290-396; its callers transpose). */
+ * (the reference's attention output is head-major, f32_fused.c:290-396; its callers transpose). An output over q, a cache or the
+ * lengths goes through scratch and one. */
 SKAINET_HIP_API int32_t skainet_hip_f32_sdpa_cache_rows_dev(const float* q, const float* k_cache, const float* v_cache, float* out,
     int32_t batch, int32_t heads, int32_t kv_heads, int32_t seq_q, int32_t seq_kv, int32_t kv_capacity, int32_t head_dim,
     float scale, int32_t causal, int32_t window, int32_t right_context, const int32_t* lengths);

@@ -190,9 +190,17 @@ int launch_sdpa_prefill(const float* q, const float* k, const float* v, float* o
 int launch_sdpa_cache(const float* q, const float* k, const float* v, float* out, int batch, int heads, int kv_heads,
                       int seq_q, int seq_kv, int kv_capacity, int head_dim, float scale, int causal, int window, int right_context,
                       const int32_t* lengths, const float* mask, int mask_b, int mask_h, int mask_q, int mask_k, int out_rows) {
+    // A workgroup of either kernel stores while others still read. Token rows lie elsewhere than the query rows they come from, so an output over an
+    // operand goes through the caller's scratch. Head-major rows lie where their queries do; a prompt's output over K or V stays with the prompt
+    // kernel, which has laid both out elsewhere before it stores.
+    const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), o1 = o0 + sizeof(float) * (size_t)batch * heads * seq_q * head_dim;
+    auto apart = [&](const void* in, size_t bytes) { const uintptr_t i0 = reinterpret_cast<uintptr_t>(in); return o1 <= i0 || i0 + bytes <= o0; };
+    const size_t kv_bytes = sizeof(float) * (size_t)batch * kv_heads * kv_capacity * head_dim;
+    const bool kv_apart = apart(k, kv_bytes) && apart(v, kv_bytes);
+    if (out_rows && !(kv_apart && apart(q, o1 - o0) && (!lengths || apart(lengths, sizeof(int32_t) * (size_t)batch)))) return 0;
     // decode and draft shapes, and the prompts that are shorter on it: the split-K cache-streaming kernel, when the head shape is one it carries
     // (a forced form of the prompt kernel keeps its prompts)
-    if (!mask && (seq_q < 16 || (sdpa_prefill_by_rule() &&
+    if (!mask && (seq_q < 16 || (kv_apart && sdpa_prefill_by_rule() &&
                                  sdpa_decode_takes_prompt(batch, heads, kv_heads, seq_q, seq_kv, head_dim, causal, window, right_context)))) {
         const int r = launch_sdpa_decode(q, k, v, out, batch, heads, kv_heads, seq_q, seq_kv, kv_capacity, head_dim, scale, causal, window,
                                          right_context, lengths, nullptr, out_rows);

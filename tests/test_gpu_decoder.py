@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from decoder_check import CheckDecoder
-from gpu_util import dev
+from gpu_util import dev, launches, normalized_err
 
 pytestmark = pytest.mark.gpu
 
@@ -353,6 +353,46 @@ def test_sdpa_cache_rows_is_the_head_major_result_transposed(hip_backend, torch_
     from skainet_amd._lib import HipError
     with pytest.raises(HipError):
         kx.sdpa_cache_rows_dev(q, kc, vc, rows, b, h, 3, sq, skv, cap, d, scale)        # heads not a multiple of kv_heads
+
+
+@pytest.mark.parametrize("b,h,hkv,sq,skv,d", [(1, 8, 2, 3, 37, 64), (2, 16, 4, 15, 300, 128), (1, 4, 2, 1, 40, 64), (1, 8, 2, 40, 56, 64), (1, 16, 4, 300, 300, 128)])
+def test_sdpa_cache_rows_over_an_operand(hip_backend, torch_cuda, b, h, hkv, sq, skv, d):
+    """An output over the queries, over part of them, over K or over V: through scratch and the transposing pass, so nothing is overwritten that another
+    workgroup still reads."""
+    torch, kx = torch_cuda, hip_backend
+    rng = np.random.default_rng(sq + d)
+    n = b * h * sq * d
+    cap = max(skv, -(-n // (b * hkv * d)) + 1)                  # K and V hold an output
+    vals = [dev(torch, rng.standard_normal(s).astype(np.float32)) for s in ((b, h, sq, d), (b, hkv, cap, d), (b, hkv, cap, d))]
+    want = torch.full((n,), float("nan"), device="cuda")
+    kx.sdpa_cache_rows_dev(*vals, want, b, h, hkv, sq, skv, cap, d, 0.1, True)
+    for which, shift in ((0, 0), (0, 2 * d), (1, 0), (2, 16)):
+        room = [torch.zeros(t.numel() + 2 * d, device="cuda") for t in vals]
+        ins = [r[:t.numel()].copy_(t.reshape(-1)) for r, t in zip(room, vals)]
+        out = room[which][shift:shift + n]
+        ran = launches(torch, lambda: kx.sdpa_cache_rows_dev(*ins, out, b, h, hkv, sq, skv, cap, d, 0.1, True))
+        assert any("heads_to_rows" in name for name, _, _ in ran), (which, ran)
+        assert torch.equal(out, want), (which, shift)
+
+
+@pytest.mark.parametrize("h,hkv,sq,d", [(8, 2, 40, 64), (4, 1, 17, 128)])
+def test_sdpa_of_a_short_prompt_over_its_keys_or_values(hip_backend, torch_cuda, h, hkv, sq, d):
+    """Head-major prompts that the streaming kernel takes by rule: over K or V they stay with the prompt kernel, whose workgroups read copies of them."""
+    torch, kx = torch_cuda, hip_backend
+    rng = np.random.default_rng(sq)
+    cap = sq * h // hkv
+    q, k, v = (dev(torch, rng.standard_normal(s).astype(np.float32)) for s in ((1, h, sq, d), (1, hkv, cap, d), (1, hkv, cap, d)))
+    want = torch.empty_like(q)
+    kx.sdpa_cache_dev(q, k, v, want, 1, h, hkv, sq, sq, cap, d, 0.1, True)
+    assert kx.last_kernel() == "sdpa_decode_kernel"
+    same = q.clone()                                            # over its own queries: each workgroup's rows are its own
+    kx.sdpa_cache_dev(same, k, v, same, 1, h, hkv, sq, sq, cap, d, 0.1, True)
+    assert kx.last_kernel() == "sdpa_decode_kernel" and torch.equal(same, want)
+    for which in (0, 1):
+        kv = [k.clone(), v.clone()]
+        kx.sdpa_cache_dev(q, kv[0], kv[1], kv[which], 1, h, hkv, sq, sq, cap, d, 0.1, True)
+        assert kx.last_kernel() == "sdpa_prefill_kernel"
+        assert normalized_err(kv[which].reshape(want.shape).cpu().numpy(), want.cpu().numpy(), eps=1.0) <= 2e-2
 
 
 def test_graph_replays_match_eager(hip_backend, torch_cuda):
