@@ -528,7 +528,8 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     // 1, three at 1720 8.3 -> 9.3).
     const int64_t tuples = (int64_t)batch * kv_heads * splits;
     const double mb = 8e-6 * batch * kv_heads * keys * head_dim;
-    if (g_sdpa_decode_dies && mb * min(subs, 8) > 34 && subs > 1 && (tuples >= 24 || (tuples + 7) / 8 * subs <= num_cus() / 8) && (tuples + 7) / 8 * 8 * subs <= 0x7FFFFFFF)
+    if (g_sdpa_decode_dies && mb * min(subs, 8) > 34 && subs > 1 && (tuples >= 24 || (tuples + 7) / 8 * subs <= num_cus() / 8) &&
+        (tuples + 7) / 8 * 8 * subs <= 0xFFFFFFFFll / 256)      // a dimension of a grid holds 2^32 work-items
         p.tuples = (int)tuples;
     if (splits > 1 || leave) {
         const size_t rows = (size_t)batch * heads * seq_q;

@@ -951,6 +951,19 @@ def test_attention_groups_of_one_die_give_the_same_bits(hip_backend, torch_cuda,
         assert not torch.isnan(got[0, keys]).any() and torch.equal(got[0, keys], got[1, keys])
 
 
+def test_attention_of_more_workgroups_than_one_grid_dimension_holds(hip_backend, torch_cuda):
+    """65 535 sequences of one key, 86 KV heads, three query heads each: 16.9 million workgroups of 256, more than 2^32 work-items, so the grid has
+    to keep its three dimensions. One key: the output is its V."""
+    torch, kx = torch_cuda, hip_backend
+    b, hkv, d = 65535, 86, 64
+    v = torch.randn((b, hkv, 1, d), device="cuda")
+    q = torch.zeros((b, 3 * hkv, 1, d), device="cuda")
+    out = torch.full_like(q, float("nan"))
+    kx.sdpa_cache_dev(q, v, v, out, b, 3 * hkv, hkv, 1, 1, 1, d, 1.0, True)
+    assert kx.last_kernel() == "sdpa_decode_kernel"
+    assert torch.equal(out.reshape(b, hkv, 3, d), v.expand(b, hkv, 3, d))
+
+
 @pytest.mark.parametrize("cols", [1, 255, 257, 4095, 4096, 4097, 15454, 16384, 65537])
 def test_argmax_at_the_edges_of_a_thread_s_walk(hip_backend, torch_cuda, cols):
     """The maximum at the first and the last column, ties between a thread's own elements and between threads, rows of -inf."""
