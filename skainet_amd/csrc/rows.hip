@@ -250,16 +250,17 @@ __global__ __launch_bounds__(256) void add_kernel(const float* __restrict__ a, c
 
 // A thread's share of [lo, hi): every ROW_THREADS-th element, upwards, so an equal value later is never lower. U loads in flight: one at a
 // time the walk is a chain of round trips to memory, 60 of them for 15 454 columns (14.1 us, 5.8 with 16 in flight; 4945 columns 6.3 and 4.0).
+// Unsigned, since a step past the last of 2^31 - 1 columns is no int.
 template <int U>
-__device__ __forceinline__ void argmax_walk(const float* x, int lo, int hi, float& bv, int& bi) {
-    for (int base = lo + threadIdx.x; base < hi; base += U * ROW_THREADS) {
+__device__ __forceinline__ void argmax_walk(const float* x, unsigned lo, unsigned hi, float& bv, int& bi) {
+    for (unsigned base = lo + threadIdx.x; base < hi; base += U * ROW_THREADS) {
         float v[U];
 #pragma unroll
         for (int j = 0; j < U; ++j) v[j] = x[min(base + j * ROW_THREADS, hi - 1)];
 #pragma unroll
         for (int j = 0; j < U; ++j) {
-            const int i = base + j * ROW_THREADS;
-            if (i < hi && (v[j] > bv || bi == 0x7FFFFFFF)) { bv = v[j]; bi = i; }
+            const unsigned i = base + j * ROW_THREADS;
+            if (i < hi && (v[j] > bv || bi == 0x7FFFFFFF)) { bv = v[j]; bi = (int)i; }
         }
     }
 }
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(ROW_THREADS) void argmax_split_kernel(const float* 
     __shared__ unsigned ticket;
     const int row = blockIdx.y, part = blockIdx.x;
     const float* x = in + (int64_t)row * cols;
-    const int per = ((cols + ARGMAX_SPLIT - 1) / ARGMAX_SPLIT + 3) & ~3;
-    const int lo = part * per, hi = min(cols, lo + per);
+    const unsigned per = (((unsigned)cols + ARGMAX_SPLIT - 1) / ARGMAX_SPLIT + 3) & ~3u;
+    const unsigned lo = part * per, hi = min((unsigned)cols, lo + per);
     float bv = -INFINITY;
     int bi = 0x7FFFFFFF;
     argmax_walk<4>(x, lo, hi, bv, bi);

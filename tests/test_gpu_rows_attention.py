@@ -976,3 +976,15 @@ def test_argmax_at_the_edges_of_a_thread_s_walk(hip_backend, torch_cuda, cols):
     idx = torch.full((5,), -1, dtype=torch.int32, device="cuda")
     kx.argmax_rows_dev(dev(torch, lg), 5, cols, idx)
     assert idx.cpu().tolist() == [int(r.argmax()) for r in lg]
+
+
+@pytest.mark.parametrize("cols", [2 ** 31 - 1, 2 ** 31 - 64, 2 ** 31 - 500])
+def test_argmax_of_a_row_up_to_the_last_int(hip_backend, torch_cuda, cols):
+    """Where the share of a workgroup, rounded up, and a thread's step past the row's end are beyond the int range."""
+    torch = torch_cuda
+    row = torch.zeros(cols, device="cuda")
+    idx = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    for at in (cols - 1, cols - 300, 0):
+        row[at] = 1.0
+        hip_backend.argmax_rows_dev(row, 1, cols, idx)
+        assert int(idx.cpu()[0]) == at
