@@ -892,9 +892,9 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
                          (enc != ENC_Q4_K || (gemm_ksw_enabled() && gemm_frag_enabled()));
     if (by_rule && (skinny_mode == 1 || skinny_mode == 3) && gemm_skinny_fits(enc, m, n, k)) {
         const double others = fmin(tile_estimate, frag_estimate), two = gemm_skinny_estimate(enc, m, n, k);
-        // One launch: 3 % below the others' estimate up to 5 us, 20 % of what is above that. Of 4 750 random products (9 to 300 rows) a quarter
-        // takes it, 1.26x on the device and 1.5x back to back from the host, where the second launch was 2.4 us; 15 of them are more than 3 % slower on
-        // the device. 3 % throughout would take 1 680 of them, 250 slower, by up to 30 %.
+        // One launch: 3 % below the others' estimate up to 5 us, 20 % of what is above that. Of 7 100 random products (9 to 300 rows, m n k up to
+        // 1.5e9) 3 252 take it, 1.24x on the device and 1.50x back to back from the host, where the second launch was 2.4 us. 111 of them are more than 3 %
+        // slower on the device, by up to 17 %: these take 0.79 of their time from the host all the same, but for 4, so the line stays here.
         const double least_of_two = fmin(others, two);
         if (skinny_mode == 1 && direct_ok && gemm_skinny_direct_estimate(enc, m, n, k) < (least_of_two <= 5.0 ? 0.97 * least_of_two : 4.85 + 0.8 * (least_of_two - 5.0)))
             return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);

@@ -558,7 +558,8 @@ double gemm_skinny_estimate(int enc, int m, int n, int k) { return gemm_skinny_t
 
 // The one-launch form of a shape and what it is estimated to take, in us, or mt = 0: outside its range. Terms as above: the launch, the result, the
 // workgroups of a CU for their shares of K. Fitted to 2 560 random products (9 to 200 rows, m n k up to 1.2e9, every format), which it meets
-// within 4 to 7 % (rms); 20 to 30 % off, and low, for few columns of more than 6144, which are left out.
+// within 4 to 7 % (rms). Rows of more than 4864 are left out: the estimate is low there (from 6144 on by 20 to 30 %), and those that took a form gained
+// nothing on the device (Q4_K 95 x 668 x 5888 8.5 us in two launches, 9.5 in one).
 SknTile gemm_skinny_direct_tile(int enc, int m, int n, int k) {
     struct Form { int mt, nt, wn; double launch, result, whole, whole_k, cost[7][2]; };          // formats: Q4_K, Q5_K, Q6_K, Q8_0, Q4_0, Q5_0, Q5_1
     static const Form forms[4] = {
@@ -568,7 +569,7 @@ SknTile gemm_skinny_direct_tile(int enc, int m, int n, int k) {
         {2, 2, 4, 3.40, 1.21e-06, 0.75, 0.46, {{2.59, 4.99}, {3.41, 5.97}, {5.94, 8.48}, {3.63, 6.63}, {2.44, 4.65}, {2.79, 3.10}, {2.93, 3.57}}},
     };
     SknTile best{0, 0, 0, 0.0};
-    if (k > 6144) return best;
+    if (k > 4864) return best;
     const int format = enc == ENC_Q4_K ? 0 : enc == ENC_Q5_K ? 1 : enc == ENC_Q6_K ? 2 : enc == ENC_Q8_0 ? 3 : enc == ENC_Q4_0 ? 4 : enc == ENC_Q5_0 ? 5 : 6;
     const int mtiles = (m + 15) / 16;
     for (const Form& f : forms) {
@@ -582,11 +583,11 @@ SknTile gemm_skinny_direct_tile(int enc, int m, int n, int k) {
     if (k % 2048 == 0) best.us *= 1.08;      // rows of 2^n KB meet in the same channels of the L2
     return best;
 }
-// From 8 us on the estimate is a tenth low for what only single waves share, for Q6_K and for one row tile of Q8_0: of 4 913 random products that took
-// these forms such ones took 1.05 of what two launches take (Q6_K 55 x 9274 x 768 11.3 -> 12.0 us, Q8_0 46 x 8548 x 768 8.2 -> 9.9), the others 0.87.
+// From 8 us on the estimate is a tenth low for what single waves read for themselves, for Q6_K and for Q8_0: such products took 1.01 to 1.05 of what two launches
+// take, on the device and from the host (Q6_K 55 x 9274 x 768 11.3 -> 12.0 us, Q8_0 46 x 8548 x 768 8.2 -> 9.9, 100 x 7267 x 1024 11.8 -> 13.2), the others 0.87.
 double gemm_skinny_direct_estimate(int enc, int m, int n, int k) {
     const SknTile t = gemm_skinny_direct_tile(enc, m, n, k);
-    return !t.mt || (t.us >= 8 && (t.wn == 1 || enc == ENC_Q6_K || (enc == ENC_Q8_0 && t.mt == 1))) ? 1e30 : t.us;
+    return !t.mt || (t.us >= 8 && (t.wn == 1 || enc == ENC_Q6_K || enc == ENC_Q8_0)) ? 1e30 : t.us;
 }
 
 // 0 never, 1 where the estimates favour it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits; 100 wn + 10 mt + nt: that

@@ -334,7 +334,7 @@ def test_gemm_of_few_rows_in_one_launch(hip_backend, torch_cuda, enc, m, n, k):
 
 
 @pytest.mark.parametrize("enc,m,n,k,kernel", [("Q4_0", 18, 924, 1024, "direct"), ("Q5_K", 91, 8978, 512, "shared"), ("Q8_0", 24, 4096, 4096, "kernel"),
-                                              ("Q4_0", 46, 1086, 9984, "kernel")])
+                                              ("Q4_0", 46, 1086, 9984, "kernel"), ("Q8_0", 100, 7267, 1024, "kernel"), ("Q4_K", 95, 668, 5888, "kernel")])
 def test_small_products_of_few_rows_take_one_launch(hip_backend, torch_cuda, enc, m, n, k, kernel):
     packed = gaussian_weight(hip_backend, enc, n, k, 31)
     x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
