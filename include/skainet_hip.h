@@ -440,7 +440,9 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * 0 = chosen from K), "gemm_ksplit" (K splits of the MFMA GEMM,
  * 0 = automatic), "gemv_few" (products of 1 to 8 rows by lanes that decode 64 weights at a time: 0 never, 1 where they are the faster ones,
  * 2 wherever they fit), "gemm_skinny" (the packed GEMM for few rows: 0 never, 1 where the launcher's estimate favours it, 2 wherever it
- * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2), "gemm_wide" (0 / 1 / 2: force the tile of 128 / 256 / 192
+ * fits, 10 mt + nt: tiles of 16 mt rows x 16 nt columns wherever it fits, mt 1, 2 or 4, nt 1 or 2; 111, 112, 411, 422: 100 waves on the same rows + 10 mt + nt,
+ * its forms that read the fp32 rows themselves, wherever they fit and take the call's rows; a value that names no form changes nothing), "gemm_skinny_direct" (0: those
+ * forms are never chosen, 1 where the launcher's estimates favour them), "gemm_wide" (0 / 1 / 2: force the tile of 128 / 256 / 192
  * columns, 192 with 128 rows being 256, -1 = chosen from the shape), "gemm_rows" (2 / 3 / 4: 128 / 192 / 256 activation rows per tile, 0 = chosen from the shape),
  * "gemm_f32" (the 128 x 128 tile on the fp32 rows instead of rounded copies: 0 never, 1 where the estimate favours it, 2 wherever that tile is taken), "gemm_ksw" (the Q4_K kernel that splits K over the
  * waves of a workgroup: 0 never, 1 where "gemm_frag" is 0 and the launcher's estimate favours it -- the fragment-order kernel
@@ -462,7 +464,7 @@ SKAINET_HIP_API void skainet_hip_graph_free(skainet_hip_graph* graph);
  * "sdpa_prefill_splits" (workgroups that share the keys of a query group that has workgroups of its own: 1 to 32, 0 = chosen from the shape), "sdpa_decode_split_keys" (least keys per split of
  * decode-shape attention, default 64), "sdpa_decode_prompts" (prompts of 16 queries and more without a mask on the kernel for decode shapes:
  * 0 never, 1 where the launcher's estimates of both favour it and no "sdpa_prefill_*" key is set, 2 wherever it fits unless one is), "sdpa_decode_one_launch" (0: short contexts are split over workgroups and merged by a
- * second launch too), "sdpa_decode_gs" (query heads per workgroup of decode-shape attention: 1, 2 or 4, 0 = chosen from
+ * second launch too), "sdpa_decode_dies" (0: workgroups that share keys are never placed on one die), "sdpa_decode_gs" (query heads per workgroup of decode-shape attention: 1, 2 or 4, 0 = chosen from
  * the shape), "attn_merge_enable" (0: skainet_hip_attn_out_proj_dev always merges the key
  * splits in a launch of its own), "attn_merge_max_keys" (most keys per split for which that entry leaves the merge to
  * the projection, default 176), "attn_merge_splits" (most key splits it then uses, 1 to 8, default 6).

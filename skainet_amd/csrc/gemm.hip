@@ -719,6 +719,7 @@ double gemm_skinny_estimate(int enc, int m, int n, int k);
 int launch_gemm_skinny_direct(int enc, const uint8_t* w, const float* x, int m, int k, int n, float* c, const float* residual, int epilogue);
 double gemm_skinny_direct_estimate(int enc, int m, int n, int k);
 int gemm_skinny_mode();
+bool gemm_skinny_direct_enabled();
 
 constexpr int GEMM_MAX_SPLITS = 24;
 static std::atomic<int> g_gemm_ksplit{0};   // 0 = choose from the tile count
@@ -818,7 +819,7 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     const bool direct_ok = !gain && !x_pairs && (x0 + sizeof(float) * (size_t)m * k <= y0 || y0 + sizeof(float) * (size_t)m * n <= x0);
     const int skinny_mode = gemm_skinny_mode();
     if (skinny_mode >= 100 && direct_ok && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);
-    if (skinny_mode != 3 && skinny_mode >= 2 && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
+    if (skinny_mode >= 2 && gemm_skinny_fits(enc, m, n, k)) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     hipStream_t s = current_stream();
     auto round_activations = [&](__bf16* a) -> int {            // fp32 -> bf16, with the RMSNorm of a fused call folded in
         const int64_t n4 = (int64_t)m * k / 4;                  // k is a multiple of 64
@@ -890,13 +891,13 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     // leaves the format to the kernels before them.
     const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 &&
                          (enc != ENC_Q4_K || (gemm_ksw_enabled() && gemm_frag_enabled()));
-    if (by_rule && (skinny_mode == 1 || skinny_mode == 3) && gemm_skinny_fits(enc, m, n, k)) {
+    if (by_rule && skinny_mode == 1 && gemm_skinny_fits(enc, m, n, k)) {
         const double others = fmin(tile_estimate, frag_estimate), two = gemm_skinny_estimate(enc, m, n, k);
         // One launch: 3 % below the others' estimate up to 5 us, 20 % of what is above that. Of 7 100 random products (9 to 300 rows, m n k up to
         // 1.5e9) 3 252 take it, 1.24x on the device and 1.50x back to back from the host, where the second launch was 2.4 us. 111 of them are more than 3 %
         // slower on the device, by up to 17 %: these take 0.79 of their time from the host all the same, but for 4, so the line stays here.
         const double least_of_two = fmin(others, two);
-        if (skinny_mode == 1 && direct_ok && gemm_skinny_direct_estimate(enc, m, n, k) < (least_of_two <= 5.0 ? 0.97 * least_of_two : 4.85 + 0.8 * (least_of_two - 5.0)))
+        if (direct_ok && gemm_skinny_direct_enabled() && gemm_skinny_direct_estimate(enc, m, n, k) < (least_of_two <= 5.0 ? 0.97 * least_of_two : 4.85 + 0.8 * (least_of_two - 5.0)))
             return launch_gemm_skinny_direct(enc, w, x, m, k, n, y, residual, epilogue);
         if (two < 0.95 * others) return launch_gemm_skinny(enc, w, x, m, k, n, y, gain, eps, residual, epilogue, x_pairs);
     }

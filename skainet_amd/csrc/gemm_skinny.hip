@@ -590,11 +590,19 @@ double gemm_skinny_direct_estimate(int enc, int m, int n, int k) {
     return !t.mt || (t.us >= 8 && (t.wn == 1 || enc == ENC_Q6_K || enc == ENC_Q8_0)) ? 1e30 : t.us;
 }
 
-// 0 never, 1 where the estimates favour it, 2 wherever it fits; 10 mt + nt: that tile, wherever it fits; 100 wn + 10 mt + nt: that
-// one-launch form (111, 112, 411, 422), wherever it fits; 3: as 1 without the one-launch forms
+// 0 never, 1 where the estimates favour it, 2 (to 10) wherever it fits; 10 mt + nt: that tile, wherever it fits; 100 wn + 10 mt + nt: that one-launch
+// form, wherever it fits. A value that names no built form changes nothing.
 static std::atomic<int> g_gemm_skinny{1};
-void set_gemm_skinny(int v) { g_gemm_skinny = v; }
+void set_gemm_skinny(int v) {
+    static const int forms[] = {11, 12, 21, 22, 41, 42, 111, 112, 411, 422};
+    bool known = v <= 10;
+    for (int f : forms) known |= v == f;
+    if (known) g_gemm_skinny = v < 0 ? 0 : v > 2 && v <= 10 ? 2 : v;
+}
 int gemm_skinny_mode() { return g_gemm_skinny.load(); }
+static std::atomic<int> g_gemm_skinny_direct{1};   // the one-launch forms by rule: 0 never, 1 where the estimates favour them
+void set_gemm_skinny_direct(int v) { g_gemm_skinny_direct = v != 0; }
+bool gemm_skinny_direct_enabled() { return g_gemm_skinny_direct.load() != 0; }
 
 template <class F>
 static int launch_skinny_format(int enc, const float* x, const float* gain, float eps, bool pairs, uint8_t* a, const uint8_t* w, float* c,

@@ -193,6 +193,7 @@ void set_gemm_rows(int v);
 void set_gemm_f32(int v);
 void set_gemm_ksw(int v);
 void set_gemm_skinny(int v);
+void set_gemm_skinny_direct(int v);
 void set_gemm_ksw_teams(int v);
 void set_gemm_ksw_stages(int v);
 void set_gemm_frag(int v);
@@ -246,6 +247,7 @@ int set_tuning(const char* key, int value) {
     if (!strcmp(key, "gemm_rows")) { set_gemm_rows(value); return 0; }
     if (!strcmp(key, "gemv_few")) { set_gemv_few(value); return 0; }
     if (!strcmp(key, "gemm_skinny")) { set_gemm_skinny(value); return 0; }
+    if (!strcmp(key, "gemm_skinny_direct")) { set_gemm_skinny_direct(value); return 0; }
     if (!strcmp(key, "gemm_ksw")) { set_gemm_ksw(value); return 0; }
     if (!strcmp(key, "gemm_ksw_teams")) { set_gemm_ksw_teams(value); return 0; }
     if (!strcmp(key, "gemm_ksw_stages")) { set_gemm_ksw_stages(value); return 0; }

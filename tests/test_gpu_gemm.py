@@ -345,6 +345,26 @@ def test_small_products_of_few_rows_take_one_launch(hip_backend, torch_cuda, enc
     check_exact(torch_cuda, enc, got[0], x, packed, n)
 
 
+def test_the_few_rows_key_takes_what_names_a_form(hip_backend, torch_cuda):
+    """2 to 10: wherever it fits; a value that names no form leaves the key as it is; the one-launch forms have a key of their own."""
+    def ran(enc, m, n, k):
+        gpu_gemm(hip_backend, torch_cuda, enc, gaussian_weight(hip_backend, enc, n, k, 31), n, k, np.ones((m, k), np.float32))
+        return hip_backend.last_kernel()
+    big, small = ("Q6_K", 1000, 2048, 1024), ("Q4_0", 18, 924, 1024)
+    try:
+        for value, kernel in ((1, "dequant_gemm_kernel"), (121, "dequant_gemm_kernel"), (13, "dequant_gemm_kernel"), (412, "dequant_gemm_kernel"),
+                              (3, "packed_gemm_skinny_kernel"), (13, "packed_gemm_skinny_kernel"), (422, "packed_gemm_skinny_shared_kernel"), (0, "dequant_gemm_kernel")):
+            hip_backend.set_tuning("gemm_skinny", value)
+            assert ran(*big) == kernel, value
+        hip_backend.set_tuning("gemm_skinny", 1)
+        for value, kernel in ((0, "packed_gemm_skinny_kernel"), (1, "packed_gemm_skinny_direct_kernel")):
+            hip_backend.set_tuning("gemm_skinny_direct", value)
+            assert ran(*small) == kernel
+    finally:
+        hip_backend.set_tuning("gemm_skinny", 1)
+        hip_backend.set_tuning("gemm_skinny_direct", 1)
+
+
 @pytest.mark.parametrize("knob", ["gemm_frag", "gemm_ksw"])
 def test_the_q4k_gemm_knobs_leave_other_formats_alone(hip_backend, torch_cuda, knob):
     """Either Q4_K kernel switched off: a product of few rows in another format takes the kernel it takes by rule, Q4_K one
