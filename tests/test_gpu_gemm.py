@@ -108,11 +108,13 @@ def test_gemm_tiles_of_192_rows_or_columns_give_the_bits_of_the_others(hip_backe
         hip_backend.set_tuning("gemm_wide", 0)
         want = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
         check_exact(torch_cuda, enc, want, x, packed, n)
-        for rows, wide in ((3, 0), (3, 2), (3, 1), (4, 2)):
+        for rows, wide, tile in ((3, 0, "3, 2"), (3, 2, "3, 3"), (3, 1, "3, 4"), (4, 2, "4, 3")):
             hip_backend.set_tuning("gemm_rows", rows)
             hip_backend.set_tuning("gemm_wide", wide)
-            got = gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)
-            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (rows, wide)
+            got = []
+            ran = launches(torch_cuda, lambda: got.append(gpu_gemm(hip_backend, torch_cuda, enc, packed, n, k, x)))
+            assert sum(f"{tile}, false>" in name for name, _, _ in ran if "dequant_gemm_kernel<" in name) == 1, (tile, ran)
+            assert np.array_equal(got[0].view(np.uint32), want.view(np.uint32)), (rows, wide)
     finally:
         hip_backend.set_tuning("gemm_ksplit", 0)
         hip_backend.set_tuning("gemm_wide", -1)
@@ -139,9 +141,15 @@ def test_gemm_tile_on_fp32_rows_gives_the_bits_of_the_rounded_rows(hip_backend, 
     """The tile rounds the rows itself instead of a pass in front: the same values, so the same bits; also where the product lies over the
     rows, which then go through the pass."""
     torch = torch_cuda
-    w = hip_backend.DeviceWeight.upload(enc, gaussian_weight(hip_backend, enc, n, k, 700 + n), n, k)
+    packed = gaussian_weight(hip_backend, enc, n, k, 700 + n)
+    w = hip_backend.DeviceWeight.upload(enc, packed, n, k)
     x = torch.from_numpy(np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)).cuda()
     got = {}
+
+    def product(rows, out, f32):                               # the tile on fp32 rows alone, or behind the pass
+        ran = [name for name, _, _ in launches(torch, lambda: w.matmul(rows, m, out, 1))]
+        assert sum(f"2, 2, {str(f32).lower()}>" in name for name in ran if "dequant_gemm_kernel<" in name) == 1, ran
+        assert any("prepass" in name for name in ran) != f32, ran
     try:
         for key, v in (("gemm_skinny", 0), ("gemm_frag", 0), ("gemm_ksw", 0), ("gemm_rows", 2), ("gemm_wide", 0), ("gemm_ksplit", ks)):
             hip_backend.set_tuning(key, v)
@@ -149,15 +157,25 @@ def test_gemm_tile_on_fp32_rows_gives_the_bits_of_the_rounded_rows(hip_backend, 
             hip_backend.set_tuning("gemm_f32", mode)
             both = torch.full((m * k + m * n,), float("nan"), device="cuda")
             xs, apart, over = both[:m * k].reshape(m, k).copy_(x), both[m * k:], both[:m * n]
-            w.matmul(xs, m, apart, 1)
+            product(xs, apart, mode == 2)
             got[mode] = apart.clone()
             if n <= k:
-                w.matmul(xs, m, over, 1)
+                product(xs, over, False)
                 assert torch.equal(over, got[mode])
     finally:
         for key, v in (("gemm_skinny", 1), ("gemm_frag", 1), ("gemm_ksw", 1), ("gemm_rows", 0), ("gemm_wide", -1), ("gemm_ksplit", 0), ("gemm_f32", 1)):
             hip_backend.set_tuning(key, v)
     assert not torch.isnan(got[0]).any() and torch.equal(got[0], got[2])
+    check_exact(torch, enc, got[2].reshape(m, n).cpu().numpy(), x.cpu().numpy(), packed, n)
+
+
+@pytest.mark.parametrize("enc,m,n,k,tile", [("Q6_K", 1000, 11008, 4096, "4, 3, false>"), ("Q5_K", 348, 1503, 2560, "2, 2, true>"), ("Q8_0", 400, 9000, 3072, "3, 2, false>")])
+def test_gemm_tiles_that_the_rule_takes(hip_backend, torch_cuda, enc, m, n, k, tile):
+    torch, (_, elems, size) = torch_cuda, hip_backend.ENCODINGS[enc]
+    w = hip_backend.DeviceWeight.wrap(enc, torch.full((n * (k // elems) * size,), 17, dtype=torch.uint8, device="cuda"), n, k)
+    x, out = torch.ones((m, k), device="cuda"), torch.empty((m, n), device="cuda")
+    ran = launches(torch, lambda: w.matmul(x, m, out, 1))
+    assert sum(tile in name for name, _, _ in ran if "dequant_gemm_kernel<" in name) == 1, ran
 
 
 @pytest.mark.parametrize("k", [96, 192, 320, 448])

@@ -78,8 +78,13 @@ def test_attention_masks_padding_and_host_entry(hip_backend, torch_cuda):
     q, k, v = sdpa_inputs(1, 12, 12, 150, 150, 64, seed=9)     # the reference's threaded shape (NativeFusedKernelsTest.kt:211)
     o = np.empty_like(q)
     want = L.sdpa(q, k, v, 1 / np.sqrt(64.0), True)
-    attn.sdpa(q, k, v, o, 1, 12, 12, 150, 150, 64, float(1 / np.sqrt(64.0)), True, 0, 0)
-    assert normalized_err(o, want, eps=1.0) <= 2e-2               # a prompt shape: bf16 operands on the matrix cores
+    hip_backend.set_tuning("sdpa_decode_prompts", 0)              # on the prompt kernel: bf16 operands on the matrix cores
+    try:
+        attn.sdpa(q, k, v, o, 1, 12, 12, 150, 150, 64, float(1 / np.sqrt(64.0)), True, 0, 0)
+        assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+    finally:
+        hip_backend.set_tuning("sdpa_decode_prompts", 1)
+    assert normalized_err(o, want, eps=1.0) <= 2e-2
     hip_backend.set_tuning("sdpa_prefill_mfma", 0)                # the same call on the fp32 kernel: the reference's tolerance
     try:
         attn.sdpa(q, k, v, o, 1, 12, 12, 150, 150, 64, float(1 / np.sqrt(64.0)), True, 0, 0)
@@ -231,6 +236,7 @@ def test_attention_prefill_config_against_torch_fp32(hip_backend, torch_cuda):
     qs, ks, vs = q[:, :, :sp].copy(), k[:, :, :sp].copy(), v[:, :, :sp].copy()
     want_s = L.sdpa(qs, ks, vs, scale, True)
     e_mfma = normalized_err(gpu_sdpa(hip_backend, torch, qs, ks, vs, scale, True), want_s, eps=1.0)
+    assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
     print(f"prefill attention 256 (matrix cores): max err / max |ref| vs oracle {e_mfma:.2e}")
     assert e_mfma <= 2e-2
     hip_backend.set_tuning("sdpa_prefill_mfma", 0)                # the fp32 kernel on the same problem, reference tolerance
@@ -248,20 +254,24 @@ def test_attention_prefill_config_against_torch_fp32(hip_backend, torch_cuda):
 def test_attention_prefill_mfma_shapes(hip_backend, torch_cuda, batch, heads, kv_heads, d, sq, skv, causal):
     """The matrix-core prompt kernel over its shape range: group sizes 1 / 2 / 4 / 8, head_dim 64 / 128, lengths that
     are not multiples of the 32-query or 64-key tiles, a query block shorter than the keys (a later prompt chunk),
-    causal and full. Bound: 2e-2 of the largest reference magnitude (bf16 operands); the RMS error is held to 5e-3."""
+    causal and full; the short ones would go to the streaming kernel, which is kept out. Bound: 2e-2 of the largest reference magnitude (bf16 operands); the RMS error is held to 5e-3."""
     rng = np.random.default_rng(sq * skv + d)
     q = rng.standard_normal((batch, heads, sq, d)).astype(np.float32)
     k = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
     v = rng.standard_normal((batch, kv_heads, skv, d)).astype(np.float32)
     scale = float(1 / np.sqrt(d))
-    got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, scale, causal)
+    hip_backend.set_tuning("sdpa_decode_prompts", 0)
+    try:
+        got = gpu_sdpa(hip_backend, torch_cuda, q, k, v, scale, causal)
+        assert hip_backend.last_kernel() == "sdpa_prefill_kernel"
+        # rows of P sum to 1: with v = 1 everywhere the output is 1 (bf16 P entries: 1e-2)
+        assert np.abs(gpu_sdpa(hip_backend, torch_cuda, q, k, np.ones_like(v), scale, causal) - 1.0).max() <= 1e-2
+    finally:
+        hip_backend.set_tuning("sdpa_decode_prompts", 1)
     want = L.sdpa(q, k, v, scale, causal)
     assert np.isfinite(got).all()
     assert normalized_err(got, want, eps=1.0) <= 2e-2
     assert np.sqrt(np.mean((got - want) ** 2)) <= 5e-3 * np.abs(want).max()
-    # rows of P sum to 1: with v = 1 everywhere the output is 1 (bf16 P entries: 1e-2)
-    ones = np.ones_like(v)
-    assert np.abs(gpu_sdpa(hip_backend, torch_cuda, q, k, ones, scale, causal) - 1.0).max() <= 1e-2
 
 
 @pytest.mark.parametrize("batch,heads,kv_heads,d,sq,skv,causal,window,rc,lengths", [
@@ -360,10 +370,9 @@ def test_attention_prefill_mfma_window_and_key_lengths(hip_backend, torch_cuda, 
             assert np.isfinite(got).all()
             assert normalized_err(got, want, eps=1.0) <= 2e-2
             assert np.sqrt(np.mean((got - want) ** 2)) <= 5e-3 * np.abs(want).max()
+            assert np.abs(gpu_sdpa(hip_backend, torch_cuda, q, k, np.ones_like(v), scale, causal, window, rc, ln) - 1.0).max() <= 1e-2
     finally:
         hip_backend.set_tuning("sdpa_prefill_teams", 0)
-    ones = np.ones_like(v)
-    assert np.abs(gpu_sdpa(hip_backend, torch_cuda, q, k, ones, scale, causal, window, rc, ln) - 1.0).max() <= 1e-2
     hip_backend.set_tuning("sdpa_prefill_mfma", 0)
     try:
         close(gpu_sdpa(hip_backend, torch_cuda, q, k, v, scale, causal, window, rc, ln), want)
