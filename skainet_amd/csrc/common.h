@@ -221,7 +221,7 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// (cos, sin) of rotation pair i at a position: one expression for every kernel that needs it, so that they agree bit for bit.
+// (cos, sin) of rotation pair i at a position: one expression for the two kernels that write a rotation table, which agree bit for bit.
 __device__ __forceinline__ float2 rope_cos_sin(int32_t pos, float theta, int i, int head_dim) {
     float sn, cs;
     sincosf((float)pos * powf(theta, -2.0f * (float)i / (float)head_dim), &sn, &cs);

@@ -37,7 +37,7 @@ constexpr int G_THREADS = G_WAVES_M * G_WAVES_N * 64;
 constexpr int GSTRIDE = GK + 8;                               // bf16 elements per LDS row (144 bytes)
 // A wave owns WTM x WTN MFMA tiles of 32 x 32, 2 to 4 of them each way (not 2 x 3): workgroup tiles of 128, 192 or 256 rows and columns, so that
 // what a product leaves of its last row of tiles and of the last round over the CUs is small. With 128 and 256 alone 300 rows took
-// three or four thirds of what they need and 1000 x 11008 left 84 of 256 CUs idle: Q6_K 1000 x 11008 x 4096 124.0 -> 112.6 us, Q8_0
+// three or four thirds of what they need and 1000 x 11008 left 84 of 256 CUs idle: Q6_K 1000 x 11008 x 4096 126.7 -> 118.4 us, Q8_0
 // 400 x 9000 x 3072 64 -> 55. Of 605 random products (100 to 1024 rows) 146 take one of the four tiles with a 192: 1.10x, 5 of all more than 3 % slower.
 constexpr int gemm_gm(int wtm) { return 32 * wtm * G_WAVES_M; }
 constexpr int gemm_gn(int wtn) { return 32 * wtn * G_WAVES_N; }
@@ -886,7 +886,8 @@ int launch_gemm_fused(int enc, const uint8_t* w, const float* x, int m, int k, i
     const bool frag_by_rule = frag_ok && gemm_frag_enabled() && gemm_ksw_enabled() && g_gemm_ksplit.load() <= 0;
     const double frag_estimate = frag_by_rule ? gemm_frag_us(m, n, k) : tile_estimate;
     // Few rows: the kernel without a row tile to fill. (The epilogue plays no part in the choice: a product takes one
-    // kernel, and sums in one order, whatever is done to it on the way out.)
+    // kernel, and sums in one order, whatever is done to it on the way out. What comes in does: a gain, (gate, up) pairs or an output over the rows
+    // keep the one-launch forms out, and the one whose waves share their rows sums K in two shares instead of eight.)
     // A forced tile or split keeps it out, and so does either of the two Q4_K kernels switched off, for Q4_K alone: that
     // leaves the format to the kernels before them.
     const bool by_rule = g_gemm_ksplit.load() <= 0 && g_gemm_wide.load() < 0 && g_gemm_rows.load() == 0 &&

@@ -42,7 +42,6 @@ struct SdpaDecodeParams {
     int subs, tuples;     // workgroups that share a split's keys, and how many such (split, kv head, sequence) there are; tuples 0: a grid of three dimensions
     int seq_q, causal;    // queries per sequence (the last ones of its positions) and whether a later key is hidden from them
     int out_rows;         // the output as [batch, seq_q, heads, D] instead of [batch, heads, seq_q, D]
-    int by_query;         // rows that share a KV head: query by query instead of head by head
 };
 
 // Scores are kept in units of ln 2 (the query is scaled by scale * log2(e) once), so every exponential of the softmax is
@@ -56,7 +55,7 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
     return m_old == -INFINITY ? 0.f : e;
 }
 
-// MQ: several queries per sequence (a draft of a few tokens). The rows that share a KV head are then its query heads times
+// ROWS: one query per sequence, a draft of a few (MQ) or a prompt. The rows that share a KV head are then its query heads times
 // the queries, GS of them to a workgroup: each has a key range of its own (causal and window move with the query) and the
 // workgroup walks the union. A key outside a row's range takes no part in that row: it scores -inf and its V is replaced by
 // zeros, since a weight of zero times an infinite or undefined element (a later token's, or the padding of a cache) is not
@@ -64,10 +63,13 @@ __device__ __forceinline__ float exp_diff(float m_old, float m_new) {
 // A draft's rows come head by head. A prompt's come query by query, so that a workgroup holds neighbouring queries, at most GS of them: head by head
 // some hold the last queries of one head and the first of the next, which share no key under a window (385 queries on 1828 keys under a
 // window of 153, 8 heads over 1: 537 keys walked by six of 770 workgroups, about 156 by the others).
-// DIES: a grid of one dimension, below. A template argument, since a run-time choice costs every call 0.03 to 0.1 us in front of its first load.
-template <int GS, int DPL, bool MQ, bool DIES>
+// DIES: a grid of one dimension, below. Both are template arguments, since a run-time choice costs every call 0.03 to 0.1 us (DIES) or a draft 0.1 to
+// 0.4 (the order of its rows) in front of its first load.
+enum DecodeRows { ROWS_ONE, ROWS_DRAFT, ROWS_PROMPT };
+template <int GS, int DPL, DecodeRows ROWS, bool DIES>
 __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
     constexpr int D = 16 * DPL;
+    constexpr bool MQ = ROWS != ROWS_ONE, BY_QUERY = ROWS == ROWS_PROMPT;
     constexpr int U = 2;                       // groups of 4 keys a wave has in flight
     __shared__ __attribute__((aligned(16))) float wacc[16][GS][D];
     __shared__ __attribute__((aligned(16))) float cw[GS][16];
@@ -93,9 +95,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_kernel(SdpaDecodeParams p) {
         sub_group = blockIdx.y % subs;
     }
     const int r0 = sub_group * GS;
-    const int row_div = p.by_query ? per_kv : p.seq_q;
-    auto head_of = [&](int r) { return !MQ ? r : p.by_query ? r % row_div : r / row_div; };
-    auto query_of = [&](int r) { return !MQ ? 0 : p.by_query ? r / row_div : r % row_div; };
+    auto head_of = [&](int r) { return !MQ ? r : BY_QUERY ? r % per_kv : r / p.seq_q; };
+    auto query_of = [&](int r) { return !MQ ? 0 : BY_QUERY ? r / per_kv : r % p.seq_q; };
     // row g of the workgroup: its place among the [batch, heads, seq_q] query rows (rows past the last are copies of it)
     int64_t row_of[GS];
     int first_of[GS], end_of[GS];
@@ -357,12 +358,12 @@ float* sdpa_workspace(size_t bytes);   // shim.hip: per-thread scratch, grown on
 static std::atomic<int> g_sdpa_decode_split_keys{64};   // least keys per split (a multiple of 16)
 void set_sdpa_decode_split_keys(int v) { if (v >= 16) g_sdpa_decode_split_keys = (v + 15) & ~15; }
 
-template <int GS, int DPL, bool MQ>
+template <int GS, int DPL, DecodeRows ROWS>
 static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge) {
     constexpr int D = 16 * DPL;
     note_kernel("sdpa_decode_kernel");
-    if (p.tuples) sdpa_decode_kernel<GS, DPL, MQ, true><<<dim3((unsigned)((p.tuples + 7) / 8 * 8 * subs)), dim3(256), 0, current_stream()>>>(p);
-    else sdpa_decode_kernel<GS, DPL, MQ, false><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
+    if (p.tuples) sdpa_decode_kernel<GS, DPL, ROWS, true><<<dim3((unsigned)((p.tuples + 7) / 8 * 8 * subs)), dim3(256), 0, current_stream()>>>(p);
+    else sdpa_decode_kernel<GS, DPL, ROWS, false><<<dim3(p.splits, p.kv_heads * subs, p.batch), dim3(256), 0, current_stream()>>>(p);
     SKH_CHECK(hipGetLastError());
     if (merge) {
         sdpa_decode_combine_kernel<D><<<dim3(p.batch * p.heads * p.seq_q), dim3(4 * D), 0, current_stream()>>>(p.part, p.ml, p.out, p.splits, p.heads, p.seq_q, p.out_rows);
@@ -370,11 +371,16 @@ static int launch_decode_variant(const SdpaDecodeParams& p, int subs, bool merge
     }
     return 1;
 }
-template <int DPL, bool MQ>
+template <int DPL, DecodeRows ROWS>
+static int launch_decode_rows(const SdpaDecodeParams& p, int gs, int subs, bool merge) {
+    if constexpr (DPL <= 8) { if (gs == 4) return launch_decode_variant<4, DPL, ROWS>(p, subs, merge); }
+    if (gs == 2) return launch_decode_variant<2, DPL, ROWS>(p, subs, merge);
+    return launch_decode_variant<1, DPL, ROWS>(p, subs, merge);
+}
+template <int DPL>
 static int launch_decode_d(const SdpaDecodeParams& p, int gs, int subs, bool merge) {
-    if constexpr (DPL <= 8) { if (gs == 4) return launch_decode_variant<4, DPL, MQ>(p, subs, merge); }
-    if (gs == 2) return launch_decode_variant<2, DPL, MQ>(p, subs, merge);
-    return launch_decode_variant<1, DPL, MQ>(p, subs, merge);
+    if constexpr (DPL <= 8) { if (p.seq_q >= 16) return launch_decode_rows<DPL, ROWS_PROMPT>(p, gs, subs, merge); }
+    return p.seq_q > 1 ? launch_decode_rows<DPL, ROWS_DRAFT>(p, gs, subs, merge) : launch_decode_rows<DPL, ROWS_ONE>(p, gs, subs, merge);
 }
 
 static std::atomic<int> g_sdpa_decode_gs{0};            // query heads per workgroup: 0 = chosen from the shape, else 1 / 2 / 4
@@ -405,8 +411,8 @@ double sdpa_prefill_estimate(int batch, int heads, int kv_heads, int seq_q, int 
 // (Straight lines through the keys, fitted up to 2048 earlier ones, took 5 % more, 973 of 21 378 slower, by up to 3.3 times: beyond the fit they
 // did not know that the other kernel splits its keys, nor under a window what its workgroups walk.)
 bool sdpa_decode_takes_prompt(int batch, int heads, int kv_heads, int seq_q, int seq_kv, int head_dim, int causal, int window, int right_context) {
-    if (g_sdpa_decode_prompts.load() != 1) return g_sdpa_decode_prompts.load() == 2;
     if ((head_dim != 64 && head_dim != 128) || seq_q > seq_kv) return false;
+    if (g_sdpa_decode_prompts.load() != 1) return g_sdpa_decode_prompts.load() == 2;
     const double cus = num_cus(), groups = (double)batch * kv_heads * (((int64_t)(heads / kv_heads) * seq_q + 3) / 4);
     double keys = causal ? seq_kv - 0.5 * (seq_q - 1) : seq_kv, most = seq_kv, all = seq_kv;       // of a query on average, of a workgroup, of the call
     if (window > 0) {
@@ -501,7 +507,7 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     const int subs = (cols + gs - 1) / gs;
     if (batch > 65535 || (int64_t)kv_heads * subs > 65535) return 0;
     SdpaDecodeParams p{q, k, v, out, batch, heads, kv_heads, seq_kv, kv_capacity, scale, window, right_context, lengths, 1,
-                       nullptr, nullptr, subs, 0, seq_q, causal, out_rows && seq_q > 1, seq_q >= 16};
+                       nullptr, nullptr, subs, 0, seq_q, causal, out_rows && seq_q > 1};
     // enough workgroups to put every CU on the cache, at least 64 keys per split (measured in the decoder at 500 to 650
     // keys: 32 or 48 keys per split 2.5 % slower per token, 96 and 128 keys the same as 64)
     const int64_t groups = (int64_t)batch * kv_heads * subs;
@@ -539,9 +545,9 @@ int launch_sdpa_decode(const float* q, const float* k, const float* v, float* ou
     }
     if (leave) *leave = AttnMergePrologue{p.part, p.ml, splits, head_dim};
     const bool merge = splits > 1 && !leave;
-    if (head_dim == 64) return draft ? launch_decode_d<4, true>(p, gs, subs, merge) : launch_decode_d<4, false>(p, gs, subs, merge);
-    if (head_dim == 128) return draft ? launch_decode_d<8, true>(p, gs, subs, merge) : launch_decode_d<8, false>(p, gs, subs, merge);
-    return draft ? launch_decode_d<16, true>(p, gs, subs, merge) : launch_decode_d<16, false>(p, gs, subs, merge);
+    if (head_dim == 64) return launch_decode_d<4>(p, gs, subs, merge);
+    if (head_dim == 128) return launch_decode_d<8>(p, gs, subs, merge);
+    return launch_decode_d<16>(p, gs, subs, merge);
 }
 
 int launch_q4k_gemv_mfma(const uint8_t* w, const float* x, float* y, int k, int n, const float* gain, float eps,
