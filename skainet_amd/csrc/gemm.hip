@@ -38,7 +38,8 @@ constexpr int GSTRIDE = GK + 8;                               // bf16 elements p
 // A wave owns WTM x WTN MFMA tiles of 32 x 32, 2 to 4 of them each way (not 2 x 3): workgroup tiles of 128, 192 or 256 rows and columns, so that
 // what a product leaves of its last row of tiles and of the last round over the CUs is small. With 128 and 256 alone 300 rows took
 // three or four thirds of what they need and 1000 x 11008 left 84 of 256 CUs idle: Q6_K 1000 x 11008 x 4096 126.7 -> 118.4 us, Q8_0
-// 400 x 9000 x 3072 64 -> 55. Of 605 random products (100 to 1024 rows) 146 take one of the four tiles with a 192: 1.10x, 5 of all more than 3 % slower.
+// 400 x 9000 x 3072 64 -> 55. Of 605 random products (100 to 1024 rows) 146 take one of the four tiles with a 192: 1.10x, 5 of all more than 3 % slower
+// (with the line against the fragment-order kernel, below, at 2 %).
 constexpr int gemm_gm(int wtm) { return 32 * wtm * G_WAVES_M; }
 constexpr int gemm_gn(int wtn) { return 32 * wtn * G_WAVES_N; }
 // Weight rows that a step decodes: two threads share a row, so whole multiples of 128. 192 columns (WTN = 3) decode 256, the last 64 of them
